@@ -148,6 +148,13 @@ struct GiPrefillArgs {
     const float* vs;
     long long sc_stride;
     long long sc_head_stride;
+    float* part;
+    int slice_tiles;
+    int nslice;
+    int pwaves;
+    int items;
+    uint32_t gmul;
+    int rows;
 };
 
 constexpr float kLog2e = 1.4426950408889634f;
@@ -166,7 +173,10 @@ constexpr int kDecWaves = 4, kDecTile = 32, kDecPairs = 8; // slice partials are
 constexpr int kSliceUnit = kDecWaves * kDecTile; // 128 keys
 constexpr int kSplitMaxBatch = 15;                // tokens per split launch (src/cuda.rs:119)
 constexpr int kTiledMinBatch = 16;                // prefill from this many tokens (src/cuda.rs:95)
-constexpr int kPrefillRows = 256; // query rows per prefill workgroup; must match the kernels' PF_BQ
+constexpr int kPrefillRows = 256; // packed query rows per workgroup of 8 waves (head sizes 64 and 128)
+constexpr int kPrefillKeys = 64;  // keys per prefill tile; must match the kernels' PF_BK
+constexpr int kPrefillMaxSlices = 64; // must match the kernels' PFC_MAXS
+constexpr int kPrefillMergeFrags = 4; // must match the kernels' PFC_FRAGS
 constexpr int kPrefill256rRows = 128; // the same for gi_prefill_fwd_h256r (PF256R_BQ)
 
 thread_local std::string g_err;
@@ -203,17 +213,17 @@ struct Module {
                                       // one column block, 4-bit one and two column blocks
     hipFunction_t dec_pm256[2] = {};  // head size 256, one pair per column, two pair sets of two waves: [f16, int8]
     hipFunction_t dec_i8_256f[2] = {}; // head size 256 over the int8 cache in f32 precision: [up to 8 pairs, above]
-    hipFunction_t prefill[2] = {};   // [int8 cache], head size 128
-    hipFunction_t prefill64[2] = {}; // [int8 cache], head size 64 (the same launch shape and block size)
+    // head sizes 128 and 64: [head size 64][f16 cache, pre-widened int8, int8 widened tile by tile][8 waves, 4 waves]
+    hipFunction_t prefill[2][3][2] = {};
     hipFunction_t dec_f32[2][6] = {}, prefill_f32[2][6] = {}; // the f32 kernels: [int8 cache][kF32Sizes index]
     hipFunction_t prefill_f32p[2][2] = {}; // f32 prompts at head sizes 64 and 128: [int8 cache][64, 128]
     hipFunction_t prefill256r = nullptr; // head size 256 (f16 cache), 16 rows per wave: one workgroup per query tile
     hipFunction_t prefill256r_fmt[2] = {}; // the same over the int8 and the 4-bit cache
-    // pre-widened staging: gi_kv_widen, then the int8 kernels that stage the widened tiles by LDS-DMA (head sizes
-    // 128, 64, 256; the widened 4-bit cache runs prefill256r)
-    hipFunction_t widen = nullptr, prefill_i8s[3] = {};
+    // pre-widened staging: gi_kv_widen, then the int8 kernels that stage the widened tiles by LDS-DMA (head size 256
+    // here; the widened 4-bit cache runs prefill256r)
+    hipFunction_t widen = nullptr, prefill256r_i8s = nullptr;
+    hipFunction_t prefill_combine[2] = {}; // merge of a sliced prefill's partials: 32 rows per wave
     hipFunction_t combine = nullptr, rope = nullptr, relayout = nullptr, hadamard = nullptr;
-    int prefill_threads[2] = {}; // each prefill kernel's block size (its launch bound: waves x 64)
     int prefill256r_threads = 0;
     // gi_attn_decode_noalloc's partials: the device address of the code object's gi_scratch array on this
     // device (the array's host-side name is no device address; the module gives the real one at load)
@@ -277,17 +287,22 @@ int load_module(const char* path, Module** out) {
             {&m.combine, "gi_decode_combine"},
             {&m.relayout, "gi_kv_relayout"},
             {&m.hadamard, "gi_hadamard_rows"},
-            {&m.prefill[0], "gi_prefill_fwd"},
-            {&m.prefill[1], "gi_prefill_fwd_i8"},
-            {&m.prefill64[0], "gi_prefill_fwd_h64"},
-            {&m.prefill64[1], "gi_prefill_fwd_h64_i8"},
+            {&m.prefill[0][0][0], "gi_prefill_fwd"},
+            {&m.prefill[0][0][1], "gi_prefill_fwd_w4"},
+            {&m.prefill[0][1][0], "gi_prefill_fwd_i8s"},
+            {&m.prefill[0][1][1], "gi_prefill_fwd_i8s_w4"},
+            {&m.prefill[0][2][0], "gi_prefill_fwd_i8"},
+            {&m.prefill[1][0][0], "gi_prefill_fwd_h64"},
+            {&m.prefill[1][0][1], "gi_prefill_fwd_h64_w4"},
+            {&m.prefill[1][1][0], "gi_prefill_fwd_h64_i8s"},
+            {&m.prefill[1][1][1], "gi_prefill_fwd_h64_i8s_w4"},
+            {&m.prefill[1][2][0], "gi_prefill_fwd_h64_i8"},
             {&m.prefill256r, "gi_prefill_fwd_h256r"},
             {&m.prefill256r_fmt[0], "gi_prefill_fwd_h256r_i8"},
             {&m.prefill256r_fmt[1], "gi_prefill_fwd_h256r_q4"},
             {&m.widen, "gi_kv_widen"},
-            {&m.prefill_i8s[0], "gi_prefill_fwd_i8s"},
-            {&m.prefill_i8s[1], "gi_prefill_fwd_h64_i8s"},
-            {&m.prefill_i8s[2], "gi_prefill_fwd_h256r_i8s"},
+            {&m.prefill256r_i8s, "gi_prefill_fwd_h256r_i8s"},
+            {&m.prefill_combine[0], "gi_prefill_combine_32"},
             {&m.rope, "gi_qk_norm_rope"},
         };
         for (auto& f : fns)
@@ -313,11 +328,7 @@ int load_module(const char* path, Module** out) {
                     return e;
                 }
             }
-        if (int e = check(hipFuncGetAttribute(&m.prefill_threads[0], HIP_FUNC_ATTRIBUTE_MAX_THREADS_PER_BLOCK, m.prefill[0]),
-                          "hipFuncGetAttribute(gi_prefill_fwd)") ||
-                    check(hipFuncGetAttribute(&m.prefill_threads[1], HIP_FUNC_ATTRIBUTE_MAX_THREADS_PER_BLOCK, m.prefill[1]),
-                          "hipFuncGetAttribute(gi_prefill_fwd_i8)") ||
-                    check(hipFuncGetAttribute(&m.prefill256r_threads, HIP_FUNC_ATTRIBUTE_MAX_THREADS_PER_BLOCK,
+        if (int e = check(hipFuncGetAttribute(&m.prefill256r_threads, HIP_FUNC_ATTRIBUTE_MAX_THREADS_PER_BLOCK,
                                               m.prefill256r),
                           "hipFuncGetAttribute(gi_prefill_fwd_h256r)")) {
             (void)hipModuleUnload(m.mod);
@@ -339,9 +350,9 @@ int load_module(const char* path, Module** out) {
 
 // ---- per-kernel timing (gi_kernel_timing): event pairs around each launch, per kernel kind
 enum Kind { kDecodePartial = 0, kDecodeCombine = 1, kPrefill = 2, kRope = 3, kRelayout = 4, kHadamard = 5, kWiden = 6,
-            kKinds = 7 };
+            kPrefillCombine = 7, kKinds = 8 };
 const char* const kKindNames[kKinds] = {"decode_partial", "decode_combine", "prefill", "qk_norm_rope", "kv_relayout",
-                                        "hadamard_rows", "kv_widen"};
+                                        "hadamard_rows", "kv_widen", "prefill_combine"};
 struct Timing {
     std::mutex mu;
     bool on = false;
@@ -682,14 +693,87 @@ size_t prefill_ws_bytes(int kv_len, int n_kv, int hd, int fmt) {
     return 2 * rows + 2 * scales;
 }
 
+// How a prefill launch at head size 64 or 128 is laid out. It has one workgroup per (kv head, tile of packed query
+// rows), and a CU holds one workgroup.
+//  - Waves: 8 (256 rows, two waves per SIMD) or 4 (128 rows, one per SIMD). One wave takes a key tile in about 0.7 of
+//    the time that two on its SIMD take for theirs together, so 4 waves win where the workgroups are few or unequal
+//    (1024 tokens of 32/8 heads of 128, f16: 33.9 us with 8, 23.7 with 4; 512 at a 2000-token prefix 64 and 44) and
+//    8 where they fill the chip several times over (8192 tokens: 505 and 580).
+//  - Slices: a short batch over a long prefix leaves most of the chip idle while each workgroup walks all of its keys
+//    (512 tokens of 32/4 heads at a 16K prefix: 64 workgroups of 264 key tiles, 350 us). Such a launch cuts the key
+//    tiles of every row tile into slices, one workgroup each, whose partial results a second launch merges (137 us).
+// A row's arithmetic does not depend on the waves, only on the slices.
+struct PrefillPlan {
+    int waves;      // 8 or 4
+    int tiles;      // key tiles per slice
+    int nslice;     // slices of the longest row tile
+};
+constexpr int kPrefillRowTiles(long long rows, int per) { return (int)((rows + per - 1) / per); }
+PrefillPlan prefill_plan(int pos0, int n, int n_heads, int n_kv, int hd) {
+    const int G = n_heads / n_kv, cus = 256, tmax = (pos0 + n + kPrefillKeys - 1) / kPrefillKeys;
+    const long long P = (long long)n * G;
+    PrefillPlan p{8, tmax, 1};
+    if ((long long)kPrefillRowTiles(P, kPrefillRows) * n_kv >= 2 * cus) return p; // longest tiles first balances these
+    // Below 16 key tiles slices save less than the merge launch costs. A prompt of up to 4096 keys taken in chunks of
+    // 256 tokens or more keeps each row's arithmetic independent of the chunking (one slice always); beyond, chunks
+    // agree to f32 rounding.
+    const bool may_slice = tmax >= 16 && (n < 256 || pos0 + n > 4096);
+    // Costs in units of one key tile of an 8-wave workgroup (1.4 to 1.9 us): rounds of workgroups over the CUs, each
+    // with a fixed cost until its first tile is in and for its output (~6 us), and for a sliced launch the merge
+    // launch (~5 us) and its read of the partials (~4 TB/s).
+    const double per_wg = 4.0, merge = 3.3;
+    double best = 0;
+    for (int waves = 8; waves >= 4; waves -= 4) {
+        const int rows = 32 * waves, items = kPrefillRowTiles(P, rows);
+        const long long wgs = (long long)items * n_kv;
+        const double tile = waves == 8 ? 1.0 : 0.7;
+        auto tiles_of = [&](int i) { // key tiles of row tile i
+            const long long last = std::min<long long>(n - 1, ((long long)(i + 1) * rows - 1) / G);
+            return (int)((pos0 + last) / kPrefillKeys + 1);
+        };
+        // one slice: the longest workgroup, or the mean load of a CU where there are several rounds
+        const double mean = (double)wgs / cus * (tile * (tiles_of(0) + tmax) / 2 + (wgs > cus ? per_wg : 0));
+        const double one = std::max(tile * tmax, mean) + per_wg;
+        if (waves == 8 || one < 0.95 * best) best = one, p = PrefillPlan{waves, tmax, 1};
+        if (!may_slice) continue;
+        const double part = std::min<long long>(P, rows) * (hd + 2) * 4.0 / 4e12 / 1.5e-6;
+        for (int S = 2; S <= std::min(kPrefillMaxSlices, tmax / 2) && wgs * S <= 4 * cus; S++) {
+            const int C = (tmax + S - 1) / S;
+            long long u = 0; // workgroups with keys
+            if (tiles_of(0) + C > tmax) u = wgs * ((tmax + C - 1) / C); // (every row tile has tmax tiles or nearly)
+            else
+                for (int i = 0; i < items; i++) u += (long long)n_kv * ((tiles_of(i) + C - 1) / C);
+            const double cost = (double)((u + cus - 1) / cus) * (tile * C + per_wg) + merge + u * part;
+            if (cost < 0.95 * best) best = cost, p = PrefillPlan{waves, C, (tmax + C - 1) / C};
+        }
+    }
+    return p;
+}
+// Rows per kv head from which the int8 keys are widened into the workspace first (one pass over all keys, ~6 bytes moved
+// per value) rather than tile by tile in the prefill: above one row tile, every tile would be widened again for each.
+// 32/8 heads of 128, tile by tile / widened: 16 tokens at a 2000-token prefix 17.6 / 21.5 us, at 16000 29.6 / 43.5; 64
+// tokens at 2000 27.7 / 26.7, at 16000 48 / 51; 256 tokens at 2000 84 / 55; 8192 tokens 634 / 588.
+constexpr int kPrefillWidenRows = kPrefillRows;
+bool prefill_widens(int n, int n_heads, int n_kv, int hd) {
+    return hd == 256 || (long long)n * (n_heads / n_kv) > kPrefillWidenRows;
+}
+// Bytes of a sliced launch's partials, in row tiles of `rows` (pwaves: waves of a row tile that hold rows)
+int prefill_pwaves(long long P, int rows) { return P > rows ? rows / 32 : (int)((P + 31) / 32); }
+size_t prefill_part_bytes(const PrefillPlan& p, int n, int n_heads, int n_kv, int hd, int rows) {
+    if (p.nslice == 1) return 0;
+    const long long P = (long long)n * (n_heads / n_kv);
+    return align256((size_t)kPrefillRowTiles(P, rows) * n_kv * p.nslice * prefill_pwaves(P, rows) * 32 * (hd + 2) * 4);
+}
+
 // gi_attn_prefill, gi_attn_prefill_i8 and gi_attn_prefill_q4: the same launch with the f16, int8 or 4-bit kernel
-// (fmt 0, 1, 2). With a workspace (int8 and 4-bit caches, head sizes 64, 128, 256) the keys 0..pos0+n-1 are first
-// widened into it (gi_kv_widen) and the prefill stages the widened tiles by LDS-DMA, as it stages the f16 cache.
+// (fmt 0, 1, 2). With a workspace and `widen` (int8 and 4-bit caches, head sizes 64, 128, 256) the keys 0..pos0+n-1
+// are first widened into it (gi_kv_widen) and the prefill stages the widened tiles by LDS-DMA, as it stages the f16
+// cache. What is left of the workspace takes the partials of a sliced launch (prefill_plan) where it holds them.
 int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, const void* kc, const void* vc,
                  const float* ks, const float* vs, long long sc_stride, long long sc_head_stride, int fmt,
                  long long kv_stride, long long kv_head_stride, void* out, int out_dtype, long long out_stride, int pos0,
                  int n, int n_heads, int n_kv, int hd, float scale, void* workspace = nullptr,
-                 size_t workspace_bytes = 0, bool f32_prompt = false) {
+                 size_t workspace_bytes = 0, bool f32_prompt = false, bool widen = true) {
     const bool i8 = fmt == 1;
     if (int e = check_shape(n_heads, n_kv, hd, true)) return e;
     if (fmt == 2 && hd != 256) return fail("the 4-bit cache takes head size 256 only (got %d)", hd);
@@ -744,17 +828,44 @@ int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, c
     a.q_f16 = q_dtype == GI_F16;
     a.out_f16 = out_dtype == GI_F16;
     a.hd = hd;
+    a.nslice = 1;
+    const int G = n_heads / n_kv;
+    a.gmul = (long long)n * G * G < 1ll << 31 ? (uint32_t)(((1ll << 31) + G - 1) / G) : 0;
+    // the launch of a prefill kernel of head size 64 or 128 over staging `st` (Module::prefill), sliced where the plan
+    // says so and the rest of the workspace holds the partials; then their merge
+    auto run = [&](int st, unsigned char* free, size_t left) {
+        const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd);
+        const int waves = st == 2 ? 8 : p.waves; // (tile by tile: 8 waves only)
+        const size_t need = prefill_part_bytes(p, n, n_heads, n_kv, hd, 32 * waves);
+        a.rows = 32 * waves;
+        a.items = kPrefillRowTiles((long long)n * G, a.rows);
+        a.pwaves = prefill_pwaves((long long)n * G, a.rows);
+        if (need && free && aligned16(free) && left >= need) {
+            a.part = (float*)free;
+            a.nslice = p.nslice;
+            a.slice_tiles = p.tiles;
+        }
+        if (int e = launch(kPrefill, m->prefill[hd == 64][st][waves == 4], dim3((unsigned)(a.items * n_kv * a.nslice), 1, 1),
+                           dim3(64 * waves), (hipStream_t)stream, &a, sizeof a))
+            return e;
+        if (a.nslice == 1) return 0;
+        return launch(kPrefillCombine, m->prefill_combine[0],
+                      dim3(a.pwaves * a.items * n_kv, 32 * hd / 256 / kPrefillMergeFrags, 1), dim3(64 * kPrefillMergeFrags),
+                      (hipStream_t)stream, &a, sizeof a);
+    };
+    unsigned char* const ws = (unsigned char*)workspace;
     if (f32_prompt && !f32_hd(hd)) // head sizes 64 and 128 in f32: one workgroup per (head, 128 query rows)
         return launch(kPrefill, m->prefill_f32p[i8][hd == 128], dim3((n + kF32Rows - 1) / kF32Rows * n_heads, 1, 1),
                       dim3(kF32Threads), (hipStream_t)stream, &a, sizeof a);
-    if (fmt && workspace && !f32_hd(hd)) {
+    if (fmt && workspace && widen && !f32_hd(hd)) {
         const int len = pos0 + n;
         const size_t need = prefill_ws_bytes(len, n_kv, hd, fmt);
         if (workspace_bytes < need)
             return fail("the prefill workspace holds %zu bytes; %zu needed (gi_attn_prefill_workspace_bytes)",
                         workspace_bytes, need);
         if ((uintptr_t)workspace & 255) return fail("the prefill workspace must be 256-byte aligned");
-        unsigned char* w = (unsigned char*)workspace;
+        if (!prefill_widens(n, n_heads, n_kv, hd)) return run(2, ws, workspace_bytes);
+        unsigned char* w = ws;
         const size_t rows = align256((size_t)n_kv * len * hd * 2), scales = fmt == 1 ? align256((size_t)n_kv * len * 4) : 0;
         GiWidenArgs wa{};
         wa.kc = kc;
@@ -786,11 +897,10 @@ int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, c
         a.sc_stride = 1;
         a.sc_head_stride = len;
         if (hd == 256)
-            return launch(kPrefill, fmt == 2 ? m->prefill256r : m->prefill_i8s[2],
+            return launch(kPrefill, fmt == 2 ? m->prefill256r : m->prefill256r_i8s,
                           dim3((n + kPrefill256rRows - 1) / kPrefill256rRows * n_heads, 1, 1), dim3(m->prefill256r_threads),
                           (hipStream_t)stream, &a, sizeof a);
-        return launch(kPrefill, m->prefill_i8s[hd == 64 ? 1 : 0], dim3((n + kPrefillRows - 1) / kPrefillRows * n_heads, 1, 1),
-                      dim3(m->prefill_threads[1]), (hipStream_t)stream, &a, sizeof a);
+        return run(1, ws + need, workspace_bytes - need);
     }
     if (f32_hd(hd)) // one workgroup per (head, 128 query rows)
         return launch(kPrefill, m->prefill_f32[i8][f32_index(hd)], dim3((n + kF32Rows - 1) / kF32Rows * n_heads, 1, 1),
@@ -798,10 +908,7 @@ int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, c
     if (hd == 256) // one workgroup per (head, 128 query rows), 16 rows per wave
         return launch(kPrefill, fmt ? m->prefill256r_fmt[fmt - 1] : m->prefill256r, dim3((n + kPrefill256rRows - 1) / kPrefill256rRows * n_heads, 1, 1),
                       dim3(m->prefill256r_threads), (hipStream_t)stream, &a, sizeof a);
-    const int qtiles = (n + kPrefillRows - 1) / kPrefillRows; // one workgroup per (head, 256 query rows)
-    return launch(kPrefill, hd == 64 ? m->prefill64[i8] : m->prefill[i8], dim3(qtiles * n_heads, 1, 1),
-                  dim3(m->prefill_threads[i8]),
-                  (hipStream_t)stream, &a, sizeof a);
+    return run(i8 ? 2 : 0, ws, workspace_bytes);
 }
 
 int attention_impl(void* stream, const float* qkv, const void* kc, const void* vc, const float* ks, const float* vs,
@@ -936,6 +1043,32 @@ size_t gi_attn_prefill_workspace_bytes(int kv_len, int n_kv, int hd, int fmt) {
     return prefill_ws_bytes(kv_len, n_kv, hd, fmt);
 }
 
+size_t gi_attn_prefill_scratch_bytes(int pos0, int n, int n_heads, int n_kv, int hd, int fmt, int flags) {
+    if (check_shape(n_heads, n_kv, hd, true) || pos0 < 0 || n <= 0 || fmt < 0 || fmt > 2 || (fmt == 2 && hd != 256)) return 0;
+    if ((flags & GI_PREFILL_F32) || f32_hd(hd)) return 0;
+    const bool widens = fmt && (flags & GI_PREFILL_WIDEN) && prefill_widens(n, n_heads, n_kv, hd);
+    const size_t widened = widens ? prefill_ws_bytes(pos0 + n, n_kv, hd, fmt) : 0;
+    if (hd == 256) return widened;
+    const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd);
+    return widened + prefill_part_bytes(p, n, n_heads, n_kv, hd, fmt && !widens ? kPrefillRows : 32 * p.waves);
+}
+
+int gi_attn_prefill_ws(void* stream, const void* q, int q_dtype, long long q_stride, const void* kc, const void* vc,
+                       const void* ks, const void* vs, int fmt, int flags, long long kv_stride, long long kv_head_stride,
+                       long long sc_stride, long long sc_head_stride, void* out, int out_dtype, long long out_stride,
+                       int pos0, int n, int n_heads, int n_kv, int hd, float scale, void* workspace,
+                       size_t workspace_bytes) {
+    if (fmt < 0 || fmt > 2) return fail("cache format %d must be 0 (f16), 1 (int8) or 2 (4-bit)", fmt);
+    if (sc_stride == 0 && sc_head_stride == 0) sc_stride = fmt == 2 ? 8LL * n_kv : n_kv, sc_head_stride = fmt == 2 ? 8 : 1;
+    const bool f32 = flags & GI_PREFILL_F32;
+    // widened staging where the workspace holds the widened keys, else tile by tile
+    const bool widen = (flags & GI_PREFILL_WIDEN) && fmt && !f32 && workspace && n > 0 && pos0 >= 0 && n_kv > 0 &&
+                       prefill_widens(n, n_heads, n_kv, hd) && workspace_bytes >= prefill_ws_bytes(pos0 + n, n_kv, hd, fmt);
+    return prefill_impl(stream, q, q_dtype, q_stride, kc, vc, fmt ? (const float*)ks : nullptr, fmt ? (const float*)vs : nullptr,
+                        fmt ? sc_stride : 0, fmt ? sc_head_stride : 0, fmt, kv_stride, kv_head_stride, out, out_dtype,
+                        out_stride, pos0, n, n_heads, n_kv, hd, scale, workspace, workspace_bytes, f32, widen);
+}
+
 int gi_attn_prefill_i8_ws(void* stream, const void* q, int q_dtype, long long q_stride, const int8_t* kc,
                           const int8_t* vc, const float* ks, const float* vs, long long kv_stride,
                           long long kv_head_stride, long long sc_stride, long long sc_head_stride, void* out,
@@ -1025,7 +1158,7 @@ int attention_impl(void* stream, const float* qkv, const void* kc, const void* v
         // the int8 and 4-bit caches: pre-widened staging when the workspace holds it
         const bool staged = fmt && workspace && workspace_bytes >= prefill_ws_bytes(pos0 + n, n_kv, hd, fmt);
         return prefill_impl(stream, qkv, GI_F32, row, kc, vc, ks, vs, scs, sch, fmt, kvs, kvh, out, GI_F32, q_dim, pos0,
-                            n, n_heads, n_kv, hd, scale, staged ? workspace : nullptr, workspace_bytes);
+                            n, n_heads, n_kv, hd, scale, workspace, workspace_bytes, false, staged);
     }
     for (int b0 = 0; b0 < n; b0 += kSplitMaxBatch) {
         int m = std::min(n - b0, kSplitMaxBatch);
@@ -1056,7 +1189,7 @@ int gi_kernel_timing_read(const char* kernel, double* total_ms, int* launches) {
         if (std::strcmp(kernel, kKindNames[k]) == 0) kind = k;
     if (kind < 0)
         return fail("unknown kernel \"%s\" (decode_partial, decode_combine, prefill, qk_norm_rope, kv_relayout, "
-                    "hadamard_rows or kv_widen)", kernel);
+                    "hadamard_rows, kv_widen or prefill_combine)", kernel);
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
     {
         std::lock_guard<std::mutex> lock(g_timing.mu);

@@ -1422,19 +1422,68 @@ struct GiPrefillArgs {
     const float* vs;
     long long sc_stride;
     long long sc_head_stride;
+    // sliced launches (nslice > 1): slice s of a row tile covers the key tiles [s*slice_tiles, (s+1)*slice_tiles) and
+    // leaves its partial result here (pf_partial), for gi_prefill_combine_*; unsliced: null, 1
+    float* part;
+    int slice_tiles;
+    int nslice;
+    int pwaves;            // waves of a row tile that hold rows (the workgroup's, or fewer where one tile holds all rows)
+    int items;             // row tiles per kv head
+    uint32_t gmul;         // ceil(2^31 / G): a packed row's token without a division (pf_token)
+    int rows;              // rows of a row tile
 };
 
-#ifndef PF_WAVES
-#define PF_WAVES 8         // waves per workgroup, 32 query rows each
-#endif
-#define PF_BQ (32 * PF_WAVES) // query rows per workgroup
-#define PF_SW (PF_WAVES / 2)  // waves staging each of K and V
+// Rows of a prefill workgroup. The query rows of one kv head are taken token-major with their G query heads side by
+// side (packed row r: token r / G, head r % G of the group), so that a row tile covers few positions: its waves end
+// at nearly the same key tile, all heads of the group share each staged K/V tile, and a few tokens still fill a
+// tile. A row's arithmetic does not depend on which rows share its tile.
+struct PfUnit {
+    int kvh, row0;       // kv head, first packed row
+    int t_begin, t_end;  // key tiles of this workgroup
+    long long unit;      // index of its partial
+};
+// row / G. The product form is exact for row * G < 2^31 (else the host passes gmul 0): 2 row ceil(2^31 / G) exceeds
+// 2^32 row / G by less than 2 row, so the quotient's fraction stays below the next integer. (A 32-bit division is
+// some 40 instructions; four in a row before the first tile's loads cost a short prompt 0.5 us.)
+__device__ __forceinline__ int pf_token(const GiPrefillArgs& a, int row) {
+    return a.gmul ? (int)__umulhi(2u * (uint32_t)row, a.gmul) : row / (a.n_heads / a.n_kv);
+}
+__device__ __forceinline__ int pf_last_token(const GiPrefillArgs& a, int row0, int rows) {
+    return min(a.n - 1, pf_token(a, row0 + rows - 1)); // the last token with a row in the tile
+}
+// Workgroup j of the grid (kv head, slice, row tile). Blocks go to the 8 XCDs round-robin; the remap gives each XCD
+// a contiguous run of the order, so that one kv head's K/V (one slice's, in a sliced launch) stays in one XCD's L2.
+// Longest row tiles first.
+__device__ __forceinline__ PfUnit pf_unit(const GiPrefillArgs& a, int BQ, int BK) {
+    const int items = a.items;
+    const int nwg = gridDim.x;
+    int j = blockIdx.x;
+    if ((nwg & 7) == 0) j = (j & 7) * (nwg >> 3) + (j >> 3);
+    const int run = j / items; // kv head * nslice + slice
+    const int item = items - 1 - (j - run * items);
+    const int kvh = a.nslice == 1 ? run : run / a.nslice, slice = run - kvh * a.nslice;
+    const int k_lim = a.pos0 + pf_last_token(a, item * BQ, BQ) + 1; // keys any row of the tile may see
+    const int ntiles = (k_lim + BK - 1) / BK;
+    const int tb = slice * a.slice_tiles;
+    return PfUnit{kvh, item * BQ, tb, a.nslice == 1 ? ntiles : min(ntiles, tb + a.slice_tiles),
+                  ((long long)kvh * items + item) * a.nslice + slice};
+}
+// A sliced launch's partials: per unit (kv head, row tile, slice) the unnormalised O^T accumulators as the lanes hold
+// them, [wave][fragment][lane] float4, so that every store and every load of the merge is 1 KB contiguous; behind
+// all of them (reference max, row sum) per unit and row. With RW rows per wave, fragment f of lane l is row l % RW,
+// dims (256 / RW) f + 4 (l / RW) .. + 3.
+template <int RW> __device__ __forceinline__ float* pf_part_o(const GiPrefillArgs& a, int hd, long long unit, int wave) {
+    return a.part + (unit * a.pwaves + wave) * (RW * hd);
+}
+template <int RW> __device__ __forceinline__ float2* pf_part_ml(const GiPrefillArgs& a, int hd, long long units, long long unit, int wave) {
+    return reinterpret_cast<float2*>(a.part + units * a.pwaves * (RW * hd)) + (unit * a.pwaves + wave) * RW;
+}
+
 // s_waitcnt immediate waiting until at most n vector memory operations are outstanding (gfx9 encoding:
 // vmcnt in bits 3:0 and 15:14, expcnt and lgkmcnt left at their maxima)
 #define GI_VMCNT(n) (0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
 // s_waitcnt immediate waiting for this wave's LDS operations (lgkmcnt 0, vmcnt and expcnt at their maxima)
 #define GI_LGKMCNT0 0xC07F
-#define PF_LPW (16 / PF_SW)   // 1 KB loads per staging wave and tile
 #define PF_NBUF 4          // LDS tile buffers
 #define PF_BK 64           // keys per tile
 #define PF_TILE 16384      // bytes of one K or V tile: 64 rows of 256 bytes
@@ -1469,24 +1518,116 @@ __device__ __forceinline__ void gi_stage16(const void* base, long long bytes, GI
     __builtin_amdgcn_raw_ptr_buffer_load_lds(gi_rsrc(base, bytes), dst, 16, voff, 0, 0, 0);
 #endif
 }
+__device__ __forceinline__ u4 gi_rsrc_rows(const void* p, int bytes) {
+    const unsigned long long b = (unsigned long long)p;
+    return u4{(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, (uint32_t)bytes, (uint32_t)GI_RSRC_FLAGS};
+}
+__device__ __forceinline__ void gi_stage16(u4 rs, GI_LDS void* dst, int voff) {
+    const uint32_t m0 = (uint32_t)(uintptr_t)dst;
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "{m0}"(m0) : "memory");
+}
+__device__ __forceinline__ void gi_stage4(u4 rs, GI_LDS void* dst, int voff) { // 4 bytes a lane, at M0 + 4i
+    const uint32_t m0 = (uint32_t)(uintptr_t)dst;
+    asm volatile("s_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "{m0}"(m0) : "memory");
+}
 // int8 cache: the value scale goes into the f16 probabilities times this power of two (undone at the
 // end) so that small products stay normal f16; with P <= 2^8 a dequantised |V| up to 127 * 65504 / (2^8 *
 // PF_I8_VBIAS) ~ 4000 fits (the reference biases by 2^10 with P <= 1, src/cuda.rs:2416-2420)
 #define PF_I8_VBIAS 8.f
 typedef short gi_s4 __attribute__((__vector_size__(8))); // 4 f16 as ds_read_b64_tr_b16 returns them
 
-// One workgroup = (head, 256 query rows); wave w of 8 owns rows 32w..32w+31 of the tile. Per 64-key tile:
+// ---------------------------------------------------------------- prefill, merge of a sliced launch's partials
+// One workgroup per (kv head, row tile, wave of its rows, PFC_FRAGS of its fragments): the slices' weights
+// exp2(m - M) / L of its rows go to LDS once, then each thread sums its float4 over the slices (loads of 1 KB per
+// wave, PFC_FRAGS waves) and writes the output.
+#define PFC_FRAGS 4
+#define PFC_MAXS 64 // most slices of a launch (must match gi_attn_host.cpp)
+template <int RW>
+__device__ __forceinline__ void gi_prefill_combine_t(const GiPrefillArgs& a) {
+    __shared__ float w_sh[PFC_MAXS][RW];
+    __shared__ float l_sh[PFC_MAXS][RW];
+    const int G = a.n_heads / a.n_kv, P = a.n * G, hd = a.hd, BQ = a.rows;
+    const int items = a.items;
+    const int wave = blockIdx.x % a.pwaves, item = blockIdx.x / a.pwaves % items, kvh = blockIdx.x / a.pwaves / items;
+    const int row0 = item * BQ + RW * wave;
+    if (row0 >= P) return;
+    const int ntiles = (a.pos0 + pf_last_token(a, item * BQ, BQ)) / PF_BK + 1;
+    const int ns = min(a.nslice, (ntiles + a.slice_tiles - 1) / a.slice_tiles); // slices that left a partial
+    const long long u0 = ((long long)kvh * items + item) * a.nslice, units = (long long)a.n_kv * items * a.nslice;
+    const int tid = threadIdx.x;
+    for (int i = tid; i < ns * RW; i += 64 * PFC_FRAGS) {
+        const float2 ml = pf_part_ml<RW>(a, hd, units, u0 + i / RW, wave)[i % RW];
+        w_sh[i / RW][i % RW] = ml.x;
+        l_sh[i / RW][i % RW] = ml.y;
+    }
+    __syncthreads();
+    if (tid < RW) {
+        float M = GI_NEG_INF, L = 0.f;
+        for (int s = 0; s < ns; s++) M = fmaxf(M, w_sh[s][tid]);
+        for (int s = 0; s < ns; s++) {
+            const float w = __builtin_amdgcn_exp2f(w_sh[s][tid] - M);
+            w_sh[s][tid] = w;
+            L = fmaf(w, l_sh[s][tid], L);
+        }
+        const float inv = 1.f / L;
+        for (int s = 0; s < ns; s++) w_sh[s][tid] *= inv;
+    }
+    __syncthreads();
+    const int lane = tid & 63, f = blockIdx.y * PFC_FRAGS + (tid >> 6);
+    if (f >= RW * hd / 256) return;
+    const int r = lane % RW;
+    const long long step = (long long)a.pwaves * (RW * hd) / 4; // float4 from one slice's partial to the next
+    const f4* po = reinterpret_cast<const f4*>(pf_part_o<RW>(a, hd, u0, wave)) + 64 * f + lane;
+    f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int s = 0; s < ns; s++) {
+        const f4 x = po[s * step];
+        const float w = w_sh[s][r];
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[e] = fmaf(x[e], w, acc[e]);
+    }
+    const int row = row0 + r;
+    if (row >= P) return;
+    const int tok = pf_token(a, row), h = kvh * G + row - tok * G;
+    const long long e0 = (long long)tok * a.out_stride + (long long)h * hd + (256 / RW) * f + 4 * (lane / RW);
+    if (a.out_f16)
+        *reinterpret_cast<h4x*>((_Float16*)a.out + e0) = h4x{(_Float16)acc[0], (_Float16)acc[1], (_Float16)acc[2], (_Float16)acc[3]};
+    else
+        *reinterpret_cast<f4*>((float*)a.out + e0) = acc;
+}
+extern "C" __global__ void __launch_bounds__(64 * PFC_FRAGS) gi_prefill_combine_32(GiPrefillArgs a) { gi_prefill_combine_t<32>(a); }
+
+template <int I> struct gi_int { static constexpr int value = I; };
+// f(gi_int<0>) ... f(gi_int<N - 1>)
+template <int N, int I = 0, typename F> __device__ __forceinline__ void gi_unroll(F&& f) {
+    if constexpr (I < N) {
+        f(gi_int<I>{});
+        gi_unroll<N, I + 1>(f);
+    }
+}
+// One workgroup = (kv head, 32 * WAVES packed query rows, key slice); wave w owns rows 32w..32w+31 of the tile. Per
+// 64-key tile:
 //   S^T[key, q] = K[key, :] . Q[q, :]       v_mfma_f32_32x32x16_f16, K from LDS (A), Q in registers (B)
 //   O^T[d, q]  += V^T[d, key] . P^T[key, q]  V^T from LDS (A, by transposing reads), P^T from S^T (B)
-// Software pipeline inside each wave: the softmax of tile t (VALU) runs between the MFMAs of QK for
-// tile t+1 and of PV for tile t, which do not depend on it, so the VALU work hides under the matrix core's
-// 32-cycle MFMAs instead of following them (a SIMD does not overlap one wave's VALU with another wave's
-// back-to-back MFMAs, so the overlap has to come from within the wave).
-// Staging: K and V tiles go global -> LDS with direct-to-LDS buffer loads (no registers, no VALU): each of
-// the 8 waves moves 4 KB per tile as 4 loads of 1 KB (64 lanes x 16 bytes, written at base + 16*lane).
-// Rows are stored unpadded with an XOR swizzle of their 16-byte units (K: unit ^ row%16, V: unit ^
-// 4*(row%4)) so the MFMA operand reads hit distinct banks. Iteration t reads V of tile t and K of tile
-// t+1; once every wave has passed its barrier tile t-1 is free and tile t+3 streams into its buffer.
+// Software pipeline inside each wave: iteration `it` runs QK of tile it+1 and P V of tile it as one sequence of slots,
+// one MFMA each, and the rest of the work is placed slot by slot under the 32-cycle MFMAs (scheduling barriers keep
+// it there): the LDS reads of the operands RING slots ahead, tile it's probabilities spread evenly up to the P V MFMA
+// that needs them, tile it+1's row max from two slots after its last QK MFMA, the staging loads. Left to the
+// compiler, the reads sat one or two MFMAs ahead and the exponentials bunched: a wave then took ~3,100 cycles per tile
+// whether its SIMD held one wave or two; with the slots ~2,300 alone (32 MFMAs are 1,024, ~290 instructions issue in
+// ~1,150, the rest are waits).
+// WAVES = 8 (two waves per SIMD, 256 rows) has the better throughput, WAVES = 4 (one per SIMD, 128 rows) the shorter
+// tile time: prefill_plan in the host file chooses. Measured, 32/8 heads of 128, f16 / pre-widened int8: 8192 tokens
+// 505 / 588 us with 8 waves, 580 / 675 with 4 (before the slots, 8 waves: 505 / 630; at head size 64 324 -> 307 /
+// 466 -> 382); 1024 tokens 33.9 / 44.3 against 23.7 / 32.0 us (before: 34.7 / 48.5); 512 tokens at a 2000-token
+// prefix 64 / 87 against 44 / 62 us (before: 65.6 / 97). At 8192 tokens the power limit sets the clock (1.86 GHz
+// against 2.14 with 4 waves): fewer cycles there did not shorten the f16 launch.
+// Staging: K and V tiles go global -> LDS with direct-to-LDS buffer loads (no registers, no VALU): half of the waves
+// move K, half V, LPW loads of 1 KB (64 lanes x 16 bytes, written at base + 16*lane) per wave and tile. Rows are stored
+// unpadded with an XOR swizzle of their 16-byte units (K: unit ^ row%16, V: unit ^ 4*(row%4)) so the MFMA operand
+// reads hit distinct banks. One barrier per iteration, RING slots before its end: it publishes K of tile it+2 and V of
+// tile it+1 (read from there on), and K of tile it+4 and V of tile it+3 then go into the buffers of K(it) and V(it-1),
+// whose readers' MFMAs all issued before it. Two iterations for each load to land.
 // Keys past the cache's end read as zeros (buffer bounds) and are masked.
 // K operand: A-row r of S^T block bb holds tile key 32bb + 16(i/2) + 8h + 4(i%2) + j for r = 8i + 4h + j,
 // so the 16 values a lane holds per block are exactly the keys its PV B operand needs (k-step 2bb + i/2,
@@ -1497,179 +1638,202 @@ typedef short gi_s4 __attribute__((__vector_size__(8))); // 4 f16 as ds_read_b64
 // moves when a tile's max exceeds it by more than 2^8 in probability (then O and l are rescaled), so
 // P <= 256 fits f16 and most tiles skip the rescale. Row sums add the f16-rounded P that PV uses
 // (v_dot2 against ones). Causal: a wave skips tiles past its last row (keeping every barrier); only
-// tiles crossing the diagonal are masked. Work order: the grid is remapped so that each of the 8 XCDs
-// (blockIdx round-robin) walks a contiguous run of (kv head, query tile, head) items, longest query
-// tiles first, so one kv head's K/V stays in one XCD's L2.
-// I8 = true: an int8 cache (the reference's KV8 prefill, src/cuda.rs:2466-2498, 2548-2605): each thread
-// loads 16 bytes of a K row and of a V row of the tile into registers one iteration ahead, widens them to
-// exact f16 and writes them into the same swizzled LDS layout (so the MFMA operand reads are unchanged),
-// and the tile's 64 key and value scales go to LDS beside it. Scores are the integer-key dot products
+// tiles crossing the diagonal are masked.
+// I8 = true: an int8 cache (the reference's KV8 prefill, src/cuda.rs:2466-2498, 2548-2605): the
+// threads load 16-byte chunks of K and V rows into registers one iteration ahead, widen them to exact f16 and write
+// them into the same swizzled LDS layout (so the MFMA operand reads are unchanged), and the tile's 64 key and
+// value scales go to LDS beside it; STG: the cache already widened to exact f16 integers in a workspace
+// (gi_kv_widen, rows [n_kv][len][hd], scales [n_kv][len], the value scales times PF_I8_VBIAS) is staged as the f16
+// cache is. Scores are the integer-key dot products
 // times the key scale (QK chains start from zero; s = acc * kscale - m); P V takes f16(p * vscale *
 // PF_I8_VBIAS) and the row sum the f16-rounded p, as the reference's pv / pf.
 // HD = 64 (attn_prefill_tc<64>, src/cuda.rs:2620): the same kernel with half the QK k-steps and O^T blocks. The
 // LDS image keeps the head-128 layout: each 128-byte row sits in a 256-byte slot, its 8 units at the swizzled
-// positions the operand reads compute (the staging loads of the other 8 positions are switched off by lane).
-template <bool I8, int HD = 128, bool STG = false>
+// positions the operand reads compute (the staging loads of the other 8 positions are out of bounds and leave zeros).
+template <bool I8, int HD, bool STG, int WAVES, int RING>
 __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     static_assert(HD == 64 || HD == 128, "head sizes 64, 128 (256: gi_prefill256r)");
     static_assert(!STG || I8, "pre-widened staging: the int8 cache");
-    // STG: the int8 cache already widened to exact f16 integers in a workspace (gi_kv_widen, rows [n_kv][len][hd],
-    // scales [n_kv][len], the value scales times PF_I8_VBIAS), staged by LDS-DMA as the f16 cache is; else int8
-    // tiles are widened through registers (RSTG)
-    constexpr bool RSTG = I8 && !STG;
-    constexpr int WAVES = PF_WAVES;
+    constexpr bool RSTG = I8 && !STG; // int8 tiles widened through registers, else LDS-DMA
     constexpr int BQ = 32 * WAVES;  // query rows per workgroup
     constexpr int SW = WAVES / 2;   // waves staging each of K and V
     constexpr int LPW = 16 / SW;    // 1 KB loads per staging wave and tile
-    constexpr int LPT = LPW + (STG ? 1 : 0); // loads per staging wave and tile (STG: plus a quarter of the scales)
+    constexpr int LPT = LPW + (STG ? 1 : 0); // loads per staging wave and tile (STG: plus its share of the scales)
     constexpr int BK = PF_BK;       // keys per tile
     constexpr int NBLK = BK / 32;   // S^T blocks of 32 keys
     constexpr int KS = HD / 16;     // QK k-steps
     constexpr int NDB = HD / 32;    // O^T blocks of 32 dims
+    constexpr int NQ = 2 * KS, NP = 4 * NDB, NS = NQ + NP; // MFMAs of QK and of P V, slots of an iteration
     __shared__ __attribute__((aligned(1024))) unsigned char smem[PF_NBUF][2][PF_TILE]; // [buffer][K, V]
-    __shared__ __attribute__((aligned(16))) float scl[I8 ? PF_NBUF : 1][2][BK];         // int8: [buffer][K, V] scales
+    __shared__ __attribute__((aligned(256))) float scl[I8 ? PF_NBUF : 1][2][BK];        // int8: [buffer][K, V] scales
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G = a.n_heads / a.n_kv;
-    const int qtiles = (a.n + BQ - 1) / BQ;
-    const int nwg = gridDim.x;
-    int j = blockIdx.x;
-    if ((nwg & 7) == 0) j = (j & 7) * (nwg >> 3) + (j >> 3);
-    const int kvh = j / (qtiles * G);
-    const int rest = j % (qtiles * G);
-    const int qt = qtiles - 1 - rest / G; // longest query tiles first
-    const int h = kvh * G + rest % G;
-    const int q0 = qt * BQ;
+    const PfUnit un = pf_unit(a, BQ, BK);
+    const int kvh = un.kvh, q0 = un.row0, t_begin = un.t_begin, ntiles = un.t_end; // key tiles t_begin .. ntiles - 1
+    if (t_begin >= ntiles) return; // a slice past the tile's last key
     const int kv_len = a.pos0 + a.n;
-    const int k_lim = min(kv_len, a.pos0 + q0 + BQ); // keys any row of the tile may see
-    const int ntiles = (k_lim + BK - 1) / BK;
     const long long kvs = a.kv_stride;
 
-    // ---- staging: the first half of the waves moves K rows, the second half V rows (SW waves each,
-    // LPW loads of 1 KB per wave and tile); wave w's load i covers tile rows 4*(LPW*(w%SW) + i)
-    // + lane/16, LDS unit lane%16 holding global unit (lane%16) ^ swizzle(row)
     const bool stage_v = wave >= SW;
     const uint16_t* sbase = (stage_v ? a.vc : a.kc) + kvh * a.kv_head_stride;
     int soff[LPW];
-    bool sval[LPW]; // head size 64: the lane's LDS unit holds one of the row's 8 units
 #pragma unroll
     for (int i = 0; i < LPW; i++) {
         const int r = 4 * (LPW * (wave % SW) + i) + (lane >> 4);
         const int u = (lane & 15) ^ (stage_v ? ((r & 3) << 2) : (r & 15));
-        soff[i] = (r * (int)kvs + 8 * u) * 2;
-        sval[i] = u < HD / 8;
+        // head size 64: half of the slot's 16 units hold the row, the other lanes' loads are out of bounds (zeros)
+        soff[i] = u < HD / 8 ? (r * (int)kvs + 8 * u) * 2 : 0x7fffffff;
     }
-    auto stage = [&](int t) {
+    const int last = ntiles - 1;
+    // this wave's share of tile t (its K if it stages K, else its V): load i of stage_at(t). A tile past the last one
+    // is loaded as zeros, without memory traffic, so that every wave has the same count of loads in flight.
+    struct StageAt { u4 rs, rs_sc; unsigned char* dst; float* dst_sc; };
+    auto stage_at = [&](int t) {
         const int t0 = t * BK;
-        const uint16_t* src = sbase + (long long)t0 * kvs;
-        const long long bytes = (long long)(kv_len - t0) * kvs * 2;
-        unsigned char* dst = &smem[t & (PF_NBUF - 1)][stage_v ? 1 : 0][1024 * LPW * (wave % SW)];
-#pragma unroll
-        for (int i = 0; i < LPW; i++)
-            if (HD == 128 || sval[i]) gi_stage16(src, bytes, (GI_LDS void*)(dst + 1024 * i), soff[i]);
-        if constexpr (STG) {
-            // this wave's quarter of the tile's 64 scales (16 floats: lanes 0-3, 16 bytes each)
-            const float* sp = (stage_v ? a.vs : a.ks) + kvh * a.sc_head_stride + t0;
-            if (lane < 4)
-                gi_stage16(sp, (long long)(kv_len - t0) * 4, (GI_LDS void*)&scl[t & (PF_NBUF - 1)][stage_v ? 1 : 0][16 * (wave % SW)],
-                           64 * (wave % SW) + 16 * lane);
+        StageAt s;
+        const int rows = t <= last ? min(kv_len - t0, BK) : 0;
+        s.rs = gi_rsrc_rows(sbase + (long long)t0 * kvs, rows * (int)kvs * 2);
+        s.dst = &smem[t & (PF_NBUF - 1)][stage_v ? 1 : 0][1024 * LPW * (wave % SW)];
+        if constexpr (STG) { // the tile's 64 scales, 4 bytes a lane (by each of the waves that stage the tile)
+            s.rs_sc = gi_rsrc_rows((stage_v ? a.vs : a.ks) + kvh * a.sc_head_stride + t0, rows * 4);
+            s.dst_sc = &scl[t & (PF_NBUF - 1)][stage_v ? 1 : 0][0];
         }
+        return s;
     };
-    // int8 staging: thread -> tile row sr, 16-byte chunk sch (dims 16sch..16sch+15) of K and of V; threads
-    // 0-63 also take the K scale of key tid, 64-127 the V scale of key tid-64 (times PF_I8_VBIAS)
-    // (head size 64: rows of 4 chunks, threads 0-255)
-    constexpr int NCH = HD / 16;
-    const int sr = tid / NCH, sch = tid % NCH;
-    const bool stager = tid < PF_BK * NCH;
+    // int8 tiles through registers: thread -> chunks of 16 bytes of the tile's K and V rows (row ch / NCH, dims 16 (ch %
+    // NCH) ..), widened to exact f16 and written into the same swizzled image; threads 0-63 take the K scale of key tid,
+    // 64-127 the V scale of key tid - 64 (times PF_I8_VBIAS). Lanes in the upper half of a row hold their chunk's two
+    // 8-byte halves swapped (and write them in that order): the 8 lanes of a row that one 16-byte LDS store serves
+    // then write 8 different units mod 8, all 32 banks, where 2ch alone would cover half of them twice.
+    constexpr int NT = 64 * WAVES, NCH = HD / 16, CH = BK * NCH, CPT = CH > NT ? CH / NT : 1;
     const int8_t* kb8 = reinterpret_cast<const int8_t*>(a.kc) + kvh * a.kv_head_stride;
     const int8_t* vb8 = reinterpret_cast<const int8_t*>(a.vc) + kvh * a.kv_head_stride;
-    const float* scb = I8 ? (tid < 64 ? a.ks : a.vs) + kvh * a.sc_head_stride : nullptr;
-    u4 rk = u4{0u, 0u, 0u, 0u}, rv = rk;
+    const float* scb = RSTG ? (tid < BK ? a.ks : a.vs) + kvh * a.sc_head_stride : nullptr;
+    struct Chunks { u4 w[CPT]; };
+    Chunks rk, rv;
     float rsc = 0.f;
-    // Lanes with sch >= 4 hold their chunk's two 8-byte halves swapped (and write them in that order below):
-    // then the 8 lanes of a row that one 16-byte LDS store serves write 8 different units mod 8, all 32
-    // banks, where 2sch alone would cover half of them twice.
-    const int flip = (sch >> 2) & 1;
-    auto load8 = [&](int t) {
-        const int t0 = t * PF_BK;
-        const int off = sr * (int)kvs + 16 * sch;
-        const __amdgpu_buffer_rsrc_t rsk = gi_rsrc(kb8 + (long long)t0 * kvs, (long long)(kv_len - t0) * kvs);
-        const __amdgpu_buffer_rsrc_t rsv = gi_rsrc(vb8 + (long long)t0 * kvs, (long long)(kv_len - t0) * kvs);
-        if (stager) {
-            const u2 k0 = gi_load8(rsk, off + 8 * flip), k1 = gi_load8(rsk, off + 8 - 8 * flip);
-            const u2 v0 = gi_load8(rsv, off + 8 * flip), v1 = gi_load8(rsv, off + 8 - 8 * flip);
-            rk = u4{k0.x, k0.y, k1.x, k1.y};
-            rv = u4{v0.x, v0.y, v1.x, v1.y};
+    auto load_rows = [&](const int8_t* base, int t, Chunks& c) {
+        const int t0 = t * BK, rows = t <= last ? min(kv_len - t0, BK) : 0;
+        const __amdgpu_buffer_rsrc_t rs = gi_rsrc(base + (long long)t0 * kvs, rows * (int)kvs);
+#pragma unroll
+        for (int i = 0; i < CPT; i++) {
+            const int ch = tid + NT * i, off = ch / NCH * (int)kvs + 16 * (ch % NCH), flip = (ch % NCH >> 2) & 1;
+            if (CH % NT && ch >= CH) continue;
+            const u2 h0 = gi_load8(rs, off + 8 * flip), h1 = gi_load8(rs, off + 8 - 8 * flip);
+            c.w[i] = u4{h0.x, h0.y, h1.x, h1.y};
         }
-        if (tid < 2 * PF_BK)
-            rsc = gi_load4f(gi_rsrc(scb + (long long)t0 * a.sc_stride, (long long)(kv_len - t0) * a.sc_stride * 4),
-                            (tid & (PF_BK - 1)) * (int)a.sc_stride * 4);
     };
-    auto write8 = [&](int t) {
-        unsigned char* K = &smem[t & (PF_NBUF - 1)][0][sr * 256];
-        unsigned char* V = &smem[t & (PF_NBUF - 1)][1][sr * 256];
+    auto load_scales = [&](int tk, int tv) {
+        const int t0 = (tid < BK ? tk : tv) * BK, rows = t0 <= last * BK ? min(kv_len - t0, BK) : 0;
+        rsc = 0.f;
+        if (tid < 2 * BK && (tid & (BK - 1)) < rows) rsc = scb[(long long)(t0 + (tid & (BK - 1))) * a.sc_stride];
+    };
+    auto write_rows = [&](int t, bool v, const Chunks& c) {
+        GI_LDS unsigned char* img = (GI_LDS unsigned char*)&smem[t & (PF_NBUF - 1)][v ? 1 : 0][0];
 #pragma unroll
-        for (int hw = 0; hw < 2; hw++) { // f16 unit 2sch + (hw ^ flip): dims 16sch + 8(hw ^ flip) .. +7
-            if (!stager) break;
-            const int u = 2 * sch + (hw ^ flip);
-            u4 kw, vw;
+        for (int i = 0; i < CPT; i++) {
+            const int ch = tid + NT * i, row = ch / NCH, flip = (ch % NCH >> 2) & 1;
+            if (CH % NT && ch >= CH) continue;
 #pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const uint32_t xk = gi_i8_in(rk[2 * hw + e]), xv = gi_i8_in(rv[2 * hw + e]);
-                kw[2 * e] = i8_f16x2(xk, GI_I8_LO);
-                kw[2 * e + 1] = i8_f16x2(xk, GI_I8_HI);
-                vw[2 * e] = i8_f16x2(xv, GI_I8_LO);
-                vw[2 * e + 1] = i8_f16x2(xv, GI_I8_HI);
+            for (int hw = 0; hw < 2; hw++) {
+                const int u = 2 * (ch % NCH) + (hw ^ flip);
+                u4 w;
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const uint32_t x = gi_i8_in(c.w[i][2 * hw + e]);
+                    w[2 * e] = i8_f16x2(x, GI_I8_LO);
+                    w[2 * e + 1] = i8_f16x2(x, GI_I8_HI);
+                }
+                *reinterpret_cast<GI_LDS u4*>(img + row * 256 + ((u ^ (v ? (row & 3) << 2 : row & 15)) << 4)) = w;
             }
-            *reinterpret_cast<u4*>(K + ((u ^ (sr & 15)) << 4)) = kw;
-            *reinterpret_cast<u4*>(V + ((u ^ ((sr & 3) << 2)) << 4)) = vw;
         }
-        if (tid < 2 * PF_BK) scl[t & (PF_NBUF - 1)][tid >> 6][tid & (PF_BK - 1)] = tid < PF_BK ? rsc : rsc * PF_I8_VBIAS;
+    };
+    auto write_scales = [&](int tk, int tv) {
+        if (tid < BK) scl[tk & (PF_NBUF - 1)][0][tid] = rsc;
+        else if (tid < 2 * BK) scl[tv & (PF_NBUF - 1)][1][tid - BK] = rsc * PF_I8_VBIAS;
+    };
+    auto stage1 = [&](const StageAt& s, int i) {
+        if (i < LPW) gi_stage16(s.rs, (GI_LDS void*)(s.dst + 1024 * i), soff[i]);
+        else if constexpr (STG) gi_stage4(s.rs_sc, (GI_LDS void*)s.dst_sc, 4 * lane);
+    };
+    auto stage = [&](int t) {
+        const StageAt s = stage_at(t);
+#pragma unroll
+        for (int i = 0; i < LPT; i++) stage1(s, i);
     };
 
     // ---- Q as B operands: lane (col = l%32, half = l/32), k-step ks: dims 16ks + 8*half .. +7
     const int qcol = lane & 31, half = lane >> 5;
-    const int qrow = q0 + 32 * wave + qcol;      // this lane's query row
-    const int qpos = a.pos0 + qrow;              // its position
+    const int qrow = q0 + 32 * wave + qcol;      // this lane's packed query row
+    const bool qlive = qrow < a.n * G;           // (rows past the last compute garbage that is never written)
+    const int qtok = qlive ? pf_token(a, qrow) : a.n - 1;
+    const int h = kvh * G + (qlive ? qrow : a.n * G - 1) - qtok * G;
+    const int qpos = a.pos0 + qtok;              // its position
     // Q is held pre-multiplied by scale*log2(e), so scores come out of the MFMA in log2 units (the f16
     // rounding of the scaled value is the same size as the rounding of Q itself)
     const float qs = a.qscale;
+    // what the first QK and the first iteration need starts loading: K of two tiles, V of one
+    Chunks rk1;
+    float rsc1 = 0.f;
+    if constexpr (RSTG) {
+        load_rows(kb8, t_begin, rk);
+        load_rows(vb8, t_begin, rv);
+        load_rows(kb8, t_begin + 1, rk1);
+        load_scales(t_begin + 1, t_begin); // K of the second tile, V of the first
+        rsc1 = rsc;
+        load_scales(t_begin, t_begin);
+    } else {
+        stage(t_begin);
+        if (!stage_v) stage(t_begin + 1);
+    }
     h8 qf[KS];
-    {
-        const int qr = qrow < a.n ? qrow : a.n - 1; // rows past n compute garbage that is never written
-        if (a.q_f16) {
-            const _Float16* qp = (const _Float16*)a.q + (long long)qr * a.q_stride + h * HD + 8 * half;
+    if (a.q_f16) {
+        const _Float16* qp = (const _Float16*)a.q + (long long)qtok * a.q_stride + h * HD + 8 * half;
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                const h8 x = __builtin_bit_cast(h8, *reinterpret_cast<const u4*>(qp + 16 * ks));
+        for (int ks = 0; ks < KS; ks++) {
+            const h8 x = __builtin_bit_cast(h8, *reinterpret_cast<const u4*>(qp + 16 * ks));
 #pragma unroll
-                for (int e = 0; e < 8; e++) qf[ks][e] = (_Float16)((float)x[e] * qs);
-            }
-        } else {
-            const float* qp = (const float*)a.q + (long long)qr * a.q_stride + h * HD + 8 * half;
+            for (int e = 0; e < 8; e++) qf[ks][e] = (_Float16)((float)x[e] * qs);
+        }
+    } else {
+        const float* qp = (const float*)a.q + (long long)qtok * a.q_stride + h * HD + 8 * half;
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                float4 x0 = *reinterpret_cast<const float4*>(qp + 16 * ks);
-                float4 x1 = *reinterpret_cast<const float4*>(qp + 16 * ks + 4);
-                qf[ks] = h8{(_Float16)(x0.x * qs), (_Float16)(x0.y * qs), (_Float16)(x0.z * qs), (_Float16)(x0.w * qs),
-                            (_Float16)(x1.x * qs), (_Float16)(x1.y * qs), (_Float16)(x1.z * qs), (_Float16)(x1.w * qs)};
-            }
+        for (int ks = 0; ks < KS; ks++) {
+            float4 x0 = *reinterpret_cast<const float4*>(qp + 16 * ks);
+            float4 x1 = *reinterpret_cast<const float4*>(qp + 16 * ks + 4);
+            qf[ks] = h8{(_Float16)(x0.x * qs), (_Float16)(x0.y * qs), (_Float16)(x0.z * qs), (_Float16)(x0.w * qs),
+                        (_Float16)(x1.x * qs), (_Float16)(x1.y * qs), (_Float16)(x1.z * qs), (_Float16)(x1.w * qs)};
         }
     }
 
+    // (the compiler's wait for the queries is also one for the loads above; the next two tiles' go out behind it)
+    if constexpr (RSTG) {
+        write_rows(t_begin, false, rk);
+        write_rows(t_begin, true, rv);
+        write_scales(t_begin, t_begin);
+        write_rows(t_begin + 1, false, rk1);
+        rsc = rsc1;
+        write_scales(t_begin + 1, t_begin);
+        load_rows(kb8, t_begin + 2, rk);
+        load_rows(vb8, t_begin + 1, rv);
+        load_scales(t_begin + 2, t_begin + 1);
+    } else {
+        stage(t_begin + (stage_v ? 1 : 2));
+        stage(t_begin + (stage_v ? 2 : 3));
+    }
     // ---- operand read offsets (bytes within a buffer's K or V tile)
     const int r = lane & 31;
     const int kperm = 16 * ((r >> 3) >> 1) + 8 * ((r >> 2) & 1) + 4 * ((r >> 3) & 1) + (r & 3);
-    // K row kperm (block 1 is 32 rows = 8192 bytes further), unit (2ks + half) ^ (kperm % 16)
-    //   = 2(ks ^ ky) + (half ^ kperm % 2)
     const int kbase = kperm * 256 + ((half ^ (kperm & 1)) << 4);
     const int ky = (kperm >> 1) & 7;
     const int tg = lane >> 4, ts = lane & 15, te = ts >> 2, tc = ts & 3;
-    // V row 8*half + te (+16ks, +4 for the second read), unit 4*(db ^ te) + 2*(tg%2) + tc/2
     const int vbase = (8 * half + te) * 256 + ((2 * (tg & 1) + (tc >> 1)) << 4) + 8 * (tc & 1);
+    // (bits 5-7 of kbase and 6-7 of vbase are free: the swizzled unit of k-step ks or dim block db is one xor)
+    const int kx = kbase | (ky << 5), vx = vbase | (te << 6);
 
-    // ---- per-lane state: O^T (4 dim blocks of 32), reference max (log2 units; tile 0 sets it), row sum
+    // ---- per-lane state: O^T (dim blocks of 32), reference max (log2 units; the first tile sets it), row sum
     f16x o[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; db++)
@@ -1680,97 +1844,85 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
 #pragma unroll
     for (int e = 0; e < 16; e++) negm[e] = 0.f;
 
-    // S^T of tile t (its K in buffer t%4) minus the row's reference max: each chain starts from C = negm,
-    // so the MFMA output is the exp2 argument itself
-    // MFMA st of a tile's 16 alternates the two key blocks (k-step st/2, key block st%2)
-    auto kfrag = [&](const unsigned char* K, int st) {
-        const int reg = st & 1, ksr = st >> 1;
-        return *reinterpret_cast<const h8*>(K + 8192 * reg + kbase + 32 * (ksr ^ ky));
+    auto buf = [&](int t) { return (t & (PF_NBUF - 1)) * (2 * PF_TILE); };
+    GI_LDS unsigned char* const lds = (GI_LDS unsigned char*)&smem[0][0][0];
+    // fragment st of a tile's QK (key block st%2, k-step st/2), fragment f of its P V (k-step f/NDB, dim block f%NDB)
+    auto kfrag = [&](int B, int st) {
+        return *reinterpret_cast<GI_LDS const h8*>(lds + ((B + kx) ^ (32 * (st >> 1))) + 8192 * (st & 1));
     };
-    auto qk = [&](int t, f16x* s) {
-        const unsigned char* K = &smem[t & (PF_NBUF - 1)][0][0];
-        // K fragments stream through a ring of PF_KPF registers, each read PF_KPF MFMAs before its use
-        h8 kf[PF_KPF];
-#pragma unroll
-        for (int st = 0; st < PF_KPF; st++) kf[st] = kfrag(K, st);
-        __builtin_amdgcn_sched_barrier(0); // the first PF_KPF reads go out before any of the MFMAs
-#pragma unroll
-        for (int st = 0; st < 2 * KS; st++) {
-            const int ks = st >> 1, bb = st & 1;
-            const h8 cur = kf[st % PF_KPF];
-            if (st + PF_KPF < 2 * KS) kf[st % PF_KPF] = kfrag(K, st + PF_KPF);
-            s[bb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur, qf[ks], ks == 0 ? (I8 ? f16x{} : negm) : s[bb], 0, 0, 0);
-        }
-    };
-    // int8: scores of tile t (its QK sums in s) times their key scales, minus the reference max. Lane holds
-    // block bb, element 4i + jj: tile key 32bb + 16(i/2) + 8*half + 4(i%2) + jj
-    auto kscale = [&](int t, f16x* s) {
-        if constexpr (I8) {
-            const float* ksl = &scl[t & (PF_NBUF - 1)][0][8 * half];
-#pragma unroll
-            for (int bb = 0; bb < 2; bb++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float4 k4 = *reinterpret_cast<const float4*>(ksl + 32 * bb + 16 * (i >> 1) + 4 * (i & 1));
-                    s[bb][4 * i] = fmaf(s[bb][4 * i], k4.x, -m_run);
-                    s[bb][4 * i + 1] = fmaf(s[bb][4 * i + 1], k4.y, -m_run);
-                    s[bb][4 * i + 2] = fmaf(s[bb][4 * i + 2], k4.z, -m_run);
-                    s[bb][4 * i + 3] = fmaf(s[bb][4 * i + 3], k4.w, -m_run);
-                }
-        }
+    auto vfrag = [&](int B, int f) {
+        GI_LDS unsigned char* vp = lds + ((B + vx) ^ (64 * (f % NDB))) + PF_TILE + 4096 * (f / NDB);
+        gi_s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GI_LDS gi_s4*)(vp));
+        gi_s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GI_LDS gi_s4*)(vp + 1024));
+        return __builtin_shufflevector(__builtin_bit_cast(h4x, lo), __builtin_bit_cast(h4x, hi), 0, 1, 2, 3, 4, 5, 6, 7);
     };
 
-    const int wave_first = a.pos0 + q0 + 32 * wave;  // position of the wave's first row
-    const int wave_last = wave_first + 31;
-    const int my_tiles = min(ntiles, wave_last / BK + 1); // tiles this wave computes
+    const int wrow = q0 + 32 * wave;                      // the wave's first row
+    const int wave_first = a.pos0 + pf_token(a, wrow);    // its position
+    const int wave_last = a.pos0 + pf_last_token(a, wrow, 32);
+    const int my_tiles = wrow < a.n * G ? min(ntiles, wave_last / BK + 1) : 0; // tiles this wave computes: up to here
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
-    // Prologue: tiles 0-2 start loading; tile 0 is waited for and published, and its QK issued. (int8:
-    // tiles 0 and 1 are loaded and written, tile 2's loads stay in flight into registers.)
-    if constexpr (RSTG) {
-        load8(0);
-        write8(0);
-        if (ntiles > 1) {
-            load8(1);
-            write8(1);
-        }
-        if (ntiles > 2) load8(2);
-        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): this thread's LDS writes are done
-    } else {
-        stage(0);
-        if (ntiles > 1) stage(1);
-        if (ntiles > 2) stage(2);
-        if (ntiles > 2) __builtin_amdgcn_s_waitcnt(GI_VMCNT(2 * LPT)); // tile 0 is in
-        else if (ntiles > 1) __builtin_amdgcn_s_waitcnt(GI_VMCNT(LPT));
-        else __builtin_amdgcn_s_waitcnt(GI_VMCNT(0));
-    }
-    asm volatile("s_barrier" ::: "memory");
-    // One pipeline step: tile it's softmax and PV, with QK of tile it+1 into sn (past this wave's last
-    // tile that QK reads a stale buffer and is never used). No branch separates the QK MFMAs from the
-    // VALU work they hide.
     // row max of a tile's scores (relative to m_run) over the row's two lane halves (lanes l and l + 32,
     // exchanged by a VALU lane swap, no LDS round trip)
+    auto halves_max = [&](float mx) {
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_int(mx), __float_as_int(mx), false, false);
+        return fmaxf(__int_as_float(p[0]), __int_as_float(p[1]));
+    };
     auto rowmax = [&](const f16x* sc) {
         float mx = GI_NEG_INF;
 #pragma unroll
         for (int bb = 0; bb < NBLK; bb++)
 #pragma unroll
             for (int e = 0; e < 16; e++) mx = fmaxf(mx, sc[bb][e]);
-        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_int(mx), __float_as_int(mx), false, false);
-        return fmaxf(__int_as_float(p[0]), __int_as_float(p[1]));
+        return halves_max(mx);
     };
-    // One pipeline step for tile it (scores s, their row max mx): the rare rescale first, then one
-    // branch-free block that issues QK of tile it+1 into sn, computes tile it's probabilities k-step by
-    // k-step under those MFMAs and the PV MFMAs of tile it, and ends with tile it+1's row max (mx on exit),
-    // so that the next step can start its exp2 work at once. Past this wave's last tile the QK reads a
-    // stale buffer and is never used.
-    auto step = [&](int it, f16x* s, f16x* sn, float& mx) {
-        const bool up = mx > PF_RESCALE_LOG2 || it == 0;
+    // int8: this lane's 4 scales of key group (bb, i): keys 32bb + 16(i/2) + 8*half + 4(i%2) .. +3
+    auto scale4 = [&](const float* sc, int g) {
+        return *reinterpret_cast<const f4*>(sc + 8 * half + 32 * (g >> 2) + 16 * ((g & 3) >> 1) + 4 * (g & 1));
+    };
+
+    h8 kf[RING], vf[RING];
+    float mx = GI_NEG_INF;
+    f16x sa[NBLK], sb[NBLK]; // scores of alternate tiles
+
+    // publish K of tile it+2 and V of tile it+1 (each wave's own loads of them are in; one tile more may be in flight),
+    // after which tile it+4's K goes into K(it)'s buffer, tile it+3's V into V(it-1)'s
+    auto publish = [&](int it) {
+        if constexpr (RSTG) __builtin_amdgcn_s_waitcnt(GI_LGKMCNT0); // this wave's widened rows are in LDS
+        else __builtin_amdgcn_s_waitcnt(GI_VMCNT(LPT));
+        asm volatile("s_barrier" ::: "memory");
+    };
+    // register staging of iteration it: the rows loaded in iteration it-1 (K of tile it+2, V of tile it+1) are widened
+    // into their buffers (last read in iterations it-3 and it-3), and the next ones' loads go out
+    auto restage_k = [&](int it) {
+        write_rows(it + 2, false, rk);
+        load_rows(kb8, it + 3, rk);
+    };
+    auto restage_v = [&](int it) {
+        write_rows(it + 1, true, rv);
+        load_rows(vb8, it + 2, rv);
+    };
+    auto restage_s = [&](int it) {
+        write_scales(it + 2, it + 1);
+        load_scales(it + 3, it + 2);
+    };
+    auto step = [&](int it, f16x* s, f16x* sn) {
+        const int t0 = it * BK;
+        if (t0 + BK - 1 > wave_first) { // the tile crosses the diagonal (or the end) somewhere in the wave
+            const int lim = qpos - t0 - 8 * half;
+#pragma unroll
+            for (int bb = 0; bb < NBLK; bb++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int jj = 0; jj < 4; jj++)
+                        if (32 * bb + 16 * (i >> 1) + 4 * (i & 1) + jj > lim) s[bb][4 * i + jj] = GI_NEG_INF;
+            mx = rowmax(s);
+        }
+        const bool up = mx > PF_RESCALE_LOG2 || it == t_begin;
         if (__builtin_amdgcn_ballot_w64(up)) {
-            // some row's max moved (tile 0: every row takes its first max): shift the reference by delta,
-            // rescale O and l (alpha = 1 for the other rows; O and l are still 0 at tile 0) and this tile's
-            // scores; the next tile's QK starts from the new reference
-            const float delta = up ? mx : 0.f;
+            const float delta = up && mx > GI_NEG_INF ? mx : 0.f;
             const float alpha = __builtin_amdgcn_exp2f(-fmaxf(delta, 0.f));
             m_run += delta;
 #pragma unroll
@@ -1781,108 +1933,153 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
 #pragma unroll
             for (int bb = 0; bb < NBLK; bb++) s[bb] -= delta;
         }
-        qk(it + 1, sn);
-        // probabilities of k-step ks feed the PV MFMAs of k-step ks
-        const unsigned char* V = &smem[it & (PF_NBUF - 1)][1][0];
+        const int B0 = buf(it), B1 = buf(it + 1), B2 = buf(it + 2);
+        StageAt st; // the tile this iteration stages
+        if constexpr (!RSTG) st = stage_at(it + (stage_v ? 3 : 4));
+        h8 pf[4];
+        float mxn = GI_NEG_INF;
+        // slot of probability pair w (of 16: every P^T operand is complete before its P V MFMAs), and of the next
+        // tile's row max over score group g (of 8), from two slots after its last QK MFMA on
+        constexpr auto pslot = [](int w) { return w * (NS - 4) / 16; };
+        constexpr auto mslot = [](int g) { return NQ + 2 + g * (NP - 2) / 8; };
+        // int8: scales of score group g in element g % SR, read when the group SR before it has taken its own
+        constexpr int SR = HD == 64 ? 4 : 2;
+        f4 ksv[SR], vsv[SR];
+        const float* const ksp = &scl[I8 ? (it + 1) & (PF_NBUF - 1) : 0][0][0];
+        const float* const vsp = &scl[I8 ? it & (PF_NBUF - 1) : 0][1][0];
+        if constexpr (I8)
 #pragma unroll
-        for (int ks = 0; ks < BK / 16; ks++) {
-            const int bb = ks >> 1;
-            h8 pf;
+            for (int g = 0; g < SR; g++) vsv[g] = scale4(vsp, g);
+        __builtin_amdgcn_sched_barrier(0);
+        gi_unroll<NS>([&](auto slot) {
+            constexpr int sl = decltype(slot)::value;
+            if constexpr (sl == NS - RING) publish(it);
+            // the slot's MFMA
+            if constexpr (sl < NQ) {
+                const int ks = sl >> 1, bb = sl & 1;
+                sn[bb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[sl % RING], qf[ks], ks == 0 ? (I8 ? f16x{} : negm) : sn[bb], 0, 0, 0);
+            } else {
+                const int f = sl - NQ;
+                o[f % NDB] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[f % RING], pf[f / NDB], o[f % NDB], 0, 0, 0);
+            }
+            // LDS reads, RING slots ahead of their MFMA
+            if constexpr (sl + RING < NQ) kf[sl % RING] = kfrag(B1, sl + RING);
+            else if constexpr (sl + RING < NS) vf[(sl + RING - NQ) % RING] = vfrag(B0, sl + RING - NQ);
+            else kf[(sl + RING - NS) % RING] = kfrag(B2, sl + RING - NS);
+            // staging behind the barrier
+            if constexpr (RSTG) {
+                if (sl == 1) restage_k(it);
+                if (sl == NQ / 2 + 1) restage_v(it);
+                if (sl == NQ - 1) restage_s(it);
+            } else {
 #pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                const int i = 2 * (ks & 1) + (e >> 2), jj = e & 3;
-                const float p0 = __builtin_amdgcn_exp2f(s[bb][4 * i + jj]);
-                const float p1 = __builtin_amdgcn_exp2f(s[bb][4 * i + jj + 1]);
-                const _Float16 h0 = (_Float16)p0, h1 = (_Float16)p1;
-                if constexpr (I8) { // P V takes p times the value scale; the row sum the rounded p
-                    const float* vsl = &scl[it & (PF_NBUF - 1)][1][32 * bb + 16 * (i >> 1) + 8 * half + 4 * (i & 1) + jj];
-                    pf[e] = (_Float16)(p0 * vsl[0]);
-                    pf[e + 1] = (_Float16)(p1 * vsl[1]);
-                } else {
-                    pf[e] = h0;
-                    pf[e + 1] = h1;
+                for (int i = 0; i < LPT; i++)
+                    if (sl == NS - RING + i * RING / LPT) stage1(st, i);
+            }
+#pragma unroll
+            for (int w = 0; w < 16; w++)
+                if (pslot(w) == sl) {
+                    const int ks = w >> 2, e = 2 * (w & 3), bb = ks >> 1, i = 2 * (ks & 1) + (e >> 2), jj = e & 3;
+                    const float p0 = __builtin_amdgcn_exp2f(s[bb][4 * i + jj]);
+                    const float p1 = __builtin_amdgcn_exp2f(s[bb][4 * i + jj + 1]);
+                    const _Float16 h0 = (_Float16)p0, h1 = (_Float16)p1;
+                    if constexpr (I8) {
+                        pf[ks][e] = (_Float16)(p0 * vsv[(w >> 1) % SR][jj]);
+                        pf[ks][e + 1] = (_Float16)(p1 * vsv[(w >> 1) % SR][jj + 1]);
+                    } else {
+                        pf[ks][e] = h0;
+                        pf[ks][e + 1] = h1;
+                    }
+                    l_run = __builtin_amdgcn_fdot2(h2{h0, h1}, h2{(_Float16)1.f, (_Float16)1.f}, l_run, false);
+                    if constexpr (I8)
+                        if ((w & 1) && (w >> 1) + SR < 8) vsv[(w >> 1) % SR] = scale4(vsp, (w >> 1) + SR);
                 }
-                l_run = __builtin_amdgcn_fdot2(h2{h0, h1}, h2{(_Float16)1.f, (_Float16)1.f}, l_run, false);
-            }
+            // the next tile's row max (int8: after its key scales)
+            if constexpr (I8 && sl == NQ - 2)
 #pragma unroll
-            for (int db = 0; db < NDB; db++) {
-                const unsigned char* vp = V + vbase + ((db ^ te) << 6) + 4096 * ks;
-                gi_s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GI_LDS gi_s4*)(vp));
-                gi_s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GI_LDS gi_s4*)(vp + 1024));
-                h8 vf = __builtin_shufflevector(__builtin_bit_cast(h4x, lo), __builtin_bit_cast(h4x, hi),
-                                                0, 1, 2, 3, 4, 5, 6, 7);
-                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf, o[db], 0, 0, 0);
-            }
-        }
-        kscale(it + 1, sn);
-        mx = rowmax(sn); // unmasked: a diagonal tile recomputes it after masking
-        // Instruction order of the QK phase: every QK MFMA is followed by the read of the K fragment PF_KPF
-        // MFMAs on (the compiler otherwise reads each fragment just before its MFMA). Interleaving the
-        // softmax VALU or the V reads by further groups measured no better.
+                for (int g = 0; g < SR; g++) ksv[g] = scale4(ksp, g);
 #pragma unroll
-        for (int i = 0; i < 2 * KS; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // MFMA
-            if (i + PF_KPF < 2 * KS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); // its K refill
-        }
+            for (int g = 0; g < 8; g++)
+                if (mslot(g) == sl) {
+                    f16x& x = sn[g >> 2];
+                    const int b = 4 * (g & 3);
+                    if constexpr (I8)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) x[b + e] = fmaf(x[b + e], ksv[g % SR][e], -m_run);
+                    mxn = fmaxf(fmaxf(mxn, x[b]), x[b + 1]);
+                    mxn = fmaxf(fmaxf(mxn, x[b + 2]), x[b + 3]);
+                    if constexpr (I8)
+                        if (g + SR < 8) ksv[g % SR] = scale4(ksp, g + SR);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        mx = halves_max(mxn);
     };
-    // Iteration it: before the barrier each wave waits for its own loads of tile it+1 (tile it+2's may
-    // stay in flight); the barrier publishes the tile and tells that every wave is done with tile it-1,
-    // whose buffer then takes tile it+3. Barriers are bare s_barrier (__syncthreads' release fence would
-    // also wait for tile it+2's loads); the memory clobber keeps LDS accesses on their side.
-    float mx = GI_NEG_INF;
-    // int8: the registers loaded in iteration it-1 (tile it+2) are written into its buffer (free: every wave
-    // has passed tile it-2) right after the barrier, and tile it+3's loads go out; a wave's LDS writes are
-    // complete before the next barrier publishes them.
     auto iteration = [&](int it, f16x* s, f16x* sn) {
-        if constexpr (RSTG) {
-            __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
-        } else {
-            if (it + 2 < ntiles) __builtin_amdgcn_s_waitcnt(GI_VMCNT(LPT)); // tile it+2's loads may stay in flight
-            else __builtin_amdgcn_s_waitcnt(GI_VMCNT(0));
-        }
-        asm volatile("s_barrier" ::: "memory");
-        if constexpr (RSTG) {
-            if (it + 2 < ntiles) {
-                write8(it + 2);
-                if (it + 3 < ntiles) load8(it + 3);
-            }
-        } else {
-            if (it + 3 < ntiles) stage(it + 3);
-        }
         if (it < my_tiles) {
-            const int t0 = it * BK;
-            if (t0 + BK - 1 > wave_first) { // the tile crosses the diagonal (or the end) somewhere in the wave
-                // lane holds, for query qcol: block bb, element 4i + jj -> tile key 32bb + 16(i/2) + 8*half + 4(i%2) + jj
-                const int lim = qpos - t0 - 8 * half;
-#pragma unroll
-                for (int bb = 0; bb < NBLK; bb++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++)
-#pragma unroll
-                        for (int jj = 0; jj < 4; jj++)
-                            if (32 * bb + 16 * (i >> 1) + 4 * (i & 1) + jj > lim) s[bb][4 * i + jj] = GI_NEG_INF;
-                mx = rowmax(s);
+            step(it, s, sn);
+        } else {
+            if constexpr (RSTG) {
+                restage_k(it);
+                restage_v(it);
+                restage_s(it);
             }
-            step(it, s, sn, mx);
+            publish(it);
+            if constexpr (!RSTG) stage(it + (stage_v ? 3 : 4));
         }
     };
-    f16x sa[NBLK], sb[NBLK]; // scores of alternate tiles
-    if (my_tiles > 0) {
-        qk(0, sa);
-        kscale(0, sa);
+
+    // prologue: K of the first two tiles and V of the first are in
+    if constexpr (RSTG) __builtin_amdgcn_s_waitcnt(GI_LGKMCNT0);
+    else __builtin_amdgcn_s_waitcnt(GI_VMCNT(2 * LPT));
+    asm volatile("s_barrier" ::: "memory");
+    if (my_tiles > t_begin) {
+        const int B0 = buf(t_begin), B1 = buf(t_begin + 1);
+#pragma unroll
+        for (int st = 0; st < RING; st++) kf[st] = kfrag(B0, st);
+#pragma unroll
+        for (int st = 0; st < NQ; st++) {
+            const int ks = st >> 1, bb = st & 1;
+            sa[bb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[st % RING], qf[ks], ks == 0 ? f16x{} : sa[bb], 0, 0, 0);
+            kf[st % RING] = st + RING < NQ ? kfrag(B0, st + RING) : kfrag(B1, st + RING - NQ);
+        }
+        if constexpr (I8) {
+#pragma unroll
+            for (int g = 0; g < 8; g++) {
+                const f4 k4 = scale4(&scl[t_begin & (PF_NBUF - 1)][0][0], g);
+#pragma unroll
+                for (int e = 0; e < 4; e++) sa[g >> 2][4 * (g & 3) + e] *= k4[e];
+            }
+        }
         mx = rowmax(sa);
     }
-    for (int it = 0; it < ntiles; it += 2) {
+    for (int it = t_begin; it < ntiles; it += 2) {
         iteration(it, sa, sb);
         if (it + 1 < ntiles) iteration(it + 1, sb, sa);
     }
+    __builtin_amdgcn_s_waitcnt(GI_VMCNT(0)); // no load may write this LDS once the workgroup has ended
 
     // ---- normalise and write: lane holds query qcol, dims 32db + 8i + 4*half + jj
     float l = l_run + __shfl_xor(l_run, 32, 64);
-    if (qrow < a.n) {
+    if (a.nslice > 1) { // a slice's partial; a row with no key here (sum 0) leaves max -inf
+        if (wave >= a.pwaves) return;
+        f4* po = reinterpret_cast<f4*>(pf_part_o<32>(a, HD, un.unit, wave)) + lane;
+#pragma unroll
+        for (int db = 0; db < NDB; db++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                f4 v = f4{o[db][4 * i], o[db][4 * i + 1], o[db][4 * i + 2], o[db][4 * i + 3]};
+                if constexpr (I8) v *= 1.f / PF_I8_VBIAS;
+                po[64 * (4 * db + i)] = v;
+            }
+        if (half == 0)
+            pf_part_ml<32>(a, HD, gridDim.x, un.unit, wave)[qcol] = make_float2(l == 0.f ? GI_NEG_INF : m_run, l);
+        return;
+    }
+    if (qlive) {
         const float inv = (I8 ? 1.f / PF_I8_VBIAS : 1.f) / l;
         if (a.out_f16) {
-            _Float16* op = (_Float16*)a.out + (long long)qrow * a.out_stride + h * HD + 4 * half;
+            _Float16* op = (_Float16*)a.out + (long long)qtok * a.out_stride + h * HD + 4 * half;
 #pragma unroll
             for (int db = 0; db < NDB; db++)
 #pragma unroll
@@ -1892,7 +2089,7 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
                     *reinterpret_cast<h4x*>(op + 32 * db + 8 * i) = v;
                 }
         } else {
-            float* op = (float*)a.out + (long long)qrow * a.out_stride + h * HD + 4 * half;
+            float* op = (float*)a.out + (long long)qtok * a.out_stride + h * HD + 4 * half;
 #pragma unroll
             for (int db = 0; db < NDB; db++)
 #pragma unroll
@@ -2328,13 +2525,25 @@ __device__ __forceinline__ void gi_prefill256r(const GiPrefillArgs& a) {
     }
 }
 
-extern "C" __global__ void __launch_bounds__(64 * PF_WAVES, 1) gi_prefill_fwd(GiPrefillArgs a) { gi_prefill_t<false>(a); }
-extern "C" __global__ void __launch_bounds__(64 * PF_WAVES, 1) gi_prefill_fwd_i8(GiPrefillArgs a) { gi_prefill_t<true>(a); }
-extern "C" __global__ void __launch_bounds__(64 * PF_WAVES, 1) gi_prefill_fwd_h64(GiPrefillArgs a) { gi_prefill_t<false, 64>(a); }
-extern "C" __global__ void __launch_bounds__(64 * PF_WAVES, 1) gi_prefill_fwd_h64_i8(GiPrefillArgs a) { gi_prefill_t<true, 64>(a); }
+// Kernels of head sizes 64 and 128 (_w4: 4 waves, 128 rows). The launch bound of 8 waves caps every form at 256
+// registers: past that the compiler keeps all MFMA accumulators in AGPRs and copies them to VGPRs for the softmax and
+// the rescale (96 to 270 copies per tile; the 4-wave form measured 702 us instead of 580 at 8192 tokens).
+#define GI_PREFILL_KERNEL(name, I8, HD, STG, WAVES, RING)                                                              \
+    extern "C" __global__ void __launch_bounds__(512) name(GiPrefillArgs a) { gi_prefill_t<I8, HD, STG, WAVES, RING>(a); }
+GI_PREFILL_KERNEL(gi_prefill_fwd, false, 128, false, 8, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_w4, false, 128, false, 4, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64, false, 64, false, 8, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64_w4, false, 64, false, 4, 4)
 // the int8 cache pre-widened by gi_kv_widen, staged as the f16 cache is
-extern "C" __global__ void __launch_bounds__(64 * PF_WAVES, 1) gi_prefill_fwd_i8s(GiPrefillArgs a) { gi_prefill_t<true, 128, true>(a); }
-extern "C" __global__ void __launch_bounds__(64 * PF_WAVES, 1) gi_prefill_fwd_h64_i8s(GiPrefillArgs a) { gi_prefill_t<true, 64, true>(a); }
+GI_PREFILL_KERNEL(gi_prefill_fwd_i8s, true, 128, true, 8, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_i8s_w4, true, 128, true, 4, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s, true, 64, true, 8, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s_w4, true, 64, true, 4, 4)
+// int8 tiles widened through registers (the chunks in flight leave room for a ring of 2; with 4 waves, twice the
+// chunks a thread, 36 registers spill and a tile takes twice as long)
+GI_PREFILL_KERNEL(gi_prefill_fwd_i8, true, 128, false, 8, 2)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8, true, 64, false, 8, 2)
+
 #ifndef PF256R_KBUF
 #define PF256R_KBUF 2 // K tile buffers of gi_prefill_fwd_h256r
 #endif

@@ -22,6 +22,8 @@ HSACO_PATH = os.path.join(HERE, "gi_attn_gfx950.hsaco")
 
 GI_F32 = 0
 GI_F16 = 1
+GI_PREFILL_WIDEN = 1
+GI_PREFILL_F32 = 2
 SPLIT_MAX_BATCH = 15  # src/cuda.rs:119
 TILED_MIN_BATCH = 16  # src/cuda.rs:95
 
@@ -42,6 +44,8 @@ SYMBOLS = (
     "gi_attn_prefill_q4",
     "gi_attn_prefill_workspace_bytes",
     "gi_attn_prefill_f32",
+    "gi_attn_prefill_scratch_bytes",
+    "gi_attn_prefill_ws",
     "gi_attn_prefill_i8_ws",
     "gi_attn_prefill_q4_ws",
     "gi_attention_q4",
@@ -106,6 +110,11 @@ def load_library(path=LIB_PATH):
     lib.gi_attn_prefill_f32.restype = i
     lib.gi_attn_prefill_workspace_bytes.argtypes = [i, i, i, i]
     lib.gi_attn_prefill_workspace_bytes.restype = sz
+    lib.gi_attn_prefill_scratch_bytes.argtypes = [i, i, i, i, i, i, i]
+    lib.gi_attn_prefill_scratch_bytes.restype = sz
+    lib.gi_attn_prefill_ws.argtypes = [vp, vp, i, ll, vp, vp, vp, vp, i, i, ll, ll, ll, ll, vp, i, ll, i, i, i, i, i, f,
+                                       vp, sz]
+    lib.gi_attn_prefill_ws.restype = i
     lib.gi_attn_prefill_i8_ws.argtypes = [vp, vp, i, ll, vp, vp, vp, vp, ll, ll, ll, ll, vp, i, ll, i, i, i, i, i, f,
                                           vp, sz]
     lib.gi_attn_prefill_i8_ws.restype = i
@@ -325,6 +334,24 @@ def prefill_workspace(kv_len, n_kv, hd, fmt, device):
     return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
 
 
+def _prefill_scratch(pos0, n, n_heads, n_kv, hd, fmt, flags, device):
+    """(scratch tensor or None, its bytes) of a prefill call: the widened keys and the partials of a sliced launch
+    (gi_attn_prefill_scratch_bytes). The tensor belongs to the current stream, where the call goes."""
+    if pos0 + n <= 960 and not flags & GI_PREFILL_WIDEN:  # fewer than 16 key tiles: never cut
+        return None, 0
+    nbytes = load_library().gi_attn_prefill_scratch_bytes(pos0, n, n_heads, n_kv, hd, fmt, flags)
+    return (torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None), nbytes
+
+
+def _prefill_ws(q, k_cache, v_cache, k_scale, v_scale, fmt, flags, strides, out, pos0, n, n_heads, n_kv, hd, scale):
+    """gi_attn_prefill_ws with a scratch of its own."""
+    scratch, nbytes = _prefill_scratch(pos0, n, n_heads, n_kv, hd, fmt, flags, q.device)
+    _check(load_library().gi_attn_prefill_ws(
+        _stream(), _ptr(q), GI_F16 if q.dtype == torch.float16 else GI_F32, q.stride(0), _ptr(k_cache), _ptr(v_cache),
+        _ptr(k_scale), _ptr(v_scale), fmt, flags, *strides, _ptr(out), GI_F16 if out.dtype == torch.float16 else GI_F32,
+        out.stride(0), pos0, n, n_heads, n_kv, hd, scale, _ptr(scratch), nbytes))
+
+
 def prefill_q4(q, k_cache, v_cache, k_scale, v_scale, pos0, n_heads, n_kv, scale=None, out=None, out_dtype=None,
                kv_layout="reference", staged=True, workspace=None):
     """Causal prefill over the 4-bit cache (head size 256; attention_prefill_tc256 with KV4, src/cuda.rs:2495-2514):
@@ -346,21 +373,17 @@ def prefill_q4(q, k_cache, v_cache, k_scale, v_scale, pos0, n_heads, n_kv, scale
     if out.dtype not in (torch.float32, torch.float16):
         raise GiAttnError("out must be float32 or float16")
     _need(out, "out", out.dtype)
-    qd = GI_F16 if q.dtype == torch.float16 else GI_F32
-    od = GI_F16 if out.dtype == torch.float16 else GI_F32
-    lib = load_library()
-    if staged and workspace is None:
-        workspace = prefill_workspace(pos0 + n, n_kv, 256, 2, q.device)
-    if staged:
+    if staged and workspace is not None:
         _need(workspace, "workspace", torch.uint8)
-        _check(lib.gi_attn_prefill_q4_ws(_stream(), _ptr(q), qd, q.stride(0), _ptr(k_cache), _ptr(v_cache),
-                                         _ptr(k_scale), _ptr(v_scale), kv_stride, kv_head_stride, sc_stride,
-                                         sc_head_stride, _ptr(out), od, out.stride(0), pos0, n, n_heads, n_kv, scale,
-                                         _ptr(workspace), workspace.numel()))
+        qd = GI_F16 if q.dtype == torch.float16 else GI_F32
+        od = GI_F16 if out.dtype == torch.float16 else GI_F32
+        _check(load_library().gi_attn_prefill_q4_ws(
+            _stream(), _ptr(q), qd, q.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(k_scale), _ptr(v_scale), kv_stride,
+            kv_head_stride, sc_stride, sc_head_stride, _ptr(out), od, out.stride(0), pos0, n, n_heads, n_kv, scale,
+            _ptr(workspace), workspace.numel()))
         return out
-    _check(lib.gi_attn_prefill_q4(_stream(), _ptr(q), qd, q.stride(0), _ptr(k_cache), _ptr(v_cache),
-                                  _ptr(k_scale), _ptr(v_scale), kv_stride, kv_head_stride, sc_stride,
-                                  sc_head_stride, _ptr(out), od, out.stride(0), pos0, n, n_heads, n_kv, scale))
+    _prefill_ws(q, k_cache, v_cache, k_scale, v_scale, 2, GI_PREFILL_WIDEN if staged else 0,
+                (kv_stride, kv_head_stride, sc_stride, sc_head_stride), out, pos0, n, n_heads, n_kv, 256, scale)
     return out
 
 
@@ -389,10 +412,12 @@ def attention_q4(qkv, k_cache, v_cache, k_scale, v_scale, pos0, n_heads, n_kv, e
             workspace = new_workspace(cap, min(n, SPLIT_MAX_BATCH), n_heads, n_kv, 256, qkv.device)
         ws_ptr, ws_bytes = _ptr(workspace), workspace.numel() * workspace.element_size()
     else:
-        # a prefill batch: the pre-widened staging, whose workspace the library checks
+        # a prefill batch: the pre-widened staging, whose workspace the library checks, and the sliced launches
         if workspace is None:
-            workspace = prefill_workspace(pos0 + n, n_kv, 256, 2, qkv.device)
-        ws_ptr, ws_bytes = _ptr(workspace), workspace.numel() * workspace.element_size()
+            workspace, ws_bytes = _prefill_scratch(pos0, n, n_heads, n_kv, 256, 2, GI_PREFILL_WIDEN, qkv.device)
+        else:
+            ws_bytes = workspace.numel() * workspace.element_size()
+        ws_ptr = _ptr(workspace)
     _check(load_library().gi_attention_q4(_stream(), _ptr(qkv), _ptr(k_cache), _ptr(v_cache), _ptr(k_scale),
                                           _ptr(v_scale), _ptr(out), ws_ptr, ws_bytes, pos0, _ptr(posp), ctx_cap, n,
                                           n_heads, n_kv, 1 if exact else 0))
@@ -437,29 +462,19 @@ def prefill(q, k_cache, v_cache, pos0, n_heads, n_kv, hd=128, scale=None, out=No
     if out.dtype not in (torch.float32, torch.float16):
         raise GiAttnError("out must be float32 or float16")
     _need(out, "out", out.dtype)
-    lib = load_library()
-    qd = GI_F16 if q.dtype == torch.float16 else GI_F32
-    od = GI_F16 if out.dtype == torch.float16 else GI_F32
-    if f32:
-        _check(lib.gi_attn_prefill_f32(_stream(), _ptr(q), qd, q.stride(0), _ptr(k_cache), _ptr(v_cache),
-                                       _ptr(k_scale) if i8 else None, _ptr(v_scale) if i8 else None, 1 if i8 else 0,
-                                       kv_stride, kv_head_stride, sc[0] if i8 else 0, sc[1] if i8 else 0, _ptr(out), od,
-                                       out.stride(0), pos0, n, n_heads, n_kv, hd, scale))
-    elif i8 and staged and hd in (64, 128, 256):
-        if workspace is None:
-            workspace = prefill_workspace(pos0 + n, n_kv, hd, 1, q.device)
+    widen = i8 and staged and hd in (64, 128, 256) and not f32
+    if widen and workspace is not None:
         _need(workspace, "workspace", torch.uint8)
-        _check(lib.gi_attn_prefill_i8_ws(_stream(), _ptr(q), qd, q.stride(0), _ptr(k_cache), _ptr(v_cache),
-                                         _ptr(k_scale), _ptr(v_scale), kv_stride, kv_head_stride, sc[0], sc[1],
-                                         _ptr(out), od, out.stride(0), pos0, n, n_heads, n_kv, hd, scale,
-                                         _ptr(workspace), workspace.numel()))
-    elif i8:
-        _check(lib.gi_attn_prefill_i8(_stream(), _ptr(q), qd, q.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(k_scale),
-                                      _ptr(v_scale), kv_stride, kv_head_stride, sc[0], sc[1], _ptr(out), od,
-                                      out.stride(0), pos0, n, n_heads, n_kv, hd, scale))
-    else:
-        _check(lib.gi_attn_prefill(_stream(), _ptr(q), qd, q.stride(0), _ptr(k_cache), _ptr(v_cache), kv_stride,
-                                   kv_head_stride, _ptr(out), od, out.stride(0), pos0, n, n_heads, n_kv, hd, scale))
+        qd = GI_F16 if q.dtype == torch.float16 else GI_F32
+        od = GI_F16 if out.dtype == torch.float16 else GI_F32
+        _check(load_library().gi_attn_prefill_i8_ws(
+            _stream(), _ptr(q), qd, q.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(k_scale), _ptr(v_scale), kv_stride,
+            kv_head_stride, sc[0], sc[1], _ptr(out), od, out.stride(0), pos0, n, n_heads, n_kv, hd, scale,
+            _ptr(workspace), workspace.numel()))
+        return out
+    _prefill_ws(q, k_cache, v_cache, k_scale if i8 else None, v_scale if i8 else None, 1 if i8 else 0,
+                (GI_PREFILL_WIDEN if widen else 0) | (GI_PREFILL_F32 if f32 else 0),
+                (kv_stride, kv_head_stride, *(sc if i8 else (0, 0))), out, pos0, n, n_heads, n_kv, hd, scale)
     return out
 
 
@@ -499,12 +514,13 @@ def attention(qkv, k_cache, v_cache, pos0, n_heads, n_kv, hd=128, exact=False, o
             cap = ctx_cap if posp is not None else pos0 + n
             workspace = new_workspace(cap, min(n, SPLIT_MAX_BATCH), n_heads, n_kv, hd, qkv.device)
         ws_ptr, ws_bytes = _ptr(workspace), workspace.numel() * workspace.element_size()
-    elif i8 and not no_tc:
+    elif i8 and not no_tc and workspace is not None:
         # a prefill batch over the int8 cache: the pre-widened staging, whose workspace the library checks
-        if workspace is None:
-            workspace = prefill_workspace(pos0 + n, n_kv, hd, 1, qkv.device)
-        if workspace is not None:
-            ws_ptr, ws_bytes = _ptr(workspace), workspace.numel() * workspace.element_size()
+        ws_ptr, ws_bytes = _ptr(workspace), workspace.numel() * workspace.element_size()
+    else:
+        flags = (GI_PREFILL_WIDEN if i8 else 0) if not no_tc else GI_PREFILL_F32
+        scratch, ws_bytes = _prefill_scratch(pos0, n, n_heads, n_kv, hd, 1 if i8 else 0, flags, qkv.device)
+        ws_ptr = _ptr(scratch)
     lib = load_library()
     if i8:
         _check(lib.gi_attention_i8(_stream(), _ptr(qkv), _ptr(k_cache), _ptr(v_cache), _ptr(k_scale), _ptr(v_scale),
@@ -621,7 +637,8 @@ def kernel_timing(on):
 
 def kernel_timing_read(kernel):
     """(total milliseconds, launches) of kernel kind "decode_partial", "decode_combine", "prefill",
-    "qk_norm_rope", "kv_relayout", "hadamard_rows" or "kv_widen" since the previous read of that kind."""
+    "prefill_combine", "qk_norm_rope", "kv_relayout", "hadamard_rows" or "kv_widen" since the previous read of that
+    kind."""
     ms, n = ctypes.c_double(), ctypes.c_int()
     _check(load_library().gi_kernel_timing_read(kernel.encode(), ctypes.byref(ms), ctypes.byref(n)))
     return ms.value, n.value

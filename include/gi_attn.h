@@ -189,6 +189,25 @@ int gi_attn_prefill_q4_ws(void* stream, const void* q, int q_dtype, long long q_
                           int out_dtype, long long out_stride, int pos0, int n, int n_heads, int n_kv, float scale,
                           void* workspace, size_t workspace_bytes);
 
+/* flags of gi_attn_prefill_ws */
+#define GI_PREFILL_WIDEN 1 /* int8 and 4-bit caches: widen the keys into the workspace first (gi_attn_prefill_i8_ws) */
+#define GI_PREFILL_F32 2   /* in f32, as gi_attn_prefill_f32 */
+
+/* Every causal prefill above in one entry point (fmt 0: f16 cache, 1: int8, 2: 4-bit; ks / vs and the scale strides
+ * as the entry points of that cache), with a scratch workspace. The workspace (16-byte aligned; 256-byte with
+ * GI_PREFILL_WIDEN) takes the widened keys and the partial results of a sliced launch: a batch too short to fill the
+ * chip over a long prefix is cut along its keys too (one workgroup per slice, merged by a second launch; rows then
+ * differ from the one-slice results by f32 rounding). gi_attn_prefill_scratch_bytes says how much a call can use; it
+ * is optional, and with a smaller one (or none) the call does without. The workspace needs no initialisation; calls that
+ * share one must be ordered. Prompts of up to 4096 keys taken in chunks of 256 tokens or more, and spans below 16
+ * tiles of 64 keys, are never cut. */
+size_t gi_attn_prefill_scratch_bytes(int pos0, int n, int n_heads, int n_kv, int hd, int fmt, int flags);
+int gi_attn_prefill_ws(void* stream, const void* q, int q_dtype, long long q_stride, const void* kc, const void* vc,
+                       const void* ks, const void* vs, int fmt, int flags, long long kv_stride, long long kv_head_stride,
+                       long long sc_stride, long long sc_head_stride, void* out, int out_dtype, long long out_stride,
+                       int pos0, int n, int n_heads, int n_kv, int hd, float scale, void* workspace,
+                       size_t workspace_bytes);
+
 /* The attention operator of one layer, as GpuModel::attention (src/cuda.rs:8448-8541) dispatches it:
  * qkv rows are [q (n_heads*hd) | k | v] f32 (stride n_heads*hd + 2*n_kv*hd, src/cuda.rs:1713), out rows
  * n_heads*hd f32. Batches of >= 16 tokens go to prefill; the rest, and every batch with bit 0 of `exact` set (a
@@ -196,7 +215,8 @@ int gi_attn_prefill_q4_ws(void* stream, const void* q, int q_dtype, long long q_
  * (SPLIT_MAX_BATCH, src/cuda.rs:119). Bit 1 of `exact` is the reference's GHOST_INFER_NO_TC_ATT
  * (src/cuda.rs:5648-5655): prefill batches take the f32 prefill (gi_attn_prefill_f32) at head sizes up to 128 over
  * the f16 and int8 caches and the split path elsewhere, and at head size 256 over the int8 cache the split path
- * computes in f32 precision instead of attention_decode_tc256's roundings. fixed_split
+ * computes in f32 precision instead of attention_decode_tc256's roundings. A prefill batch uses the workspace as
+ * gi_attn_prefill_ws does, where it is large enough. fixed_split
  * with posp: the grid is sized for ctx_cap (the session capacity), as max_splits does. scale is
  * 1/sqrt(hd) as in the reference. */
 int gi_attention(void* stream, const float* qkv, const uint16_t* kc, const uint16_t* vc, float* out,
@@ -273,7 +293,7 @@ int gi_kv_relayout(void* stream, const void* src, long long src_stride, long lon
 int gi_kernel_timing(int on);
 
 /* Total milliseconds and launch count of kernel kind `kernel` ("decode_partial", "decode_combine",
- * "prefill", "qk_norm_rope", "kv_relayout" or "hadamard_rows") recorded since the previous read of that kind; waits for the recorded events and
+ * "prefill", "prefill_combine", "qk_norm_rope", "kv_widen", "kv_relayout" or "hadamard_rows") recorded since the previous read of that kind; waits for the recorded events and
  * releases them. */
 int gi_kernel_timing_read(const char* kernel, double* total_ms, int* launches);
 

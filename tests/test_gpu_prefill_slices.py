@@ -1,0 +1,98 @@
+"""Prefill launches cut along their keys (gi_attn_prefill_ws, the partials merged by gi_prefill_combine_*) and the packed
+row tiles they share: short batches over long prefixes, against float64, and against the launch without a workspace, which
+is never cut. Sizes at the edges: 16 and 17 key tiles, a last slice that only part of the rows sees, rows that end inside
+a wave, inside a row tile and at its end, groups that do not divide a wave."""
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+import gi_attn
+from attn_common import assert_close, make_inputs, make_inputs_i8, reference_f64, reference_f64_i8
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # (n, pos0, n_heads, n_kv, hd)
+    (16, 16 * 64 - 16, 4, 4, 128),    # 16 tiles, one row per token and head
+    (17, 16 * 64 - 16, 8, 1, 128),    # 17 tiles, the last one seen by the last token only
+    (43, 2000, 6, 1, 128),            # G 6: 258 rows, two rows past a tile of 256
+    (64, 4033, 8, 1, 128),
+    (200, 3000, 32, 8, 128),
+    (255, 1500, 9, 3, 64),
+    (31, 9000, 9, 3, 64),
+    (300, 5000, 16, 4, 128),          # over 4096 keys, 256 tokens or more
+    (300, 5000, 8, 8, 64),
+]
+
+
+def dev(x, gpu, *shape):
+    return torch.from_numpy(np.ascontiguousarray(x)).to(gpu).view(*shape)
+
+
+def sliced(n, pos0, n_heads, n_kv, hd, fmt):
+    return gi_attn.load_library().gi_attn_prefill_scratch_bytes(pos0, n, n_heads, n_kv, hd, fmt, 0) > 0
+
+
+@pytest.mark.parametrize("n,pos0,n_heads,n_kv,hd", SHAPES)
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.float16])
+def test_sliced_prefill_f16(gpu, n, pos0, n_heads, n_kv, hd, out_dtype):
+    print("[case] sliced prefill f16", n, pos0, n_heads, n_kv, hd, out_dtype, flush=True)
+    assert sliced(n, pos0, n_heads, n_kv, hd, 0)
+    q, k, v = make_inputs(9100 + n + hd, n, pos0 + n, n_heads, n_kv, hd=hd)
+    qt = dev(q, gpu, n, n_heads * hd)
+    kt, vt = (dev(x.view(np.int16), gpu, -1, n_kv, hd).view(torch.float16) for x in (k, v))
+    got = gi_attn.prefill(qt, kt, vt, pos0, n_heads, n_kv, hd=hd, out_dtype=out_dtype)
+    whole = torch.empty_like(got)
+    code = gi_attn.GI_F16 if out_dtype == torch.float16 else gi_attn.GI_F32
+    gi_attn._check(gi_attn.load_library().gi_attn_prefill(
+        gi_attn._stream(), qt.data_ptr(), gi_attn.GI_F32, n_heads * hd, kt.data_ptr(), vt.data_ptr(), n_kv * hd, hd,
+        whole.data_ptr(), code, n_heads * hd, pos0, n, n_heads, n_kv, hd, hd ** -0.5))
+    torch.cuda.synchronize()
+    # both round Q and P to f16 and differ in P's reference max per slice: within the bar of each from float64
+    rows = sorted({0, 1, n // 2, n - 2, n - 1})
+    for r in rows:
+        want = reference_f64(q[r:r + 1], k, v, pos0 + r, n_heads, n_kv, hd=hd)
+        assert_close(got[r:r + 1].float().cpu().numpy(), want, what=f"sliced row {r}")
+    assert_close(got.float().cpu().numpy(), whole.float().cpu().numpy(), what="sliced against whole")
+
+
+@pytest.mark.parametrize("n,pos0,n_heads,n_kv,hd", SHAPES)
+def test_sliced_prefill_i8_same_for_both_stagings(gpu, n, pos0, n_heads, n_kv, hd):
+    print("[case] sliced prefill i8", n, pos0, n_heads, n_kv, hd, flush=True)
+    assert sliced(n, pos0, n_heads, n_kv, hd, 1)
+    q, k, v, ks, vs = make_inputs_i8(9200 + n + hd, n, pos0 + n, n_heads, n_kv, hd=hd)
+    qt = dev(q, gpu, n, n_heads * hd)
+    kt, vt = (dev(x, gpu, -1, n_kv, hd) for x in (k, v))
+    kst, vst = (dev(x, gpu, -1, n_kv) for x in (ks, vs))
+    kw = dict(hd=hd, out_dtype=torch.float32, k_scale=kst, v_scale=vst)
+    got = gi_attn.prefill(qt, kt, vt, pos0, n_heads, n_kv, staged=True, **kw)
+    tile = gi_attn.prefill(qt, kt, vt, pos0, n_heads, n_kv, staged=False, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(got, tile)
+    for r in sorted({0, 1, n // 2, n - 1}):
+        want = reference_f64_i8(q[r:r + 1], k, v, ks, vs, pos0 + r, n_heads, n_kv, hd=hd)
+        assert_close(got[r:r + 1].cpu().numpy(), want, what=f"sliced i8 row {r}")
+
+
+def test_sliced_prefill_graph_replay(gpu):
+    # the sliced launch and its merge captured together, replayed with new queries and eager work between the replays
+    n, pos0, n_heads, n_kv = 40, 3000, 8, 2
+    _, k, v = make_inputs(9300, 1, pos0 + n, n_heads, n_kv)
+    kt, vt = (dev(x.view(np.int16), gpu, -1, n_kv, 128).view(torch.float16) for x in (k, v))
+    q = torch.randn((n, n_heads * 128), device=gpu)
+    out = torch.empty_like(q)
+    gi_attn.prefill(q, kt, vt, pos0, n_heads, n_kv, out=out)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        gi_attn.prefill(q, kt, vt, pos0, n_heads, n_kv, out=out)
+    for r in range(3):
+        q.copy_(torch.randn_like(q))
+        want = gi_attn.prefill(q, kt, vt, pos0, n_heads, n_kv)
+        torch.cuda.synchronize()
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), f"replay {r}"
