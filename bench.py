@@ -616,7 +616,7 @@ def run_prefill(torch, gi_attn, dev, w, steps, warmup):
     r = prefill_workload(torch, gi_attn, dev, 8192, nh, nkv, steps, warmup, 99, i8=i8, hd=hd, f32=f32)
     tf = r["flops"] / r["seconds"] / 1e12
     # (the int8 cache: the kernels staging the pre-widened keys, *_i8s; the 4-bit cache widened runs the f16 kernel)
-    kernel = ("gi_prefill_fwd_h256r" + ("_i8s" if i8 is True else "") if hd == 256
+    kernel = ("gi_prefill_fwd_h256" + ("_i8s" if i8 is True else "") if hd == 256
               else "gi_prefill_fwd_h64" + ("_i8s" if i8 else "") if hd == 64
               else "gi_prefill_f32" + ("_i8" if i8 else "") + f"_h{hd}" if hd not in (64, 128)
               else "gi_prefill_f32_h128" if f32

@@ -177,7 +177,6 @@ constexpr int kPrefillRows = 256; // packed query rows per workgroup of 8 waves 
 constexpr int kPrefillKeys = 64;  // keys per prefill tile; must match the kernels' PF_BK
 constexpr int kPrefillMaxSlices = 64; // must match the kernels' PFC_MAXS
 constexpr int kPrefillMergeFrags = 4; // must match the kernels' PFC_FRAGS
-constexpr int kPrefill256rRows = 128; // the same for gi_prefill_fwd_h256r (PF256R_BQ)
 
 thread_local std::string g_err;
 
@@ -213,18 +212,15 @@ struct Module {
                                       // one column block, 4-bit one and two column blocks
     hipFunction_t dec_pm256[2] = {};  // head size 256, one pair per column, two pair sets of two waves: [f16, int8]
     hipFunction_t dec_i8_256f[2] = {}; // head size 256 over the int8 cache in f32 precision: [up to 8 pairs, above]
-    // head sizes 128 and 64: [head size 64][f16 cache, pre-widened int8, int8 widened tile by tile][8 waves, 4 waves]
-    hipFunction_t prefill[2][3][2] = {};
+    // [head size 128, 64, 256][f16 cache, pre-widened int8, int8 or 4-bit widened tile by tile][8 waves, 4 waves; head
+    // size 256: 4, 2] (the pre-widened 4-bit cache runs the f16 kernel; head size 256 tile by tile in prefill256)
+    hipFunction_t prefill[3][3][2] = {};
+    hipFunction_t prefill256[2] = {}; // head size 256 tile by tile: int8, 4-bit
     hipFunction_t dec_f32[2][6] = {}, prefill_f32[2][6] = {}; // the f32 kernels: [int8 cache][kF32Sizes index]
     hipFunction_t prefill_f32p[2][2] = {}; // f32 prompts at head sizes 64 and 128: [int8 cache][64, 128]
-    hipFunction_t prefill256r = nullptr; // head size 256 (f16 cache), 16 rows per wave: one workgroup per query tile
-    hipFunction_t prefill256r_fmt[2] = {}; // the same over the int8 and the 4-bit cache
-    // pre-widened staging: gi_kv_widen, then the int8 kernels that stage the widened tiles by LDS-DMA (head size 256
-    // here; the widened 4-bit cache runs prefill256r)
-    hipFunction_t widen = nullptr, prefill256r_i8s = nullptr;
+    hipFunction_t widen = nullptr; // the int8 and 4-bit keys widened into a workspace
     hipFunction_t prefill_combine[2] = {}; // merge of a sliced prefill's partials: 32 rows per wave
     hipFunction_t combine = nullptr, rope = nullptr, relayout = nullptr, hadamard = nullptr;
-    int prefill256r_threads = 0;
     // gi_attn_decode_noalloc's partials: the device address of the code object's gi_scratch array on this
     // device (the array's host-side name is no device address; the module gives the real one at load)
     void* scratch = nullptr;
@@ -297,11 +293,13 @@ int load_module(const char* path, Module** out) {
             {&m.prefill[1][1][0], "gi_prefill_fwd_h64_i8s"},
             {&m.prefill[1][1][1], "gi_prefill_fwd_h64_i8s_w4"},
             {&m.prefill[1][2][0], "gi_prefill_fwd_h64_i8"},
-            {&m.prefill256r, "gi_prefill_fwd_h256r"},
-            {&m.prefill256r_fmt[0], "gi_prefill_fwd_h256r_i8"},
-            {&m.prefill256r_fmt[1], "gi_prefill_fwd_h256r_q4"},
+            {&m.prefill[2][0][0], "gi_prefill_fwd_h256"},
+            {&m.prefill[2][0][1], "gi_prefill_fwd_h256_w2"},
+            {&m.prefill[2][1][0], "gi_prefill_fwd_h256_i8s"},
+            {&m.prefill[2][1][1], "gi_prefill_fwd_h256_i8s_w2"},
+            {&m.prefill256[0], "gi_prefill_fwd_h256_i8"},
+            {&m.prefill256[1], "gi_prefill_fwd_h256_q4"},
             {&m.widen, "gi_kv_widen"},
-            {&m.prefill256r_i8s, "gi_prefill_fwd_h256r_i8s"},
             {&m.prefill_combine[0], "gi_prefill_combine_32"},
             {&m.rope, "gi_qk_norm_rope"},
         };
@@ -328,13 +326,6 @@ int load_module(const char* path, Module** out) {
                     return e;
                 }
             }
-        if (int e = check(hipFuncGetAttribute(&m.prefill256r_threads, HIP_FUNC_ATTRIBUTE_MAX_THREADS_PER_BLOCK,
-                                              m.prefill256r),
-                          "hipFuncGetAttribute(gi_prefill_fwd_h256r)")) {
-            (void)hipModuleUnload(m.mod);
-            m.mod = nullptr;
-            return e;
-        }
         hipDeviceptr_t sp = nullptr;
         if (int e = check(hipModuleGetGlobal(&sp, &m.scratch_bytes, m.mod, "gi_scratch"), "hipModuleGetGlobal(gi_scratch)")) {
             (void)hipModuleUnload(m.mod);
@@ -693,18 +684,18 @@ size_t prefill_ws_bytes(int kv_len, int n_kv, int hd, int fmt) {
     return 2 * rows + 2 * scales;
 }
 
-// How a prefill launch at head size 64 or 128 is laid out. It has one workgroup per (kv head, tile of packed query
+// How an MFMA prefill launch is laid out. It has one workgroup per (kv head, tile of packed query
 // rows), and a CU holds one workgroup.
 //  - Waves: 8 (256 rows, two waves per SIMD) or 4 (128 rows, one per SIMD). One wave takes a key tile in about 0.7 of
 //    the time that two on its SIMD take for theirs together, so 4 waves win where the workgroups are few or unequal
 //    (1024 tokens of 32/8 heads of 128, f16: 33.9 us with 8, 23.7 with 4; 512 at a 2000-token prefix 64 and 44) and
-//    8 where they fill the chip several times over (8192 tokens: 505 and 580).
+//    8 where they fill the chip several times over (8192 tokens: 505 and 580). Head size 256: 4 or 2.
 //  - Slices: a short batch over a long prefix leaves most of the chip idle while each workgroup walks all of its keys
 //    (512 tokens of 32/4 heads at a 16K prefix: 64 workgroups of 264 key tiles, 350 us). Such a launch cuts the key
 //    tiles of every row tile into slices, one workgroup each, whose partial results a second launch merges (137 us).
 // A row's arithmetic does not depend on the waves, only on the slices.
 struct PrefillPlan {
-    int waves;      // 8 or 4
+    int waves;      // 8 or 4; head size 256: 4 or 2
     int tiles;      // key tiles per slice
     int nslice;     // slices of the longest row tile
 };
@@ -712,21 +703,22 @@ constexpr int kPrefillRowTiles(long long rows, int per) { return (int)((rows + p
 PrefillPlan prefill_plan(int pos0, int n, int n_heads, int n_kv, int hd) {
     const int G = n_heads / n_kv, cus = 256, tmax = (pos0 + n + kPrefillKeys - 1) / kPrefillKeys;
     const long long P = (long long)n * G;
-    PrefillPlan p{8, tmax, 1};
-    if ((long long)kPrefillRowTiles(P, kPrefillRows) * n_kv >= 2 * cus) return p; // longest tiles first balances these
+    const int most = hd == 256 ? 4 : 8;
+    PrefillPlan p{most, tmax, 1};
+    if ((long long)kPrefillRowTiles(P, 32 * most) * n_kv >= 2 * cus) return p; // longest tiles first balances these
     // Below 16 key tiles slices save less than the merge launch costs. A prompt of up to 4096 keys taken in chunks of
     // 256 tokens or more keeps each row's arithmetic independent of the chunking (one slice always); beyond, chunks
     // agree to f32 rounding.
     const bool may_slice = tmax >= 16 && (n < 256 || pos0 + n > 4096);
-    // Costs in units of one key tile of an 8-wave workgroup (1.4 to 1.9 us): rounds of workgroups over the CUs, each
+    // Costs in units of one key tile of an 8-wave workgroup (1.4 to 1.9 us; head size 256: of a 4-wave one): rounds of workgroups over the CUs, each
     // with a fixed cost until its first tile is in and for its output (~6 us), and for a sliced launch the merge
     // launch (~5 us) and its read of the partials (~4 TB/s).
     const double per_wg = 4.0, merge = 3.3;
     double best = 0;
-    for (int waves = 8; waves >= 4; waves -= 4) {
+    for (int waves = most; waves >= most / 2; waves -= most / 2) {
         const int rows = 32 * waves, items = kPrefillRowTiles(P, rows);
         const long long wgs = (long long)items * n_kv;
-        const double tile = waves == 8 ? 1.0 : 0.7;
+        const double tile = waves == most ? 1.0 : hd == 256 ? 0.85 : 0.7;
         auto tiles_of = [&](int i) { // key tiles of row tile i
             const long long last = std::min<long long>(n - 1, ((long long)(i + 1) * rows - 1) / G);
             return (int)((pos0 + last) / kPrefillKeys + 1);
@@ -734,7 +726,7 @@ PrefillPlan prefill_plan(int pos0, int n, int n_heads, int n_kv, int hd) {
         // one slice: the longest workgroup, or the mean load of a CU where there are several rounds
         const double mean = (double)wgs / cus * (tile * (tiles_of(0) + tmax) / 2 + (wgs > cus ? per_wg : 0));
         const double one = std::max(tile * tmax, mean) + per_wg;
-        if (waves == 8 || one < 0.95 * best) best = one, p = PrefillPlan{waves, tmax, 1};
+        if (waves == most || one < 0.95 * best) best = one, p = PrefillPlan{waves, tmax, 1};
         if (!may_slice) continue;
         const double part = std::min<long long>(P, rows) * (hd + 2) * 4.0 / 4e12 / 1.5e-6;
         for (int S = 2; S <= std::min(kPrefillMaxSlices, tmax / 2) && wgs * S <= 4 * cus; S++) {
@@ -831,11 +823,10 @@ int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, c
     a.nslice = 1;
     const int G = n_heads / n_kv;
     a.gmul = (long long)n * G * G < 1ll << 31 ? (uint32_t)(((1ll << 31) + G - 1) / G) : 0;
-    // the launch of a prefill kernel of head size 64 or 128 over staging `st` (Module::prefill), sliced where the plan
-    // says so and the rest of the workspace holds the partials; then their merge
+    // the launch of an MFMA prefill kernel over staging `st` (Module::prefill), sliced where the plan says so and the rest of the workspace holds the partials; then their merge
     auto run = [&](int st, unsigned char* free, size_t left) {
         const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd);
-        const int waves = st == 2 ? 8 : p.waves; // (tile by tile: 8 waves only)
+        const int waves = st == 2 ? (hd == 256 ? 4 : 8) : p.waves; // (tile by tile: the larger form only)
         const size_t need = prefill_part_bytes(p, n, n_heads, n_kv, hd, 32 * waves);
         a.rows = 32 * waves;
         a.items = kPrefillRowTiles((long long)n * G, a.rows);
@@ -845,7 +836,8 @@ int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, c
             a.nslice = p.nslice;
             a.slice_tiles = p.tiles;
         }
-        if (int e = launch(kPrefill, m->prefill[hd == 64][st][waves == 4], dim3((unsigned)(a.items * n_kv * a.nslice), 1, 1),
+        const hipFunction_t f = st == 2 && hd == 256 ? m->prefill256[fmt - 1] : m->prefill[hd == 64 ? 1 : hd == 256 ? 2 : 0][st][waves == (hd == 256 ? 2 : 4)];
+        if (int e = launch(kPrefill, f, dim3((unsigned)(a.items * n_kv * a.nslice), 1, 1),
                            dim3(64 * waves), (hipStream_t)stream, &a, sizeof a))
             return e;
         if (a.nslice == 1) return 0;
@@ -896,19 +888,12 @@ int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, c
         a.vs = wa.vsw;
         a.sc_stride = 1;
         a.sc_head_stride = len;
-        if (hd == 256)
-            return launch(kPrefill, fmt == 2 ? m->prefill256r : m->prefill256r_i8s,
-                          dim3((n + kPrefill256rRows - 1) / kPrefill256rRows * n_heads, 1, 1), dim3(m->prefill256r_threads),
-                          (hipStream_t)stream, &a, sizeof a);
-        return run(1, ws + need, workspace_bytes - need);
+        return run(fmt == 2 ? 0 : 1, ws + need, workspace_bytes - need);
     }
     if (f32_hd(hd)) // one workgroup per (head, 128 query rows)
         return launch(kPrefill, m->prefill_f32[i8][f32_index(hd)], dim3((n + kF32Rows - 1) / kF32Rows * n_heads, 1, 1),
                       dim3(kF32Threads), (hipStream_t)stream, &a, sizeof a);
-    if (hd == 256) // one workgroup per (head, 128 query rows), 16 rows per wave
-        return launch(kPrefill, fmt ? m->prefill256r_fmt[fmt - 1] : m->prefill256r, dim3((n + kPrefill256rRows - 1) / kPrefill256rRows * n_heads, 1, 1),
-                      dim3(m->prefill256r_threads), (hipStream_t)stream, &a, sizeof a);
-    return run(i8 ? 2 : 0, ws, workspace_bytes);
+    return run(fmt ? 2 : 0, ws, workspace_bytes);
 }
 
 int attention_impl(void* stream, const float* qkv, const void* kc, const void* vc, const float* ks, const float* vs,
@@ -1048,9 +1033,8 @@ size_t gi_attn_prefill_scratch_bytes(int pos0, int n, int n_heads, int n_kv, int
     if ((flags & GI_PREFILL_F32) || f32_hd(hd)) return 0;
     const bool widens = fmt && (flags & GI_PREFILL_WIDEN) && prefill_widens(n, n_heads, n_kv, hd);
     const size_t widened = widens ? prefill_ws_bytes(pos0 + n, n_kv, hd, fmt) : 0;
-    if (hd == 256) return widened;
     const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd);
-    return widened + prefill_part_bytes(p, n, n_heads, n_kv, hd, fmt && !widens ? kPrefillRows : 32 * p.waves);
+    return widened + prefill_part_bytes(p, n, n_heads, n_kv, hd, fmt && !widens ? (hd == 256 ? 128 : kPrefillRows) : 32 * p.waves);
 }
 
 int gi_attn_prefill_ws(void* stream, const void* q, int q_dtype, long long q_stride, const void* kc, const void* vc,

@@ -1451,16 +1451,16 @@ __device__ __forceinline__ int pf_token(const GiPrefillArgs& a, int row) {
 __device__ __forceinline__ int pf_last_token(const GiPrefillArgs& a, int row0, int rows) {
     return min(a.n - 1, pf_token(a, row0 + rows - 1)); // the last token with a row in the tile
 }
-// Workgroup j of the grid (kv head, slice, row tile). Blocks go to the 8 XCDs round-robin; the remap gives each XCD
-// a contiguous run of the order, so that one kv head's K/V (one slice's, in a sliced launch) stays in one XCD's L2.
-// Longest row tiles first.
+// Workgroup j of the grid takes run j % runs (kv head and slice: the workgroups that read the same keys) and the row tiles
+// of all runs longest first. Blocks go to the 8 XCDs round-robin, so with 8 runs (or a divisor or multiple) each run stays
+// in the L2 of its own XCDs and every XCD gets row tiles of every length. (Giving each XCD a contiguous stretch of the
+// (kv head, row tile) order keeps the locality too, but with fewer than 8 kv heads one XCD then gets a kv head's longest
+// tiles and another its shortest: 8192 tokens of 16/2 heads of 256 took 880 us with half of the CUs idle, 32/4 heads
+// of 128 604 us against 505 for 32/8.)
 __device__ __forceinline__ PfUnit pf_unit(const GiPrefillArgs& a, int BQ, int BK) {
-    const int items = a.items;
-    const int nwg = gridDim.x;
-    int j = blockIdx.x;
-    if ((nwg & 7) == 0) j = (j & 7) * (nwg >> 3) + (j >> 3);
-    const int run = j / items; // kv head * nslice + slice
-    const int item = items - 1 - (j - run * items);
+    const int items = a.items, runs = a.n_kv * a.nslice;
+    const int lot = (int)blockIdx.x / runs, run = (int)blockIdx.x - lot * runs; // run: kv head * nslice + slice
+    const int item = items - 1 - lot;
     const int kvh = a.nslice == 1 ? run : run / a.nslice, slice = run - kvh * a.nslice;
     const int k_lim = a.pos0 + pf_last_token(a, item * BQ, BQ) + 1; // keys any row of the tile may see
     const int ntiles = (k_lim + BK - 1) / BK;
@@ -1650,22 +1650,33 @@ template <int N, int I = 0, typename F> __device__ __forceinline__ void gi_unrol
 // HD = 64 (attn_prefill_tc<64>, src/cuda.rs:2620): the same kernel with half the QK k-steps and O^T blocks. The
 // LDS image keeps the head-128 layout: each 128-byte row sits in a 256-byte slot, its 8 units at the swizzled
 // positions the operand reads compute (the staging loads of the other 8 positions are out of bounds and leave zeros).
-template <bool I8, int HD, bool STG, int WAVES, int RING>
+template <int FMT, int HD, bool STG, int WAVES, int RING, int VRING = RING>
 __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
-    static_assert(HD == 64 || HD == 128, "head sizes 64, 128 (256: gi_prefill256r)");
-    static_assert(!STG || I8, "pre-widened staging: the int8 cache");
-    constexpr bool RSTG = I8 && !STG; // int8 tiles widened through registers, else LDS-DMA
+    static_assert(HD == 64 || HD == 128 || HD == 256, "head sizes 64, 128, 256");
+    static_assert(!STG || FMT == 1, "pre-widened staging: the int8 cache (the 4-bit one widens to the f16 kernel's input)");
+    static_assert(FMT != 2 || HD == 256, "the 4-bit cache: head size 256");
+    constexpr bool I8 = FMT == 1;
+    constexpr bool RSTG = FMT != 0 && !STG; // int8 and 4-bit tiles widened through registers, else LDS-DMA
+    constexpr bool WIDE = HD == 256;
+    constexpr int IMG = WIDE ? 2 : 1;       // 16 KB images of a K or V tile (128 dims each)
+    constexpr int NKB = WIDE ? 2 : 4, NVB = NKB; // K and V tile buffers
+    constexpr float VB = WIDE ? 1024.f : PF_I8_VBIAS; // int8: the probabilities' bias
     constexpr int BQ = 32 * WAVES;  // query rows per workgroup
     constexpr int SW = WAVES / 2;   // waves staging each of K and V
-    constexpr int LPW = 16 / SW;    // 1 KB loads per staging wave and tile
+    constexpr int LPW = 16 * IMG / SW; // 1 KB loads per staging wave and tile
     constexpr int LPT = LPW + (STG ? 1 : 0); // loads per staging wave and tile (STG: plus its share of the scales)
     constexpr int BK = PF_BK;       // keys per tile
     constexpr int NBLK = BK / 32;   // S^T blocks of 32 keys
     constexpr int KS = HD / 16;     // QK k-steps
     constexpr int NDB = HD / 32;    // O^T blocks of 32 dims
     constexpr int NQ = 2 * KS, NP = 4 * NDB, NS = NQ + NP; // MFMAs of QK and of P V, slots of an iteration
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[PF_NBUF][2][PF_TILE]; // [buffer][K, V]
-    __shared__ __attribute__((aligned(256))) float scl[I8 ? PF_NBUF : 1][2][BK];        // int8: [buffer][K, V] scales
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[(NKB + NVB) * IMG * PF_TILE]; // K buffers, V buffers
+    __shared__ __attribute__((aligned(256))) float scl[I8 ? NKB + NVB : 1][BK];         // int8: their scales
+    constexpr int TILE = IMG * PF_TILE;
+    auto kbuf = [&](int t) { return t % NKB * TILE; };
+    auto vbuf = [&](int t) { return (NKB + t % NVB) * TILE; };
+    auto kscl = [&](int t) { return &scl[I8 ? t % NKB : 0][0]; };
+    auto vscl = [&](int t) { return &scl[I8 ? NKB + t % NVB : 0][0]; };
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1681,10 +1692,10 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     int soff[LPW];
 #pragma unroll
     for (int i = 0; i < LPW; i++) {
-        const int r = 4 * (LPW * (wave % SW) + i) + (lane >> 4);
+        const int r = 4 * (LPW * (wave % SW) + i) + (lane >> 4); // image row: key r % 64, dims 128 (r / 64) ..
         const int u = (lane & 15) ^ (stage_v ? ((r & 3) << 2) : (r & 15));
         // head size 64: half of the slot's 16 units hold the row, the other lanes' loads are out of bounds (zeros)
-        soff[i] = u < HD / 8 ? (r * (int)kvs + 8 * u) * 2 : 0x7fffffff;
+        soff[i] = u < HD / 8 ? ((r % BK) * (int)kvs + 128 * (r / BK) + 8 * u) * 2 : 0x7fffffff;
     }
     const int last = ntiles - 1;
     // this wave's share of tile t (its K if it stages K, else its V): load i of stage_at(t). A tile past the last one
@@ -1695,64 +1706,78 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
         StageAt s;
         const int rows = t <= last ? min(kv_len - t0, BK) : 0;
         s.rs = gi_rsrc_rows(sbase + (long long)t0 * kvs, rows * (int)kvs * 2);
-        s.dst = &smem[t & (PF_NBUF - 1)][stage_v ? 1 : 0][1024 * LPW * (wave % SW)];
+        s.dst = smem + (stage_v ? vbuf(t) : kbuf(t)) + 1024 * LPW * (wave % SW);
         if constexpr (STG) { // the tile's 64 scales, 4 bytes a lane (by each of the waves that stage the tile)
             s.rs_sc = gi_rsrc_rows((stage_v ? a.vs : a.ks) + kvh * a.sc_head_stride + t0, rows * 4);
-            s.dst_sc = &scl[t & (PF_NBUF - 1)][stage_v ? 1 : 0][0];
+            s.dst_sc = stage_v ? vscl(t) : kscl(t);
         }
         return s;
     };
-    // int8 tiles through registers: thread -> chunks of 16 bytes of the tile's K and V rows (row ch / NCH, dims 16 (ch %
-    // NCH) ..), widened to exact f16 and written into the same swizzled image; threads 0-63 take the K scale of key tid,
-    // 64-127 the V scale of key tid - 64 (times PF_I8_VBIAS). Lanes in the upper half of a row hold their chunk's two
-    // 8-byte halves swapped (and write them in that order): the 8 lanes of a row that one 16-byte LDS store serves
-    // then write 8 different units mod 8, all 32 banks, where 2ch alone would cover half of them twice.
-    constexpr int NT = 64 * WAVES, NCH = HD / 16, CH = BK * NCH, CPT = CH > NT ? CH / NT : 1;
-    const int8_t* kb8 = reinterpret_cast<const int8_t*>(a.kc) + kvh * a.kv_head_stride;
-    const int8_t* vb8 = reinterpret_cast<const int8_t*>(a.vc) + kvh * a.kv_head_stride;
-    const float* scb = RSTG ? (tid < BK ? a.ks : a.vs) + kvh * a.sc_head_stride : nullptr;
-    struct Chunks { u4 w[CPT]; };
+    // int8 and 4-bit tiles through registers: thread -> chunks of 16 bytes of the tile's K and V rows (row ch / NCH, 16 or
+    // 32 values), widened to f16 (int8: the exact integers; 4-bit: f16((n - 8) * scale), the chunk's one scale) and
+    // written into the same swizzled image; int8: threads 0-63 take the K scale of key tid, 64-127 the V scale of key
+    // tid - 64 (times the bias). int8 lanes in the upper half of a 128-value row hold their chunk's two 8-byte halves
+    // swapped (and write them in that order): the 8 lanes of a row that one 16-byte LDS store serves then write 8
+    // different units mod 8, all 32 banks, where 2ch alone would cover half of them twice.
+    constexpr int NT = 64 * WAVES, VPC = FMT == 2 ? 32 : 16, NCH = HD / VPC, CH = BK * NCH, CPT = CH > NT ? CH / NT : 1;
+    const unsigned char* kb8 = reinterpret_cast<const unsigned char*>(a.kc) + kvh * a.kv_head_stride;
+    const unsigned char* vb8 = reinterpret_cast<const unsigned char*>(a.vc) + kvh * a.kv_head_stride;
+    const float* scb = RSTG && I8 ? (tid < BK ? a.ks : a.vs) + kvh * a.sc_head_stride : nullptr;
+    struct Chunks { u4 w[CPT]; uint16_t sc[FMT == 2 ? CPT : 1]; };
     Chunks rk, rv;
     float rsc = 0.f;
-    auto load_rows = [&](const int8_t* base, int t, Chunks& c) {
+    auto load_rows = [&](bool v, int t, Chunks& c) {
         const int t0 = t * BK, rows = t <= last ? min(kv_len - t0, BK) : 0;
-        const __amdgpu_buffer_rsrc_t rs = gi_rsrc(base + (long long)t0 * kvs, rows * (int)kvs);
+        const __amdgpu_buffer_rsrc_t rs = gi_rsrc((v ? vb8 : kb8) + (long long)t0 * kvs, rows * (int)kvs);
+        const uint16_t* sp = FMT == 2 ? reinterpret_cast<const uint16_t*>(v ? a.vs : a.ks) + kvh * a.sc_head_stride + (long long)t0 * a.sc_stride : nullptr;
+        const __amdgpu_buffer_rsrc_t rss = gi_rsrc(sp, FMT == 2 ? rows * (int)a.sc_stride * 2 : 0);
 #pragma unroll
         for (int i = 0; i < CPT; i++) {
             const int ch = tid + NT * i, off = ch / NCH * (int)kvs + 16 * (ch % NCH), flip = (ch % NCH >> 2) & 1;
             if (CH % NT && ch >= CH) continue;
-            const u2 h0 = gi_load8(rs, off + 8 * flip), h1 = gi_load8(rs, off + 8 - 8 * flip);
-            c.w[i] = u4{h0.x, h0.y, h1.x, h1.y};
+            if constexpr (FMT == 2) {
+                c.w[i] = gi_load16(rs, off);
+                c.sc[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rss, (ch / NCH * (int)a.sc_stride + ch % NCH) * 2, 0, 0);
+            } else {
+                const u2 h0 = gi_load8(rs, off + 8 * flip), h1 = gi_load8(rs, off + 8 - 8 * flip);
+                c.w[i] = u4{h0.x, h0.y, h1.x, h1.y};
+            }
         }
     };
     auto load_scales = [&](int tk, int tv) {
-        const int t0 = (tid < BK ? tk : tv) * BK, rows = t0 <= last * BK ? min(kv_len - t0, BK) : 0;
-        rsc = 0.f;
-        if (tid < 2 * BK && (tid & (BK - 1)) < rows) rsc = scb[(long long)(t0 + (tid & (BK - 1))) * a.sc_stride];
+        if constexpr (I8) {
+            const int t0 = (tid < BK ? tk : tv) * BK, rows = t0 <= last * BK ? min(kv_len - t0, BK) : 0;
+            rsc = 0.f;
+            if (tid < 2 * BK && (tid & (BK - 1)) < rows) rsc = scb[(long long)(t0 + (tid & (BK - 1))) * a.sc_stride];
+        }
     };
-    auto write_rows = [&](int t, bool v, const Chunks& c) {
-        GI_LDS unsigned char* img = (GI_LDS unsigned char*)&smem[t & (PF_NBUF - 1)][v ? 1 : 0][0];
+    auto write_rows = [&](bool v, int t, const Chunks& c) {
+        GI_LDS unsigned char* img = (GI_LDS unsigned char*)smem + (v ? vbuf(t) : kbuf(t));
 #pragma unroll
         for (int i = 0; i < CPT; i++) {
-            const int ch = tid + NT * i, row = ch / NCH, flip = (ch % NCH >> 2) & 1;
+            const int ch = tid + NT * i, row = ch / NCH, flip = FMT == 1 ? (ch % NCH >> 2) & 1 : 0;
             if (CH % NT && ch >= CH) continue;
 #pragma unroll
-            for (int hw = 0; hw < 2; hw++) {
-                const int u = 2 * (ch % NCH) + (hw ^ flip);
+            for (int q = 0; q < VPC / 8; q++) { // unit of 8 values
+                const int u = VPC / 8 * (ch % NCH) + (q ^ flip);
                 u4 w;
-#pragma unroll
-                for (int e = 0; e < 2; e++) {
-                    const uint32_t x = gi_i8_in(c.w[i][2 * hw + e]);
-                    w[2 * e] = i8_f16x2(x, GI_I8_LO);
-                    w[2 * e + 1] = i8_f16x2(x, GI_I8_HI);
+                if constexpr (FMT == 2) {
+                    const uint32_t x = c.w[i][q];
+                    const h2x sc = __builtin_bit_cast(h2x, (uint32_t)c.sc[i] * 0x10001u);
+                    w = u4{q4_f16x2(x >> 4, x, 0, sc), q4_f16x2(x >> 4, x, 1, sc), q4_f16x2(x >> 4, x, 2, sc), q4_f16x2(x >> 4, x, 3, sc)};
+                } else {
+                    const uint32_t x0 = gi_i8_in(c.w[i][2 * q]), x1 = gi_i8_in(c.w[i][2 * q + 1]);
+                    w = u4{i8_f16x2(x0, GI_I8_LO), i8_f16x2(x0, GI_I8_HI), i8_f16x2(x1, GI_I8_LO), i8_f16x2(x1, GI_I8_HI)};
                 }
-                *reinterpret_cast<GI_LDS u4*>(img + row * 256 + ((u ^ (v ? (row & 3) << 2 : row & 15)) << 4)) = w;
+                *reinterpret_cast<GI_LDS u4*>(img + (u / 16) * PF_TILE + row * 256 + (((u % 16) ^ (v ? (row & 3) << 2 : row & 15)) << 4)) = w;
             }
         }
     };
     auto write_scales = [&](int tk, int tv) {
-        if (tid < BK) scl[tk & (PF_NBUF - 1)][0][tid] = rsc;
-        else if (tid < 2 * BK) scl[tv & (PF_NBUF - 1)][1][tid - BK] = rsc * PF_I8_VBIAS;
+        if constexpr (I8) {
+            if (tid < BK) kscl(tk)[tid] = rsc;
+            else if (tid < 2 * BK) vscl(tv)[tid - BK] = WIDE ? rsc : rsc * VB;
+        }
     };
     auto stage1 = [&](const StageAt& s, int i) {
         if (i < LPW) gi_stage16(s.rs, (GI_LDS void*)(s.dst + 1024 * i), soff[i]);
@@ -1774,19 +1799,19 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     // Q is held pre-multiplied by scale*log2(e), so scores come out of the MFMA in log2 units (the f16
     // rounding of the scaled value is the same size as the rounding of Q itself)
     const float qs = a.qscale;
-    // what the first QK and the first iteration need starts loading: K of two tiles, V of one
+    // the first tile's K and V (four buffers: the second's K too) start loading
     Chunks rk1;
     float rsc1 = 0.f;
     if constexpr (RSTG) {
-        load_rows(kb8, t_begin, rk);
-        load_rows(vb8, t_begin, rv);
-        load_rows(kb8, t_begin + 1, rk1);
+        load_rows(false, t_begin, rk);
+        load_rows(true, t_begin, rv);
+        load_rows(false, t_begin + 1, rk1);
         load_scales(t_begin + 1, t_begin); // K of the second tile, V of the first
         rsc1 = rsc;
         load_scales(t_begin, t_begin);
     } else {
         stage(t_begin);
-        if (!stage_v) stage(t_begin + 1);
+        if (!WIDE && !stage_v) stage(t_begin + 1);
     }
     h8 qf[KS];
     if (a.q_f16) {
@@ -1808,17 +1833,19 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
         }
     }
 
-    // (the compiler's wait for the queries is also one for the loads above; the next two tiles' go out behind it)
+    // (the compiler's wait for the queries is also one for the loads above; the next tiles' go out behind it)
     if constexpr (RSTG) {
-        write_rows(t_begin, false, rk);
-        write_rows(t_begin, true, rv);
+        write_rows(false, t_begin, rk);
+        write_rows(true, t_begin, rv);
         write_scales(t_begin, t_begin);
-        write_rows(t_begin + 1, false, rk1);
+        write_rows(false, t_begin + 1, rk1);
         rsc = rsc1;
         write_scales(t_begin + 1, t_begin);
-        load_rows(kb8, t_begin + 2, rk);
-        load_rows(vb8, t_begin + 1, rv);
+        load_rows(false, t_begin + 2, rk);
+        load_rows(true, t_begin + 1, rv);
         load_scales(t_begin + 2, t_begin + 1);
+    } else if constexpr (WIDE) {
+        if (!stage_v) stage(t_begin + 1);
     } else {
         stage(t_begin + (stage_v ? 1 : 2));
         stage(t_begin + (stage_v ? 2 : 3));
@@ -1844,14 +1871,13 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
 #pragma unroll
     for (int e = 0; e < 16; e++) negm[e] = 0.f;
 
-    auto buf = [&](int t) { return (t & (PF_NBUF - 1)) * (2 * PF_TILE); };
-    GI_LDS unsigned char* const lds = (GI_LDS unsigned char*)&smem[0][0][0];
+    GI_LDS unsigned char* const lds = (GI_LDS unsigned char*)smem;
     // fragment st of a tile's QK (key block st%2, k-step st/2), fragment f of its P V (k-step f/NDB, dim block f%NDB)
     auto kfrag = [&](int B, int st) {
-        return *reinterpret_cast<GI_LDS const h8*>(lds + ((B + kx) ^ (32 * (st >> 1))) + 8192 * (st & 1));
+        return *reinterpret_cast<GI_LDS const h8*>(lds + ((B + kx) ^ (32 * (st >> 1 & 7))) + 8192 * (st & 1) + PF_TILE * (st >> 4));
     };
     auto vfrag = [&](int B, int f) {
-        GI_LDS unsigned char* vp = lds + ((B + vx) ^ (64 * (f % NDB))) + PF_TILE + 4096 * (f / NDB);
+        GI_LDS unsigned char* vp = lds + ((B + vx) ^ (64 * (f % NDB & 3))) + PF_TILE * (f % NDB >> 2) + 4096 * (f / NDB);
         gi_s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GI_LDS gi_s4*)(vp));
         gi_s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GI_LDS gi_s4*)(vp + 1024));
         return __builtin_shufflevector(__builtin_bit_cast(h4x, lo), __builtin_bit_cast(h4x, hi), 0, 1, 2, 3, 4, 5, 6, 7);
@@ -1882,32 +1908,37 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
         return *reinterpret_cast<const f4*>(sc + 8 * half + 32 * (g >> 2) + 16 * ((g & 3) >> 1) + 4 * (g & 1));
     };
 
-    h8 kf[RING], vf[RING];
+    h8 kf[RING], vf[VRING];
     float mx = GI_NEG_INF;
     f16x sa[NBLK], sb[NBLK]; // scores of alternate tiles
 
-    // publish K of tile it+2 and V of tile it+1 (each wave's own loads of them are in; one tile more may be in flight),
-    // after which tile it+4's K goes into K(it)'s buffer, tile it+3's V into V(it-1)'s
+    // publish K of tile it+2 and V of tile it+1 (each wave's own loads of them are in), after which the tiles of
+    // stage_tile(it) go into buffers that no wave reads any more. Four buffers: K(it+4) into K(it)'s, V(it+3) into
+    // V(it-1)'s, whose readers' MFMAs all issued before the barrier; one tile more may be in flight at it. Two buffers:
+    // K(it+3) into K(it+1)'s and V(it+2) into V(it)'s, whose last reads are waited for before the barrier (they went
+    // out VRING slots ahead of their MFMAs, so they are back by then).
     auto publish = [&](int it) {
-        if constexpr (RSTG) __builtin_amdgcn_s_waitcnt(GI_LGKMCNT0); // this wave's widened rows are in LDS
-        else __builtin_amdgcn_s_waitcnt(GI_VMCNT(LPT));
+        if constexpr (RSTG || WIDE) __builtin_amdgcn_s_waitcnt(GI_LGKMCNT0); // (RSTG: and this wave's widened rows are in LDS)
+        if constexpr (!RSTG) __builtin_amdgcn_s_waitcnt(GI_VMCNT(WIDE ? 0 : LPT));
         asm volatile("s_barrier" ::: "memory");
     };
+    auto stage_tile = [&](int it) { return it + (WIDE ? 3 : 4) - (stage_v ? 1 : 0); };
     // register staging of iteration it: the rows loaded in iteration it-1 (K of tile it+2, V of tile it+1) are widened
-    // into their buffers (last read in iterations it-3 and it-3), and the next ones' loads go out
+    // into their buffers (free since the barrier of it-1), and the next ones' loads go out
     auto restage_k = [&](int it) {
-        write_rows(it + 2, false, rk);
-        load_rows(kb8, it + 3, rk);
+        write_rows(false, it + 2, rk);
+        load_rows(false, it + 3, rk);
     };
     auto restage_v = [&](int it) {
-        write_rows(it + 1, true, rv);
-        load_rows(vb8, it + 2, rv);
+        write_rows(true, it + 1, rv);
+        load_rows(true, it + 2, rv);
     };
     auto restage_s = [&](int it) {
         write_scales(it + 2, it + 1);
         load_scales(it + 3, it + 2);
     };
-    auto step = [&](int it, f16x* s, f16x* sn) {
+    // the causal mask of a tile that crosses the diagonal (or the end) somewhere in the wave, and its row max again
+    auto mask = [&](int it, f16x* s) {
         const int t0 = it * BK;
         if (t0 + BK - 1 > wave_first) { // the tile crosses the diagonal (or the end) somewhere in the wave
             const int lim = qpos - t0 - 8 * half;
@@ -1920,33 +1951,39 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
                         if (32 * bb + 16 * (i >> 1) + 4 * (i & 1) + jj > lim) s[bb][4 * i + jj] = GI_NEG_INF;
             mx = rowmax(s);
         }
-        const bool up = mx > PF_RESCALE_LOG2 || it == t_begin;
+    };
+    auto step = [&](int it, f16x* s, f16x* sn) {
+        mask(it, s);
+        const bool up = mx > PF_RESCALE_LOG2;
         if (__builtin_amdgcn_ballot_w64(up)) {
-            const float delta = up && mx > GI_NEG_INF ? mx : 0.f;
-            const float alpha = __builtin_amdgcn_exp2f(-fmaxf(delta, 0.f));
+            // some row's max moved: shift the reference by delta, rescale O and l (alpha = 1 for the other rows) and this
+            // tile's scores; the next tile's QK starts from the new reference
+            const float delta = up ? mx : 0.f;
+            const float alpha = __builtin_amdgcn_exp2f(-delta);
             m_run += delta;
 #pragma unroll
             for (int e = 0; e < 16; e++) negm[e] = -m_run;
             l_run *= alpha;
 #pragma unroll
-            for (int db = 0; db < NDB; db++) gi_acc_scale<false>(o[db], alpha);
+            for (int db = 0; db < NDB; db++) gi_acc_scale<WIDE>(o[db], alpha);
 #pragma unroll
             for (int bb = 0; bb < NBLK; bb++) s[bb] -= delta;
         }
-        const int B0 = buf(it), B1 = buf(it + 1), B2 = buf(it + 2);
+        const int B0 = vbuf(it), B1 = kbuf(it + 1), B2 = kbuf(it + 2);
         StageAt st; // the tile this iteration stages
-        if constexpr (!RSTG) st = stage_at(it + (stage_v ? 3 : 4));
+        if constexpr (!RSTG) st = stage_at(stage_tile(WIDE ? it - 1 : it));
         h8 pf[4];
         float mxn = GI_NEG_INF;
-        // slot of probability pair w (of 16: every P^T operand is complete before its P V MFMAs), and of the next
+        // slot of exponential x (of 32: every P^T operand is complete before its P V MFMAs), and of the next
         // tile's row max over score group g (of 8), from two slots after its last QK MFMA on
-        constexpr auto pslot = [](int w) { return w * (NS - 4) / 16; };
+        constexpr auto pslot = [](int x) { return x * (NS - NDB) / 32; };
         constexpr auto mslot = [](int g) { return NQ + 2 + g * (NP - 2) / 8; };
         // int8: scales of score group g in element g % SR, read when the group SR before it has taken its own
         constexpr int SR = HD == 64 ? 4 : 2;
         f4 ksv[SR], vsv[SR];
-        const float* const ksp = &scl[I8 ? (it + 1) & (PF_NBUF - 1) : 0][0][0];
-        const float* const vsp = &scl[I8 ? it & (PF_NBUF - 1) : 0][1][0];
+        float p0 = 0.f;
+        const float* const ksp = kscl(it + 1);
+        const float* const vsp = vscl(it);
         if constexpr (I8)
 #pragma unroll
             for (int g = 0; g < SR; g++) vsv[g] = scale4(vsp, g);
@@ -1960,12 +1997,12 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
                 sn[bb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[sl % RING], qf[ks], ks == 0 ? (I8 ? f16x{} : negm) : sn[bb], 0, 0, 0);
             } else {
                 const int f = sl - NQ;
-                o[f % NDB] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[f % RING], pf[f / NDB], o[f % NDB], 0, 0, 0);
+                o[f % NDB] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[f % VRING], pf[f / NDB], o[f % NDB], 0, 0, 0);
             }
-            // LDS reads, RING slots ahead of their MFMA
+            // LDS reads, RING (V: VRING) slots ahead of their MFMA
             if constexpr (sl + RING < NQ) kf[sl % RING] = kfrag(B1, sl + RING);
-            else if constexpr (sl + RING < NS) vf[(sl + RING - NQ) % RING] = vfrag(B0, sl + RING - NQ);
-            else kf[(sl + RING - NS) % RING] = kfrag(B2, sl + RING - NS);
+            if constexpr (sl + VRING >= NQ && sl + VRING < NS) vf[(sl + VRING - NQ) % VRING] = vfrag(B0, sl + VRING - NQ);
+            if constexpr (sl + RING >= NS) kf[(sl + RING - NS) % RING] = kfrag(B2, sl + RING - NS);
             // staging behind the barrier
             if constexpr (RSTG) {
                 if (sl == 1) restage_k(it);
@@ -1974,18 +2011,21 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
             } else {
 #pragma unroll
                 for (int i = 0; i < LPT; i++)
-                    if (sl == NS - RING + i * RING / LPT) stage1(st, i);
+                    if (sl == (WIDE ? i : NS - RING + i * RING / LPT)) stage1(st, i);
             }
 #pragma unroll
-            for (int w = 0; w < 16; w++)
-                if (pslot(w) == sl) {
-                    const int ks = w >> 2, e = 2 * (w & 3), bb = ks >> 1, i = 2 * (ks & 1) + (e >> 2), jj = e & 3;
-                    const float p0 = __builtin_amdgcn_exp2f(s[bb][4 * i + jj]);
+            for (int x = 0; x < 32; x++)
+                if (pslot(x) == sl) {
+                    const int w = x >> 1, ks = w >> 2, e = 2 * (w & 3), bb = ks >> 1, i = 2 * (ks & 1) + (e >> 2), jj = e & 3;
+                    if (!(x & 1)) {
+                        p0 = __builtin_amdgcn_exp2f(s[bb][4 * i + jj]);
+                        continue;
+                    }
                     const float p1 = __builtin_amdgcn_exp2f(s[bb][4 * i + jj + 1]);
                     const _Float16 h0 = (_Float16)p0, h1 = (_Float16)p1;
                     if constexpr (I8) {
-                        pf[ks][e] = (_Float16)(p0 * vsv[(w >> 1) % SR][jj]);
-                        pf[ks][e + 1] = (_Float16)(p1 * vsv[(w >> 1) % SR][jj + 1]);
+                        pf[ks][e] = (_Float16)(p0 * (WIDE ? vsv[(w >> 1) % SR][jj] * VB : vsv[(w >> 1) % SR][jj]));
+                        pf[ks][e + 1] = (_Float16)(p1 * (WIDE ? vsv[(w >> 1) % SR][jj + 1] * VB : vsv[(w >> 1) % SR][jj + 1]));
                     } else {
                         pf[ks][e] = h0;
                         pf[ks][e + 1] = h1;
@@ -2018,40 +2058,59 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     auto iteration = [&](int it, f16x* s, f16x* sn) {
         if (it < my_tiles) {
             step(it, s, sn);
-        } else {
+        } else { // past its last tile a wave goes on staging and keeping the barriers
             if constexpr (RSTG) {
                 restage_k(it);
                 restage_v(it);
                 restage_s(it);
             }
+            if constexpr (!RSTG && WIDE) stage(stage_tile(it - 1));
             publish(it);
-            if constexpr (!RSTG) stage(it + (stage_v ? 3 : 4));
+            if constexpr (!RSTG && !WIDE) stage(stage_tile(it));
         }
     };
 
-    // prologue: K of the first two tiles and V of the first are in
+    // prologue: K of the first tile is in (four buffers: K of the first two tiles and V of the first), and its QK runs
+    constexpr bool ONE = !WIDE; // one barrier: the second tile's K is there for the operand ring
     if constexpr (RSTG) __builtin_amdgcn_s_waitcnt(GI_LGKMCNT0);
-    else __builtin_amdgcn_s_waitcnt(GI_VMCNT(2 * LPT));
+    else __builtin_amdgcn_s_waitcnt(GI_VMCNT(ONE ? 2 * LPT : LPT)); // (two buffers: V waves have issued one tile, known to be in)
     asm volatile("s_barrier" ::: "memory");
     if (my_tiles > t_begin) {
-        const int B0 = buf(t_begin), B1 = buf(t_begin + 1);
+        const int B0 = kbuf(t_begin), B1 = kbuf(t_begin + 1);
 #pragma unroll
         for (int st = 0; st < RING; st++) kf[st] = kfrag(B0, st);
 #pragma unroll
         for (int st = 0; st < NQ; st++) {
             const int ks = st >> 1, bb = st & 1;
             sa[bb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[st % RING], qf[ks], ks == 0 ? f16x{} : sa[bb], 0, 0, 0);
-            kf[st % RING] = st + RING < NQ ? kfrag(B0, st + RING) : kfrag(B1, st + RING - NQ);
+            if (st + RING < NQ) kf[st % RING] = kfrag(B0, st + RING);
+            else if (ONE) kf[st % RING] = kfrag(B1, st + RING - NQ);
         }
         if constexpr (I8) {
 #pragma unroll
             for (int g = 0; g < 8; g++) {
-                const f4 k4 = scale4(&scl[t_begin & (PF_NBUF - 1)][0][0], g);
+                const f4 k4 = scale4(kscl(t_begin), g);
 #pragma unroll
                 for (int e = 0; e < 4; e++) sa[g >> 2][4 * (g & 3) + e] *= k4[e];
             }
         }
         mx = rowmax(sa);
+        // every row takes its first max as its reference (a row that sees no key of a slice's first tile sees none of
+        // its later ones: its reference stays 0 and its sum 0)
+        mask(t_begin, sa);
+        m_run = mx > GI_NEG_INF ? mx : 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; e++) negm[e] = -m_run;
+#pragma unroll
+        for (int bb = 0; bb < NBLK; bb++) sa[bb] -= m_run;
+        mx -= m_run;
+    }
+    if constexpr (!ONE) { // K of the second tile is in, and the first's buffer free for the third's
+        __builtin_amdgcn_s_waitcnt(GI_LGKMCNT0);
+        if constexpr (!RSTG) __builtin_amdgcn_s_waitcnt(GI_VMCNT(0));
+        asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+        for (int st = 0; st < RING; st++) kf[st] = kfrag(kbuf(t_begin + 1), st);
     }
     for (int it = t_begin; it < ntiles; it += 2) {
         iteration(it, sa, sb);
@@ -2069,7 +2128,7 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 f4 v = f4{o[db][4 * i], o[db][4 * i + 1], o[db][4 * i + 2], o[db][4 * i + 3]};
-                if constexpr (I8) v *= 1.f / PF_I8_VBIAS;
+                if constexpr (I8) v *= 1.f / VB;
                 po[64 * (4 * db + i)] = v;
             }
         if (half == 0)
@@ -2077,7 +2136,7 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
         return;
     }
     if (qlive) {
-        const float inv = (I8 ? 1.f / PF_I8_VBIAS : 1.f) / l;
+        const float inv = (I8 ? 1.f / VB : 1.f) / l;
         if (a.out_f16) {
             _Float16* op = (_Float16*)a.out + (long long)qtok * a.out_stride + h * HD + 4 * half;
 #pragma unroll
@@ -2100,469 +2159,35 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     }
 }
 
-// ---------------------------------------------------------------- prefill, head size 256, 16 rows per wave
-// One workgroup per (head, 128 query rows): 8 waves of 16 rows, each with all 256 output dims, so QK and the
-// softmax are computed once per row (the reference's attention_prefill_tc256 splits the output dims over
-// two blocks that both compute QK, src/cuda.rs:2622-2623). On v_mfma_f32_16x16x32_f16, per 64-key tile:
-//  - S^T (4 blocks of 16 keys x 16 queries) = K Q^T over 8 k-steps of 32 dims, each chain starting from
-//    C = -(reference max). Lane l holds query column c = l%16 and rows 4g + r (g = l/16) of each block.
-//    A-row rho of key block kb reads tile key 8(rho/4) + 4(kb%2) + 32(kb/2) + rho%4, so the lane's rows
-//    are keys 32(kb/2) + 8g + 4(kb%2) + r: exactly the keys 32kp + 8g + e (kp = kb/2, e = 4(kb%2) + r) it
-//    holds in the P^T operand of k-step kp of P V, with no data movement.
-//  - O^T (16 blocks of 16 dims x 16 queries) += V^T P^T: per 16-dim block one MFMA for each 32 keys, V^T
-//    from two transposing reads (keys 8g..8g+3 and 8g+4..8g+7 of the 32, 16 dims).
-// LDS image of a K or V tile (32 KB): row r holds key r%64, dims 128(r/64) .. +127 (256 bytes), its 16-byte
-// units XOR-swizzled (pf256r_swz_k / pf256r_swz_v). Per tile a wave issues 64 MFMAs against 64 KB of LDS
-// operand reads, twice the bytes per flop of the head-size-128 kernel's 32-row waves.
-__device__ __forceinline__ int pf256r_swz_k(int r) { return (r & 15) ^ (((r >> 4) & 1) << 2); }
-__device__ __forceinline__ int pf256r_swz_v(int r) { return ((r & 3) << 2) | (((r >> 3) & 1) << 1); }
-#define PF256R_WAVES 8
-#define PF256R_ROWS 16
-#define PF256R_BQ (PF256R_ROWS * PF256R_WAVES) // query rows per workgroup
-// K and V rings: NKBUF and NVBUF buffers of one tile each (NKBUF + NVBUF <= 5 in 160 KB of LDS). Iteration
-// it reads K of tile it+1 (its QK) and V of tile it (its P V); after its barrier the buffers of K(it) and
-// V(it-1) have no reader left, so it refills them with K(it + NKBUF) and V(it + NVBUF - 1): each tile is
-// issued NKBUF - 1 (K) or NVBUF - 1 (V) iterations before its use. Half the waves stage K, half V, and
-// each waits for its own loads only, then the barrier publishes them.
-// FMT 1 (the int8 cache, attention_prefill_tc256 with KV8, src/cuda.rs:2466-2498, 2548-2605) and 2 (the 4-bit
-// cache, with KV4, src/cuda.rs:2495-2514): the staging waves load the compressed rows into registers, widen them
-// to f16 (int8: the exact integers; 4-bit: f16((n - 8) * scale)) and write the same swizzled f16 image, one tile
-// ahead of the barrier that publishes it. int8 also stages each tile's key and value scales: a score is the dot
-// product with the integer key times the key's scale, P V takes f16(p * vscale * 2^10), the row sum the f16 p,
-// and the output is divided by 2^10.
-template <int NKBUF, int NVBUF, int FMT = 0, bool STG = false>
-__device__ __forceinline__ void gi_prefill256r(const GiPrefillArgs& a) {
-    static_assert(NKBUF >= 2 && NVBUF >= 2 && NKBUF + NVBUF <= 5, "K and V rings within 160 KB");
-    static_assert(!STG || FMT == 1, "pre-widened staging: the int8 cache (the 4-bit one widens to the f16 kernel's input)");
-    // STG: the int8 cache already widened to exact f16 integers in a workspace (gi_kv_widen: rows [n_kv][len][256],
-    // raw scales [n_kv][len]), staged by LDS-DMA as the f16 cache is
-    constexpr bool REG = FMT != 0 && !STG; // staging through registers
-    constexpr int HD = 256, WAVES = PF256R_WAVES, BQ = PF256R_BQ, BK = 64;
-    constexpr int SW = WAVES / 2;            // waves staging each of K and V
-    constexpr int LPW = (BK / 2) / SW;       // 1 KB loads per staging wave and tile (K or V: BK * 512 bytes)
-    constexpr int LPT = LPW + (STG ? 1 : 0); // loads per staging wave and tile (STG: plus a quarter of the scales)
-    constexpr int KS = HD / 32;              // QK k-steps
-    constexpr int NKB = BK / 16;             // S^T blocks of 16 keys
-    constexpr int NDB = HD / 16;             // O^T blocks of 16 dims
-    constexpr int TILE = BK * 512;           // bytes of one K or V tile image
-    constexpr int VPF = REG ? 4 : 0;         // V^T fragments read ahead in P V (0: the compiler's order)
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[(NKBUF + NVBUF) * TILE];
-    __shared__ __attribute__((aligned(16))) float sc_sh[FMT == 1 ? NKBUF + NVBUF : 1][BK]; // int8: tile scales
-    auto kbuf = [&](int t) { return smem + (t % NKBUF) * TILE; };
-    auto vbuf = [&](int t) { return smem + (NKBUF + t % NVBUF) * TILE; };
-    auto kscl = [&](int t) { return &sc_sh[t % NKBUF][0]; };
-    auto vscl = [&](int t) { return &sc_sh[FMT == 1 ? NKBUF + t % NVBUF : 0][0]; };
-    // wait until at most n (0..2) of this wave's tile loads are outstanding
-    auto wait_tiles = [&](int n) {
-        if constexpr (REG) return; // (register staging: the compiler waits for the loads it issued)
-        if (n >= 2) __builtin_amdgcn_s_waitcnt(GI_VMCNT(2 * LPT));
-        else if (n == 1) __builtin_amdgcn_s_waitcnt(GI_VMCNT(LPT));
-        else __builtin_amdgcn_s_waitcnt(GI_VMCNT(0));
-    };
-    static_assert(NKBUF <= 4 && NVBUF <= 4, "wait_tiles covers two tiles in flight past the one waited for");
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int G = a.n_heads / a.n_kv;
-    const int qtiles = (a.n + BQ - 1) / BQ;
-    const int nwg = gridDim.x;
-    int j = blockIdx.x;
-    if ((nwg & 7) == 0) j = (j & 7) * (nwg >> 3) + (j >> 3); // each XCD a contiguous run of items
-    const int kvh = j / (qtiles * G);
-    const int rest = j % (qtiles * G);
-    const int qt = qtiles - 1 - rest / G; // longest query tiles first
-    const int h = kvh * G + rest % G;
-    const int q0 = qt * BQ;
-    const int kv_len = a.pos0 + a.n;
-    const int k_lim = min(kv_len, a.pos0 + q0 + BQ);
-    const int ntiles = (k_lim + BK - 1) / BK;
-    const long long kvs = a.kv_stride;
-
-    // ---- staging: wave w's load i covers image rows 4*(LPW*(w%SW) + i) + lane/16 (row r = key r%BK, dims
-    // 128*(r/BK)..), LDS unit lane%16 holding global unit (lane%16) ^ swizzle(r). K: the key's low 4 bits with bit 4 folded into bit 2, so
-    // that the 16 rows one K fragment read touches (keys 8(c/4) + c%4 (+4), c = 0..15: low 4 bits repeat at
-    // c and c + 8) fall on 16 different unit positions. V: (key % 4) << 2 with bit 3 into bit 1, so that lane
-    // groups g and g + 1 of a transposing read (keys 8g + te and 8g + 8 + te) use disjoint banks.
-    const bool stage_v = wave >= SW;
-    const uint16_t* sbase = (stage_v ? a.vc : a.kc) + kvh * a.kv_head_stride;
-    int soff[LPW];
-#pragma unroll
-    for (int i = 0; i < LPW; i++) {
-        const int r = 4 * (LPW * (wave % SW) + i) + (lane >> 4);
-        const int u = (lane & 15) ^ (stage_v ? pf256r_swz_v(r) : pf256r_swz_k(r));
-        soff[i] = ((r & (BK - 1)) * (int)kvs + 128 * (r / BK) + 8 * u) * 2;
-    }
-    // this wave's share of tile t (its K if it stages K, else its V)
-    auto stage = [&](int t) {
-        const int t0 = t * BK;
-        const uint16_t* src = sbase + (long long)t0 * kvs;
-        const long long bytes = (long long)(kv_len - t0) * kvs * 2;
-        unsigned char* dst = (stage_v ? vbuf(t) : kbuf(t)) + 1024 * LPW * (wave % SW);
-#pragma unroll
-        for (int i = 0; i < LPW; i++) gi_stage16(src, bytes, (GI_LDS void*)(dst + 1024 * i), soff[i]);
-        if constexpr (STG) {
-            // this wave's quarter of the tile's 64 scales (16 floats: lanes 0-3, 16 bytes each)
-            static_assert(SW * 16 == BK, "a quarter of the scales per staging wave");
-            const float* sp = (stage_v ? a.vs : a.ks) + kvh * a.sc_head_stride + t0;
-            if (lane < 4)
-                gi_stage16(sp, (long long)(kv_len - t0) * 4, (GI_LDS void*)((stage_v ? vscl(t) : kscl(t)) + 16 * (wave % SW)),
-                           64 * (wave % SW) + 16 * lane);
-        }
-    };
-    // ---- register staging (FMT 1, 2): staging lane l takes a quarter (l/16) of key 16(wave % SW) + l%16's row,
-    // values 64 quarter .. +63, i.e. image row key + 64(quarter/2), units 8(quarter%2) .. +7 (swizzled as above):
-    // the 16 lanes of a quarter write 16 keys' rows, whose swizzles put their 16-byte units on distinct banks
-    // (one quarter per lane and key instead measured 12% slower). These LDS writes, not the widening, are what
-    // the register path costs against the f16 cache's LDS-DMA staging (widening without the writes: 0.77 ms at
-    // 8192 tokens, 16/2; the writes without the widening: 1.31 ms).
-    // int8 rows: 4 16-byte loads and the key's f32 scale (quarter 0's lane); 4-bit rows: 2 16-byte loads and the
-    // two f16 scales of its groups. `pend` holds one tile's loads from its issue to its widening.
-    const int skey = 16 * (wave % SW) + (lane & 15), squart = lane >> 4;
-    const int srow = skey + BK * (squart >> 1);
-    struct Pend { u4 w[FMT == 1 ? 4 : 2]; uint32_t sc; int t; } pend;
-    pend.t = -1;
-    const unsigned char* sbase8 = reinterpret_cast<const unsigned char*>(stage_v ? a.vc : a.kc) + kvh * a.kv_head_stride;
-    const void* scbase = nullptr;
-    if constexpr (FMT == 1) scbase = (stage_v ? a.vs : a.ks) + kvh * a.sc_head_stride;
-    if constexpr (FMT == 2) scbase = reinterpret_cast<const uint16_t*>(stage_v ? a.vs : a.ks) + kvh * a.sc_head_stride;
-    auto issue = [&](int t) {
-        const int t0 = t * BK;
-        const __amdgpu_buffer_rsrc_t r = gi_rsrc(sbase8 + (long long)t0 * kvs, (long long)(kv_len - t0) * kvs);
-        if constexpr (FMT == 1) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) pend.w[i] = gi_load16(r, skey * (int)kvs + 64 * squart + 16 * i);
-            const float* sp = reinterpret_cast<const float*>(scbase) + (long long)t0 * a.sc_stride;
-            pend.sc = __builtin_amdgcn_raw_buffer_load_b32(gi_rsrc(sp, (long long)(kv_len - t0) * a.sc_stride * 4),
-                                                           skey * (int)a.sc_stride * 4, 0, 0);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 2; i++) pend.w[i] = gi_load16(r, skey * (int)kvs + 32 * squart + 16 * i);
-            const uint16_t* sp = reinterpret_cast<const uint16_t*>(scbase) + (long long)t0 * a.sc_stride;
-            pend.sc = __builtin_amdgcn_raw_buffer_load_b32(gi_rsrc(sp, (long long)(kv_len - t0) * a.sc_stride * 2),
-                                                           (skey * (int)a.sc_stride + 2 * squart) * 2, 0, 0);
-        }
-        pend.t = t;
-    };
-    // widen the pending tile into its buffer (the next barrier publishes it, after this wave's LDS writes are
-    // waited for)
-    auto commit = [&]() {
-        if (pend.t < 0) return;
-        const int t = pend.t;
-        unsigned char* img = stage_v ? vbuf(t) : kbuf(t);
-        const int swz = stage_v ? pf256r_swz_v(srow) : pf256r_swz_k(srow);
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            u4 h;
-            if constexpr (FMT == 1) {
-                const uint32_t x0 = gi_i8_in(pend.w[i >> 1][2 * (i & 1)]), x1 = gi_i8_in(pend.w[i >> 1][2 * (i & 1) + 1]);
-                h = u4{i8_f16x2(x0, GI_I8_LO), i8_f16x2(x0, GI_I8_HI), i8_f16x2(x1, GI_I8_LO), i8_f16x2(x1, GI_I8_HI)};
-            } else {
-                const uint32_t x = pend.w[i >> 2][i & 3];
-                const h2x sc = __builtin_bit_cast(h2x, (i >> 2) ? (pend.sc >> 16) * 0x10001u : (pend.sc & 0xffffu) * 0x10001u);
-                h = u4{q4_f16x2(x >> 4, x, 0, sc), q4_f16x2(x >> 4, x, 1, sc), q4_f16x2(x >> 4, x, 2, sc),
-                       q4_f16x2(x >> 4, x, 3, sc)};
-            }
-            const int unit = (8 * (squart & 1) + i) ^ swz;
-            *reinterpret_cast<GI_LDS u4*>((GI_LDS unsigned char*)img + srow * 256 + (unit << 4)) = h;
-        }
-        if constexpr (FMT == 1)
-            if (squart == 0) (stage_v ? vscl(t) : kscl(t))[skey] = __uint_as_float(pend.sc);
-        pend.t = -1;
-    };
-    // iteration it's staging: the pending tile (K: it + NKBUF into K(it)'s buffer; V: it + NVBUF - 1 into
-    // V(it-1)'s; both free since the barrier of it) is widened, and the loads of the next one are issued, so
-    // each tile's loads have a whole iteration to land and its widening runs among the wave's MFMAs
-    auto restage = [&](int it) {
-        commit();
-        if (!stage_v && it + NKBUF + 1 < ntiles) issue(it + NKBUF + 1);
-        if (stage_v && it + NVBUF < ntiles) issue(it + NVBUF);
-    };
-
-    // ---- Q as B operands: lane (column c, k-group g), k-step ks: dims 32ks + 8g .. +7, times scale*log2(e)
-    const int c = lane & 15, g = lane >> 4;
-    const int qrow = q0 + PF256R_ROWS * wave + c;
-    const int qpos = a.pos0 + qrow;
-    const float qs = a.qscale;
-    h8 qf[KS];
-    {
-        const int qr = qrow < a.n ? qrow : a.n - 1; // rows past n compute garbage that is never written
-        if (a.q_f16) {
-            const _Float16* qp = (const _Float16*)a.q + (long long)qr * a.q_stride + h * HD + 8 * g;
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                const h8 x = __builtin_bit_cast(h8, *reinterpret_cast<const u4*>(qp + 32 * ks));
-#pragma unroll
-                for (int e = 0; e < 8; e++) qf[ks][e] = (_Float16)((float)x[e] * qs);
-            }
-        } else {
-            const float* qp = (const float*)a.q + (long long)qr * a.q_stride + h * HD + 8 * g;
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                const float4 x0 = *reinterpret_cast<const float4*>(qp + 32 * ks);
-                const float4 x1 = *reinterpret_cast<const float4*>(qp + 32 * ks + 4);
-                qf[ks] = h8{(_Float16)(x0.x * qs), (_Float16)(x0.y * qs), (_Float16)(x0.z * qs), (_Float16)(x0.w * qs),
-                            (_Float16)(x1.x * qs), (_Float16)(x1.y * qs), (_Float16)(x1.z * qs), (_Float16)(x1.w * qs)};
-            }
-        }
-    }
-
-    // ---- operand read offsets (bytes within a buffer's K or V image)
-    // K: block kb, k-step ks: key krow + 4(kb%2) + 32(kb/2) (krow = 8(c/4) + c%4), image half ks/4, unit
-    // 4(ks%4) + g swizzled
-    const int krow = 8 * (c >> 2) + (c & 3);
-    auto kfrag = [&](const unsigned char* K, int st) { // MFMA st of a tile's NKB*KS: block st%NKB, k-step st/NKB
-        const int kb = st % NKB, ks = st / NKB;
-        const int key = krow + 4 * (kb & 1) + 32 * (kb >> 1);
-        const int unit = (4 * (ks & 3) + g) ^ pf256r_swz_k(key);
-        return *reinterpret_cast<const h8*>(K + (key + BK * (ks >> 2)) * 256 + (unit << 4));
-    };
-    // V: block db (dims 16db..), keys 8g + te (+4): image row 32*(db/8) + 8g + te, unit 2*(db%8) + tc/2 swizzled,
-    // plus 8 bytes for odd tc (te = (lane%16)/4, tc = lane%4); the +4 rows of the second read keep the swizzle
-    // (BK = 64: k-step kp of P V takes keys 32kp + ..)
-    const int te = c >> 2, tc = c & 3;
-    const int vbase = (8 * g + te) * 256 + 8 * (tc & 1);
-    auto vfrag = [&](const unsigned char* V, int db, int kp) {
-        const int off = vbase + 8192 * kp + BK * 256 * (db >> 3) +
-                        (((2 * (db & 7) + (tc >> 1)) ^ pf256r_swz_v(8 * g + te)) << 4);
-        gi_s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GI_LDS gi_s4*)(V + off));
-        gi_s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GI_LDS gi_s4*)(V + off + 1024));
-        return __builtin_shufflevector(__builtin_bit_cast(h4x, lo), __builtin_bit_cast(h4x, hi), 0, 1, 2, 3, 4, 5,
-                                       6, 7);
-    };
-
-    // ---- per-lane state: O^T (16 blocks of 16 dims; this lane dims 16db + 4g + r), reference max, row sum
-    f4 o[NDB];
-#pragma unroll
-    for (int db = 0; db < NDB; db++) o[db] = f4{0.f, 0.f, 0.f, 0.f};
-    float m_run = 0.f, l_run = 0.f;
-    f4 negm = f4{0.f, 0.f, 0.f, 0.f}; // -m_run: the C operand that starts each QK chain
-
-    // this lane's keys of a tile: 32(kb/2) + 8g + 4(kb%2) + r, 4 consecutive per block
-    auto key_scales = [&](const float* sc, f4* out) {
-#pragma unroll
-        for (int kb = 0; kb < NKB; kb++)
-            out[kb] = *reinterpret_cast<const f4*>(sc + 32 * (kb >> 1) + 8 * g + 4 * (kb & 1));
-    };
-    auto qk = [&](int t, f4* s) {
-        const unsigned char* K = kbuf(t);
-        h8 kf[PF_KPF];
-#pragma unroll
-        for (int st = 0; st < PF_KPF; st++) kf[st] = kfrag(K, st);
-        __builtin_amdgcn_sched_barrier(0);
-        const f4 zero = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int st = 0; st < NKB * KS; st++) {
-            const int kb = st % NKB, ks = st / NKB;
-            const h8 cur = kf[st % PF_KPF];
-            if (st + PF_KPF < NKB * KS) kf[st % PF_KPF] = kfrag(K, st + PF_KPF);
-            s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cur, qf[ks], ks == 0 ? (FMT == 1 ? zero : negm) : s[kb], 0, 0,
-                                                           0);
-        }
-        if constexpr (FMT == 1) { // the score: the integer key's dot product times its scale, less the max
-            f4 ksv[NKB];
-            key_scales(kscl(t), ksv);
-#pragma unroll
-            for (int kb = 0; kb < NKB; kb++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) s[kb][r] = fmaf(s[kb][r], ksv[kb][r], -m_run);
-        }
-    };
-    auto rowmax = [&](const f4* sc) {
-        float mx = GI_NEG_INF;
-#pragma unroll
-        for (int kb = 0; kb < NKB; kb++) mx = fmaxf(mx, fmaxf(fmaxf(sc[kb][0], sc[kb][1]), fmaxf(sc[kb][2], sc[kb][3])));
-        return rows_max(mx);
-    };
-    const int wave_first = a.pos0 + q0 + PF256R_ROWS * wave; // position of the wave's first row
-    const int wave_last = wave_first + PF256R_ROWS - 1;
-    const int my_tiles = min(ntiles, wave_last / BK + 1);
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-
-    // one step: the rare rescale, then QK of tile it+1 into sn under tile it's probabilities and P V, and tile
-    // it+1's row max (mx on exit)
-    auto step = [&](int it, f4* s, f4* sn, float& mx) {
-        const bool up = mx > PF_RESCALE_LOG2 || it == 0;
-        if (__builtin_amdgcn_ballot_w64(up)) {
-            const float delta = up ? mx : 0.f;
-            const float alpha = __builtin_amdgcn_exp2f(-fmaxf(delta, 0.f));
-            m_run += delta;
-            negm = f4{-m_run, -m_run, -m_run, -m_run};
-            l_run *= alpha;
-#pragma unroll
-            for (int db = 0; db < NDB; db++) gi_acc_scale<false>(o[db], alpha);
-#pragma unroll
-            for (int kb = 0; kb < NKB; kb++) s[kb] -= delta;
-        }
-        qk(it + 1, sn);
-        h8 pf[NKB / 2]; // k-step kp: keys 32kp + 8g + e, e = 4(kb%2) + r for block kb = 2kp + kb%2
-        f4 vsv[FMT == 1 ? NKB : 1];
-        if constexpr (FMT == 1) key_scales(vscl(it), vsv);
-#pragma unroll
-        for (int kb = 0; kb < NKB; kb++)
-#pragma unroll
-            for (int r = 0; r < 4; r += 2) {
-                const float p0 = __builtin_amdgcn_exp2f(s[kb][r]), p1 = __builtin_amdgcn_exp2f(s[kb][r + 1]);
-                const _Float16 h0 = (_Float16)p0, h1 = (_Float16)p1;
-                if constexpr (FMT == 1) { // P V weights: f16(p * vscale * 2^10)
-                    pf[kb >> 1][4 * (kb & 1) + r] = (_Float16)(p0 * (vsv[kb][r] * 1024.f));
-                    pf[kb >> 1][4 * (kb & 1) + r + 1] = (_Float16)(p1 * (vsv[kb][r + 1] * 1024.f));
-                } else {
-                    pf[kb >> 1][4 * (kb & 1) + r] = h0;
-                    pf[kb >> 1][4 * (kb & 1) + r + 1] = h1;
-                }
-                l_run = __builtin_amdgcn_fdot2(h2{h0, h1}, h2{(_Float16)1.f, (_Float16)1.f}, l_run, false);
-            }
-        const unsigned char* V = vbuf(it);
-        if constexpr (VPF > 0) {
-            // register staging: V^T fragments stream through a ring of VPF registers, each read VPF MFMAs
-            // before its use (the f16 kernel measured faster with the compiler's own order)
-            constexpr int NPV = (NKB / 2) * NDB;
-            h8 vq[VPF > 0 ? VPF : 1];
-#pragma unroll
-            for (int i = 0; i < VPF; i++) vq[i] = vfrag(V, i % NDB, i / NDB);
-#pragma unroll
-            for (int i = 0; i < NPV; i++) {
-                const int kp = i / NDB, db = i % NDB;
-                const h8 cur = vq[i % VPF];
-                if (i + VPF < NPV) vq[i % VPF] = vfrag(V, (i + VPF) % NDB, (i + VPF) / NDB);
-                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cur, pf[kp], o[db], 0, 0, 0);
-            }
-        } else {
-#pragma unroll
-            for (int kp = 0; kp < NKB / 2; kp++)
-#pragma unroll
-                for (int db = 0; db < NDB; db++)
-                    o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vfrag(V, db, kp), pf[kp], o[db], 0, 0, 0);
-        }
-        mx = rowmax(sn);
-#pragma unroll
-        for (int i = 0; i < NKB * KS; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (i + PF_KPF < NKB * KS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-        if constexpr (VPF > 0) { // then the first V reads, and each P V MFMA followed by its ring refill
-            __builtin_amdgcn_sched_group_barrier(0x100, 2 * VPF, 0);
-#pragma unroll
-            for (int i = 0; i < (NKB / 2) * NDB; i++) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                if (i + VPF < (NKB / 2) * NDB) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-            }
-        }
-    };
-
-    // prologue: K of tiles 0..NKBUF-1 and V of tiles 0..NVBUF-2 start loading; K(0) is waited for and
-    // published (the rest are waited for by the iterations that first read them)
-    const int last_k0 = min(NKBUF - 1, ntiles - 1), last_v0 = min(NVBUF - 2, ntiles - 1);
-    for (int t = 0; t <= (stage_v ? last_v0 : last_k0); t++) {
-        if constexpr (REG) {
-            issue(t);
-            commit();
-        } else {
-            stage(t);
-        }
-    }
-    if constexpr (REG) { // the tile iteration 0 widens
-        if (!stage_v && NKBUF < ntiles) issue(NKBUF);
-        if (stage_v && NVBUF - 1 < ntiles) issue(NVBUF - 1);
-        __builtin_amdgcn_s_waitcnt(GI_LGKMCNT0);
-    }
-    if (!stage_v) wait_tiles(last_k0);
-    asm volatile("s_barrier" ::: "memory");
-    float mx = GI_NEG_INF;
-    auto iteration = [&](int it, f4* s, f4* sn) {
-        // K waves need K(it+1), having issued up to K(it + NKBUF - 1); V waves need V(it), issued up to
-        // V(it + NVBUF - 2)
-        if (stage_v) wait_tiles(max(min(it + NVBUF - 2, ntiles - 1) - it, 0));
-        else wait_tiles(max(min(it + NKBUF - 1, ntiles - 1) - (it + 1), 0));
-        if constexpr (REG) __builtin_amdgcn_s_waitcnt(GI_LGKMCNT0); // the widened tile's writes, before they publish
-        asm volatile("s_barrier" ::: "memory");
-        if constexpr (!REG) {
-            if (!stage_v && it + NKBUF < ntiles) stage(it + NKBUF);    // into K(it)'s buffer
-            if (stage_v && it + NVBUF - 1 < ntiles) stage(it + NVBUF - 1); // into V(it-1)'s buffer
-        }
-        if (it < my_tiles) {
-            const int t0 = it * BK;
-            if (t0 + BK - 1 > wave_first) { // the tile crosses the diagonal somewhere in the wave
-                const int lim = qpos - t0;
-#pragma unroll
-                for (int kb = 0; kb < NKB; kb++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (32 * (kb >> 1) + 8 * g + 4 * (kb & 1) + r > lim) s[kb][r] = GI_NEG_INF;
-                mx = rowmax(s);
-            }
-            step(it, s, sn, mx);
-        }
-        if constexpr (REG) restage(it);
-    };
-    f4 sa[NKB], sb[NKB];
-    if (my_tiles > 0) {
-        qk(0, sa);
-        mx = rowmax(sa);
-    }
-    for (int it = 0; it < ntiles; it += 2) {
-        iteration(it, sa, sb);
-        if (it + 1 < ntiles) iteration(it + 1, sb, sa);
-    }
-
-    // ---- normalise and write: lane holds query c, dims 16db + 4g + r
-    const float l = rows_sum(l_run);
-    if (qrow < a.n) {
-        const float inv = FMT == 1 ? (1.f / 1024.f) / l : 1.f / l;
-        if (a.out_f16) {
-            _Float16* op = (_Float16*)a.out + (long long)qrow * a.out_stride + h * HD + 4 * g;
-#pragma unroll
-            for (int db = 0; db < NDB; db++)
-                *reinterpret_cast<h4x*>(op + 16 * db) = h4x{(_Float16)(o[db][0] * inv), (_Float16)(o[db][1] * inv),
-                                                            (_Float16)(o[db][2] * inv), (_Float16)(o[db][3] * inv)};
-        } else {
-            float* op = (float*)a.out + (long long)qrow * a.out_stride + h * HD + 4 * g;
-#pragma unroll
-            for (int db = 0; db < NDB; db++)
-                *reinterpret_cast<float4*>(op + 16 * db) =
-                    make_float4(o[db][0] * inv, o[db][1] * inv, o[db][2] * inv, o[db][3] * inv);
-        }
-    }
-}
-
 // Kernels of head sizes 64 and 128 (_w4: 4 waves, 128 rows). The launch bound of 8 waves caps every form at 256
 // registers: past that the compiler keeps all MFMA accumulators in AGPRs and copies them to VGPRs for the softmax and
 // the rescale (96 to 270 copies per tile; the 4-wave form measured 702 us instead of 580 at 8192 tokens).
-#define GI_PREFILL_KERNEL(name, I8, HD, STG, WAVES, RING)                                                              \
-    extern "C" __global__ void __launch_bounds__(512) name(GiPrefillArgs a) { gi_prefill_t<I8, HD, STG, WAVES, RING>(a); }
-GI_PREFILL_KERNEL(gi_prefill_fwd, false, 128, false, 8, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_w4, false, 128, false, 4, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_h64, false, 64, false, 8, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_h64_w4, false, 64, false, 4, 4)
+#define GI_PREFILL_KERNEL(name, FMT, HD, STG, WAVES, RING)                                                              \
+    extern "C" __global__ void __launch_bounds__(512) name(GiPrefillArgs a) { gi_prefill_t<FMT, HD, STG, WAVES, RING>(a); }
+GI_PREFILL_KERNEL(gi_prefill_fwd, 0, 128, false, 8, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_w4, 0, 128, false, 4, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64, 0, 64, false, 8, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64_w4, 0, 64, false, 4, 4)
 // the int8 cache pre-widened by gi_kv_widen, staged as the f16 cache is
-GI_PREFILL_KERNEL(gi_prefill_fwd_i8s, true, 128, true, 8, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_i8s_w4, true, 128, true, 4, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s, true, 64, true, 8, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s_w4, true, 64, true, 4, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_i8s, 1, 128, true, 8, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_i8s_w4, 1, 128, true, 4, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s, 1, 64, true, 8, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s_w4, 1, 64, true, 4, 4)
 // int8 tiles widened through registers (the chunks in flight leave room for a ring of 2; with 4 waves, twice the
 // chunks a thread, 36 registers spill and a tile takes twice as long)
-GI_PREFILL_KERNEL(gi_prefill_fwd_i8, true, 128, false, 8, 2)
-GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8, true, 64, false, 8, 2)
+GI_PREFILL_KERNEL(gi_prefill_fwd_i8, 1, 128, false, 8, 2)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8, 1, 64, false, 8, 2)
 
-#ifndef PF256R_KBUF
-#define PF256R_KBUF 2 // K tile buffers of gi_prefill_fwd_h256r
-#endif
-#ifndef PF256R_VBUF
-#define PF256R_VBUF 2 // V tile buffers of gi_prefill_fwd_h256r
-#endif
-extern "C" __global__ void __launch_bounds__(64 * PF256R_WAVES, 1) gi_prefill_fwd_h256r(GiPrefillArgs a) {
-    gi_prefill256r<PF256R_KBUF, PF256R_VBUF>(a);
-}
-extern "C" __global__ void __launch_bounds__(64 * PF256R_WAVES, 1) gi_prefill_fwd_h256r_i8(GiPrefillArgs a) {
-    gi_prefill256r<PF256R_KBUF, PF256R_VBUF, 1>(a);
-}
-extern "C" __global__ void __launch_bounds__(64 * PF256R_WAVES, 1) gi_prefill_fwd_h256r_q4(GiPrefillArgs a) {
-    gi_prefill256r<PF256R_KBUF, PF256R_VBUF, 2>(a);
-}
+// Head size 256 (4 waves, 128 rows; _w2: 2 waves, 64 rows): 32-row waves need 424 to 472 registers (O^T alone 128), so one wave
+// per SIMD and the accumulators in AGPRs; O^T stays there through the rescale (gi_acc_scale), the scores are copied out, 32
+// per tile, with issue slots to spare under 2,048 MFMA cycles a tile.
+extern "C" __global__ void __launch_bounds__(256, 1) gi_prefill_fwd_h256(GiPrefillArgs a) { gi_prefill_t<0, 256, false, 4, 8, 8>(a); }
+extern "C" __global__ void __launch_bounds__(128, 1) gi_prefill_fwd_h256_w2(GiPrefillArgs a) { gi_prefill_t<0, 256, false, 2, 8, 8>(a); }
+extern "C" __global__ void __launch_bounds__(128, 1) gi_prefill_fwd_h256_i8s_w2(GiPrefillArgs a) { gi_prefill_t<1, 256, true, 2, 8, 8>(a); }
+extern "C" __global__ void __launch_bounds__(256, 1) gi_prefill_fwd_h256_i8(GiPrefillArgs a) { gi_prefill_t<1, 256, false, 4, 4, 8>(a); }
+extern "C" __global__ void __launch_bounds__(256, 1) gi_prefill_fwd_h256_q4(GiPrefillArgs a) { gi_prefill_t<2, 256, false, 4, 4, 8>(a); }
 // the int8 cache pre-widened by gi_kv_widen (the 4-bit cache pre-widened runs gi_prefill_fwd_h256r itself)
-extern "C" __global__ void __launch_bounds__(64 * PF256R_WAVES, 1) gi_prefill_fwd_h256r_i8s(GiPrefillArgs a) {
-    gi_prefill256r<PF256R_KBUF, PF256R_VBUF, 1, true>(a);
-}
+extern "C" __global__ void __launch_bounds__(256, 1) gi_prefill_fwd_h256_i8s(GiPrefillArgs a) { gi_prefill_t<1, 256, true, 4, 8, 8>(a); }
 
 // ------------------------------------------------------------------------------------------------ KV store
 

@@ -9,7 +9,8 @@ import pytest
 import torch
 
 import gi_attn
-from attn_common import assert_close, make_inputs, make_inputs_i8, reference_f64, reference_f64_i8
+from attn_common import (assert_close, make_inputs, make_inputs_i8, make_inputs_q4, reference_f64, reference_f64_i8,
+                         reference_f64_q4)
 
 pytestmark = pytest.mark.gpu
 
@@ -96,3 +97,32 @@ def test_sliced_prefill_graph_replay(gpu):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want), f"replay {r}"
+
+
+@pytest.mark.parametrize("n,pos0,n_heads,n_kv", [(16, 1008, 4, 4), (17, 1008, 16, 2), (50, 2500, 12, 2), (255, 1200, 8, 1),
+                                                 (300, 4000, 16, 2)])
+def test_sliced_prefill_h256_every_cache(gpu, n, pos0, n_heads, n_kv):
+    # head size 256: f16, int8 and 4-bit, both stagings alike, rows at the edges of waves and of tiles of 64 and 128
+    print("[case] sliced prefill h256", n, pos0, n_heads, n_kv, flush=True)
+    hd = 256
+    assert sliced(n, pos0, n_heads, n_kv, hd, 0)
+    q, k, v = make_inputs(9400 + n, n, pos0 + n, n_heads, n_kv, hd=hd)
+    qt = dev(q, gpu, n, n_heads * hd)
+    kt, vt = (dev(x.view(np.int16), gpu, -1, n_kv, hd).view(torch.float16) for x in (k, v))
+    got = gi_attn.prefill(qt, kt, vt, pos0, n_heads, n_kv, hd=hd)
+    q8, k8, v8, ks, vs = make_inputs_i8(9500 + n, n, pos0 + n, n_heads, n_kv, hd=hd)
+    q8t, kt, vt = dev(q8, gpu, n, n_heads * hd), dev(k8, gpu, -1, n_kv, hd), dev(v8, gpu, -1, n_kv, hd)
+    kw = dict(hd=hd, k_scale=dev(ks, gpu, -1, n_kv), v_scale=dev(vs, gpu, -1, n_kv))
+    got8, tile8 = (gi_attn.prefill(q8t, kt, vt, pos0, n_heads, n_kv, staged=s, **kw) for s in (True, False))
+    q4, kc, vc, ks4, vs4 = make_inputs_q4(9600 + n, n, pos0 + n, n_heads, n_kv)
+    t4 = [dev(q4, gpu, n, n_heads * hd), dev(kc, gpu, -1, n_kv, 128), dev(vc, gpu, -1, n_kv, 128)]
+    t4 += [dev(np.ascontiguousarray(x).view(np.int16), gpu, -1, n_kv, 8).view(torch.float16) for x in (ks4, vs4)]
+    got4, tile4 = (gi_attn.prefill_q4(*t4, pos0, n_heads, n_kv, staged=s) for s in (True, False))
+    torch.cuda.synchronize()
+    assert torch.equal(got8, tile8) and torch.equal(got4, tile4)
+    for r in sorted({0, 1, n // 2, n - 1}):
+        assert_close(got[r:r + 1].cpu().numpy(), reference_f64(q[r:r + 1], k, v, pos0 + r, n_heads, n_kv, hd=hd), what=f"row {r}")
+        assert_close(got8[r:r + 1].cpu().numpy(), reference_f64_i8(q8[r:r + 1], k8, v8, ks, vs, pos0 + r, n_heads, n_kv, hd=hd),
+                     what=f"i8 row {r}")
+        assert_close(got4[r:r + 1].cpu().numpy(), reference_f64_q4(q4[r:r + 1], kc, vc, ks4, vs4, pos0 + r, n_heads, n_kv),
+                     what=f"q4 row {r}")
