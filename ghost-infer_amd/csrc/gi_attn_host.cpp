@@ -167,7 +167,7 @@ bool f32_hd(int hd) { return hd % 16 == 0 && hd >= 16 && hd <= 112 && hd != 64; 
 constexpr int kF32Sizes[6] = {16, 32, 48, 80, 96, 112}; // the f32 kernels' builds, in this order
 int f32_index(int hd) { return hd < 64 ? hd / 16 - 1 : hd / 16 - 2; }
 constexpr int kMaxDevices = 64;
-constexpr int kRopeHeads = 16; // heads per gi_qk_norm_rope workgroup; must match the kernels' ROPE_HEADS
+constexpr int kRopeHeads = 16; // heads per gi_qk_norm_rope workgroup (gi_qk_norm_rope_1: 4)
 constexpr int kCombineSplit = 8; // combine workgroups per (head, token); must match the kernels' CMB_DSPLIT
 constexpr int kDecWaves = 4, kDecTile = 32, kDecPairs = 8; // slice partials are hd + 4 floats
 constexpr int kSliceUnit = kDecWaves * kDecTile; // 128 keys
@@ -220,7 +220,7 @@ struct Module {
     hipFunction_t prefill_f32p[2][2] = {}; // f32 prompts at head sizes 64 and 128: [int8 cache][64, 128]
     hipFunction_t widen = nullptr; // the int8 and 4-bit keys widened into a workspace
     hipFunction_t prefill_combine[2] = {}; // merge of a sliced prefill's partials: 32 rows per wave
-    hipFunction_t combine = nullptr, rope = nullptr, relayout = nullptr, hadamard = nullptr;
+    hipFunction_t combine = nullptr, rope = nullptr, rope1 = nullptr, relayout = nullptr, hadamard = nullptr;
     // gi_attn_decode_noalloc's partials: the device address of the code object's gi_scratch array on this
     // device (the array's host-side name is no device address; the module gives the real one at load)
     void* scratch = nullptr;
@@ -302,6 +302,7 @@ int load_module(const char* path, Module** out) {
             {&m.widen, "gi_kv_widen"},
             {&m.prefill_combine[0], "gi_prefill_combine_32"},
             {&m.rope, "gi_qk_norm_rope"},
+            {&m.rope1, "gi_qk_norm_rope_1"},
         };
         for (auto& f : fns)
             if (int e = check(hipModuleGetFunction(f.f, m.mod, f.name), f.name)) {
@@ -672,8 +673,11 @@ int rope_impl(void* stream, float* qkv, const float* qn, const float* kn, void* 
     a.base = base;
     a.eps = eps;
     a.neox = neox != 0;
-    const int groups = (n_heads + 2 * n_kv + kRopeHeads - 1) / kRopeHeads; // workgroups per token
-    return launch(kRope, m->rope, dim3(groups, n, 1), dim3(256), (hipStream_t)stream, &a, sizeof a);
+    // few tokens: one head per wave, so that a launch of less than a workgroup per CU is four times as wide
+    const int items = n_heads + 2 * n_kv;
+    const bool wide = (long long)n * ((items + kRopeHeads - 1) / kRopeHeads) < 256;
+    const int per = wide ? 4 : kRopeHeads, groups = (items + per - 1) / per; // workgroups per token
+    return launch(kRope, wide ? m->rope1 : m->rope, dim3(groups, n, 1), dim3(256), (hipStream_t)stream, &a, sizeof a);
 }
 
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }

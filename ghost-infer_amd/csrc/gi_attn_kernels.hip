@@ -2228,32 +2228,83 @@ struct GiRopeArgs {
 // A q or k head: RMSNorm (ss = sum of squares over the head, scale = rsqrt(ss/hd + eps), times the
 // weights), then RoPE on rope_dim/2 pairs (freq_i = base^(-2i/rope_dim) / ff[i], angle = pos * freq_i, all
 // f32), written back into qkv; a k head also goes to the K cache. A v head goes to the V cache unchanged.
-// Cache values are rounded to nearest even. One workgroup per (token, group of ROPE_HEADS heads of the
+// Cache values are rounded to nearest even. One workgroup per (token, group of 4 or 16 heads of the
 // packed row: q heads, then k, then v): the pairs' sines and cosines depend only on the position, so the
-// workgroup computes them once into LDS for all its heads; each wave loads its ROPE_HEADS/4 heads at once
-// and takes them one at a time through a per-wave LDS row (any two dims can pair).
-#define ROPE_HEADS 16
+// workgroup computes them once into LDS for all its heads; each wave loads its heads at once and takes them one at a
+// time, pairs through a lane swap (whole heads rotated in halves) or a per-wave LDS row (any two dims can pair).
 // The normalized 256-point Walsh-Hadamard transform of a row held 4 values per lane (lane l: values 4l..4l+3):
 // kv4_fwht's stages (src/cuda.rs:242-256) in its order, h = 1, 2 inside the lane, h = 4..128 across lanes
 // l and l ^ (h/4). Each stage gives the lower element a + c and the upper one a - c, single f32 operations as
 // the reference's, so the result is bit-identical to it; then every value times 1/16.
+// Lane l's value of lane l ^ M, on the VALU (a shuffle would be an LDS round trip, and the rows here need 6 to 24 of them in
+// a dependent chain).
+template <int M> __device__ __forceinline__ float gi_xor_lane(float v) {
+    static_assert(M == 1 || M == 2 || M == 4 || M == 8, "within a 16-lane row");
+    const int x = __float_as_int(v);
+    if constexpr (M == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, true)); // quad_perm [1,0,3,2]
+    if constexpr (M == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, true)); // quad_perm [2,3,0,1]
+    if constexpr (M == 4) // row_half_mirror (l ^ 7), then quad_perm [3,2,1,0] (l ^ 3)
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true));
+    return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x128, 0xF, 0xF, true)); // row_ror 8
+}
+// lo: the value of the lane of the pair (l, l ^ M) with bit M clear, hi: of the other
+struct GiPair { float lo, hi; };
+template <int M> __device__ __forceinline__ GiPair gi_pair(float v) {
+    static_assert(M == 16 || M == 32, "across 16-lane rows");
+    const int x = __float_as_int(v);
+    if constexpr (M == 16) {
+        const auto p = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        return GiPair{__int_as_float(p[0]), __int_as_float(p[1])};
+    } else {
+        const auto p = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        return GiPair{__int_as_float(p[0]), __int_as_float(p[1])};
+    }
+}
+// sum and max over the wave, in the order of shuffles by 32, 16, .. 1
+__device__ __forceinline__ float gi_wave_sum(float v) {
+    GiPair p = gi_pair<32>(v);
+    v = p.lo + p.hi;
+    p = gi_pair<16>(v);
+    v = p.lo + p.hi;
+    v += gi_xor_lane<8>(v);
+    v += gi_xor_lane<4>(v);
+    v += gi_xor_lane<2>(v);
+    return v + gi_xor_lane<1>(v);
+}
+__device__ __forceinline__ float gi_oct_max(float v) { // over lanes l ^ 1, 2, 4
+    v = fmaxf(v, gi_xor_lane<4>(v));
+    v = fmaxf(v, gi_xor_lane<2>(v));
+    return fmaxf(v, gi_xor_lane<1>(v));
+}
+__device__ __forceinline__ float gi_wave_max(float v) {
+    GiPair p = gi_pair<32>(v);
+    v = fmaxf(p.lo, p.hi);
+    p = gi_pair<16>(v);
+    v = fmaxf(p.lo, p.hi);
+    return gi_oct_max(fmaxf(v, gi_xor_lane<8>(v)));
+}
 __device__ __forceinline__ void gi_fwht256(float __attribute__((ext_vector_type(4))) & x, int lane) {
     float t;
     t = x[0]; x[0] = t + x[1]; x[1] = t - x[1];
     t = x[2]; x[2] = t + x[3]; x[3] = t - x[3];
     t = x[0]; x[0] = t + x[2]; x[2] = t - x[2];
     t = x[1]; x[1] = t + x[3]; x[3] = t - x[3];
+    // a stage across lanes: the lower lane own + partner, the upper partner - own (the products by +-1 are exact)
+    const float s1 = lane & 1 ? -1.f : 1.f, s2 = lane & 2 ? -1.f : 1.f, s4 = lane & 4 ? -1.f : 1.f,
+                s8 = lane & 8 ? -1.f : 1.f, s16 = lane & 16 ? -1.f : 1.f, s32 = lane & 32 ? -1.f : 1.f;
 #pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-        const bool upper = lane & m;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float p = __shfl_xor(x[j], m, 64);
-            x[j] = upper ? p - x[j] : x[j] + p;
-        }
+    for (int j = 0; j < 4; j++) {
+        float v = x[j];
+        v = fmaf(v, s1, gi_xor_lane<1>(v));
+        v = fmaf(v, s2, gi_xor_lane<2>(v));
+        v = fmaf(v, s4, gi_xor_lane<4>(v));
+        v = fmaf(v, s8, gi_xor_lane<8>(v));
+        GiPair p = gi_pair<16>(v);
+        v = fmaf(p.hi, s16, p.lo);
+        p = gi_pair<32>(v);
+        v = fmaf(p.hi, s32, p.lo);
+        x[j] = v * 0.0625f;
     }
-#pragma unroll
-    for (int j = 0; j < 4; j++) x[j] *= 0.0625f;
 }
 
 // One head row (PER values per lane) into a cache row. f16: rounded to nearest even. int8 (kv_store's KV8,
@@ -2277,7 +2328,7 @@ __device__ __forceinline__ void gi_store_row(const GiRopeArgs& a, uint16_t* cach
     for (int j = 0; j < PER; j++) amax = fmaxf(amax, fabsf(x[j]));
     if constexpr (PER == 4) {
         if (a.fmt == 2) {
-            for (int m = 4; m > 0; m >>= 1) amax = fmaxf(amax, __shfl_xor(amax, m, 64));
+            amax = gi_oct_max(amax);
             const _Float16 dh = (_Float16)__fdiv_rn(amax, 7.f);
             const float dd = (float)dh, inv = dd != 0.f ? __fdiv_rn(1.f, dd) : 0.f;
             uint32_t w = 0;
@@ -2291,7 +2342,7 @@ __device__ __forceinline__ void gi_store_row(const GiRopeArgs& a, uint16_t* cach
             return;
         }
     }
-    for (int m = 32; m > 0; m >>= 1) amax = fmaxf(amax, __shfl_xor(amax, m, 64));
+    amax = gi_wave_max(amax);
     const float dd = __fdiv_rn(amax, 127.f), inv = dd != 0.f ? __fdiv_rn(1.f, dd) : 0.f;
     typedef int8_t bv __attribute__((ext_vector_type(PER)));
     bv q;
@@ -2304,7 +2355,10 @@ __device__ __forceinline__ void gi_store_row(const GiRopeArgs& a, uint16_t* cach
 // PER = hd / 64 values per lane, dims PER*lane .. PER*lane + PER - 1 (one 4, 8 or 16-byte access per row).
 // MASKED (PER = 2): any even head size up to 128 (the f32 kernels' head sizes): lanes past hd / 2 hold zeros and
 // neither load nor store.
-template <int PER, bool MASKED = false>
+// HPW: heads of the row per wave (a workgroup: 4 HPW). 4 where the tokens fill the chip; 1 for a few tokens, whose time is
+// one wave's chain (one token of 32/8 heads of 128 into the int8 cache: 5.8 us with 4, 3.4 us with 1; 1500 tokens 22.5
+// us before the loads went ahead of the sines and the row reductions to the VALU, 18.6 us after).
+template <int PER, int HPW, bool MASKED = false>
 __device__ __forceinline__ void gi_qk_norm_rope_t(const GiRopeArgs& a, float (*cs_sh)[2], float (*row_sh)[256]) {
     typedef float fv __attribute__((ext_vector_type(PER)));
     static_assert(!MASKED || PER == 2, "the lane-masked form: two values per lane");
@@ -2312,9 +2366,24 @@ __device__ __forceinline__ void gi_qk_norm_rope_t(const GiRopeArgs& a, float (*c
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const bool act = !MASKED || PER * lane < HD; // the lane holds dims of the head
     const int items = a.n_heads + 2 * a.n_kv;
-    const int b = blockIdx.y, h0 = blockIdx.x * ROPE_HEADS;
-    const int pos = (a.posp ? *a.posp : a.pos0) + b;
+    const int b = blockIdx.y, h0 = blockIdx.x * 4 * HPW;
     const int half = a.rope_dim >> 1;
+    float* row = a.qkv + (long long)b * a.row_stride;
+    float* sh = row_sh[wave];
+    // all of this wave's head rows and the norms' weights are loaded first and arrive under the sines
+    fv v[HPW];
+#pragma unroll
+    for (int k = 0; k < HPW; k++) {
+        const int h = h0 + wave + 4 * k;
+        v[k] = fv{};
+        if (h < items && act) v[k] = *reinterpret_cast<const fv*>(row + (long long)h * HD + PER * lane); // q, k, v heads in turn
+    }
+    fv qw = fv{}, kw = fv{};
+    if (a.qn && act) {
+        if (h0 < a.n_heads) qw = *reinterpret_cast<const fv*>(a.qn + PER * lane);
+        if (h0 + 4 * HPW > a.n_heads) kw = *reinterpret_cast<const fv*>(a.kn + PER * lane);
+    }
+    const int pos = (a.posp ? *a.posp : a.pos0) + b;
     if (tid < half && h0 < a.n_heads + a.n_kv) { // (a workgroup of v heads only rotates nothing)
         float freq = powf(a.base, -2.0f * (float)tid / (float)a.rope_dim);
         if (a.ff) freq /= a.ff[tid];
@@ -2324,17 +2393,17 @@ __device__ __forceinline__ void gi_qk_norm_rope_t(const GiRopeArgs& a, float (*c
         cs_sh[tid][1] = s;
     }
     __syncthreads();
-    float* row = a.qkv + (long long)b * a.row_stride;
-    float* sh = row_sh[wave];
-    // all of this wave's head rows are loaded up front (more bytes in flight per wave), then processed
-    constexpr int HPW = ROPE_HEADS / 4;
-    fv v[HPW];
+    // the whole head rotated in pairs (i, i + hd/2): lanes l and l ^ 32 hold a pair, swapped on the VALU, the pair's cosine
+    // and sine in registers for all heads
+    const bool swap = !MASKED && a.neox && a.rope_dim == HD;
+    fv cc = fv{}, ss = fv{};
+    if (swap)
 #pragma unroll
-    for (int k = 0; k < HPW; k++) {
-        const int h = h0 + wave + 4 * k;
-        v[k] = fv{};
-        if (h < items && act) v[k] = *reinterpret_cast<const fv*>(row + (long long)h * HD + PER * lane); // q, k, v heads in turn
-    }
+        for (int j = 0; j < PER; j++) {
+            const int i = (PER * lane + j) & (HD / 2 - 1);
+            cc[j] = cs_sh[i][0];
+            ss[j] = cs_sh[i][1];
+        }
 #pragma unroll
     for (int k = 0; k < HPW; k++) {
         const int h = h0 + wave + 4 * k;
@@ -2348,26 +2417,32 @@ __device__ __forceinline__ void gi_qk_norm_rope_t(const GiRopeArgs& a, float (*c
         }
         fv x = v[k];
         if (a.qn) {
-            const float* w = h < a.n_heads ? a.qn : a.kn;
-            float ss = 0.f;
+            const fv wv = h < a.n_heads ? qw : kw;
+            float sq = 0.f;
 #pragma unroll
-            for (int j = 0; j < PER; j++) ss = fmaf(x[j], x[j], ss);
-            for (int m = 32; m > 0; m >>= 1) ss += __shfl_xor(ss, m, 64);
-            const float scale = __frsqrt_rn(ss / (float)HD + a.eps);
-            const fv wv = act ? *reinterpret_cast<const fv*>(w + PER * lane) : fv{};
+            for (int j = 0; j < PER; j++) sq = fmaf(x[j], x[j], sq);
+            const float scale = __frsqrt_rn(gi_wave_sum(sq) / (float)HD + a.eps);
 #pragma unroll
             for (int j = 0; j < PER; j++) x[j] = x[j] * scale * wv[j];
         }
-        if (act) *reinterpret_cast<fv*>(sh + PER * lane) = x;
-        __builtin_amdgcn_wave_barrier();
-        for (int i = lane; i < half; i += 64) {
-            const int ia = a.neox ? i : 2 * i, ib = a.neox ? i + half : 2 * i + 1;
-            const float p = sh[ia], q = sh[ib], c = cs_sh[i][0], s = cs_sh[i][1];
-            sh[ia] = p * c - q * s;
-            sh[ib] = p * s + q * c;
+        if (swap) {
+#pragma unroll
+            for (int j = 0; j < PER; j++) {
+                const GiPair p = gi_pair<32>(x[j]);
+                x[j] = lane < 32 ? p.lo * cc[j] - p.hi * ss[j] : p.lo * ss[j] + p.hi * cc[j];
+            }
+        } else {
+            if (act) *reinterpret_cast<fv*>(sh + PER * lane) = x;
+            __builtin_amdgcn_wave_barrier();
+            for (int i = lane; i < half; i += 64) {
+                const int ia = a.neox ? i : 2 * i, ib = a.neox ? i + half : 2 * i + 1;
+                const float p = sh[ia], q = sh[ib], c = cs_sh[i][0], s = cs_sh[i][1];
+                sh[ia] = p * c - q * s;
+                sh[ib] = p * s + q * c;
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (act) x = *reinterpret_cast<const fv*>(sh + PER * lane);
         }
-        __builtin_amdgcn_wave_barrier();
-        if (act) x = *reinterpret_cast<const fv*>(sh + PER * lane);
         // the 4-bit cache (src/cuda.rs:472-479): q and k heads rotated alike, so their dot products are kept
         if constexpr (PER == 4)
             if (a.fmt == 2) gi_fwht256(x, lane);
@@ -2376,14 +2451,17 @@ __device__ __forceinline__ void gi_qk_norm_rope_t(const GiRopeArgs& a, float (*c
         __builtin_amdgcn_wave_barrier(); // the row buffer is reused by the wave's next head
     }
 }
-extern "C" __global__ void __launch_bounds__(256) gi_qk_norm_rope(GiRopeArgs a) {
-    __shared__ float cs_sh[128][2];  // cos, sin of pair i
-    __shared__ float row_sh[4][256]; // a head row per wave
-    if (a.hd == 64) gi_qk_norm_rope_t<1>(a, cs_sh, row_sh);
-    else if (a.hd == 128) gi_qk_norm_rope_t<2>(a, cs_sh, row_sh);
-    else if (a.hd == 256) gi_qk_norm_rope_t<4>(a, cs_sh, row_sh);
-    else gi_qk_norm_rope_t<2, true>(a, cs_sh, row_sh);
-}
+#define GI_ROPE_KERNEL(name, HPW)                                                                                      \
+    extern "C" __global__ void __launch_bounds__(256) name(GiRopeArgs a) {                                             \
+        __shared__ float cs_sh[128][2];  /* cos, sin of pair i */                                                      \
+        __shared__ float row_sh[4][256]; /* a head row per wave */                                                     \
+        if (a.hd == 64) gi_qk_norm_rope_t<1, HPW>(a, cs_sh, row_sh);                                                   \
+        else if (a.hd == 128) gi_qk_norm_rope_t<2, HPW>(a, cs_sh, row_sh);                                             \
+        else if (a.hd == 256) gi_qk_norm_rope_t<4, HPW>(a, cs_sh, row_sh);                                             \
+        else gi_qk_norm_rope_t<2, HPW, true>(a, cs_sh, row_sh);                                                        \
+    }
+GI_ROPE_KERNEL(gi_qk_norm_rope, 4)
+GI_ROPE_KERNEL(gi_qk_norm_rope_1, 1)
 
 // ------------------------------------------------------------------------------- output rotation (4-bit cache)
 
