@@ -13,7 +13,7 @@
 // (times the key's scale for int8); the workgroup takes the tile's max and an online base-2 softmax; the value
 // scale rides on p. The slice's (unnormalised O, max, sum) go to the partial rows gi_decode_combine merges; one
 // slice writes the output.
-// Prefill (gi_prefill_f32_*): one workgroup of 8 waves per (head, 128 query rows), on v_mfma_f32_16x16x4f32 (f32
+// Prefill (gi_prefill_f32_*): one workgroup of 8 waves per (kv head, 128 packed query rows, key slice: PfUnit), on v_mfma_f32_16x16x4f32 (f32
 // operands, f32 accumulation). Tiles of 64 keys are widened to f32 in LDS (int8: times their scales) through
 // registers, the next tile's loads in flight while the current one is used. A wave holds 16 query rows: S^T blocks
 // (16 keys x 16 queries) from K (A) and Q^T (B, in registers); a lane then holds the scores of keys 4(l/16)..+3 of
@@ -171,16 +171,19 @@ __device__ __forceinline__ void gi_prefill_f32_t(const GiPrefillArgs& a) {
     __shared__ __attribute__((aligned(16))) float Ks[PF32_KT * LD];
     __shared__ __attribute__((aligned(16))) float Vs[PF32_KT * LD];
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, lc = l & 15, lg = l >> 4;
-    const int G = a.n_heads / a.n_kv;
-    const int qtiles = (a.n + PF32_ROWS - 1) / PF32_ROWS;
-    const int h = blockIdx.x % a.n_heads, q0 = (qtiles - 1 - blockIdx.x / a.n_heads) * PF32_ROWS; // longest first
-    const int kvh = h / G;
+    const int G = a.n_heads / a.n_kv, P = a.n * G;
+    const PfUnit un = pf_unit(a, PF32_ROWS, PF32_KT);
+    const int kvh = un.kvh;
+    if (un.t_begin >= un.t_end) return; // a slice past the tile's last key
     const int kv_len = a.pos0 + a.n;
-    const int kend = min(kv_len, a.pos0 + q0 + PF32_ROWS); // keys the workgroup's rows see
-    const int wq0 = q0 + 16 * w;                            // the wave's first row
-    const int wend = min(kv_len, a.pos0 + wq0 + 16);        // keys the wave's rows see
-    const int qrow = wq0 + lc;                              // this lane's query row
-    const int lim = a.pos0 + qrow;                          // its last visible key
+    const int kbeg = un.t_begin * PF32_KT, kend = un.t_end * PF32_KT; // keys of this workgroup's tiles
+    const int wrow = un.row0 + 16 * w;                                // the wave's first packed row
+    const int wfirst = a.pos0 + pf_token(a, wrow);                    // its position
+    const int wend = wrow < P ? a.pos0 + pf_last_token(a, wrow, 16) + 1 : 0; // keys the wave's rows see
+    const int qrow = wrow + lc;                                       // this lane's row
+    const int qtok = qrow < P ? pf_token(a, qrow) : a.n - 1;
+    const int h = kvh * G + (qrow < P ? qrow : P - 1) - qtok * G;
+    const int lim = a.pos0 + qtok;                                    // its last visible key
     const long long kvs = a.kv_stride, kbase = (long long)kvh * a.kv_head_stride;
     const long long sbase = (long long)kvh * a.sc_head_stride;
 
@@ -188,7 +191,7 @@ __device__ __forceinline__ void gi_prefill_f32_t(const GiPrefillArgs& a) {
     // k-steps is one 16-byte LDS read
     float qv[HD / 4];
     {
-        const long long e0 = (long long)min(qrow, a.n - 1) * a.q_stride + (long long)h * HD + 4 * lg;
+        const long long e0 = (long long)qtok * a.q_stride + (long long)h * HD + 4 * lg;
 #pragma unroll
         for (int j = 0; j < HD / 16; j++)
 #pragma unroll
@@ -248,8 +251,8 @@ __device__ __forceinline__ void gi_prefill_f32_t(const GiPrefillArgs& a) {
 #pragma unroll
     for (int d = 0; d < DB; d++) o[d] = f4{0.f, 0.f, 0.f, 0.f};
     float m_run = GI_NEG_INF, l_run = 0.f; // l_run: this lane's keys only, summed over the row's lanes at the end
-    load_tile(0);
-    for (int t0 = 0; t0 < kend; t0 += PF32_KT) {
+    load_tile(kbeg);
+    for (int t0 = kbeg; t0 < kend; t0 += PF32_KT) {
         __syncthreads(); // every wave is done with the previous tile
         store_tile();
         if (t0 + PF32_KT < kend) load_tile(t0 + PF32_KT);
@@ -268,7 +271,7 @@ __device__ __forceinline__ void gi_prefill_f32_t(const GiPrefillArgs& a) {
                 for (int i = 0; i < 4; i++) s[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kx[i], qv[4 * j + i], s[kb], 0, 0, 0);
             }
         // lane l holds key t0 + 16 kb + 4(l/16) + r of query row qrow in s[kb][r]
-        const bool edge = t0 + PF32_KT - 1 > a.pos0 + wq0 || t0 + PF32_KT > kv_len; // a mask reaches this tile
+        const bool edge = t0 + PF32_KT - 1 > wfirst || t0 + PF32_KT > kv_len; // a mask reaches this tile
         float mx = GI_NEG_INF;
 #pragma unroll
         for (int kb = 0; kb < 4; kb++)
@@ -280,14 +283,16 @@ __device__ __forceinline__ void gi_prefill_f32_t(const GiPrefillArgs& a) {
             }
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fmaxf(m_run, mx); // key 0 is visible to every row, so finite from the first tile on
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        const float m_new = fmaxf(m_run, mx);
+        // (a row that sees no key of a slice keeps max -inf and sum 0; with key 0 in the slice every row's is finite)
+        const float ref = m_new > GI_NEG_INF ? m_new : 0.f;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - ref);
         float ls = 0.f;
 #pragma unroll
         for (int kb = 0; kb < 4; kb++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                s[kb][r] = __builtin_amdgcn_exp2f(s[kb][r] - m_new);
+                s[kb][r] = __builtin_amdgcn_exp2f(s[kb][r] - ref);
                 ls += s[kb][r];
             }
         l_run = l_run * alpha + ls;
@@ -306,10 +311,18 @@ __device__ __forceinline__ void gi_prefill_f32_t(const GiPrefillArgs& a) {
     }
     l_run += __shfl_xor(l_run, 16, 64);
     l_run += __shfl_xor(l_run, 32, 64);
-    if (qrow < a.n) {
+    if (a.nslice > 1) { // a slice's partial (pf_part_o: fragment d holds the O^T block d)
+        if (w >= a.pwaves) return;
+        f4* po = reinterpret_cast<f4*>(pf_part_o<16>(a, HD, un.unit, w)) + l;
+#pragma unroll
+        for (int d = 0; d < DB; d++) po[64 * d] = o[d];
+        if (lg == 0) pf_part_ml<16>(a, HD, gridDim.x, un.unit, w)[lc] = make_float2(m_run, l_run);
+        return;
+    }
+    if (qrow < P) {
         // lane l holds dims 16 d + 4(l/16) + i of query row qrow
         const float inv = 1.f / l_run;
-        const long long e0 = (long long)qrow * a.out_stride + (long long)h * HD + 4 * lg;
+        const long long e0 = (long long)qtok * a.out_stride + (long long)h * HD + 4 * lg;
 #pragma unroll
         for (int d = 0; d < DB; d++)
 #pragma unroll

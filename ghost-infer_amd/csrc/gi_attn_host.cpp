@@ -159,7 +159,6 @@ struct GiPrefillArgs {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kF32Rows = 128;   // query rows per gi_prefill_f32_* workgroup; must match the kernels' PF32_ROWS
-constexpr int kF32Threads = 512; // its block size (8 waves of 16 rows)
 
 // Head sizes of the f32 kernels (gi_attn_f32.hip): the multiples of 16 up to 112 that the MFMA kernels do not
 // take, the reference's f32 fallback cases (attention_partial / attention_prefill, src/cuda.rs:1866-2041).
@@ -219,7 +218,7 @@ struct Module {
     hipFunction_t dec_f32[2][6] = {}, prefill_f32[2][6] = {}; // the f32 kernels: [int8 cache][kF32Sizes index]
     hipFunction_t prefill_f32p[2][2] = {}; // f32 prompts at head sizes 64 and 128: [int8 cache][64, 128]
     hipFunction_t widen = nullptr; // the int8 and 4-bit keys widened into a workspace
-    hipFunction_t prefill_combine[2] = {}; // merge of a sliced prefill's partials: 32 rows per wave
+    hipFunction_t prefill_combine[2] = {}; // merge of a sliced prefill's partials: 32 rows per wave, 16 (f32)
     hipFunction_t combine = nullptr, rope = nullptr, rope1 = nullptr, relayout = nullptr, hadamard = nullptr;
     // gi_attn_decode_noalloc's partials: the device address of the code object's gi_scratch array on this
     // device (the array's host-side name is no device address; the module gives the real one at load)
@@ -301,6 +300,7 @@ int load_module(const char* path, Module** out) {
             {&m.prefill256[1], "gi_prefill_fwd_h256_q4"},
             {&m.widen, "gi_kv_widen"},
             {&m.prefill_combine[0], "gi_prefill_combine_32"},
+            {&m.prefill_combine[1], "gi_prefill_combine_16"},
             {&m.rope, "gi_qk_norm_rope"},
             {&m.rope1, "gi_qk_norm_rope_1"},
         };
@@ -697,30 +697,32 @@ size_t prefill_ws_bytes(int kv_len, int n_kv, int hd, int fmt) {
 //  - Slices: a short batch over a long prefix leaves most of the chip idle while each workgroup walks all of its keys
 //    (512 tokens of 32/4 heads at a 16K prefix: 64 workgroups of 264 key tiles, 350 us). Such a launch cuts the key
 //    tiles of every row tile into slices, one workgroup each, whose partial results a second launch merges (137 us).
+//    An f32 tile takes three to five times as long, so those launches gain from shorter spans on (200 tokens of 32/32
+//    heads of 96 at 1800: 64 workgroups of 32 tiles, 227 us; sliced 69 us).
 // A row's arithmetic does not depend on the waves, only on the slices.
 struct PrefillPlan {
-    int waves;      // 8 or 4; head size 256: 4 or 2
+    int waves;      // 8 or 4; head size 256: 4 or 2; f32: 8 (of 16 rows)
     int tiles;      // key tiles per slice
     int nslice;     // slices of the longest row tile
 };
 constexpr int kPrefillRowTiles(long long rows, int per) { return (int)((rows + per - 1) / per); }
-PrefillPlan prefill_plan(int pos0, int n, int n_heads, int n_kv, int hd) {
+PrefillPlan prefill_plan(int pos0, int n, int n_heads, int n_kv, int hd, bool f32 = false) {
     const int G = n_heads / n_kv, cus = 256, tmax = (pos0 + n + kPrefillKeys - 1) / kPrefillKeys;
     const long long P = (long long)n * G;
-    const int most = hd == 256 ? 4 : 8;
+    const int most = hd == 256 ? 4 : 8, rw = f32 ? 16 : 32;
     PrefillPlan p{most, tmax, 1};
-    if ((long long)kPrefillRowTiles(P, 32 * most) * n_kv >= 2 * cus) return p; // longest tiles first balances these
+    if ((long long)kPrefillRowTiles(P, rw * most) * n_kv >= 2 * cus) return p; // longest tiles first balances these
     // Below 16 key tiles slices save less than the merge launch costs. A prompt of up to 4096 keys taken in chunks of
     // 256 tokens or more keeps each row's arithmetic independent of the chunking (one slice always); beyond, chunks
     // agree to f32 rounding.
-    const bool may_slice = tmax >= 16 && (n < 256 || pos0 + n > 4096);
+    const bool may_slice = tmax >= (f32 ? 4 : 16) && (n < 256 || pos0 + n > 4096);
     // Costs in units of one key tile of an 8-wave workgroup (1.4 to 1.9 us; head size 256: of a 4-wave one): rounds of workgroups over the CUs, each
     // with a fixed cost until its first tile is in and for its output (~6 us), and for a sliced launch the merge
     // launch (~5 us) and its read of the partials (~4 TB/s).
-    const double per_wg = 4.0, merge = 3.3;
+    const double tile_s = f32 ? 5e-6 : 1.5e-6, per_wg = f32 ? 1.2 : 4.0, merge = f32 ? 1.0 : 3.3;
     double best = 0;
-    for (int waves = most; waves >= most / 2; waves -= most / 2) {
-        const int rows = 32 * waves, items = kPrefillRowTiles(P, rows);
+    for (int waves = most; waves >= (f32 ? most : most / 2); waves -= most / 2) {
+        const int rows = rw * waves, items = kPrefillRowTiles(P, rows);
         const long long wgs = (long long)items * n_kv;
         const double tile = waves == most ? 1.0 : hd == 256 ? 0.85 : 0.7;
         auto tiles_of = [&](int i) { // key tiles of row tile i
@@ -732,7 +734,7 @@ PrefillPlan prefill_plan(int pos0, int n, int n_heads, int n_kv, int hd) {
         const double one = std::max(tile * tmax, mean) + per_wg;
         if (waves == most || one < 0.95 * best) best = one, p = PrefillPlan{waves, tmax, 1};
         if (!may_slice) continue;
-        const double part = std::min<long long>(P, rows) * (hd + 2) * 4.0 / 4e12 / 1.5e-6;
+        const double part = std::min<long long>(P, rows) * (hd + 2) * 4.0 / 4e12 / tile_s;
         for (int S = 2; S <= std::min(kPrefillMaxSlices, tmax / 2) && wgs * S <= 4 * cus; S++) {
             const int C = (tmax + S - 1) / S;
             long long u = 0; // workgroups with keys
@@ -754,11 +756,11 @@ bool prefill_widens(int n, int n_heads, int n_kv, int hd) {
     return hd == 256 || (long long)n * (n_heads / n_kv) > kPrefillWidenRows;
 }
 // Bytes of a sliced launch's partials, in row tiles of `rows` (pwaves: waves of a row tile that hold rows)
-int prefill_pwaves(long long P, int rows) { return P > rows ? rows / 32 : (int)((P + 31) / 32); }
-size_t prefill_part_bytes(const PrefillPlan& p, int n, int n_heads, int n_kv, int hd, int rows) {
+int prefill_pwaves(long long P, int rows, int rw) { return P > rows ? rows / rw : (int)((P + rw - 1) / rw); }
+size_t prefill_part_bytes(const PrefillPlan& p, int n, int n_heads, int n_kv, int hd, int rows, int rw = 32) {
     if (p.nslice == 1) return 0;
     const long long P = (long long)n * (n_heads / n_kv);
-    return align256((size_t)kPrefillRowTiles(P, rows) * n_kv * p.nslice * prefill_pwaves(P, rows) * 32 * (hd + 2) * 4);
+    return align256((size_t)kPrefillRowTiles(P, rows) * n_kv * p.nslice * prefill_pwaves(P, rows, rw) * rw * (hd + 2) * 4);
 }
 
 // gi_attn_prefill, gi_attn_prefill_i8 and gi_attn_prefill_q4: the same launch with the f16, int8 or 4-bit kernel
@@ -827,32 +829,38 @@ int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, c
     a.nslice = 1;
     const int G = n_heads / n_kv;
     a.gmul = (long long)n * G * G < 1ll << 31 ? (uint32_t)(((1ll << 31) + G - 1) / G) : 0;
-    // the launch of an MFMA prefill kernel over staging `st` (Module::prefill), sliced where the plan says so and the rest of the workspace holds the partials; then their merge
-    auto run = [&](int st, unsigned char* free, size_t left) {
-        const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd);
-        const int waves = st == 2 ? (hd == 256 ? 4 : 8) : p.waves; // (tile by tile: the larger form only)
-        const size_t need = prefill_part_bytes(p, n, n_heads, n_kv, hd, 32 * waves);
-        a.rows = 32 * waves;
+    // the launch of kernel f with `waves` waves of rw rows, sliced where the plan says so and the rest of the workspace
+    // holds the partials; then their merge
+    auto run_plan = [&](const PrefillPlan& p, hipFunction_t f, int waves, int rw, unsigned char* free, size_t left) {
+        const size_t need = prefill_part_bytes(p, n, n_heads, n_kv, hd, rw * waves, rw);
+        a.rows = rw * waves;
         a.items = kPrefillRowTiles((long long)n * G, a.rows);
-        a.pwaves = prefill_pwaves((long long)n * G, a.rows);
+        a.pwaves = prefill_pwaves((long long)n * G, a.rows, rw);
         if (need && free && aligned16(free) && left >= need) {
             a.part = (float*)free;
             a.nslice = p.nslice;
             a.slice_tiles = p.tiles;
         }
-        const hipFunction_t f = st == 2 && hd == 256 ? m->prefill256[fmt - 1] : m->prefill[hd == 64 ? 1 : hd == 256 ? 2 : 0][st][waves == (hd == 256 ? 2 : 4)];
-        if (int e = launch(kPrefill, f, dim3((unsigned)(a.items * n_kv * a.nslice), 1, 1),
-                           dim3(64 * waves), (hipStream_t)stream, &a, sizeof a))
+        if (int e = launch(kPrefill, f, dim3((unsigned)(a.items * n_kv * a.nslice), 1, 1), dim3(64 * waves),
+                           (hipStream_t)stream, &a, sizeof a))
             return e;
         if (a.nslice == 1) return 0;
-        return launch(kPrefillCombine, m->prefill_combine[0],
-                      dim3(a.pwaves * a.items * n_kv, 32 * hd / 256 / kPrefillMergeFrags, 1), dim3(64 * kPrefillMergeFrags),
-                      (hipStream_t)stream, &a, sizeof a);
+        return launch(kPrefillCombine, m->prefill_combine[rw == 16],
+                      dim3(a.pwaves * a.items * n_kv, (rw * hd / 256 + kPrefillMergeFrags - 1) / kPrefillMergeFrags, 1),
+                      dim3(64 * kPrefillMergeFrags), (hipStream_t)stream, &a, sizeof a);
+    };
+    // an f16 MFMA kernel over staging `st` (Module::prefill)
+    auto run = [&](int st, unsigned char* free, size_t left) {
+        const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd);
+        const int waves = st == 2 ? (hd == 256 ? 4 : 8) : p.waves; // (tile by tile: the larger form only)
+        const hipFunction_t f = st == 2 && hd == 256 ? m->prefill256[fmt - 1]
+                                                     : m->prefill[hd == 64 ? 1 : hd == 256 ? 2 : 0][st][waves == (hd == 256 ? 2 : 4)];
+        return run_plan(p, f, waves, 32, free, left);
     };
     unsigned char* const ws = (unsigned char*)workspace;
-    if (f32_prompt && !f32_hd(hd)) // head sizes 64 and 128 in f32: one workgroup per (head, 128 query rows)
-        return launch(kPrefill, m->prefill_f32p[i8][hd == 128], dim3((n + kF32Rows - 1) / kF32Rows * n_heads, 1, 1),
-                      dim3(kF32Threads), (hipStream_t)stream, &a, sizeof a);
+    if (f32_prompt || f32_hd(hd))
+        return run_plan(prefill_plan(pos0, n, n_heads, n_kv, hd, true),
+                        f32_hd(hd) ? m->prefill_f32[i8][f32_index(hd)] : m->prefill_f32p[i8][hd == 128], 8, 16, ws, workspace_bytes);
     if (fmt && workspace && widen && !f32_hd(hd)) {
         const int len = pos0 + n;
         const size_t need = prefill_ws_bytes(len, n_kv, hd, fmt);
@@ -894,9 +902,6 @@ int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, c
         a.sc_head_stride = len;
         return run(fmt == 2 ? 0 : 1, ws + need, workspace_bytes - need);
     }
-    if (f32_hd(hd)) // one workgroup per (head, 128 query rows)
-        return launch(kPrefill, m->prefill_f32[i8][f32_index(hd)], dim3((n + kF32Rows - 1) / kF32Rows * n_heads, 1, 1),
-                      dim3(kF32Threads), (hipStream_t)stream, &a, sizeof a);
     return run(fmt ? 2 : 0, ws, workspace_bytes);
 }
 
@@ -1034,7 +1039,10 @@ size_t gi_attn_prefill_workspace_bytes(int kv_len, int n_kv, int hd, int fmt) {
 
 size_t gi_attn_prefill_scratch_bytes(int pos0, int n, int n_heads, int n_kv, int hd, int fmt, int flags) {
     if (check_shape(n_heads, n_kv, hd, true) || pos0 < 0 || n <= 0 || fmt < 0 || fmt > 2 || (fmt == 2 && hd != 256)) return 0;
-    if ((flags & GI_PREFILL_F32) || f32_hd(hd)) return 0;
+    if ((flags & GI_PREFILL_F32) || f32_hd(hd)) {
+        if (fmt == 2 || hd > 128) return 0;
+        return prefill_part_bytes(prefill_plan(pos0, n, n_heads, n_kv, hd, true), n, n_heads, n_kv, hd, kF32Rows, 16);
+    }
     const bool widens = fmt && (flags & GI_PREFILL_WIDEN) && prefill_widens(n, n_heads, n_kv, hd);
     const size_t widened = widens ? prefill_ws_bytes(pos0 + n, n_kv, hd, fmt) : 0;
     const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd);
@@ -1139,7 +1147,7 @@ int attention_impl(void* stream, const float* qkv, const void* kc, const void* v
     if (n >= kTiledMinBatch && !verify && no_tc && fmt != 2 && hd <= 128) {
         if (posp) return fail("a device position (posp) is only taken by the split path");
         return prefill_impl(stream, qkv, GI_F32, row, kc, vc, ks, vs, scs, sch, fmt, kvs, kvh, out, GI_F32, q_dim, pos0,
-                            n, n_heads, n_kv, hd, scale, nullptr, 0, true);
+                            n, n_heads, n_kv, hd, scale, workspace, workspace_bytes, true, false);
     }
     if (n >= kTiledMinBatch && !verify && !no_tc) {
         if (posp) return fail("a device position (posp) is only taken by the split path");

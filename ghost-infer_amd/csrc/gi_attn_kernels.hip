@@ -1596,6 +1596,7 @@ __device__ __forceinline__ void gi_prefill_combine_t(const GiPrefillArgs& a) {
         *reinterpret_cast<f4*>((float*)a.out + e0) = acc;
 }
 extern "C" __global__ void __launch_bounds__(64 * PFC_FRAGS) gi_prefill_combine_32(GiPrefillArgs a) { gi_prefill_combine_t<32>(a); }
+extern "C" __global__ void __launch_bounds__(64 * PFC_FRAGS) gi_prefill_combine_16(GiPrefillArgs a) { gi_prefill_combine_t<16>(a); }
 
 template <int I> struct gi_int { static constexpr int value = I; };
 // f(gi_int<0>) ... f(gi_int<N - 1>)

@@ -337,7 +337,8 @@ def prefill_workspace(kv_len, n_kv, hd, fmt, device):
 def _prefill_scratch(pos0, n, n_heads, n_kv, hd, fmt, flags, device):
     """(scratch tensor or None, its bytes) of a prefill call: the widened keys and the partials of a sliced launch
     (gi_attn_prefill_scratch_bytes). The tensor belongs to the current stream, where the call goes."""
-    if pos0 + n <= 960 and not flags & GI_PREFILL_WIDEN:  # fewer than 16 key tiles: never cut
+    if pos0 + n <= (960 if hd in (64, 128, 256) and not flags & GI_PREFILL_F32 else 192) and not flags & GI_PREFILL_WIDEN:
+        # fewer than 16 key tiles (4 in f32): never cut
         return None, 0
     nbytes = load_library().gi_attn_prefill_scratch_bytes(pos0, n, n_heads, n_kv, hd, fmt, flags)
     return (torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None), nbytes

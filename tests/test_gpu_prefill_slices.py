@@ -126,3 +126,25 @@ def test_sliced_prefill_h256_every_cache(gpu, n, pos0, n_heads, n_kv):
                      what=f"i8 row {r}")
         assert_close(got4[r:r + 1].cpu().numpy(), reference_f64_q4(q4[r:r + 1], kc, vc, ks4, vs4, pos0 + r, n_heads, n_kv),
                      what=f"q4 row {r}")
+
+
+@pytest.mark.parametrize("n,pos0,n_heads,n_kv,hd,i8", [(16, 240, 4, 4, 80, False), (17, 700, 6, 2, 96, True),
+                                                       (130, 900, 4, 4, 96, False), (255, 200, 9, 3, 48, True),
+                                                       (40, 3000, 8, 8, 112, False), (60, 1500, 8, 2, 16, False)])
+def test_sliced_prefill_f32(gpu, n, pos0, n_heads, n_kv, hd, i8):
+    # the f32 kernels: rows that end inside a wave of 16 and a tile of 128, hd / 16 fragments that do not fill a merge block
+    print("[case] sliced prefill f32", n, pos0, n_heads, n_kv, hd, i8, flush=True)
+    assert sliced(n, pos0, n_heads, n_kv, hd, int(i8))
+    if i8:
+        q, k, v, ks, vs = make_inputs_i8(9700 + n + hd, n, pos0 + n, n_heads, n_kv, hd=hd)
+        kw = dict(k_scale=dev(ks, gpu, -1, n_kv), v_scale=dev(vs, gpu, -1, n_kv))
+        kt, vt = dev(k, gpu, -1, n_kv, hd), dev(v, gpu, -1, n_kv, hd)
+        want = reference_f64_i8(q, k, v, ks, vs, pos0, n_heads, n_kv, hd=hd)
+    else:
+        q, k, v = make_inputs(9700 + n + hd, n, pos0 + n, n_heads, n_kv, hd=hd)
+        kw = {}
+        kt, vt = (dev(x.view(np.int16), gpu, -1, n_kv, hd).view(torch.float16) for x in (k, v))
+        want = reference_f64(q, k, v, pos0, n_heads, n_kv, hd=hd)
+    got = gi_attn.prefill(dev(q, gpu, n, n_heads * hd), kt, vt, pos0, n_heads, n_kv, hd=hd, **kw)
+    torch.cuda.synchronize()
+    assert_close(got.cpu().numpy(), want, max_abs=2e-5, rel_l2=2e-5, what="sliced f32")
