@@ -149,6 +149,53 @@ __device__ __forceinline__ float rows_sum(float v) {
     return __int_as_float(q[0]) + __int_as_float(q[1]);
 }
 
+// Lane l's value of lane l ^ M, on the VALU (a shuffle would be an LDS round trip, and the rows here need 6 to 24 of them in
+// a dependent chain).
+template <int M> __device__ __forceinline__ float gi_xor_lane(float v) {
+    static_assert(M == 1 || M == 2 || M == 4 || M == 8, "within a 16-lane row");
+    const int x = __float_as_int(v);
+    if constexpr (M == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, true)); // quad_perm [1,0,3,2]
+    if constexpr (M == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, true)); // quad_perm [2,3,0,1]
+    if constexpr (M == 4) // row_half_mirror (l ^ 7), then quad_perm [3,2,1,0] (l ^ 3)
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true));
+    return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x128, 0xF, 0xF, true)); // row_ror 8
+}
+// lo: the value of the lane of the pair (l, l ^ M) with bit M clear, hi: of the other
+struct GiPair { float lo, hi; };
+template <int M> __device__ __forceinline__ GiPair gi_pair(float v) {
+    static_assert(M == 16 || M == 32, "across 16-lane rows");
+    const int x = __float_as_int(v);
+    if constexpr (M == 16) {
+        const auto p = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        return GiPair{__int_as_float(p[0]), __int_as_float(p[1])};
+    } else {
+        const auto p = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        return GiPair{__int_as_float(p[0]), __int_as_float(p[1])};
+    }
+}
+// sum and max over the wave, in the order of shuffles by 32, 16, .. 1
+__device__ __forceinline__ float gi_wave_sum(float v) {
+    GiPair p = gi_pair<32>(v);
+    v = p.lo + p.hi;
+    p = gi_pair<16>(v);
+    v = p.lo + p.hi;
+    v += gi_xor_lane<8>(v);
+    v += gi_xor_lane<4>(v);
+    v += gi_xor_lane<2>(v);
+    return v + gi_xor_lane<1>(v);
+}
+__device__ __forceinline__ float gi_oct_max(float v) { // over lanes l ^ 1, 2, 4
+    v = fmaxf(v, gi_xor_lane<4>(v));
+    v = fmaxf(v, gi_xor_lane<2>(v));
+    return fmaxf(v, gi_xor_lane<1>(v));
+}
+__device__ __forceinline__ float gi_wave_max(float v) {
+    GiPair p = gi_pair<32>(v);
+    v = fmaxf(p.lo, p.hi);
+    p = gi_pair<16>(v);
+    v = fmaxf(p.lo, p.hi);
+    return gi_oct_max(fmaxf(v, gi_xor_lane<8>(v)));
+}
 // Buffer resource over `bytes` bytes from p: loads at offsets >= bytes return zeros without touching memory.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t gi_rsrc(const void* p, long long bytes) {
     int n = (int)(bytes < 0 ? 0 : (bytes > 0x7ffffff0ll ? 0x7ffffff0ll : bytes));
@@ -1347,14 +1394,14 @@ extern "C" __global__ void __launch_bounds__(256, DEC_MINWG) gi_decode_pm_ws2_1_
 // (attention_combine's maths in base 2; empty slices carry m = -inf and weigh nothing). One wave per
 // (head, token, 128/CMB_DSPLIT dims): lane l takes slices l, l + 64, ..., issuing all of a slice's loads
 // at once and folding its slices with a running max, so up to 64 slices cost one memory round trip;
-// shuffles agree on the max and the sum, and LDS sums the lanes' O. Many small workgroups keep the merge
-// short: it runs between two launches, on the critical path of every decode step.
+// the reductions over the lanes stay on the VALU (with shuffles through LDS and an LDS sum of the lanes' O a 65536-key step of
+// 32/4 heads took 25.8 us, now 25.1; a 16-layer token step at 2900 keys 230 -> 219.5). Many small workgroups keep the
+// merge short: it runs between two launches, on the critical path of every decode step.
 #ifndef CMB_DSPLIT
 #define CMB_DSPLIT 8 // workgroups per (head, token), each over 128 / CMB_DSPLIT dims
 #endif
 #define CMB_DIMS (128 / CMB_DSPLIT) // dims per workgroup (grid z = hd / CMB_DIMS)
 extern "C" __global__ void __launch_bounds__(64) gi_decode_combine(GiDecodeArgs a) {
-    __shared__ float acc_o[64][CMB_DIMS + 1];
     const int h = blockIdx.x, t = blockIdx.y, d0 = blockIdx.z * CMB_DIMS, lane = threadIdx.x;
     const int hd = a.hd, part = hd + 4;
     const float* p = a.part + ((long long)t * a.n_heads + h) * a.nsplit * part;
@@ -1380,20 +1427,31 @@ extern "C" __global__ void __launch_bounds__(64) gi_decode_combine(GiDecodeArgs 
             o[4 * i + 3] = o[4 * i + 3] * a_old + v[i].w * a_new;
         }
     }
-    float M = m;
-    for (int x = 32; x > 0; x >>= 1) M = fmaxf(M, __shfl_xor(M, x, 64));
+    const float M = gi_wave_max(m);
     const float w = m == GI_NEG_INF ? 0.f : __builtin_amdgcn_exp2f(m - M);
-    float LL = L * w;
-    for (int x = 32; x > 0; x >>= 1) LL += __shfl_xor(LL, x, 64);
+    const float LL = gi_wave_sum(L * w);
+    // the lanes' O: each exchange halves the dims that a lane still sums (lane bits 5, 4, 3, 2 end as dim bits 3, 2, 1,
+    // 0), on the VALU
+    static_assert(CMB_DIMS == 16, "16 dims over four exchanges");
 #pragma unroll
-    for (int i = 0; i < CMB_DIMS; i++) acc_o[lane][i] = o[i] * w;
-    __syncthreads();
-    if (lane < CMB_DIMS) {
-        float O = 0.f;
-#pragma unroll 8
-        for (int k = 0; k < 64; k++) O += acc_o[k][lane];
-        a.out[(long long)t * a.out_stride + (long long)h * hd + d0 + lane] = O / LL;
+    for (int i = 0; i < 16; i++) o[i] *= w;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_int(o[i]), __float_as_int(o[i + 8]), false, false);
+        o[i] = __int_as_float(p[0]) + __int_as_float(p[1]);
     }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_int(o[i]), __float_as_int(o[i + 4]), false, false);
+        o[i] = __int_as_float(p[0]) + __int_as_float(p[1]);
+    }
+    const bool b8 = lane & 8, b4 = lane & 4;
+#pragma unroll
+    for (int i = 0; i < 2; i++) o[i] = (b8 ? o[i + 2] : o[i]) + gi_xor_lane<8>(b8 ? o[i] : o[i + 2]);
+    float O = (b4 ? o[1] : o[0]) + gi_xor_lane<4>(b4 ? o[0] : o[1]);
+    O += gi_xor_lane<2>(O);
+    O += gi_xor_lane<1>(O);
+    if ((lane & 3) == 0) a.out[(long long)t * a.out_stride + (long long)h * hd + d0 + (lane >> 2)] = O / LL;
 }
 
 // ------------------------------------------------------------------------------------------------ prefill
@@ -2237,53 +2295,6 @@ struct GiRopeArgs {
 // kv4_fwht's stages (src/cuda.rs:242-256) in its order, h = 1, 2 inside the lane, h = 4..128 across lanes
 // l and l ^ (h/4). Each stage gives the lower element a + c and the upper one a - c, single f32 operations as
 // the reference's, so the result is bit-identical to it; then every value times 1/16.
-// Lane l's value of lane l ^ M, on the VALU (a shuffle would be an LDS round trip, and the rows here need 6 to 24 of them in
-// a dependent chain).
-template <int M> __device__ __forceinline__ float gi_xor_lane(float v) {
-    static_assert(M == 1 || M == 2 || M == 4 || M == 8, "within a 16-lane row");
-    const int x = __float_as_int(v);
-    if constexpr (M == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, true)); // quad_perm [1,0,3,2]
-    if constexpr (M == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, true)); // quad_perm [2,3,0,1]
-    if constexpr (M == 4) // row_half_mirror (l ^ 7), then quad_perm [3,2,1,0] (l ^ 3)
-        return __int_as_float(__builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true));
-    return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x128, 0xF, 0xF, true)); // row_ror 8
-}
-// lo: the value of the lane of the pair (l, l ^ M) with bit M clear, hi: of the other
-struct GiPair { float lo, hi; };
-template <int M> __device__ __forceinline__ GiPair gi_pair(float v) {
-    static_assert(M == 16 || M == 32, "across 16-lane rows");
-    const int x = __float_as_int(v);
-    if constexpr (M == 16) {
-        const auto p = __builtin_amdgcn_permlane16_swap(x, x, false, false);
-        return GiPair{__int_as_float(p[0]), __int_as_float(p[1])};
-    } else {
-        const auto p = __builtin_amdgcn_permlane32_swap(x, x, false, false);
-        return GiPair{__int_as_float(p[0]), __int_as_float(p[1])};
-    }
-}
-// sum and max over the wave, in the order of shuffles by 32, 16, .. 1
-__device__ __forceinline__ float gi_wave_sum(float v) {
-    GiPair p = gi_pair<32>(v);
-    v = p.lo + p.hi;
-    p = gi_pair<16>(v);
-    v = p.lo + p.hi;
-    v += gi_xor_lane<8>(v);
-    v += gi_xor_lane<4>(v);
-    v += gi_xor_lane<2>(v);
-    return v + gi_xor_lane<1>(v);
-}
-__device__ __forceinline__ float gi_oct_max(float v) { // over lanes l ^ 1, 2, 4
-    v = fmaxf(v, gi_xor_lane<4>(v));
-    v = fmaxf(v, gi_xor_lane<2>(v));
-    return fmaxf(v, gi_xor_lane<1>(v));
-}
-__device__ __forceinline__ float gi_wave_max(float v) {
-    GiPair p = gi_pair<32>(v);
-    v = fmaxf(p.lo, p.hi);
-    p = gi_pair<16>(v);
-    v = fmaxf(p.lo, p.hi);
-    return gi_oct_max(fmaxf(v, gi_xor_lane<8>(v)));
-}
 __device__ __forceinline__ void gi_fwht256(float __attribute__((ext_vector_type(4))) & x, int lane) {
     float t;
     t = x[0]; x[0] = t + x[1]; x[1] = t - x[1];
