@@ -26,7 +26,7 @@
 #define PF32_KT 64                  // prefill: keys per tile
 
 __device__ __forceinline__ float gi_block_max(float v, float* red) {
-    for (int m = 32; m > 0; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
+    v = gi_wave_max(v);
     const int w = threadIdx.x >> 6;
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[w] = v;
@@ -34,7 +34,7 @@ __device__ __forceinline__ float gi_block_max(float v, float* red) {
     return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 __device__ __forceinline__ float gi_block_sum(float v, float* red) {
-    for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m, 64);
+    v = gi_wave_sum(v);
     const int w = threadIdx.x >> 6;
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[w] = v;
@@ -281,8 +281,7 @@ __device__ __forceinline__ void gi_prefill_f32_t(const GiPrefillArgs& a) {
                 if (edge && (kp > lim || kp >= kv_len)) s[kb][r] = GI_NEG_INF;
                 mx = fmaxf(mx, s[kb][r]);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = rows_max(mx);
         const float m_new = fmaxf(m_run, mx);
         // (a row that sees no key of a slice keeps max -inf and sum 0; with key 0 in the slice every row's is finite)
         const float ref = m_new > GI_NEG_INF ? m_new : 0.f;
@@ -309,8 +308,7 @@ __device__ __forceinline__ void gi_prefill_f32_t(const GiPrefillArgs& a) {
                     o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(Vs[(16 * kb + 4 * lg + r) * LD + 16 * d + lc], s[kb][r],
                                                                 o[d], 0, 0, 0);
     }
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = rows_sum(l_run);
     if (a.nslice > 1) { // a slice's partial (pf_part_o: fragment d holds the O^T block d)
         if (w >= a.pwaves) return;
         f4* po = reinterpret_cast<f4*>(pf_part_o<16>(a, HD, un.unit, w)) + l;
