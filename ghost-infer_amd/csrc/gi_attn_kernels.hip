@@ -35,7 +35,6 @@ typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h4x __attribute__((ext_vector_type(4)));
 
 #define GI_NEG_INF (-__builtin_inff())
-#define GI_LOG2E 1.4426950408889634f
 
 // ------------------------------------------------------------------------------------------------ decode
 
@@ -118,7 +117,6 @@ typedef int i4v __attribute__((ext_vector_type(4)));
 #define DEC_REF_VB 4.f
 #define GI_RSRC_FLAGS 0x00020000
 
-__device__ __forceinline__ float wave_xor(float v, int m) { return __shfl_xor(v, m, 64); }
 // Scales an MFMA accumulator (held in AGPRs) by alpha in the rare rescale branch of an online softmax. The empty
 // asm statements pin the accumulator to AGPRs on both sides of the multiply, so the AGPR -> VGPR copies it needs are
 // made inside the branch; without them the compiler hoists those copies into every tile iteration (up to 135
@@ -1542,13 +1540,9 @@ template <int RW> __device__ __forceinline__ float2* pf_part_ml(const GiPrefillA
 #define GI_VMCNT(n) (0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
 // s_waitcnt immediate waiting for this wave's LDS operations (lgkmcnt 0, vmcnt and expcnt at their maxima)
 #define GI_LGKMCNT0 0xC07F
-#define PF_NBUF 4          // LDS tile buffers
 #define PF_BK 64           // keys per tile
 #define PF_TILE 16384      // bytes of one K or V tile: 64 rows of 256 bytes
 #define PF_RESCALE_LOG2 8.0f
-#ifndef PF_KPF
-#define PF_KPF 8           // K fragments in flight in the QK loop
-#endif
 #define GI_LDS __attribute__((address_space(3)))
 // Tile staging from HBM straight into LDS (buffer_load_dwordx4 ... lds: lane i's 16 bytes land at
 // M0 + 16i). Issued from inline asm, so the compiler does not track these loads: were it to see them, it
@@ -1557,29 +1551,12 @@ template <int RW> __device__ __forceinline__ float2* pf_part_ml(const GiPrefillA
 // loads themselves (s_waitcnt vmcnt on the issuing wave, then s_barrier). Vector memory loads retire in
 // order, so the compiler's own vmcnt(N) waits for the loads it knows stay correct with these in flight
 // (more younger loads only make such a wait stricter).
-#ifndef GI_DMA_ASM
-#define GI_DMA_ASM 1
-#endif
-__device__ __forceinline__ u4 gi_rsrc_words(const void* p, long long bytes) {
-    const uint32_t n = (uint32_t)(bytes < 0 ? 0 : (bytes > 0x7ffffff0ll ? 0x7ffffff0ll : bytes));
-    const unsigned long long b = (unsigned long long)p;
-    return u4{(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, n, (uint32_t)GI_RSRC_FLAGS};
-}
-__device__ __forceinline__ void gi_stage16(const void* base, long long bytes, GI_LDS void* dst, int voff) {
-#if GI_DMA_ASM
-    const u4 rs = gi_rsrc_words(base, bytes);
-    const uint32_t m0 = (uint32_t)(uintptr_t)dst;
-    // (s_nop 0: the one wait state an M0 write needs before an LDS-DMA load reads it; the compiler cannot see
-    // the load inside the asm, so it would not insert it)
-    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "{m0}"(m0) : "memory");
-#else
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(gi_rsrc(base, bytes), dst, 16, voff, 0, 0, 0);
-#endif
-}
 __device__ __forceinline__ u4 gi_rsrc_rows(const void* p, int bytes) {
     const unsigned long long b = (unsigned long long)p;
     return u4{(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, (uint32_t)bytes, (uint32_t)GI_RSRC_FLAGS};
 }
+// (s_nop 0: the one wait state an M0 write needs before an LDS-DMA load reads it; the compiler cannot see the load
+// inside the asm, so it would not insert it)
 __device__ __forceinline__ void gi_stage16(u4 rs, GI_LDS void* dst, int voff) {
     const uint32_t m0 = (uint32_t)(uintptr_t)dst;
     asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "{m0}"(m0) : "memory");
@@ -1693,12 +1670,12 @@ template <int N, int I = 0, typename F> __device__ __forceinline__ void gi_unrol
 // element 4(i%2) + j). V^T operand: ds_read_b64_tr_b16 gives output lane i of a 16-lane group element
 // i%4 of the 8 bytes source lane 4e + i/4 addresses, as its element e; with source lane (e, c) pointing at
 // key e, dims 16*(group%2) + 4c of the dim block, lane i receives V[key e][dim i]: the A operand rows.
-// Softmax: scores stay raw, scale*log2(e) is folded into the exp2 argument; a row's reference max only
+// Softmax: scale*log2(e) is folded into Q, so scores are in log2 units; a row's reference max only
 // moves when a tile's max exceeds it by more than 2^8 in probability (then O and l are rescaled), so
 // P <= 256 fits f16 and most tiles skip the rescale. Row sums add the f16-rounded P that PV uses
 // (v_dot2 against ones). Causal: a wave skips tiles past its last row (keeping every barrier); only
 // tiles crossing the diagonal are masked.
-// I8 = true: an int8 cache (the reference's KV8 prefill, src/cuda.rs:2466-2498, 2548-2605): the
+// FMT = 1: an int8 cache (the reference's KV8 prefill, src/cuda.rs:2466-2498, 2548-2605): the
 // threads load 16-byte chunks of K and V rows into registers one iteration ahead, widen them to exact f16 and write
 // them into the same swizzled LDS layout (so the MFMA operand reads are unchanged), and the tile's 64 key and
 // value scales go to LDS beside it; STG: the cache already widened to exact f16 integers in a workspace
@@ -2245,7 +2222,7 @@ extern "C" __global__ void __launch_bounds__(128, 1) gi_prefill_fwd_h256_w2(GiPr
 extern "C" __global__ void __launch_bounds__(128, 1) gi_prefill_fwd_h256_i8s_w2(GiPrefillArgs a) { gi_prefill_t<1, 256, true, 2, 8, 8>(a); }
 extern "C" __global__ void __launch_bounds__(256, 1) gi_prefill_fwd_h256_i8(GiPrefillArgs a) { gi_prefill_t<1, 256, false, 4, 4, 8>(a); }
 extern "C" __global__ void __launch_bounds__(256, 1) gi_prefill_fwd_h256_q4(GiPrefillArgs a) { gi_prefill_t<2, 256, false, 4, 4, 8>(a); }
-// the int8 cache pre-widened by gi_kv_widen (the 4-bit cache pre-widened runs gi_prefill_fwd_h256r itself)
+// the int8 cache pre-widened by gi_kv_widen (the 4-bit cache pre-widened is an f16 cache: gi_prefill_fwd_h256)
 extern "C" __global__ void __launch_bounds__(256, 1) gi_prefill_fwd_h256_i8s(GiPrefillArgs a) { gi_prefill_t<1, 256, true, 4, 8, 8>(a); }
 
 // ------------------------------------------------------------------------------------------------ KV store

@@ -175,8 +175,10 @@ size_t gi_attn_prefill_workspace_bytes(int kv_len, int n_kv, int hd, int fmt);
 /* gi_attn_prefill_i8 / gi_attn_prefill_q4 with a caller-owned workspace (256-byte aligned, at least
  * gi_attn_prefill_workspace_bytes(pos0 + n, ...) bytes): the keys 0..pos0+n-1 are first widened into it to the f16
  * values the tiles take (int8: the exact integers, the scales kept apart; 4-bit: f16((n - 8) * scale)), and the
- * prefill then stages the widened tiles as it stages the f16 cache. The same arithmetic and outputs, bit for bit, as
- * the entry points without a workspace (replaces what they replace). gi_attention_i8 / gi_attention_q4 take this
+ * prefill then stages the widened tiles as it stages the f16 cache. (Head sizes 64 and 128 with at most 256 query rows per
+ * kv head: the tiles are widened inside the prefill, once each, which is faster there.) The same arithmetic and outputs,
+ * bit for bit, as the entry points without a workspace (replaces what they replace); in a workspace larger than
+ * gi_attn_prefill_workspace_bytes the launch may also be cut along its keys, as in gi_attn_prefill_ws. gi_attention_i8 / gi_attention_q4 take this
  * path for prefill batches whenever their workspace holds it. */
 int gi_attn_prefill_i8_ws(void* stream, const void* q, int q_dtype, long long q_stride, const int8_t* kc,
                           const int8_t* vc, const float* ks, const float* vs, long long kv_stride,
@@ -200,7 +202,7 @@ int gi_attn_prefill_q4_ws(void* stream, const void* q, int q_dtype, long long q_
  * differ from the one-slice results by f32 rounding). gi_attn_prefill_scratch_bytes says how much a call can use; it
  * is optional, and with a smaller one (or none) the call does without. The workspace needs no initialisation; calls that
  * share one must be ordered. Prompts of up to 4096 keys taken in chunks of 256 tokens or more, and spans below 16
- * tiles of 64 keys, are never cut. */
+ * tiles of 64 keys (f32: below 4), are never cut. */
 size_t gi_attn_prefill_scratch_bytes(int pos0, int n, int n_heads, int n_kv, int hd, int fmt, int flags);
 int gi_attn_prefill_ws(void* stream, const void* q, int q_dtype, long long q_stride, const void* kc, const void* vc,
                        const void* ks, const void* vs, int fmt, int flags, long long kv_stride, long long kv_head_stride,
