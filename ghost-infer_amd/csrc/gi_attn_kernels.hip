@@ -2341,6 +2341,12 @@ __device__ __forceinline__ void gi_store_row(const GiRopeArgs& a, uint16_t* cach
     if (lane == 0) scale[(long long)pos * a.sc_stride + (long long)kh * a.sc_head_stride] = dd;
 }
 
+// The rotated pair, one product of each sum rounded first: written out so that the compiler's choice of the contracted
+// product cannot differ between the two ways that gi_qk_norm_rope_t pairs (a cached int8 value on a rounding edge
+// would then depend on the way).
+__device__ __forceinline__ float rope_a(float p, float q, float c, float s) { return fmaf(p, c, -(q * s)); }
+__device__ __forceinline__ float rope_b(float p, float q, float c, float s) { return fmaf(q, c, p * s); }
+
 // PER = hd / 64 values per lane, dims PER*lane .. PER*lane + PER - 1 (one 4, 8 or 16-byte access per row).
 // MASKED (PER = 2): any even head size up to 128 (the f32 kernels' head sizes): lanes past hd / 2 hold zeros and
 // neither load nor store.
@@ -2418,7 +2424,7 @@ __device__ __forceinline__ void gi_qk_norm_rope_t(const GiRopeArgs& a, float (*c
 #pragma unroll
             for (int j = 0; j < PER; j++) {
                 const GiPair p = gi_pair<32>(x[j]);
-                x[j] = lane < 32 ? p.lo * cc[j] - p.hi * ss[j] : p.lo * ss[j] + p.hi * cc[j];
+                x[j] = lane < 32 ? rope_a(p.lo, p.hi, cc[j], ss[j]) : rope_b(p.lo, p.hi, cc[j], ss[j]);
             }
         } else {
             if (act) *reinterpret_cast<fv*>(sh + PER * lane) = x;
@@ -2426,8 +2432,8 @@ __device__ __forceinline__ void gi_qk_norm_rope_t(const GiRopeArgs& a, float (*c
             for (int i = lane; i < half; i += 64) {
                 const int ia = a.neox ? i : 2 * i, ib = a.neox ? i + half : 2 * i + 1;
                 const float p = sh[ia], q = sh[ib], c = cs_sh[i][0], s = cs_sh[i][1];
-                sh[ia] = p * c - q * s;
-                sh[ib] = p * s + q * c;
+                sh[ia] = rope_a(p, q, c, s);
+                sh[ib] = rope_b(p, q, c, s);
             }
             __builtin_amdgcn_wave_barrier();
             if (act) x = *reinterpret_cast<const fv*>(sh + PER * lane);

@@ -68,3 +68,33 @@ def test_batch_equals_tokens_and_float64(gpu, fmt, hd, heads, n_kv, rope_dim, ne
     got = a.cpu().numpy().reshape(n, -1, hd)[:, :heads + n_kv]
     # the f32 angle of a position below 1534 is off by up to 1534 * 2^-23 * 1.5 = 2.7e-4 of a radian at |y| <= 8
     assert np.abs(got - z).max() <= 2.2e-3
+
+
+@pytest.mark.parametrize("hd,rope_dim,neox", [(64, 64, True), (128, 128, True), (128, 128, False), (128, 64, True),
+                                              (256, 256, True), (96, 96, True)])
+def test_rotated_pair_rounds_one_product(gpu, hd, rope_dim, neox):
+    """Every way of pairing gives a = round(p c - round(q s)) and b = round(q c + round(p s)), to the bit (a 64-bit mantissa
+    holds the unrounded sums to well below f32's half step). Head 0's pairs are (1, 0) and come out as the pair's (c, s)."""
+    print("[case] rope pair", hd, rope_dim, neox, flush=True)
+    n, heads, n_kv, pos0 = 70, 8, 1, 4321
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(hd)
+    x = torch.randn((n, (heads + 2 * n_kv) * hd), generator=gen, device=gpu)
+    half = rope_dim // 2
+    i = np.arange(half)
+    ia, ib = (i, i + half) if neox else (2 * i, 2 * i + 1)
+    x[:, :hd] = 0
+    x[:, torch.as_tensor(ia, device=gpu)] = 1
+    y = x.clone()
+    c = caches("f16", pos0 + n, n_kv, hd, gpu)
+    write("f16", y, c, pos0, heads, n_kv, hd, rope_dim=rope_dim, neox=neox, base=1e6)
+    xs = x.cpu().numpy().reshape(n, -1, hd)[:, 1:heads + n_kv]
+    ys = y.cpu().numpy().reshape(n, -1, hd)
+    co, si = ys[:, :1, ia], ys[:, :1, ib]
+    ld = np.longdouble
+    p, q = xs[..., ia], xs[..., ib]
+    a = (ld(p) * ld(co) - ld(q * si)).astype(np.float32)
+    b = (ld(q) * ld(co) + ld(p * si)).astype(np.float32)
+    got = ys[:, 1:heads + n_kv]
+    assert np.array_equal(got[..., ia], a)
+    assert np.array_equal(got[..., ib], b)
