@@ -2010,9 +2010,10 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
         if constexpr (!RSTG) st = stage_at(stage_tile(WIDE ? it - 1 : it));
         h8 pf[4];
         float mxn = GI_NEG_INF;
-        // slot of exponential x (of 32: every P^T operand is complete before its P V MFMAs), and of the next
+        // slot of exponential x (of 32: every P^T operand is complete before its P V MFMAs; none in the first and last
+        // eighth of the slots), and of the next
         // tile's row max over score group g (of 8), from two slots after its last QK MFMA on
-        constexpr auto pslot = [](int x) { return x * (NS - NDB) / 32; };
+        constexpr auto pslot = [](int x) { return x * (NS - NDB - NS / 4) / 32 + NS / 8; };
         constexpr auto mslot = [](int g) { return NQ + 2 + g * (NP - 2) / 8; };
         // int8: scales of score group g in element g % SR, read when the group SR before it has taken its own
         constexpr int SR = HD == 64 ? 4 : 2;
@@ -2120,8 +2121,11 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
             const int ks = st >> 1, bb = st & 1;
             sa[bb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[st % RING], qf[ks], ks == 0 ? f16x{} : sa[bb], 0, 0, 0);
             if (st + RING < NQ) kf[st % RING] = kfrag(B0, st + RING);
-            else if (ONE) kf[st % RING] = kfrag(B1, st + RING - NQ);
+            else if (ONE && NQ % RING == 0) kf[st % RING] = kfrag(B1, st + RING - NQ);
         }
+        if constexpr (ONE && NQ % RING != 0) // (the ring starts the next tile at its first fragment again)
+#pragma unroll
+            for (int st = 0; st < RING; st++) kf[st] = kfrag(B1, st);
         if constexpr (I8) {
 #pragma unroll
             for (int g = 0; g < 8; g++) {
@@ -2198,17 +2202,20 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
 // Kernels of head sizes 64 and 128 (_w4: 4 waves, 128 rows). The launch bound of 8 waves caps every form at 256
 // registers: past that the compiler keeps all MFMA accumulators in AGPRs and copies them to VGPRs for the softmax and
 // the rescale (96 to 270 copies per tile; the 4-wave form measured 702 us instead of 580 at 8192 tokens).
+// Operand ring of 6 slots and exponentials away from an iteration's ends, against a ring of 4 and exponentials from the
+// first slot on, one box: 131072 f16 tokens of 32/4 heads of 128 in chunks of 2048 120.6 -> 119.1 ms (ring of 8: 120.3, of
+// 2: 121.9); 8192 of 32/8 512 -> 505 us, int8 590 -> 584; head size 64 319 -> 306; 1024 tokens (_w4) 25.3 -> 24.6.
 #define GI_PREFILL_KERNEL(name, FMT, HD, STG, WAVES, RING)                                                              \
     extern "C" __global__ void __launch_bounds__(512) name(GiPrefillArgs a) { gi_prefill_t<FMT, HD, STG, WAVES, RING>(a); }
-GI_PREFILL_KERNEL(gi_prefill_fwd, 0, 128, false, 8, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_w4, 0, 128, false, 4, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_h64, 0, 64, false, 8, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_h64_w4, 0, 64, false, 4, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd, 0, 128, false, 8, 6)
+GI_PREFILL_KERNEL(gi_prefill_fwd_w4, 0, 128, false, 4, 6)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64, 0, 64, false, 8, 6)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64_w4, 0, 64, false, 4, 6)
 // the int8 cache pre-widened by gi_kv_widen, staged as the f16 cache is
-GI_PREFILL_KERNEL(gi_prefill_fwd_i8s, 1, 128, true, 8, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_i8s_w4, 1, 128, true, 4, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s, 1, 64, true, 8, 4)
-GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s_w4, 1, 64, true, 4, 4)
+GI_PREFILL_KERNEL(gi_prefill_fwd_i8s, 1, 128, true, 8, 6)
+GI_PREFILL_KERNEL(gi_prefill_fwd_i8s_w4, 1, 128, true, 4, 6)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s, 1, 64, true, 8, 6)
+GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s_w4, 1, 64, true, 4, 6)
 // int8 tiles widened through registers (the chunks in flight leave room for a ring of 2; with 4 waves, twice the
 // chunks a thread, 36 registers spill and a tile takes twice as long)
 GI_PREFILL_KERNEL(gi_prefill_fwd_i8, 1, 128, false, 8, 2)
