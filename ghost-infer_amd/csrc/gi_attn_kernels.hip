@@ -2203,8 +2203,9 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
 // registers: past that the compiler keeps all MFMA accumulators in AGPRs and copies them to VGPRs for the softmax and
 // the rescale (96 to 270 copies per tile; the 4-wave form measured 702 us instead of 580 at 8192 tokens).
 // Operand ring of 6 slots and exponentials away from an iteration's ends, against a ring of 4 and exponentials from the
-// first slot on, one box: 131072 f16 tokens of 32/4 heads of 128 in chunks of 2048 120.6 -> 119.1 ms (ring of 8: 120.3, of
-// 2: 121.9); 8192 of 32/8 512 -> 505 us, int8 590 -> 584; head size 64 319 -> 306; 1024 tokens (_w4) 25.3 -> 24.6.
+// first slot on (32/8 heads of 128, f16; two boxes): 1024 tokens (_w4) 25.3 -> 24.7 us, 512 at a 2000-token prefix 45.0 ->
+// 43.4; 8192 tokens of head size 64 319 -> 308. The launches at the power limit stay within what two boxes differ by
+// (8192 tokens of head size 128 510 and 515 us).
 #define GI_PREFILL_KERNEL(name, FMT, HD, STG, WAVES, RING)                                                              \
     extern "C" __global__ void __launch_bounds__(512) name(GiPrefillArgs a) { gi_prefill_t<FMT, HD, STG, WAVES, RING>(a); }
 GI_PREFILL_KERNEL(gi_prefill_fwd, 0, 128, false, 8, 6)
