@@ -1569,6 +1569,13 @@ __device__ __forceinline__ void gi_stage4(u4 rs, GI_LDS void* dst, int voff) { /
 // end) so that small products stay normal f16; with P <= 2^8 a dequantised |V| up to 127 * 65504 / (2^8 *
 // PF_I8_VBIAS) ~ 4000 fits (the reference biases by 2^10 with P <= 1, src/cuda.rs:2416-2420)
 #define PF_I8_VBIAS 8.f
+// Head size 256: a bias of 2^10, so that the small probabilities of a long context keep more bits. Value scales up to 0.249
+// leave room for P <= 2^8; a tile that holds a larger one (to V scales of 63, |V| of 8,000) moves the rows' references
+// from a smaller excess on, so that p * vscale * 2^10 <= 2^15.99 there: P <= 2^(5.99 - log2(vscale)), at least 1. (A
+// bias of 4 instead would take any such scale with P <= 2^8 and lose 8 bits of every p below 2^-16 / vscale.) The scale
+// read and its test cost 1%: 1024 tokens of 16/2 heads at a 3000-token prefix 128.6 -> 129.6 us.
+#define PF_WIDE_VFREE 0.249f
+#define PF_WIDE_VCAP 5.99f
 typedef short gi_s4 __attribute__((__vector_size__(8))); // 4 f16 as ds_read_b64_tr_b16 returns them
 
 // ---------------------------------------------------------------- prefill, merge of a sliced launch's partials
@@ -1682,7 +1689,7 @@ template <int N, int I = 0, typename F> __device__ __forceinline__ void gi_unrol
 // (gi_kv_widen, rows [n_kv][len][hd], scales [n_kv][len], the value scales times PF_I8_VBIAS) is staged as the f16
 // cache is. Scores are the integer-key dot products
 // times the key scale (QK chains start from zero; s = acc * kscale - m); P V takes f16(p * vscale *
-// PF_I8_VBIAS) and the row sum the f16-rounded p, as the reference's pv / pf.
+// PF_I8_VBIAS; head size 256: * 2^10) and the row sum the f16-rounded p, as the reference's pv / pf.
 // HD = 64 (attn_prefill_tc<64>, src/cuda.rs:2620): the same kernel with half the QK k-steps and O^T blocks. The
 // LDS image keeps the head-128 layout: each 128-byte row sits in a 256-byte slot, its 8 units at the swizzled
 // positions the operand reads compute (the staging loads of the other 8 positions are out of bounds and leave zeros).
@@ -1947,6 +1954,9 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     h8 kf[RING], vf[VRING];
     float mx = GI_NEG_INF;
     f16x sa[NBLK], sb[NBLK]; // scores of alternate tiles
+    // int8 at head size 256: the value scale of tile key `lane` (of the tile whose P V comes next)
+    constexpr bool VCAP = I8 && WIDE;
+    float vkey = 0.f;
 
     // publish K of tile it+2 and V of tile it+1 (each wave's own loads of them are in), after which the tiles of
     // stage_tile(it) go into buffers that no wave reads any more. Four buffers: K(it+4) into K(it)'s, V(it+3) into
@@ -1990,7 +2000,11 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     };
     auto step = [&](int it, f16x* s, f16x* sn) {
         mask(it, s);
-        const bool up = mx > PF_RESCALE_LOG2;
+        float top = PF_RESCALE_LOG2; // the score above its row's reference that a tile may reach
+        if constexpr (VCAP)
+            if (__builtin_amdgcn_ballot_w64(fabsf(vkey) > PF_WIDE_VFREE)) // p * vscale * 2^10 stays within f16
+                top = fmaxf(PF_WIDE_VCAP - __builtin_amdgcn_logf(gi_wave_max(fabsf(vkey))), 0.f);
+        const bool up = mx > top;
         if (__builtin_amdgcn_ballot_w64(up)) {
             // some row's max moved: shift the reference by delta, rescale O and l (alpha = 1 for the other rows) and this
             // tile's scores; the next tile's QK starts from the new reference
@@ -2028,6 +2042,7 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
         gi_unroll<NS>([&](auto slot) {
             constexpr int sl = decltype(slot)::value;
             if constexpr (sl == NS - RING) publish(it);
+            if constexpr (VCAP && sl == NS - RING + 1) vkey = vscl(it + 1)[lane];
             // the slot's MFMA
             if constexpr (sl < NQ) {
                 const int ks = sl >> 1, bb = sl & 1;
@@ -2151,6 +2166,7 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
         asm volatile("s_barrier" ::: "memory");
 #pragma unroll
         for (int st = 0; st < RING; st++) kf[st] = kfrag(kbuf(t_begin + 1), st);
+        if constexpr (VCAP) vkey = vscl(t_begin)[lane];
     }
     for (int it = t_begin; it < ntiles; it += 2) {
         iteration(it, sa, sb);

@@ -185,3 +185,26 @@ def test_decode_rising_scores_q4(gpu, n_tok):
                  what="rising scores, q4 decode vs oracle")
     assert_close(got, reference_f64_q4(q, kc, vc, ks, vs, pos0, n_heads, n_kv), *F64_TOL,
                  what="rising scores, q4 decode vs f64")
+
+
+@pytest.mark.parametrize("n,pos0", [(1000, 0), (100, 1500)])
+@pytest.mark.parametrize("staged", [True, False])
+@pytest.mark.parametrize("hd", [64, 128, 256])
+def test_prefill_rising_scores_i8_large_values(gpu, hd, staged, n, pos0):
+    # value scales from 0.02 to 30 (|V| up to 3,800; the entry points take 4,000) under rising scores: f16(p * vscale *
+    # bias) stays finite although p passes 1 under the lazy rescale. One call is cut along its keys, one is not
+    n_heads, n_kv = 4, 2
+    say("rescale prefill i8 large values", hd, staged, n, pos0)
+    q, kc, vc, ks, vs = ramp_inputs(7500 + hd + n, n, pos0 + n, n_heads, n_kv, hd, i8=True)
+    rng = np.random.default_rng(7501 + hd)
+    vs = np.exp(rng.uniform(np.log(0.02), np.log(30.0), vs.shape)).astype(np.float32)
+    t = [torch.from_numpy(x).to(gpu) for x in (q, kc, vc, ks, vs)]
+    out = gi_attn.prefill(t[0], t[1], t[2], pos0, n_heads, n_kv, hd=hd, out_dtype=torch.float32, k_scale=t[3],
+                          v_scale=t[4], staged=staged)
+    torch.cuda.synchronize()
+    # The bar is for values of standard deviation 1. An output's error is at most (f16 steps of P and Q) times the
+    # magnitude of the values that it averages, and a row may see mostly keys of the largest scale (an int8 row has a
+    # standard deviation of about 40 scales), so the unit is that of the largest scale.
+    unit = 40 * float(vs.max())
+    want = O.prefill_tc_semantics_i8(q, kc, vc, ks, vs, pos0, n_heads, n_kv, hd=hd)
+    assert_close(out.cpu().numpy() / unit, np.asarray(want) / unit, what=f"rising scores, large values, int8 prefill hd {hd}")
