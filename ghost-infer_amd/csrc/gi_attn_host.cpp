@@ -868,7 +868,9 @@ int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, c
             return fail("the prefill workspace holds %zu bytes; %zu needed (gi_attn_prefill_workspace_bytes)",
                         workspace_bytes, need);
         if ((uintptr_t)workspace & 255) return fail("the prefill workspace must be 256-byte aligned");
-        if (!prefill_widens(n, n_heads, n_kv, hd)) return run(2, ws, workspace_bytes);
+        // (a launch is cut only in what the caller gives beyond these bytes: within them the outputs are, bit for bit,
+        // those of the call without a workspace)
+        if (!prefill_widens(n, n_heads, n_kv, hd)) return run(2, ws + need, workspace_bytes - need);
         unsigned char* w = ws;
         const size_t rows = align256((size_t)n_kv * len * hd * 2), scales = fmt == 1 ? align256((size_t)n_kv * len * 4) : 0;
         GiWidenArgs wa{};
@@ -1151,10 +1153,11 @@ int attention_impl(void* stream, const float* qkv, const void* kc, const void* v
     }
     if (n >= kTiledMinBatch && !verify && !no_tc) {
         if (posp) return fail("a device position (posp) is only taken by the split path");
-        // the int8 and 4-bit caches: pre-widened staging when the workspace holds it
-        const bool staged = fmt && workspace && workspace_bytes >= prefill_ws_bytes(pos0 + n, n_kv, hd, fmt);
+        // the int8 and 4-bit caches: pre-widened staging when the workspace holds it, else as without one (the same
+        // outputs bit for bit); the f16 cache and the f32 kernels: as gi_attn_prefill_ws
+        if (fmt && !f32_hd(hd) && workspace_bytes < prefill_ws_bytes(pos0 + n, n_kv, hd, fmt)) workspace = nullptr;
         return prefill_impl(stream, qkv, GI_F32, row, kc, vc, ks, vs, scs, sch, fmt, kvs, kvh, out, GI_F32, q_dim, pos0,
-                            n, n_heads, n_kv, hd, scale, workspace, workspace_bytes, false, staged);
+                            n, n_heads, n_kv, hd, scale, workspace, workspace ? workspace_bytes : 0);
     }
     for (int b0 = 0; b0 < n; b0 += kSplitMaxBatch) {
         int m = std::min(n - b0, kSplitMaxBatch);

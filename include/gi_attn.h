@@ -176,10 +176,11 @@ size_t gi_attn_prefill_workspace_bytes(int kv_len, int n_kv, int hd, int fmt);
  * gi_attn_prefill_workspace_bytes(pos0 + n, ...) bytes): the keys 0..pos0+n-1 are first widened into it to the f16
  * values the tiles take (int8: the exact integers, the scales kept apart; 4-bit: f16((n - 8) * scale)), and the
  * prefill then stages the widened tiles as it stages the f16 cache. (Head sizes 64 and 128 with at most 256 query rows per
- * kv head: the tiles are widened inside the prefill, once each, which is faster there.) The same arithmetic and outputs,
- * bit for bit, as the entry points without a workspace (replaces what they replace); in a workspace larger than
- * gi_attn_prefill_workspace_bytes the launch may also be cut along its keys, as in gi_attn_prefill_ws. gi_attention_i8 / gi_attention_q4 take this
- * path for prefill batches whenever their workspace holds it. */
+ * kv head: the tiles are widened inside the prefill, once each, which is faster there.) With a workspace of exactly
+ * gi_attn_prefill_workspace_bytes the arithmetic and the outputs are, bit for bit, those of the entry points without a
+ * workspace (replaces what they replace); in what a larger one holds beyond that the launch may also be cut along its
+ * keys, as in gi_attn_prefill_ws. gi_attention_i8 / gi_attention_q4 take prefill batches this way whenever their
+ * workspace holds gi_attn_prefill_workspace_bytes(pos0 + n, ...), and as without a workspace otherwise. */
 int gi_attn_prefill_i8_ws(void* stream, const void* q, int q_dtype, long long q_stride, const int8_t* kc,
                           const int8_t* vc, const float* ks, const float* vs, long long kv_stride,
                           long long kv_head_stride, long long sc_stride, long long sc_head_stride, void* out,
@@ -217,9 +218,9 @@ int gi_attn_prefill_ws(void* stream, const void* q, int q_dtype, long long q_str
  * (SPLIT_MAX_BATCH, src/cuda.rs:119). Bit 1 of `exact` is the reference's GHOST_INFER_NO_TC_ATT
  * (src/cuda.rs:5648-5655): prefill batches take the f32 prefill (gi_attn_prefill_f32) at head sizes up to 128 over
  * the f16 and int8 caches and the split path elsewhere, and at head size 256 over the int8 cache the split path
- * computes in f32 precision instead of attention_decode_tc256's roundings. A prefill batch uses the workspace as
- * gi_attn_prefill_ws does, where it is large enough. fixed_split
- * with posp: the grid is sized for ctx_cap (the session capacity), as max_splits does. scale is
+ * computes in f32 precision instead of attention_decode_tc256's roundings. A prefill batch over the f16 cache, or in
+ * f32, uses the workspace as gi_attn_prefill_ws does, where it is large enough (over the int8 and 4-bit caches: as
+ * gi_attn_prefill_i8_ws). fixed_split with posp: the grid is sized for ctx_cap (the session capacity), as max_splits does. scale is
  * 1/sqrt(hd) as in the reference. */
 int gi_attention(void* stream, const float* qkv, const uint16_t* kc, const uint16_t* vc, float* out,
                  void* workspace, size_t workspace_bytes, int pos0, const int* posp, int ctx_cap, int n, int n_heads,
