@@ -353,13 +353,25 @@ def _prefill_scratch(pos0, n, n_heads, n_kv, hd, fmt, flags, device):
     return (torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None), nbytes
 
 
-def _prefill_ws(q, k_cache, v_cache, k_scale, v_scale, fmt, flags, strides, out, pos0, n, n_heads, n_kv, hd, scale):
-    """gi_attn_prefill_ws with a scratch of its own."""
-    scratch, nbytes = _prefill_scratch(pos0, n, n_heads, n_kv, hd, fmt, flags, q.device)
+def _workspace(t):
+    """(pointer, bytes) of a workspace that the caller gives, of any type."""
+    if not isinstance(t, torch.Tensor) or not t.is_cuda:
+        raise GiAttnError("workspace must be a CUDA tensor")
+    return t.data_ptr(), t.numel() * t.element_size()
+
+
+def _prefill_ws(q, k_cache, v_cache, k_scale, v_scale, fmt, flags, strides, out, pos0, n, n_heads, n_kv, hd, scale,
+                workspace=None):
+    """gi_attn_prefill_ws in the workspace given, else with a scratch of its own."""
+    if workspace is not None:
+        scratch, nbytes = _workspace(workspace)
+    else:
+        scratch, nbytes = _prefill_scratch(pos0, n, n_heads, n_kv, hd, fmt, flags, q.device)
+        scratch = _ptr(scratch)
     _check(load_library().gi_attn_prefill_ws(
         _stream(), _ptr(q), GI_F16 if q.dtype == torch.float16 else GI_F32, q.stride(0), _ptr(k_cache), _ptr(v_cache),
         _ptr(k_scale), _ptr(v_scale), fmt, flags, *strides, _ptr(out), GI_F16 if out.dtype == torch.float16 else GI_F32,
-        out.stride(0), pos0, n, n_heads, n_kv, hd, scale, _ptr(scratch), nbytes))
+        out.stride(0), pos0, n, n_heads, n_kv, hd, scale, scratch, nbytes))
 
 
 def prefill_q4(q, k_cache, v_cache, k_scale, v_scale, pos0, n_heads, n_kv, scale=None, out=None, out_dtype=None,
@@ -367,7 +379,7 @@ def prefill_q4(q, k_cache, v_cache, k_scale, v_scale, pos0, n_heads, n_kv, scale
     """Causal prefill over the 4-bit cache (head size 256; attention_prefill_tc256 with KV4, src/cuda.rs:2495-2514):
     q the rotated queries, f32 or f16 [n, >= n_heads*256]; returns rotated rows of out_dtype (default q's).
     staged: widen the keys into a workspace first (allocated here unless given) and stage the widened tiles as the
-    f16 cache's are (the same outputs); else the kernel widens each tile as it stages it."""
+    f16 cache's are (the same outputs); else the kernel widens each tile as it stages it. workspace: as prefill's."""
     if q.dtype not in (torch.float32, torch.float16):
         raise GiAttnError("q must be float32 or float16")
     _need(q, "q", q.dtype)
@@ -393,7 +405,7 @@ def prefill_q4(q, k_cache, v_cache, k_scale, v_scale, pos0, n_heads, n_kv, scale
             _ptr(workspace), workspace.numel()))
         return out
     _prefill_ws(q, k_cache, v_cache, k_scale, v_scale, 2, GI_PREFILL_WIDEN if staged else 0,
-                (kv_stride, kv_head_stride, sc_stride, sc_head_stride), out, pos0, n, n_heads, n_kv, 256, scale)
+                (kv_stride, kv_head_stride, sc_stride, sc_head_stride), out, pos0, n, n_heads, n_kv, 256, scale, workspace)
     return out
 
 
@@ -453,6 +465,9 @@ def prefill(q, k_cache, v_cache, pos0, n_heads, n_kv, hd=128, scale=None, out=No
     widened into a workspace first (allocated here unless given) and the widened tiles staged as the f16 cache's
     are (the same outputs); else the kernel widens each tile as it stages it. f32: the prompt in f32 (no f16
     rounding of Q or P), the reference's attention_prefill with its tensor-core prefill off (head sizes up to 128).
+    workspace: a CUDA tensor that also takes the partial results of a launch cut along its keys, in place of a scratch
+    allocated here; a smaller one (an empty one) means no cut (gi_attn_prefill_scratch_bytes). Given with staged over the
+    int8 cache it is uint8 and holds the widened keys at least (prefill_workspace).
     """
     if q.dtype not in (torch.float32, torch.float16):
         raise GiAttnError("q must be float32 or float16")
@@ -484,7 +499,7 @@ def prefill(q, k_cache, v_cache, pos0, n_heads, n_kv, hd=128, scale=None, out=No
         return out
     _prefill_ws(q, k_cache, v_cache, k_scale if i8 else None, v_scale if i8 else None, 1 if i8 else 0,
                 (GI_PREFILL_WIDEN if widen else 0) | (GI_PREFILL_F32 if f32 else 0),
-                (kv_stride, kv_head_stride, *(sc if i8 else (0, 0))), out, pos0, n, n_heads, n_kv, hd, scale)
+                (kv_stride, kv_head_stride, *(sc if i8 else (0, 0))), out, pos0, n, n_heads, n_kv, hd, scale, workspace)
     return out
 
 
@@ -498,7 +513,8 @@ def attention(qkv, k_cache, v_cache, pos0, n_heads, n_kv, hd=128, exact=False, o
     reference's [capacity, n_kv, hd]: f16, or int8 with f32 scales [capacity, n_kv] (its (kc, vc, ks, vs)).
     no_tc: the reference's GHOST_INFER_NO_TC_ATT: batches of >= 16 tokens in f32 (head sizes up to 128; above, the
     split path), and at head size 256 over the int8 cache the split path in f32 precision instead of the tc256
-    roundings.
+    roundings. workspace: the call's only scratch when given (nothing is allocated then); a prefill batch is cut along its
+    keys only where it holds the partial results.
     """
     _need(qkv, "qkv", torch.float32)
     n = qkv.shape[0]
@@ -530,9 +546,10 @@ def attention(qkv, k_cache, v_cache, pos0, n_heads, n_kv, hd=128, exact=False, o
             cap = ctx_cap if posp is not None else pos0 + n
             workspace = new_workspace(cap, min(n, SPLIT_MAX_BATCH), n_heads, n_kv, hd, qkv.device)
         ws_ptr, ws_bytes = _ptr(workspace), workspace.numel() * workspace.element_size()
-    elif i8 and not no_tc and workspace is not None:
-        # a prefill batch over the int8 cache: the pre-widened staging, whose workspace the library checks
-        ws_ptr, ws_bytes = _ptr(workspace), workspace.numel() * workspace.element_size()
+    elif workspace is not None:
+        # a prefill batch in the caller's workspace: the library takes what it holds (the widened keys of the int8 cache,
+        # a cut launch's partials) and does without the rest
+        ws_ptr, ws_bytes = _workspace(workspace)
     else:
         flags = (GI_PREFILL_WIDEN if i8 else 0) if not no_tc else GI_PREFILL_F32
         scratch, ws_bytes = _prefill_scratch(pos0, n, n_heads, n_kv, hd, 1 if i8 else 0, flags, qkv.device)

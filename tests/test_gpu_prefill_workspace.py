@@ -62,3 +62,49 @@ def test_i8_workspace_up_to_the_widened_keys_changes_no_bit(gpu, n, pos0, n_head
         out.zero_()
         assert merges(call) == 1
         assert_close(out.cpu().numpy(), none.cpu().numpy(), what="cut")
+
+
+# (n, pos0, n_heads, n_kv, hd, f32)
+ANY_SHAPES = [(57, 3000, 16, 4, 128, False), (40, 2000, 9, 3, 64, False), (40, 1500, 8, 2, 256, False), (40, 1000, 8, 2, 96, False),
+              (40, 1000, 8, 2, 128, True)]
+
+
+@pytest.mark.parametrize("n,pos0,n_heads,n_kv,hd,f32", ANY_SHAPES)
+def test_f16_and_f32_calls_take_the_workspace_they_are_given(gpu, n, pos0, n_heads, n_kv, hd, f32):
+    # enough room: the launch is cut as with a scratch of its own, the same bits, and nothing is allocated; too small for
+    # any cut, misaligned or empty: it is not cut, as the entry points without a workspace
+    print("[case] given workspace", n, pos0, n_heads, n_kv, hd, f32, flush=True)
+    lib = gi_attn.load_library()
+    part = lib.gi_attn_prefill_scratch_bytes(pos0, n, n_heads, n_kv, hd, 0, gi_attn.GI_PREFILL_F32 if f32 else 0)
+    assert part > 0
+    gen = torch.Generator(device=gpu).manual_seed(9950 + hd)
+    qkv = torch.randn((n, (n_heads + 2 * n_kv) * hd), device=gpu, generator=gen)
+    kt, vt = (torch.randn((pos0 + n, n_kv, hd), device=gpu, generator=gen).half() for _ in range(2))
+    q, scale = qkv[:, :n_heads * hd], 1.0 / ctypes.c_float(hd ** 0.5).value
+    out, uncut = (torch.empty((n, n_heads * hd), device=gpu) for _ in range(2))
+    args = (gi_attn._stream(), qkv.data_ptr(), gi_attn.GI_F32, qkv.shape[1], kt.data_ptr(), vt.data_ptr())
+    tail = (n_kv * hd, hd)
+    if f32:
+        gi_attn._check(lib.gi_attn_prefill_f32(*args, None, None, 0, *tail, 0, 0, uncut.data_ptr(), gi_attn.GI_F32, n_heads * hd, pos0, n,
+                                               n_heads, n_kv, hd, scale))
+    else:
+        gi_attn._check(lib.gi_attn_prefill(*args, *tail, uncut.data_ptr(), gi_attn.GI_F32, n_heads * hd, pos0, n, n_heads, n_kv, hd, scale))
+    room = torch.empty(part + 16, dtype=torch.uint8, device=gpu)
+    calls = (lambda ws: gi_attn.prefill(q, kt, vt, pos0, n_heads, n_kv, hd=hd, scale=scale, out=out, f32=f32, workspace=ws),
+             lambda ws: gi_attn.attention(qkv, kt, vt, pos0, n_heads, n_kv, hd=hd, out=out, no_tc=f32, workspace=ws))
+    for call in calls:
+        call(None)
+        own = out.clone()
+        assert_close(own.cpu().numpy(), uncut.cpu().numpy(), what="cut")
+        out.zero_()
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        assert merges(lambda: call(room)) == 1
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+        assert torch.equal(out, own)
+        for ws in (room[:4096], room[8:], room[:0]):
+            out.zero_()
+            assert merges(lambda: call(ws)) == 0
+            assert torch.equal(out, uncut)
+        with pytest.raises(gi_attn.GiAttnError, match="workspace must be a CUDA tensor"):
+            call(torch.empty(part, dtype=torch.uint8))
