@@ -1543,6 +1543,8 @@ template <int RW> __device__ __forceinline__ float2* pf_part_ml(const GiPrefillA
 #define PF_BK 64           // keys per tile
 #define PF_TILE 16384      // bytes of one K or V tile: 64 rows of 256 bytes
 #define PF_RESCALE_LOG2 8.0f
+#define PF_ENTER 0x41000000     // the bits of PF_RESCALE_LOG2
+#define PF_ENTER_ANY 0xff800000 // of -inf
 #define GI_LDS __attribute__((address_space(3)))
 // Tile staging from HBM straight into LDS (buffer_load_dwordx4 ... lds: lane i's 16 bytes land at
 // M0 + 16i). Issued from inline asm, so the compiler does not track these loads: were it to see them, it
@@ -1938,6 +1940,10 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
         const auto p = __builtin_amdgcn_permlane32_swap(__float_as_int(mx), __float_as_int(mx), false, false);
         return fmaxf(__int_as_float(p[0]), __int_as_float(p[1]));
     };
+    auto halves_sum = [&](float v) {
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+        return __int_as_float(p[0]) + __int_as_float(p[1]);
+    };
     auto rowmax = [&](const f16x* sc) {
         float mx = GI_NEG_INF;
 #pragma unroll
@@ -1953,6 +1959,9 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
 
     h8 kf[RING], vf[VRING];
     float mx = GI_NEG_INF;
+    // max above which a tile goes through the rescale, as bits (one scalar register); -inf while some row of the wave has
+    // no reference yet (none of its scores so far was above -inf)
+    int enter = PF_ENTER;
     f16x sa[NBLK], sb[NBLK]; // scores of alternate tiles
     // int8 at head size 256: the value scale of tile key `lane` (of the tile whose P V comes next)
     constexpr bool VCAP = I8 && WIDE;
@@ -2004,12 +2013,14 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
         if constexpr (VCAP)
             if (__builtin_amdgcn_ballot_w64(fabsf(vkey) > PF_WIDE_VFREE)) // p * vscale * 2^10 stays within f16
                 top = fmaxf(PF_WIDE_VCAP - __builtin_amdgcn_logf(gi_wave_max(fabsf(vkey))), 0.f);
-        const bool up = mx > top;
-        if (__builtin_amdgcn_ballot_w64(up)) {
+        if (__builtin_amdgcn_ballot_w64(mx > (VCAP ? fminf(top, __int_as_float(enter)) : __int_as_float(enter)))) {
             // some row's max moved: shift the reference by delta, rescale O and l (alpha = 1 for the other rows) and this
-            // tile's scores; the next tile's QK starts from the new reference
+            // tile's scores; the next tile's QK starts from the new reference. A row that has no sum yet takes any finite
+            // max (its O and l are 0: no alpha above 1).
+            const bool none = halves_sum(l_run) == 0.f, up = mx > top || (none && mx > GI_NEG_INF);
+            enter = __builtin_amdgcn_ballot_w64(none && !up) ? PF_ENTER_ANY : PF_ENTER;
             const float delta = up ? mx : 0.f;
-            const float alpha = __builtin_amdgcn_exp2f(-delta);
+            const float alpha = __builtin_amdgcn_exp2f(-fmaxf(delta, 0.f));
             m_run += delta;
 #pragma unroll
             for (int e = 0; e < 16; e++) negm[e] = -m_run;
@@ -2151,9 +2162,11 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
         }
         mx = rowmax(sa);
         // every row takes its first max as its reference (a row that sees no key of a slice's first tile sees none of
-        // its later ones: its reference stays 0 and its sum 0)
+        // its later ones: its reference stays 0 and its sum 0; one that sees only scores of -inf there takes the first
+        // finite max of its later tiles)
         mask(t_begin, sa);
         m_run = mx > GI_NEG_INF ? mx : 0.f;
+        enter = __builtin_amdgcn_ballot_w64(!(mx > GI_NEG_INF)) ? PF_ENTER_ANY : PF_ENTER;
 #pragma unroll
         for (int e = 0; e < 16; e++) negm[e] = -m_run;
 #pragma unroll
@@ -2175,7 +2188,7 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     __builtin_amdgcn_s_waitcnt(GI_VMCNT(0)); // no load may write this LDS once the workgroup has ended
 
     // ---- normalise and write: lane holds query qcol, dims 32db + 8i + 4*half + jj
-    float l = l_run + __shfl_xor(l_run, 32, 64);
+    const float l = halves_sum(l_run);
     if (a.nslice > 1) { // a slice's partial; a row with no key here (sum 0) leaves max -inf
         if (wave >= a.pwaves) return;
         f4* po = reinterpret_cast<f4*>(pf_part_o<32>(a, HD, un.unit, wave)) + lane;

@@ -208,3 +208,28 @@ def test_prefill_rising_scores_i8_large_values(gpu, hd, staged, n, pos0):
     unit = 40 * float(vs.max())
     want = O.prefill_tc_semantics_i8(q, kc, vc, ks, vs, pos0, n_heads, n_kv, hd=hd)
     assert_close(out.cpu().numpy() / unit, np.asarray(want) / unit, what=f"rising scores, large values, int8 prefill hd {hd}")
+
+
+@pytest.mark.parametrize("n,pos0", [(200, 0), (100, 1500), (300, 4000)])
+@pytest.mark.parametrize("hd", [64, 96, 128, 256])
+def test_prefill_tiles_whose_scores_are_all_minus_infinity(gpu, hd, n, pos0):
+    # every other tile of 64 keys, the first one of each among them, scores -inf (an overflowed key), the rest around -40
+    # log2 units, where f16 probabilities against a reference of 0 would all vanish: a row's first tile of a slice then
+    # gives it no reference, and the first later one has to. Rows that see only such keys have no answer (NaN)
+    n_heads, n_kv = 4, 2
+    say("minus infinity", hd, n, pos0)
+    rng = np.random.default_rng(7600 + hd + n)
+    ctx = pos0 + n
+    q, k, v = (rng.standard_normal((m, h, hd)).astype(np.float32) for m, h in ((n, n_heads), (ctx, n_kv), (ctx, n_kv)))
+    q[..., 0], q[..., 1] = 4.0, 16.0
+    k[..., 1] = -40.0 * np.sqrt(hd) / np.log2(np.e) / 16.0
+    dead = np.arange(ctx) // 64 % 2 == 0
+    k[dead, :, 0] = -np.inf
+    q = q.reshape(n, -1)
+    k, v = (x.reshape(ctx, -1).astype(np.float16).view(np.uint16) for x in (k, v))
+    out = gi_attn.prefill(torch.from_numpy(q).to(gpu), f16_dev(k, gpu), f16_dev(v, gpu), pos0, n_heads, n_kv, hd=hd)
+    torch.cuda.synchronize()
+    live = pos0 + np.arange(n) >= 64
+    want = reference_f64(q[live], k, v, pos0 + int((~live).sum()), n_heads, n_kv, hd=hd)
+    assert_close(out.cpu().numpy()[live], want, what=f"minus infinity, hd {hd}")
+    assert np.isnan(out.cpu().numpy()[~live]).all()
