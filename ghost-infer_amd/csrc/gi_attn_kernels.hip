@@ -199,6 +199,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t gi_rsrc(const void* p, long lo
     int n = (int)(bytes < 0 ? 0 : (bytes > 0x7ffffff0ll ? 0x7ffffff0ll : bytes));
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, n, GI_RSRC_FLAGS);
 }
+// The same for a tile's rows, 0 <= n < 2^31. (gi_rsrc's two bounds on a 32-bit count become one v_med3: the descriptor is
+// then in vector registers, and every load a loop over the lanes' descriptors. 1024 tokens at a 3000-token prefix, 16/2
+// heads of 256, tiles widened through registers: int8 198 us with these loops, 170 without; 4-bit 187 and 181.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gi_rsrc_tile(const void* p, int n) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, n, GI_RSRC_FLAGS);
+}
 __device__ __forceinline__ u4 gi_load16(__amdgpu_buffer_rsrc_t r, int off) {
     return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
 }
@@ -274,9 +280,10 @@ template <typename A, typename B> struct gi_pick<false, A, B> { typedef B type; 
 // the and-or keeps the nibbles under the f16 bits 0x6400 (1024 + n), the packed subtract leaves n - 8 exactly
 // and the packed multiply by the scales rounds (n - 8) * s to nearest even once, as the reference's conversion
 // of the exact f32 product does.
-__device__ __forceinline__ uint32_t q4_f16x2(uint32_t hi, uint32_t lo, int j, h2x sc) {
+__device__ __forceinline__ uint32_t q4_f16x2(uint32_t hi, uint32_t lo, int j, h2x sc, uint32_t keep = 0x000f000fu,
+                                             uint32_t bits = 0x64006400u) {
     const uint32_t sel = (uint32_t)j | 0x0c00u | (uint32_t)(4 + j) << 16 | 0x0c000000u;
-    const uint32_t w = (__builtin_amdgcn_perm(hi, lo, sel) & 0x000f000fu) | 0x64006400u;
+    const uint32_t w = (__builtin_amdgcn_perm(hi, lo, sel) & keep) | bits;
     const h2x v = (__builtin_bit_cast(h2x, w) - h2x{(_Float16)1032.f, (_Float16)1032.f}) * sc;
     return __builtin_bit_cast(uint32_t, v);
 }
@@ -1760,68 +1767,73 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     };
     // int8 and 4-bit tiles through registers: thread -> chunks of 16 bytes of the tile's K and V rows (row ch / NCH, 16 or
     // 32 values), widened to f16 (int8: the exact integers; 4-bit: f16((n - 8) * scale), the chunk's one scale) and
-    // written into the same swizzled image; int8: threads 0-63 take the K scale of key tid, 64-127 the V scale of key
-    // tid - 64 (times the bias). int8 lanes in the upper half of a 128-value row hold their chunk's two 8-byte halves
+    // written into the same swizzled image; int8: wave 0 takes the K scales of the tile's 64 keys, wave 1 the V scales
+    // (times the bias). int8 lanes in the upper half of a 128-value row hold their chunk's two 8-byte halves
     // swapped (and write them in that order): the 8 lanes of a row that one 16-byte LDS store serves then write 8
     // different units mod 8, all 32 banks, where 2ch alone would cover half of them twice.
     constexpr int NT = 64 * WAVES, VPC = FMT == 2 ? 32 : 16, NCH = HD / VPC, CH = BK * NCH, CPT = CH > NT ? CH / NT : 1;
     const unsigned char* kb8 = reinterpret_cast<const unsigned char*>(a.kc) + kvh * a.kv_head_stride;
     const unsigned char* vb8 = reinterpret_cast<const unsigned char*>(a.vc) + kvh * a.kv_head_stride;
-    const float* scb = RSTG && I8 ? (tid < BK ? a.ks : a.vs) + kvh * a.sc_head_stride : nullptr;
+    const float* scb = RSTG && I8 ? (wave ? a.vs : a.ks) + kvh * a.sc_head_stride : nullptr;
     struct Chunks { u4 w[CPT]; uint16_t sc[FMT == 2 ? CPT : 1]; };
     Chunks rk, rv;
     float rsc = 0.f;
-    auto load_rows = [&](bool v, int t, Chunks& c) {
+    auto load_chunk = [&](bool v, int t, Chunks& c, int i) {
         const int t0 = t * BK, rows = t <= last ? min(kv_len - t0, BK) : 0;
-        const __amdgpu_buffer_rsrc_t rs = gi_rsrc((v ? vb8 : kb8) + (long long)t0 * kvs, rows * (int)kvs);
+        const __amdgpu_buffer_rsrc_t rs = gi_rsrc_tile((v ? vb8 : kb8) + (long long)t0 * kvs, rows * (int)kvs);
         const uint16_t* sp = FMT == 2 ? reinterpret_cast<const uint16_t*>(v ? a.vs : a.ks) + kvh * a.sc_head_stride + (long long)t0 * a.sc_stride : nullptr;
-        const __amdgpu_buffer_rsrc_t rss = gi_rsrc(sp, FMT == 2 ? rows * (int)a.sc_stride * 2 : 0);
-#pragma unroll
-        for (int i = 0; i < CPT; i++) {
-            const int ch = tid + NT * i, off = ch / NCH * (int)kvs + 16 * (ch % NCH), flip = (ch % NCH >> 2) & 1;
-            if (CH % NT && ch >= CH) continue;
-            if constexpr (FMT == 2) {
-                c.w[i] = gi_load16(rs, off);
-                c.sc[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rss, (ch / NCH * (int)a.sc_stride + ch % NCH) * 2, 0, 0);
-            } else {
-                const u2 h0 = gi_load8(rs, off + 8 * flip), h1 = gi_load8(rs, off + 8 - 8 * flip);
-                c.w[i] = u4{h0.x, h0.y, h1.x, h1.y};
-            }
+        const __amdgpu_buffer_rsrc_t rss = gi_rsrc_tile(sp, FMT == 2 ? rows * (int)a.sc_stride * 2 : 0);
+        const int ch = tid + NT * i, off = ch / NCH * (int)kvs + 16 * (ch % NCH), flip = (ch % NCH >> 2) & 1;
+        if (CH % NT && ch >= CH) return;
+        if constexpr (FMT == 2) {
+            c.w[i] = gi_load16(rs, off);
+            c.sc[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rss, (ch / NCH * (int)a.sc_stride + ch % NCH) * 2, 0, 0);
+        } else {
+            const u2 h0 = gi_load8(rs, off + 8 * flip), h1 = gi_load8(rs, off + 8 - 8 * flip);
+            c.w[i] = u4{h0.x, h0.y, h1.x, h1.y};
         }
+    };
+    auto load_rows = [&](bool v, int t, Chunks& c) {
+#pragma unroll
+        for (int i = 0; i < CPT; i++) load_chunk(v, t, c, i);
     };
     auto load_scales = [&](int tk, int tv) {
         if constexpr (I8) {
-            const int t0 = (tid < BK ? tk : tv) * BK, rows = t0 <= last * BK ? min(kv_len - t0, BK) : 0;
-            rsc = 0.f;
-            if (tid < 2 * BK && (tid & (BK - 1)) < rows) rsc = scb[(long long)(t0 + (tid & (BK - 1))) * a.sc_stride];
+            if (wave > 1) return;
+            const int t = wave ? tv : tk, t0 = t * BK, rows = t <= last ? min(kv_len - t0, BK) : 0;
+            rsc = gi_load4f(gi_rsrc_tile(scb + (long long)t0 * a.sc_stride, rows * (int)a.sc_stride * 4), lane * (int)a.sc_stride * 4);
         }
     };
-    auto write_rows = [&](bool v, int t, const Chunks& c) {
-        GI_LDS unsigned char* img = (GI_LDS unsigned char*)smem + (v ? vbuf(t) : kbuf(t));
-#pragma unroll
-        for (int i = 0; i < CPT; i++) {
-            const int ch = tid + NT * i, row = ch / NCH, flip = FMT == 1 ? (ch % NCH >> 2) & 1 : 0;
-            if (CH % NT && ch >= CH) continue;
-#pragma unroll
-            for (int q = 0; q < VPC / 8; q++) { // unit of 8 values
-                const int u = VPC / 8 * (ch % NCH) + (q ^ flip);
-                u4 w;
-                if constexpr (FMT == 2) {
-                    const uint32_t x = c.w[i][q];
-                    const h2x sc = __builtin_bit_cast(h2x, (uint32_t)c.sc[i] * 0x10001u);
-                    w = u4{q4_f16x2(x >> 4, x, 0, sc), q4_f16x2(x >> 4, x, 1, sc), q4_f16x2(x >> 4, x, 2, sc), q4_f16x2(x >> 4, x, 3, sc)};
-                } else {
-                    const uint32_t x0 = gi_i8_in(c.w[i][2 * q]), x1 = gi_i8_in(c.w[i][2 * q + 1]);
-                    w = u4{i8_f16x2(x0, GI_I8_LO), i8_f16x2(x0, GI_I8_HI), i8_f16x2(x1, GI_I8_LO), i8_f16x2(x1, GI_I8_HI)};
-                }
-                *reinterpret_cast<GI_LDS u4*>(img + (u / 16) * PF_TILE + row * 256 + (((u % 16) ^ (v ? (row & 3) << 2 : row & 15)) << 4)) = w;
-            }
+    constexpr int UPC = VPC / 8; // units of 8 values of a chunk
+    // (4-bit: the and-or takes one instruction with its constants in registers, two with literals)
+    uint32_t q4_keep = 0x000f000fu, q4_bits = 0x64006400u;
+    if constexpr (FMT == 2) asm("" : "+v"(q4_keep), "+v"(q4_bits));
+    // word e (2 values) of unit q of chunk i, widened; and the unit's store
+    auto widen2 = [&](const Chunks& c, int i, int q, int e) {
+        if constexpr (FMT == 2) {
+            const uint32_t x = c.w[i][q];
+            return q4_f16x2(x >> 4, x, e, __builtin_bit_cast(h2x, (uint32_t)c.sc[i] * 0x10001u), q4_keep, q4_bits);
+        } else {
+            return i8_f16x2(gi_i8_in(c.w[i][2 * q + (e >> 1)]), e & 1 ? GI_I8_HI : GI_I8_LO);
         }
+    };
+    auto write_unit = [&](bool v, int t, int i, int q, u4 w) {
+        GI_LDS unsigned char* img = (GI_LDS unsigned char*)smem + (v ? vbuf(t) : kbuf(t));
+        const int ch = tid + NT * i, row = ch / NCH, flip = FMT == 1 ? (ch % NCH >> 2) & 1 : 0, u = UPC * (ch % NCH) + (q ^ flip);
+        if (CH % NT && ch >= CH) return;
+        *reinterpret_cast<GI_LDS u4*>(img + (u / 16) * PF_TILE + row * 256 + (((u % 16) ^ (v ? (row & 3) << 2 : row & 15)) << 4)) = w;
+    };
+    auto write_rows = [&](bool v, int t, const Chunks& c) {
+#pragma unroll
+        for (int i = 0; i < CPT; i++)
+#pragma unroll
+            for (int q = 0; q < UPC; q++)
+                write_unit(v, t, i, q, u4{widen2(c, i, q, 0), widen2(c, i, q, 1), widen2(c, i, q, 2), widen2(c, i, q, 3)});
     };
     auto write_scales = [&](int tk, int tv) {
         if constexpr (I8) {
-            if (tid < BK) kscl(tk)[tid] = rsc;
-            else if (tid < 2 * BK) vscl(tv)[tid - BK] = WIDE ? rsc : rsc * VB;
+            if (wave == 0) kscl(tk)[lane] = rsc;
+            else if (wave == 1) vscl(tv)[lane] = WIDE ? rsc : rsc * VB;
         }
     };
     auto stage1 = [&](const StageAt& s, int i) {
@@ -1979,14 +1991,18 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     };
     auto stage_tile = [&](int it) { return it + (WIDE ? 3 : 4) - (stage_v ? 1 : 0); };
     // register staging of iteration it: the rows loaded in iteration it-1 (K of tile it+2, V of tile it+1) are widened
-    // into their buffers (free since the barrier of it-1), and the next ones' loads go out
-    auto restage_k = [&](int it) {
-        write_rows(false, it + 2, rk);
-        load_rows(false, it + 3, rk);
-    };
-    auto restage_v = [&](int it) {
-        write_rows(true, it + 1, rv);
-        load_rows(true, it + 2, rv);
+    // into their buffers (free since the barrier of it-1), and the next ones' loads go out. Piece j of RPC widens one word
+    // (2 values; K's chunks first, then V's), the last word of a unit stores it, the last unit of a chunk loads the next:
+    // a few instructions under each MFMA (whole units at a time, 20 instructions under every fourth: 170 us instead of 166
+    // for the int8 cache at the sizes above, 181 instead of 171 for the 4-bit one)
+    constexpr int RPC = 2 * CPT * UPC * 4;
+    u4 rw = u4{0u, 0u, 0u, 0u};
+    auto restage = [&](int it, int j) {
+        const bool v = j >= RPC / 2;
+        const int e = j % 4, q = j / 4 % UPC, i = j % (RPC / 2) / (4 * UPC);
+        rw[e] = widen2(v ? rv : rk, i, q, e);
+        if (e == 3) write_unit(v, v ? it + 1 : it + 2, i, q, rw);
+        if (e == 3 && q == UPC - 1) load_chunk(v, v ? it + 2 : it + 3, v ? rv : rk, i);
     };
     auto restage_s = [&](int it) {
         write_scales(it + 2, it + 1);
@@ -2068,8 +2084,9 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
             if constexpr (sl + RING >= NS) kf[(sl + RING - NS) % RING] = kfrag(B2, sl + RING - NS);
             // staging behind the barrier
             if constexpr (RSTG) {
-                if (sl == 1) restage_k(it);
-                if (sl == NQ / 2 + 1) restage_v(it);
+#pragma unroll
+                for (int j = 0; j < RPC; j++)
+                    if (sl == j * (NS - RING - 2) / RPC) restage(it, j);
                 if (sl == NQ - 1) restage_s(it);
             } else {
 #pragma unroll
@@ -2123,8 +2140,8 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
             step(it, s, sn);
         } else { // past its last tile a wave goes on staging and keeping the barriers
             if constexpr (RSTG) {
-                restage_k(it);
-                restage_v(it);
+#pragma unroll
+                for (int j = 0; j < RPC; j++) restage(it, j);
                 restage_s(it);
             }
             if constexpr (!RSTG && WIDE) stage(stage_tile(it - 1));
