@@ -13,7 +13,7 @@
 // (times the key's scale for int8); the workgroup takes the tile's max and an online base-2 softmax; the value
 // scale rides on p. The slice's (unnormalised O, max, sum) go to the partial rows gi_decode_combine merges; one
 // slice writes the output.
-// Prefill (gi_prefill_f32_*): one workgroup of 8 waves per (kv head, 128 packed query rows, key slice: PfUnit), on v_mfma_f32_16x16x4f32 (f32
+// Prefill (gi_prefill_f32_*): one workgroup of 8 waves per (set of a kv head's query heads, 128 packed query rows, key slice: PfUnit), on v_mfma_f32_16x16x4f32 (f32
 // operands, f32 accumulation). Tiles of 64 keys are widened to f32 in LDS (int8: times their scales) through
 // registers, the next tile's loads in flight while the current one is used. A wave holds 16 query rows: S^T blocks
 // (16 keys x 16 queries) from K (A) and Q^T (B, in registers); a lane then holds the scores of keys 4(l/16)..+3 of
@@ -171,7 +171,7 @@ __device__ __forceinline__ void gi_prefill_f32_t(const GiPrefillArgs& a) {
     __shared__ __attribute__((aligned(16))) float Ks[PF32_KT * LD];
     __shared__ __attribute__((aligned(16))) float Vs[PF32_KT * LD];
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, lc = l & 15, lg = l >> 4;
-    const int G = a.n_heads / a.n_kv, P = a.n * G;
+    const int G = a.group, P = a.n * G;
     const PfUnit un = pf_unit(a, PF32_ROWS, PF32_KT);
     const int kvh = un.kvh;
     if (un.t_begin >= un.t_end) return; // a slice past the tile's last key
@@ -182,7 +182,7 @@ __device__ __forceinline__ void gi_prefill_f32_t(const GiPrefillArgs& a) {
     const int wend = wrow < P ? a.pos0 + pf_last_token(a, wrow, 16) + 1 : 0; // keys the wave's rows see
     const int qrow = wrow + lc;                                       // this lane's row
     const int qtok = qrow < P ? pf_token(a, qrow) : a.n - 1;
-    const int h = kvh * G + (qrow < P ? qrow : P - 1) - qtok * G;
+    const int h = un.head0 + (qrow < P ? qrow : P - 1) - qtok * G;
     const int lim = a.pos0 + qtok;                                    // its last visible key
     const long long kvs = a.kv_stride, kbase = (long long)kvh * a.kv_head_stride;
     const long long sbase = (long long)kvh * a.sc_head_stride;

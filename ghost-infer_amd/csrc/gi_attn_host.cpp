@@ -5,6 +5,8 @@
 // hipModuleLoad once per device and launched by name with hipModuleLaunchKernel on the caller's stream.
 // No entry point allocates device memory or synchronises the host.
 #include "gi_attn.h"
+#include "gi_prefill_plan.h"
+#include "gi_prefill_rows.h"
 
 #include <hip/hip_runtime.h>
 
@@ -155,10 +157,11 @@ struct GiPrefillArgs {
     int items;
     uint32_t gmul;
     int rows;
+    int group;
+    int sets;
 };
 
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr int kF32Rows = 128;   // query rows per gi_prefill_f32_* workgroup; must match the kernels' PF32_ROWS
 
 // Head sizes of the f32 kernels (gi_attn_f32.hip): the multiples of 16 up to 112 that the MFMA kernels do not
 // take, the reference's f32 fallback cases (attention_partial / attention_prefill, src/cuda.rs:1866-2041).
@@ -173,8 +176,6 @@ constexpr int kSliceUnit = kDecWaves * kDecTile; // 128 keys
 constexpr int kSplitMaxBatch = 15;                // tokens per split launch (src/cuda.rs:119)
 constexpr int kTiledMinBatch = 16;                // prefill from this many tokens (src/cuda.rs:95)
 constexpr int kPrefillRows = 256; // packed query rows per workgroup of 8 waves (head sizes 64 and 128)
-constexpr int kPrefillKeys = 64;  // keys per prefill tile; must match the kernels' PF_BK
-constexpr int kPrefillMaxSlices = 64; // must match the kernels' PFC_MAXS
 constexpr int kPrefillMergeFrags = 4; // must match the kernels' PFC_FRAGS
 
 thread_local std::string g_err;
@@ -688,65 +689,6 @@ size_t prefill_ws_bytes(int kv_len, int n_kv, int hd, int fmt) {
     return 2 * rows + 2 * scales;
 }
 
-// How an MFMA prefill launch is laid out. It has one workgroup per (kv head, tile of packed query
-// rows), and a CU holds one workgroup.
-//  - Waves: 8 (256 rows, two waves per SIMD) or 4 (128 rows, one per SIMD). One wave takes a key tile in about 0.7 of
-//    the time that two on its SIMD take for theirs together, so 4 waves win where the workgroups are few or unequal
-//    (1024 tokens of 32/8 heads of 128, f16: 33.9 us with 8, 23.7 with 4; 512 at a 2000-token prefix 64 and 44) and
-//    8 where they fill the chip several times over (8192 tokens: 505 and 580). Head size 256: 4 or 2.
-//  - Slices: a short batch over a long prefix leaves most of the chip idle while each workgroup walks all of its keys
-//    (512 tokens of 32/4 heads at a 16K prefix: 64 workgroups of 264 key tiles, 350 us). Such a launch cuts the key
-//    tiles of every row tile into slices, one workgroup each, whose partial results a second launch merges (137 us).
-//    An f32 tile takes three to five times as long, so those launches gain from shorter spans on (200 tokens of 32/32
-//    heads of 96 at 1800: 64 workgroups of 32 tiles, 227 us; sliced 69 us).
-// A row's arithmetic does not depend on the waves, only on the slices.
-struct PrefillPlan {
-    int waves;      // 8 or 4; head size 256: 4 or 2; f32: 8 (of 16 rows)
-    int tiles;      // key tiles per slice
-    int nslice;     // slices of the longest row tile
-};
-constexpr int kPrefillRowTiles(long long rows, int per) { return (int)((rows + per - 1) / per); }
-PrefillPlan prefill_plan(int pos0, int n, int n_heads, int n_kv, int hd, bool f32 = false) {
-    const int G = n_heads / n_kv, cus = 256, tmax = (pos0 + n + kPrefillKeys - 1) / kPrefillKeys;
-    const long long P = (long long)n * G;
-    const int most = hd == 256 ? 4 : 8, rw = f32 ? 16 : 32;
-    PrefillPlan p{most, tmax, 1};
-    if ((long long)kPrefillRowTiles(P, rw * most) * n_kv >= 2 * cus) return p; // longest tiles first balances these
-    // Below 16 key tiles slices save less than the merge launch costs. A prompt of up to 4096 keys taken in chunks of
-    // 256 tokens or more keeps each row's arithmetic independent of the chunking (one slice always); beyond, chunks
-    // agree to f32 rounding.
-    const bool may_slice = tmax >= (f32 ? 4 : 16) && (n < 256 || pos0 + n > 4096);
-    // Costs in units of one key tile of an 8-wave workgroup (1.4 to 1.9 us; head size 256: of a 4-wave one): rounds of workgroups over the CUs, each
-    // with a fixed cost until its first tile is in and for its output (~6 us), and for a sliced launch the merge
-    // launch (~5 us) and its read of the partials (~4 TB/s).
-    const double tile_s = f32 ? 5e-6 : 1.5e-6, per_wg = f32 ? 1.2 : 4.0, merge = f32 ? 1.0 : 3.3;
-    double best = 0;
-    for (int waves = most; waves >= (f32 ? most : most / 2); waves -= most / 2) {
-        const int rows = rw * waves, items = kPrefillRowTiles(P, rows);
-        const long long wgs = (long long)items * n_kv;
-        const double tile = waves == most ? 1.0 : hd == 256 ? 0.85 : 0.7;
-        auto tiles_of = [&](int i) { // key tiles of row tile i
-            const long long last = std::min<long long>(n - 1, ((long long)(i + 1) * rows - 1) / G);
-            return (int)((pos0 + last) / kPrefillKeys + 1);
-        };
-        // one slice: the longest workgroup, or the mean load of a CU where there are several rounds
-        const double mean = (double)wgs / cus * (tile * (tiles_of(0) + tmax) / 2 + (wgs > cus ? per_wg : 0));
-        const double one = std::max(tile * tmax, mean) + per_wg;
-        if (waves == most || one < 0.95 * best) best = one, p = PrefillPlan{waves, tmax, 1};
-        if (!may_slice) continue;
-        const double part = std::min<long long>(P, rows) * (hd + 2) * 4.0 / 4e12 / tile_s;
-        for (int S = 2; S <= std::min(kPrefillMaxSlices, tmax / 2) && wgs * S <= 4 * cus; S++) {
-            const int C = (tmax + S - 1) / S;
-            long long u = 0; // workgroups with keys
-            if (tiles_of(0) + C > tmax) u = wgs * ((tmax + C - 1) / C); // (every row tile has tmax tiles or nearly)
-            else
-                for (int i = 0; i < items; i++) u += (long long)n_kv * ((tiles_of(i) + C - 1) / C);
-            const double cost = (double)((u + cus - 1) / cus) * (tile * C + per_wg) + merge + u * part;
-            if (cost < 0.95 * best) best = cost, p = PrefillPlan{waves, C, (tmax + C - 1) / C};
-        }
-    }
-    return p;
-}
 // Rows per kv head from which the int8 keys are widened into the workspace first (one pass over all keys, ~6 bytes moved
 // per value) rather than tile by tile in the prefill: above one row tile, every tile would be widened again for each.
 // 32/8 heads of 128, tile by tile / widened: 16 tokens at a 2000-token prefix 17.6 / 21.5 us, at 16000 29.6 / 43.5; 64
@@ -755,14 +697,6 @@ constexpr int kPrefillWidenRows = kPrefillRows;
 bool prefill_widens(int n, int n_heads, int n_kv, int hd) {
     return hd == 256 || (long long)n * (n_heads / n_kv) > kPrefillWidenRows;
 }
-// Bytes of a sliced launch's partials, in row tiles of `rows` (pwaves: waves of a row tile that hold rows)
-int prefill_pwaves(long long P, int rows, int rw) { return P > rows ? rows / rw : (int)((P + rw - 1) / rw); }
-size_t prefill_part_bytes(const PrefillPlan& p, int n, int n_heads, int n_kv, int hd, int rows, int rw = 32) {
-    if (p.nslice == 1) return 0;
-    const long long P = (long long)n * (n_heads / n_kv);
-    return align256((size_t)kPrefillRowTiles(P, rows) * n_kv * p.nslice * prefill_pwaves(P, rows, rw) * rw * (hd + 2) * 4);
-}
-
 // gi_attn_prefill, gi_attn_prefill_i8 and gi_attn_prefill_q4: the same launch with the f16, int8 or 4-bit kernel
 // (fmt 0, 1, 2). With a workspace and `widen` (int8 and 4-bit caches, head sizes 64, 128, 256) the keys 0..pos0+n-1
 // are first widened into it (gi_kv_widen) and the prefill stages the widened tiles by LDS-DMA, as it stages the f16
@@ -826,41 +760,38 @@ int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, c
     a.q_f16 = q_dtype == GI_F16;
     a.out_f16 = out_dtype == GI_F16;
     a.hd = hd;
-    a.nslice = 1;
-    const int G = n_heads / n_kv;
-    a.gmul = (long long)n * G * G < 1ll << 31 ? (uint32_t)(((1ll << 31) + G - 1) / G) : 0;
-    // the launch of kernel f with `waves` waves of rw rows, sliced where the plan says so and the rest of the workspace
-    // holds the partials; then their merge
-    auto run_plan = [&](const PrefillPlan& p, hipFunction_t f, int waves, int rw, unsigned char* free, size_t left) {
-        const size_t need = prefill_part_bytes(p, n, n_heads, n_kv, hd, rw * waves, rw);
-        a.rows = rw * waves;
-        a.items = kPrefillRowTiles((long long)n * G, a.rows);
-        a.pwaves = prefill_pwaves((long long)n * G, a.rows, rw);
-        if (need && free && aligned16(free) && left >= need) {
-            a.part = (float*)free;
-            a.nslice = p.nslice;
-            a.slice_tiles = p.tiles;
-        }
-        if (int e = launch(kPrefill, f, dim3((unsigned)(a.items * n_kv * a.nslice), 1, 1), dim3(64 * waves),
+    // the launch of kernel f of a kind, laid out by the plan for what is left of the workspace, then the merge of its slices
+    auto run_plan = [&](PrefillKind kind, unsigned char* free, size_t left, auto kernel) {
+        const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd, kind, free && aligned16(free) ? left : 0);
+        const int rw = prefill_wave_rows(kind), sets = n_heads / n_kv / p.group;
+        a.rows = rw * p.waves;
+        a.group = p.group;
+        a.sets = sets;
+        a.gmul = gi_row_mul(n, p.group);
+        a.items = prefill_row_tiles((long long)n * p.group, a.rows);
+        a.pwaves = prefill_pwaves((long long)n * p.group, a.rows, rw);
+        a.nslice = p.nslice;
+        a.slice_tiles = p.tiles;
+        if (p.nslice > 1) a.part = (float*)free;
+        if (int e = launch(kPrefill, kernel(p.waves), dim3((unsigned)(a.items * n_kv * sets * a.nslice), 1, 1), dim3(64 * p.waves),
                            (hipStream_t)stream, &a, sizeof a))
             return e;
         if (a.nslice == 1) return 0;
         return launch(kPrefillCombine, m->prefill_combine[rw == 16],
-                      dim3(a.pwaves * a.items * n_kv, (rw * hd / 256 + kPrefillMergeFrags - 1) / kPrefillMergeFrags, 1),
+                      dim3(a.pwaves * a.items * n_kv * sets, (rw * hd / 256 + kPrefillMergeFrags - 1) / kPrefillMergeFrags, 1),
                       dim3(64 * kPrefillMergeFrags), (hipStream_t)stream, &a, sizeof a);
     };
-    // an f16 MFMA kernel over staging `st` (Module::prefill)
+    // an f16 MFMA kernel over staging `st` (Module::prefill; 2: tile by tile)
     auto run = [&](int st, unsigned char* free, size_t left) {
-        const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd);
-        const int waves = st == 2 ? (hd == 256 ? 4 : 8) : p.waves; // (tile by tile: the larger form only)
-        const hipFunction_t f = st == 2 && hd == 256 ? m->prefill256[fmt - 1]
-                                                     : m->prefill[hd == 64 ? 1 : hd == 256 ? 2 : 0][st][waves == (hd == 256 ? 2 : 4)];
-        return run_plan(p, f, waves, 32, free, left);
+        return run_plan(st == 2 ? kPrefillTile : kPrefillStaged, free, left, [&](int waves) {
+            return st == 2 && hd == 256 ? m->prefill256[fmt - 1]
+                                        : m->prefill[hd == 64 ? 1 : hd == 256 ? 2 : 0][st][waves == (hd == 256 ? 2 : 4)];
+        });
     };
     unsigned char* const ws = (unsigned char*)workspace;
     if (f32_prompt || f32_hd(hd))
-        return run_plan(prefill_plan(pos0, n, n_heads, n_kv, hd, true),
-                        f32_hd(hd) ? m->prefill_f32[i8][f32_index(hd)] : m->prefill_f32p[i8][hd == 128], 8, 16, ws, workspace_bytes);
+        return run_plan(kPrefillF32, ws, workspace_bytes,
+                        [&](int) { return f32_hd(hd) ? m->prefill_f32[i8][f32_index(hd)] : m->prefill_f32p[i8][hd == 128]; });
     if (fmt && workspace && widen && !f32_hd(hd)) {
         const int len = pos0 + n;
         const size_t need = prefill_ws_bytes(len, n_kv, hd, fmt);
@@ -1041,14 +972,13 @@ size_t gi_attn_prefill_workspace_bytes(int kv_len, int n_kv, int hd, int fmt) {
 
 size_t gi_attn_prefill_scratch_bytes(int pos0, int n, int n_heads, int n_kv, int hd, int fmt, int flags) {
     if (check_shape(n_heads, n_kv, hd, true) || pos0 < 0 || n <= 0 || fmt < 0 || fmt > 2 || (fmt == 2 && hd != 256)) return 0;
-    if ((flags & GI_PREFILL_F32) || f32_hd(hd)) {
-        if (fmt == 2 || hd > 128) return 0;
-        return prefill_part_bytes(prefill_plan(pos0, n, n_heads, n_kv, hd, true), n, n_heads, n_kv, hd, kF32Rows, 16);
-    }
-    const bool widens = fmt && (flags & GI_PREFILL_WIDEN) && prefill_widens(n, n_heads, n_kv, hd);
+    const bool f32 = (flags & GI_PREFILL_F32) || f32_hd(hd);
+    if (f32 && (fmt == 2 || hd > 128)) return 0;
+    const bool widens = !f32 && fmt && (flags & GI_PREFILL_WIDEN) && prefill_widens(n, n_heads, n_kv, hd);
     const size_t widened = widens ? prefill_ws_bytes(pos0 + n, n_kv, hd, fmt) : 0;
-    const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd);
-    return widened + prefill_part_bytes(p, n, n_heads, n_kv, hd, fmt && !widens ? (hd == 256 ? 128 : kPrefillRows) : 32 * p.waves);
+    const PrefillKind kind = f32 ? kPrefillF32 : fmt && !widens ? kPrefillTile : kPrefillStaged;
+    const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd, kind, SIZE_MAX);
+    return widened + prefill_part_bytes(p.nslice, p.waves, kind, n, n_heads, n_kv, hd);
 }
 
 int gi_attn_prefill_ws(void* stream, const void* q, int q_dtype, long long q_stride, const void* kc, const void* vc,

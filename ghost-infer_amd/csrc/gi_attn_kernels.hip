@@ -28,6 +28,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "gi_prefill_rows.h"
+
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f16x __attribute__((ext_vector_type(16)));
@@ -1486,52 +1488,50 @@ struct GiPrefillArgs {
     long long sc_stride;
     long long sc_head_stride;
     // sliced launches (nslice > 1): slice s of a row tile covers the key tiles [s*slice_tiles, (s+1)*slice_tiles) and
-    // leaves its partial result here (pf_partial), for gi_prefill_combine_*; unsliced: null, 1
+    // leaves its partial result here (pf_part_o, pf_part_ml), for gi_prefill_combine_*; unsliced: null, 1
     float* part;
     int slice_tiles;
     int nslice;
     int pwaves;            // waves of a row tile that hold rows (the workgroup's, or fewer where one tile holds all rows)
     int items;             // row tiles per kv head
-    uint32_t gmul;         // ceil(2^31 / G): a packed row's token without a division (pf_token)
+    uint32_t gmul;         // gi_row_mul: a packed row's token without a division (pf_token)
     int rows;              // rows of a row tile
+    int group;             // query heads of a set, whose rows are packed together: a kv head's group, or a part of it
+    int sets;              // sets per kv head
 };
 
-// Rows of a prefill workgroup. The query rows of one kv head are taken token-major with their G query heads side by
-// side (packed row r: token r / G, head r % G of the group), so that a row tile covers few positions: its waves end
-// at nearly the same key tile, all heads of the group share each staged K/V tile, and a few tokens still fill a
-// tile. A row's arithmetic does not depend on which rows share its tile.
+// Rows of a prefill workgroup. The query rows of one kv head are taken token-major with their query heads side by side
+// (packed row r: token r / group, head r % group), so that a row tile covers few positions: its waves end at nearly the
+// same key tile, all heads of the group share each staged K/V tile, and a few tokens still fill a tile. Where that leaves
+// CUs without a workgroup the group is split into sets of heads, each with row tiles of its own (prefill_plan). A row's
+// arithmetic does not depend on which rows share its tile.
 struct PfUnit {
-    int kvh, row0;       // kv head, first packed row
-    int t_begin, t_end;  // key tiles of this workgroup
-    long long unit;      // index of its partial
+    int kvh, head0, row0; // kv head, first query head of the set, first packed row
+    int t_begin, t_end;   // key tiles of this workgroup
+    long long unit;       // index of its partial
 };
-// row / G. The product form is exact for row * G < 2^31 (else the host passes gmul 0): 2 row ceil(2^31 / G) exceeds
-// 2^32 row / G by less than 2 row, so the quotient's fraction stays below the next integer. (A 32-bit division is
-// some 40 instructions; four in a row before the first tile's loads cost a short prompt 0.5 us.)
-__device__ __forceinline__ int pf_token(const GiPrefillArgs& a, int row) {
-    return a.gmul ? (int)__umulhi(2u * (uint32_t)row, a.gmul) : row / (a.n_heads / a.n_kv);
-}
+__device__ __forceinline__ int pf_token(const GiPrefillArgs& a, int row) { return gi_row_token(row, a.gmul, a.group); }
 __device__ __forceinline__ int pf_last_token(const GiPrefillArgs& a, int row0, int rows) {
     return min(a.n - 1, pf_token(a, row0 + rows - 1)); // the last token with a row in the tile
 }
-// Workgroup j of the grid takes run j % runs (kv head and slice: the workgroups that read the same keys) and the row tiles
-// of all runs longest first. Blocks go to the 8 XCDs round-robin, so with 8 runs (or a divisor or multiple) each run stays
-// in the L2 of its own XCDs and every XCD gets row tiles of every length. (Giving each XCD a contiguous stretch of the
+// Workgroup j of the grid takes run j % runs (set of heads and slice: the workgroups that read the same keys) and the row
+// tiles of all runs longest first. Blocks go to the 8 XCDs round-robin, so with 8 runs (or a divisor or multiple) each run
+// stays in the L2 of its own XCDs and every XCD gets row tiles of every length. (Giving each XCD a contiguous stretch of the
 // (kv head, row tile) order keeps the locality too, but with fewer than 8 kv heads one XCD then gets a kv head's longest
 // tiles and another its shortest: 8192 tokens of 16/2 heads of 256 took 880 us with half of the CUs idle, 32/4 heads
 // of 128 604 us against 505 for 32/8.)
 __device__ __forceinline__ PfUnit pf_unit(const GiPrefillArgs& a, int BQ, int BK) {
-    const int items = a.items, runs = a.n_kv * a.nslice;
-    const int lot = (int)blockIdx.x / runs, run = (int)blockIdx.x - lot * runs; // run: kv head * nslice + slice
+    const int items = a.items, runs = a.n_kv * a.sets * a.nslice;
+    const int lot = (int)blockIdx.x / runs, run = (int)blockIdx.x - lot * runs; // run: set * nslice + slice
     const int item = items - 1 - lot;
-    const int kvh = a.nslice == 1 ? run : run / a.nslice, slice = run - kvh * a.nslice;
+    const int set = a.nslice == 1 ? run : run / a.nslice, slice = run - set * a.nslice;
     const int k_lim = a.pos0 + pf_last_token(a, item * BQ, BQ) + 1; // keys any row of the tile may see
     const int ntiles = (k_lim + BK - 1) / BK;
     const int tb = slice * a.slice_tiles;
-    return PfUnit{kvh, item * BQ, tb, a.nslice == 1 ? ntiles : min(ntiles, tb + a.slice_tiles),
-                  ((long long)kvh * items + item) * a.nslice + slice};
+    return PfUnit{a.sets == 1 ? set : set / a.sets, set * a.group, item * BQ, tb,
+                  a.nslice == 1 ? ntiles : min(ntiles, tb + a.slice_tiles), ((long long)set * items + item) * a.nslice + slice};
 }
-// A sliced launch's partials: per unit (kv head, row tile, slice) the unnormalised O^T accumulators as the lanes hold
+// A sliced launch's partials: per unit (set of heads, row tile, slice) the unnormalised O^T accumulators as the lanes hold
 // them, [wave][fragment][lane] float4, so that every store and every load of the merge is 1 KB contiguous; behind
 // all of them (reference max, row sum) per unit and row. With RW rows per wave, fragment f of lane l is row l % RW,
 // dims (256 / RW) f + 4 (l / RW) .. + 3.
@@ -1588,7 +1588,7 @@ __device__ __forceinline__ void gi_stage4(u4 rs, GI_LDS void* dst, int voff) { /
 typedef short gi_s4 __attribute__((__vector_size__(8))); // 4 f16 as ds_read_b64_tr_b16 returns them
 
 // ---------------------------------------------------------------- prefill, merge of a sliced launch's partials
-// One workgroup per (kv head, row tile, wave of its rows, PFC_FRAGS of its fragments): the slices' weights
+// One workgroup per (set of heads, row tile, wave of its rows, PFC_FRAGS of its fragments): the slices' weights
 // exp2(m - M) / L of its rows go to LDS once, then each thread sums its float4 over the slices (loads of 1 KB per
 // wave, PFC_FRAGS waves) and writes the output.
 #define PFC_FRAGS 4
@@ -1597,14 +1597,14 @@ template <int RW>
 __device__ __forceinline__ void gi_prefill_combine_t(const GiPrefillArgs& a) {
     __shared__ float w_sh[PFC_MAXS][RW];
     __shared__ float l_sh[PFC_MAXS][RW];
-    const int G = a.n_heads / a.n_kv, P = a.n * G, hd = a.hd, BQ = a.rows;
+    const int G = a.group, P = a.n * G, hd = a.hd, BQ = a.rows;
     const int items = a.items;
-    const int wave = blockIdx.x % a.pwaves, item = blockIdx.x / a.pwaves % items, kvh = blockIdx.x / a.pwaves / items;
+    const int wave = blockIdx.x % a.pwaves, item = blockIdx.x / a.pwaves % items, set = blockIdx.x / a.pwaves / items;
     const int row0 = item * BQ + RW * wave;
     if (row0 >= P) return;
     const int ntiles = (a.pos0 + pf_last_token(a, item * BQ, BQ)) / PF_BK + 1;
     const int ns = min(a.nslice, (ntiles + a.slice_tiles - 1) / a.slice_tiles); // slices that left a partial
-    const long long u0 = ((long long)kvh * items + item) * a.nslice, units = (long long)a.n_kv * items * a.nslice;
+    const long long u0 = ((long long)set * items + item) * a.nslice, units = (long long)a.n_kv * a.sets * items * a.nslice;
     const int tid = threadIdx.x;
     for (int i = tid; i < ns * RW; i += 64 * PFC_FRAGS) {
         const float2 ml = pf_part_ml<RW>(a, hd, units, u0 + i / RW, wave)[i % RW];
@@ -1639,7 +1639,7 @@ __device__ __forceinline__ void gi_prefill_combine_t(const GiPrefillArgs& a) {
     }
     const int row = row0 + r;
     if (row >= P) return;
-    const int tok = pf_token(a, row), h = kvh * G + row - tok * G;
+    const int tok = pf_token(a, row), h = set * G + row - tok * G;
     const long long e0 = (long long)tok * a.out_stride + (long long)h * hd + (256 / RW) * f + 4 * (lane / RW);
     if (a.out_f16)
         *reinterpret_cast<h4x*>((_Float16*)a.out + e0) = h4x{(_Float16)acc[0], (_Float16)acc[1], (_Float16)acc[2], (_Float16)acc[3]};
@@ -1657,7 +1657,7 @@ template <int N, int I = 0, typename F> __device__ __forceinline__ void gi_unrol
         gi_unroll<N, I + 1>(f);
     }
 }
-// One workgroup = (kv head, 32 * WAVES packed query rows, key slice); wave w owns rows 32w..32w+31 of the tile. Per
+// One workgroup = (set of a kv head's query heads, 32 * WAVES packed query rows, key slice); wave w owns rows 32w..32w+31 of the tile. Per
 // 64-key tile:
 //   S^T[key, q] = K[key, :] . Q[q, :]       v_mfma_f32_32x32x16_f16, K from LDS (A), Q in registers (B)
 //   O^T[d, q]  += V^T[d, key] . P^T[key, q]  V^T from LDS (A, by transposing reads), P^T from S^T (B)
@@ -1732,7 +1732,7 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int G = a.n_heads / a.n_kv;
+    const int G = a.group;
     const PfUnit un = pf_unit(a, BQ, BK);
     const int kvh = un.kvh, q0 = un.row0, t_begin = un.t_begin, ntiles = un.t_end; // key tiles t_begin .. ntiles - 1
     if (t_begin >= ntiles) return; // a slice past the tile's last key
@@ -1851,7 +1851,7 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     const int qrow = q0 + 32 * wave + qcol;      // this lane's packed query row
     const bool qlive = qrow < a.n * G;           // (rows past the last compute garbage that is never written)
     const int qtok = qlive ? pf_token(a, qrow) : a.n - 1;
-    const int h = kvh * G + (qlive ? qrow : a.n * G - 1) - qtok * G;
+    const int h = un.head0 + (qlive ? qrow : a.n * G - 1) - qtok * G;
     const int qpos = a.pos0 + qtok;              // its position
     // Q is held pre-multiplied by scale*log2(e), so scores come out of the MFMA in log2 units (the f16
     // rounding of the scaled value is the same size as the rounding of Q itself)

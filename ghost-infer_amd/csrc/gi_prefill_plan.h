@@ -1,0 +1,126 @@
+// How a prefill launch is laid out: rows per workgroup, heads per set of packed rows, slices along the keys. Host code.
+#ifndef GI_PREFILL_PLAN_H
+#define GI_PREFILL_PLAN_H
+
+#include <algorithm>
+#include <cstddef>
+#include <cstdint>
+
+constexpr int kPrefillCUs = 256;      // compute units of a gfx950 device; a prefill workgroup takes one of its own
+constexpr int kPrefillKeys = 64;      // keys per prefill tile; must match the kernels' PF_BK
+constexpr int kPrefillMaxSlices = 64; // must match the kernels' PFC_MAXS
+
+// The kernels of a launch: MFMA kernels over tiles staged as they are in memory (two sizes of workgroup), MFMA kernels that
+// widen each int8 or 4-bit tile as they stage it (the larger workgroup only), and the f32 kernels (8 waves of 16 rows).
+enum PrefillKind { kPrefillStaged, kPrefillTile, kPrefillF32 };
+
+struct PrefillPlan {
+    int waves;      // per workgroup: 8 or 4; head size 256: 4 or 2; f32: 8
+    int group;      // query heads that share row tiles
+    int tiles;      // key tiles per slice
+    int nslice;     // slices of the longest row tile
+};
+
+inline int prefill_row_tiles(long long rows, int per) { return (int)((rows + per - 1) / per); }
+inline int prefill_wave_rows(PrefillKind kind) { return kind == kPrefillF32 ? 16 : 32; }
+inline int prefill_most_waves(PrefillKind kind, int hd) { return hd == 256 && kind != kPrefillF32 ? 4 : 8; }
+// waves of a row tile of `rows` that hold any of P rows
+inline int prefill_pwaves(long long P, int rows, int rw) { return P > rows ? rows / rw : (int)((P + rw - 1) / rw); }
+// Bytes of a sliced launch's partials
+inline size_t prefill_part_bytes(int nslice, int waves, PrefillKind kind, int n, int n_heads, int n_kv, int hd) {
+    if (nslice == 1) return 0;
+    const int rw = prefill_wave_rows(kind), rows = rw * waves;
+    const long long P = (long long)n * (n_heads / n_kv);
+    const size_t b = (size_t)prefill_row_tiles(P, rows) * n_kv * nslice * prefill_pwaves(P, rows, rw) * rw * (hd + 2) * 4;
+    return (b + 255) / 256 * 256;
+}
+
+// A launch has one workgroup per (kv head, tile of packed query rows), and a CU holds one workgroup.
+//  - Waves: 8 (256 rows, two waves per SIMD) or 4 (128 rows, one per SIMD). One wave takes a key tile in about 0.7 of
+//    the time that two on its SIMD take for theirs together, so 4 waves win where the workgroups are few or unequal
+//    (1024 tokens of 32/8 heads of 128, f16: 33.9 us with 8, 23.7 with 4; 512 at a 2000-token prefix 64 and 44) and
+//    8 where they fill the chip several times over (8192 tokens: 505 and 580). Head size 256: 4 or 2.
+//  - Slices: a short batch over a long prefix leaves most of the chip idle while each workgroup walks all of its keys
+//    (512 tokens of 32/4 heads at a 16K prefix: 64 workgroups of 264 key tiles, 350 us). Such a launch cuts the key
+//    tiles of every row tile into slices, one workgroup each, whose partial results a second launch merges (137 us).
+//    An f32 tile takes three to five times as long, so those launches gain from shorter spans on (200 tokens of 32/32
+//    heads of 96 at 1800: 64 workgroups of 32 tiles, 227 us; sliced 69 us).
+// A row's arithmetic does not depend on the waves or the set, only on the slices. Of a sliced launch the partials fit
+// `room` bytes.
+inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, PrefillKind kind, size_t room) {
+    const bool f32 = kind == kPrefillF32;
+    const int G = n_heads / n_kv, cus = kPrefillCUs, tmax = (pos0 + n + kPrefillKeys - 1) / kPrefillKeys;
+    const long long P = (long long)n * G;
+    const int most = prefill_most_waves(kind, hd), rw = prefill_wave_rows(kind);
+    PrefillPlan p{most, G, tmax, 1};
+    if ((long long)prefill_row_tiles(P, rw * most) * n_kv >= 2 * cus) return p; // longest tiles first balances these
+    // Below 16 key tiles slices save less than the merge launch costs. A prompt of up to 4096 keys taken in chunks of
+    // 256 tokens or more keeps each row's arithmetic independent of the chunking (one slice always); beyond, chunks
+    // agree to f32 rounding.
+    const bool may_slice = room && tmax >= (f32 ? 4 : 16) && (n < 256 || pos0 + n > 4096);
+    // Costs in units of one key tile of an 8-wave workgroup (1.4 to 1.9 us; head size 256: of a 4-wave one): rounds of
+    // workgroups over the CUs, each with a fixed cost until its first tile is in and for its output (~6 us), and for a
+    // sliced launch the merge launch (~5 us) and its read of the partials (~4 TB/s).
+    const double tile_s = f32 ? 5e-6 : 1.5e-6, per_wg = f32 ? 1.2 : 4.0, merge = f32 ? 1.0 : 3.3;
+    double best = 0;
+    for (int waves = most; waves >= (f32 ? most : most / 2); waves -= most / 2) {
+        const int rows = rw * waves, items = prefill_row_tiles(P, rows);
+        const long long wgs = (long long)items * n_kv;
+        const double tile = waves == most ? 1.0 : hd == 256 ? 0.85 : 0.7;
+        auto tiles_of = [&](int i) { // key tiles of row tile i
+            const long long last = std::min<long long>(n - 1, ((long long)(i + 1) * rows - 1) / G);
+            return (int)((pos0 + last) / kPrefillKeys + 1);
+        };
+        // one slice: the longest workgroup, or the mean load of a CU where there are several rounds
+        const double mean = (double)wgs / cus * (tile * (tiles_of(0) + tmax) / 2 + (wgs > cus ? per_wg : 0));
+        const double one = std::max(tile * tmax, mean) + per_wg;
+        if (waves == most || one < 0.95 * best) best = one, p = PrefillPlan{waves, G, tmax, 1};
+        if (!may_slice) continue;
+        const double part = std::min<long long>(P, rows) * (hd + 2) * 4.0 / 4e12 / tile_s;
+        for (int S = 2; S <= std::min(kPrefillMaxSlices, tmax / 2) && wgs * S <= 4 * cus; S++) {
+            const int C = (tmax + S - 1) / S, slices = (tmax + C - 1) / C;
+            if (prefill_part_bytes(slices, kind == kPrefillTile ? most : waves, kind, n, n_heads, n_kv, hd) > room) continue;
+            long long u = 0; // workgroups with keys
+            if (tiles_of(0) + C > tmax) u = wgs * slices; // (every row tile has tmax tiles or nearly)
+            else
+                for (int i = 0; i < items; i++) u += (long long)n_kv * ((tiles_of(i) + C - 1) / C);
+            const double cost = (double)((u + cus - 1) / cus) * (tile * C + per_wg) + merge + u * part;
+            if (cost < 0.95 * best) best = cost, p = PrefillPlan{waves, G, C, slices};
+        }
+    }
+    return p;
+}
+
+// The plan of a call whose workspace has `room` bytes for partials.
+// A launch that is not cut and leaves CUs idle splits the group of a kv head's query heads into sets, each with row tiles of
+// its own, and takes the smaller workgroup, where that gives at least half as many workgroups again (one each CU at
+// most): a workgroup loads its rows' queries and stores its outputs by itself, and 128 rows of 256 f32 take it 7 us longer
+// than 16. Prompts at position 0, replayed graph, whole groups / sets: 32/8 heads of 128, f16, 16 tokens 7.3 / 6.4 us, 64
+// tokens 8.8 / 7.6; 16/2 heads of 256, 16 tokens 14.2 / 8.7, 64 tokens 14.5 / 10.9.
+// The f32 kernels, bound by their MFMAs with two waves a SIMD, always take one head a set: waves of a tile of 128 tokens of
+// one head skip the key tiles past their own last row, where 128 rows of 4 heads all end at the same one (32/8 heads of
+// 96, whole groups / sets: 32 tokens 19.3 / 10.0 us, 256 tokens 40.2 / 36.3, 4096 tokens 867 / 864).
+inline PrefillPlan prefill_plan(int pos0, int n, int n_heads, int n_kv, int hd, PrefillKind kind, size_t room) {
+    PrefillPlan p = prefill_rate(pos0, n, n_heads, n_kv, hd, kind, room ? SIZE_MAX : 0);
+    const int most = prefill_most_waves(kind, hd), G = n_heads / n_kv;
+    if (kind == kPrefillTile) p.waves = most;
+    if (prefill_part_bytes(p.nslice, p.waves, kind, n, n_heads, n_kv, hd) > room) {
+        p = prefill_rate(pos0, n, n_heads, n_kv, hd, kind, room);
+        if (kind == kPrefillTile) p.waves = most;
+    }
+    if (p.nslice > 1) return p;
+    if (kind == kPrefillF32) {
+        p.group = 1;
+        return p;
+    }
+    auto wgs = [&](int waves, int group) {
+        return (long long)n_heads / group * prefill_row_tiles((long long)n * group, prefill_wave_rows(kind) * waves);
+    };
+    long long have = wgs(p.waves, p.group);
+    if (kind == kPrefillStaged && wgs(most / 2, G) <= kPrefillCUs && wgs(most / 2, G) * 2 >= have * 3) p.waves = most / 2, have = wgs(p.waves, G);
+    for (int g = G - 1; g >= 1; g--)
+        if (G % g == 0 && wgs(p.waves, g) <= kPrefillCUs && wgs(p.waves, g) * 2 >= have * 3) p.group = g, have = wgs(p.waves, g);
+    return p;
+}
+
+#endif
