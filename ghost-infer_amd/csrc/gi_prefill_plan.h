@@ -55,8 +55,11 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
     PrefillPlan p{most, G, tmax, 1};
     if ((long long)prefill_row_tiles(P, rw * most) * n_kv >= 2 * cus) return p; // longest tiles first balances these
     // Below 16 key tiles slices save less than the merge launch costs. A prompt of up to 4096 keys taken in chunks of
-    // 256 tokens or more keeps each row's arithmetic independent of the chunking (one slice always); beyond, chunks
-    // agree to f32 rounding.
+    // 256 tokens or more keeps each row's arithmetic independent of the chunking (one slice always); beyond, and in
+    // shorter chunks, rows differ from the uncut ones by f16's step (each slice rounds its P against its own maximum).
+    // What that costs such chunks, 255 (cut) and 256 tokens (not): 32/8 heads of 128, f16, at 1500 keys 25 and 32 us, at
+    // 3000 30 and 51; 16/2 heads of 256 at 3000 37 and 83; in f32 (32/8 heads of 128) at 500 50 and 117, at 3000 135 and
+    // 462. (Never cut, 256 tokens took 49, 80, 99, 117 and 462 before the row tiles were packed.)
     const bool may_slice = room && tmax >= (f32 ? 4 : 16) && (n < 256 || pos0 + n > 4096);
     // Costs in units of one key tile of an 8-wave workgroup (1.4 to 1.9 us; head size 256: of a 4-wave one): rounds of
     // workgroups over the CUs, each with a fixed cost until its first tile is in and for its output (~6 us), and for a

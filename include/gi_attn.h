@@ -199,11 +199,14 @@ int gi_attn_prefill_q4_ws(void* stream, const void* q, int q_dtype, long long q_
 /* Every causal prefill above in one entry point (fmt 0: f16 cache, 1: int8, 2: 4-bit; ks / vs and the scale strides
  * as the entry points of that cache), with a scratch workspace. The workspace (16-byte aligned; 256-byte with
  * GI_PREFILL_WIDEN) takes the widened keys and the partial results of a sliced launch: a batch too short to fill the
- * chip over a long prefix is cut along its keys too (one workgroup per slice, merged by a second launch; rows then
- * differ from the one-slice results by f32 rounding). gi_attn_prefill_scratch_bytes says how much a call can use; it
- * is optional, and with a smaller one (or none) the call does without. The workspace needs no initialisation; calls that
- * share one must be ordered. Prompts of up to 4096 keys taken in chunks of 256 tokens or more, and spans below 16
- * tiles of 64 keys (f32: below 4), are never cut. */
+ * chip over a long prefix is cut along its keys too (one workgroup per slice, merged by a second launch). The rows of a cut
+ * call differ from those of an uncut one: each slice rounds its probabilities to f16 against its own maximum (about 3e-4
+ * relative, as far as either is from float64; in f32 by f32 rounding). gi_attn_prefill_scratch_bytes says how much a call
+ * can use; it is optional: with a smaller one the call takes fewer slices, with none (or fewer than 16 bytes, or a
+ * misaligned one) it is not cut. The workspace needs no initialisation; calls that share one must be ordered. Calls of
+ * 256 tokens or more over up to 4096 keys, and spans below 16 tiles of 64 keys (f32: below 4), are never cut: a prompt
+ * of up to 4096 keys taken in chunks equals the whole one bit for bit as long as every chunk has 256 tokens; a shorter
+ * last chunk may be cut, and equals it only when the call has no room for slices. */
 size_t gi_attn_prefill_scratch_bytes(int pos0, int n, int n_heads, int n_kv, int hd, int fmt, int flags);
 int gi_attn_prefill_ws(void* stream, const void* q, int q_dtype, long long q_stride, const void* kc, const void* vc,
                        const void* ks, const void* vs, int fmt, int flags, long long kv_stride, long long kv_head_stride,

@@ -1,7 +1,7 @@
 """The committed golden fixtures (tests/golden/*.npz: seeded inputs and float64 expected outputs, written by
 tests/golden/make_golden.py) through the HIP path: the decode / verify cases through gi_attn_decode(_i8, _q4)
 and, packed as the reference's qkv rows, through the operator gi_attention(_i8, _q4) (src/cuda.rs:8448-8541);
-the prefill cases through gi_attn_prefill(_i8, _q4).
+the prefill cases through prefill() and prefill_q4() (gi_attn_prefill_ws).
 
 Bar: decode and verify within 2e-5 of float64 (the split path keeps f32 precision), prefill within the
 north star's 2e-3 / 1e-3 (it rounds P to f16 as the reference does), and so is decode at head size 256 over the

@@ -148,3 +148,34 @@ def test_sliced_prefill_f32(gpu, n, pos0, n_heads, n_kv, hd, i8):
     got = gi_attn.prefill(dev(q, gpu, n, n_heads * hd), kt, vt, pos0, n_heads, n_kv, hd=hd, **kw)
     torch.cuda.synchronize()
     assert_close(got.cpu().numpy(), want, max_abs=2e-5, rel_l2=2e-5, what="sliced f32")
+
+
+@pytest.mark.parametrize("fmt,hd", [("f16", 128), ("f16", 64), ("f16", 256), ("i8", 128), ("i8", 256), ("q4", 256), ("f32", 96)])
+def test_chunked_prompt_with_a_short_last_chunk(gpu, fmt, hd):
+    # a prompt of 1100 tokens in chunks of 512: the full chunks equal the whole prompt bit for bit; the last one, of 76
+    # tokens, is cut along its keys and agrees within the bar, and equals it too where its workspace has no room
+    n, chunk, n_heads, n_kv = 1100, 512, (16 if hd == 256 else 8), 2
+    print("[case] short last chunk", fmt, hd, flush=True)
+    gen = torch.Generator(device=gpu).manual_seed(9990 + hd)
+    q = torch.randn((n, n_heads * hd), device=gpu, generator=gen)
+    code = {"i8": 1, "q4": 2}.get(fmt, 0)
+    if fmt == "q4":
+        cache = [torch.randint(0, 256, (n, n_kv, 128), device=gpu, dtype=torch.uint8, generator=gen) for _ in range(2)]
+        cache += [(0.2 + 0.15 * torch.rand((n, n_kv, 8), device=gpu, generator=gen)).half() for _ in range(2)]
+        call = lambda x, pos, ws=None: gi_attn.prefill_q4(x, *cache, pos, n_heads, n_kv, workspace=ws)
+    elif fmt == "i8":
+        kv = [torch.randint(-127, 128, (n, n_kv, hd), device=gpu, dtype=torch.int8, generator=gen) for _ in range(2)]
+        ks, vs = (0.01 + 0.01 * torch.rand((n, n_kv), device=gpu, generator=gen) for _ in range(2))
+        call = lambda x, pos, ws=None: gi_attn.prefill(x, *kv, pos, n_heads, n_kv, hd=hd, k_scale=ks, v_scale=vs, workspace=ws)
+    else:
+        kv = [torch.randn((n, n_kv, hd), device=gpu, generator=gen).half() for _ in range(2)]
+        call = lambda x, pos, ws=None: gi_attn.prefill(x, *kv, pos, n_heads, n_kv, hd=hd, f32=fmt == "f32", workspace=ws)
+    whole = call(q, 0)
+    for c0 in (0, 512):
+        assert torch.equal(call(q[c0:c0 + chunk], c0), whole[c0:c0 + chunk]), c0
+    tail = q[1024:].contiguous()
+    assert gi_attn.load_library().gi_attn_prefill_scratch_bytes(1024, n - 1024, n_heads, n_kv, hd, code, 0) > 0
+    got = call(tail, 1024)
+    assert_close(got.cpu().numpy(), whole[1024:].cpu().numpy(), what="last chunk, cut")
+    room = gi_attn.load_library().gi_attn_prefill_workspace_bytes(n, n_kv, hd, code)
+    assert torch.equal(call(tail, 1024, torch.empty(room, dtype=torch.uint8, device=gpu)), whole[1024:])

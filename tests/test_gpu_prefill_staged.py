@@ -1,6 +1,6 @@
 """The pre-widened prefill over the int8 and 4-bit caches (gi_kv_widen, then the prefill kernels that stage the
-widened tiles by LDS-DMA: gi_attn_prefill_i8_ws / gi_attn_prefill_q4_ws, and the operators' prefill batches) against
-the kernels that widen each tile as they stage it (gi_attn_prefill_i8 / gi_attn_prefill_q4). Both feed the same f16
+widened tiles by LDS-DMA: gi_attn_prefill_ws with GI_PREFILL_WIDEN, gi_attn_prefill_i8_ws, and the operators' prefill
+batches) against the kernels that widen each tile as they stage it (gi_attn_prefill_ws without it). Both feed the same f16
 values and scales to the same MFMA and softmax code, so the outputs must agree bit for bit; the oracle checks of the
 int8 and 4-bit prefill (test_gpu_int8.py, test_gpu_hd256.py, test_gpu_q4.py, test_gpu_hd64.py) run the widened path,
 which is the default. Semantics: attention_prefill_tc64/128/256 with KV8 (src/cuda.rs:2466-2498, 2548-2605) and
