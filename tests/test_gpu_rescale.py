@@ -233,3 +233,25 @@ def test_prefill_tiles_whose_scores_are_all_minus_infinity(gpu, hd, n, pos0):
     want = reference_f64(q[live], k, v, pos0 + int((~live).sum()), n_heads, n_kv, hd=hd)
     assert_close(out.cpu().numpy()[live], want, what=f"minus infinity, hd {hd}")
     assert np.isnan(out.cpu().numpy()[~live]).all()
+
+
+@pytest.mark.parametrize("n,pos0", [(40, 1500), (300, 4000)])
+@pytest.mark.parametrize("fmt,hd", [("f16", 64), ("f16", 128), ("f16", 256), ("i8", 64), ("i8", 128), ("i8", 256), ("f32", 96), ("f32", 128)])
+def test_cut_prefill_rising_scores(gpu, fmt, hd, n, pos0):
+    # launches cut along their keys: 60 log2 units over the prompt, so that references move within a slice and the slices'
+    # maxima lie far apart in the merge
+    n_heads, n_kv = 4, 2
+    say("rescale cut prefill", fmt, hd, n, pos0)
+    code, f32 = int(fmt == "i8"), fmt == "f32"
+    assert gi_attn.load_library().gi_attn_prefill_scratch_bytes(pos0, n, n_heads, n_kv, hd, code, 2 if f32 else 0) > 0
+    q, *kv = ramp_inputs(7700 + hd + n, n, pos0 + n, n_heads, n_kv, hd, i8=fmt == "i8", log2_span=60.0)
+    qt = torch.from_numpy(q).to(gpu)
+    if fmt == "i8":
+        t = [torch.from_numpy(x).to(gpu) for x in kv]
+        out = gi_attn.prefill(qt, t[0], t[1], pos0, n_heads, n_kv, hd=hd, k_scale=t[2], v_scale=t[3])
+        want = O.prefill_tc_semantics_i8(q, *kv, pos0, n_heads, n_kv, hd=hd)
+    else:
+        out = gi_attn.prefill(qt, *(f16_dev(x, gpu) for x in kv), pos0, n_heads, n_kv, hd=hd, f32=f32)
+        want = reference_f64(q, *kv, pos0, n_heads, n_kv, hd=hd) if f32 else O.prefill_tc_semantics(q, *kv, pos0, n_heads, n_kv, hd=hd)
+    torch.cuda.synchronize()
+    assert_close(out.cpu().numpy(), want, *(SPLIT_F64_TOL if f32 else ()), what=f"rising scores, cut prefill {fmt} {hd}")
