@@ -96,9 +96,11 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
 
 // The plan of a call whose workspace has `room` bytes for partials.
 // A launch that is not cut and leaves CUs idle splits the group of a kv head's query heads into sets, each with row tiles of
-// its own, and takes the smaller workgroup, where that gives at least half as many workgroups again (one each CU at
-// most): a workgroup loads its rows' queries and stores its outputs by itself, and 128 rows of 256 f32 take it 7 us longer
-// than 16. Prompts at position 0, replayed graph, whole groups / sets: 32/8 heads of 128, f16, 16 tokens 7.3 / 6.4 us, 64
+// its own, and takes the smaller workgroup, where that gives more workgroups (at most one each CU): a workgroup loads its
+// rows' queries and stores its outputs by itself, and 128 rows of 256 f32 take it 7 us longer than 16. It has to give a
+// quarter more over a few key tiles (16/2 heads of 256, 200 tokens 15.1 / 13.6 us, 64 workgroups for 50), half as many
+// again over longer spans, where that share counts for less (32/4 heads of 128, 300 tokens at 1500: 96 workgroups for 76
+// take 33.4 us, 76 32.2). Prompts at position 0, replayed graph, whole groups / sets: 32/8 heads of 128, f16, 16 tokens 7.3 / 6.4 us, 64
 // tokens 8.8 / 7.6; 16/2 heads of 256, 16 tokens 14.2 / 8.7, 64 tokens 14.5 / 10.9.
 // The f32 kernels, bound by their MFMAs with two waves a SIMD, always take one head a set: waves of a tile of 128 tokens of
 // one head skip the key tiles past their own last row, where 128 rows of 4 heads all end at the same one (32/8 heads of
@@ -120,9 +122,11 @@ inline PrefillPlan prefill_plan(int pos0, int n, int n_heads, int n_kv, int hd, 
         return (long long)n_heads / group * prefill_row_tiles((long long)n * group, prefill_wave_rows(kind) * waves);
     };
     long long have = wgs(p.waves, p.group);
-    if (kind == kPrefillStaged && wgs(most / 2, G) <= kPrefillCUs && wgs(most / 2, G) * 2 >= have * 3) p.waves = most / 2, have = wgs(p.waves, G);
+    const int gain = p.tiles < 16 ? 25 : 50; // percent more workgroups that a split has to give
+    auto better = [&](long long w) { return w <= kPrefillCUs && w * 100 >= have * (100 + gain); };
+    if (kind == kPrefillStaged && better(wgs(most / 2, G))) p.waves = most / 2, have = wgs(p.waves, G);
     for (int g = G - 1; g >= 1; g--)
-        if (G % g == 0 && wgs(p.waves, g) <= kPrefillCUs && wgs(p.waves, g) * 2 >= have * 3) p.group = g, have = wgs(p.waves, g);
+        if (G % g == 0 && better(wgs(p.waves, g))) p.group = g, have = wgs(p.waves, g);
     return p;
 }
 
