@@ -535,12 +535,6 @@ def attention(qkv, k_cache, v_cache, pos0, n_heads, n_kv, hd=128, exact=False, o
     ws_ptr, ws_bytes = None, 0
     code = (1 if exact else 0) | (2 if no_tc else 0)  # the library's exact bits: verify, no tensor-core kernels
     split = n < TILED_MIN_BATCH or exact or (no_tc and hd > 128)
-    if i8 and not split and not no_tc and workspace is None and posp is None:
-        # a prefill batch over the int8 cache with a scratch of its own (gi_attention_i8 would cut the launch only in
-        # what a workspace holds beyond the widened keys); the scale as the library rounds it
-        _prefill_ws(qkv, k_cache, v_cache, k_scale, v_scale, 1, GI_PREFILL_WIDEN, (n_kv * hd, hd, n_kv, 1), out, pos0, n,
-                    n_heads, n_kv, hd, 1.0 / ctypes.c_float(math.sqrt(hd)).value)
-        return out
     if split:
         if workspace is None:
             cap = ctx_cap if posp is not None else pos0 + n
@@ -550,6 +544,12 @@ def attention(qkv, k_cache, v_cache, pos0, n_heads, n_kv, hd=128, exact=False, o
         # a prefill batch in the caller's workspace: the library takes what it holds (the widened keys of the int8 cache,
         # a cut launch's partials) and does without the rest
         ws_ptr, ws_bytes = _workspace(workspace)
+    elif i8 and not no_tc and posp is None:
+        # a prefill batch over the int8 cache with a scratch of its own (gi_attention_i8 would cut the launch only in
+        # what a workspace holds beyond the widened keys); the scale as the library rounds it
+        _prefill_ws(qkv, k_cache, v_cache, k_scale, v_scale, 1, GI_PREFILL_WIDEN, (n_kv * hd, hd, n_kv, 1), out, pos0, n,
+                    n_heads, n_kv, hd, 1.0 / ctypes.c_float(math.sqrt(hd)).value)
+        return out
     else:
         flags = (GI_PREFILL_WIDEN if i8 else 0) if not no_tc else GI_PREFILL_F32
         scratch, ws_bytes = _prefill_scratch(pos0, n, n_heads, n_kv, hd, 1 if i8 else 0, flags, qkv.device)
