@@ -1802,7 +1802,8 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
         if constexpr (I8) {
             if (wave > 1) return;
             const int t = wave ? tv : tk, t0 = t * BK, rows = t <= last ? min(kv_len - t0, BK) : 0;
-            rsc = gi_load4f(gi_rsrc_tile(scb + (long long)t0 * a.sc_stride, rows * (int)a.sc_stride * 4), lane * (int)a.sc_stride * 4);
+            // (64-bit offsets: 64 keys of scales may span more than a descriptor does)
+            rsc = lane < rows ? scb[(long long)(t0 + lane) * a.sc_stride] : 0.f;
         }
     };
     constexpr int UPC = VPC / 8; // units of 8 values of a chunk

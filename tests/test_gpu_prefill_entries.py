@@ -114,3 +114,29 @@ def test_nan_and_infinities_through_the_merge(gpu, hd):
     assert heads[:, 0, 5].isinf().all() and heads[n - 20:, 2:].isnan().all() and not heads[:n - 20, 2:].isnan().any()
     fin = cut.isfinite()
     assert_close(cut[fin].cpu().numpy(), whole[fin].cpu().numpy(), what="finite outputs")
+
+
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("stride", [1 << 23, 1 << 24])
+def test_i8_scales_far_apart(gpu, hd, stride):
+    # scales of one position 32 and 64 MiB from the next: a tile's 64 span 2 and 4 GiB, more than 32-bit offsets reach
+    n, n_heads, n_kv = 70, 4, 2
+    print("[case] far scales", hd, stride, flush=True)
+    lib, row = gi_attn.load_library(), n_heads * hd
+    q, k, v, ks, vs = make_inputs_i8(9100 + hd, n, n, n_heads, n_kv, hd=hd)
+    qt, kt, vt = dev(q, gpu, n, row), dev(k, gpu, n, n_kv, hd), dev(v, gpu, n, n_kv, hd)
+    near = [dev(x, gpu, n, n_kv) for x in (ks, vs)]
+    far = [torch.empty((n - 1) * stride + n_kv, device=gpu) for _ in range(2)]
+    for f, s in zip(far, near):
+        f.as_strided((n, n_kv), (stride, 1)).copy_(s)
+
+    def run(scales, sc_stride):
+        out = torch.full((n, row), float("nan"), device=gpu)
+        gi_attn._check(lib.gi_attn_prefill_i8(gi_attn._stream(), qt.data_ptr(), gi_attn.GI_F32, row, *ptrs(kt, vt, *scales), n_kv * hd, hd,
+                                              sc_stride, 1, out.data_ptr(), gi_attn.GI_F32, row, 0, n, n_heads, n_kv, hd, hd ** -0.5))
+        torch.cuda.synchronize()
+        return out
+
+    got = run(near, n_kv)
+    assert_close(got.cpu().numpy(), reference_f64_i8(q, k, v, ks, vs, 0, n_heads, n_kv, hd=hd), what="near")
+    assert torch.equal(run(far, stride), got)
