@@ -175,7 +175,6 @@ constexpr int kDecWaves = 4, kDecTile = 32, kDecPairs = 8; // slice partials are
 constexpr int kSliceUnit = kDecWaves * kDecTile; // 128 keys
 constexpr int kSplitMaxBatch = 15;                // tokens per split launch (src/cuda.rs:119)
 constexpr int kTiledMinBatch = 16;                // prefill from this many tokens (src/cuda.rs:95)
-constexpr int kPrefillRows = 256; // packed query rows per workgroup of 8 waves (head sizes 64 and 128)
 constexpr int kPrefillMergeFrags = 4; // must match the kernels' PFC_FRAGS
 
 thread_local std::string g_err;
@@ -689,14 +688,6 @@ size_t prefill_ws_bytes(int kv_len, int n_kv, int hd, int fmt) {
     return 2 * rows + 2 * scales;
 }
 
-// Rows per kv head from which the int8 keys are widened into the workspace first (one pass over all keys, ~6 bytes moved
-// per value) rather than tile by tile in the prefill: above one row tile, every tile would be widened again for each.
-// 32/8 heads of 128, tile by tile / widened: 16 tokens at a 2000-token prefix 17.6 / 21.5 us, at 16000 29.6 / 43.5; 64
-// tokens at 2000 27.7 / 26.7, at 16000 48 / 51; 256 tokens at 2000 84 / 55; 8192 tokens 634 / 588.
-constexpr int kPrefillWidenRows = kPrefillRows;
-bool prefill_widens(int n, int n_heads, int n_kv, int hd) {
-    return hd == 256 || (long long)n * (n_heads / n_kv) > kPrefillWidenRows;
-}
 // gi_attn_prefill, gi_attn_prefill_i8 and gi_attn_prefill_q4: the same launch with the f16, int8 or 4-bit kernel
 // (fmt 0, 1, 2). With a workspace and `widen` (int8 and 4-bit caches, head sizes 64, 128, 256) the keys 0..pos0+n-1
 // are first widened into it (gi_kv_widen) and the prefill stages the widened tiles by LDS-DMA, as it stages the f16

@@ -35,6 +35,15 @@ inline size_t prefill_part_bytes(int nslice, int waves, PrefillKind kind, int n,
     return (b + 255) / 256 * 256;
 }
 
+// Rows per kv head from which the int8 keys are widened into the workspace first (one pass over all keys, ~6 bytes moved
+// per value) rather than tile by tile in the prefill: above one row tile (of 8 waves), every tile would be widened again for each.
+// 32/8 heads of 128, tile by tile / widened: 16 tokens at a 2000-token prefix 17.6 / 21.5 us, at 16000 29.6 / 43.5; 64
+// tokens at 2000 27.7 / 26.7, at 16000 48 / 51; 256 tokens at 2000 84 / 55; 8192 tokens 634 / 588.
+constexpr int kPrefillWidenRows = 256;
+inline bool prefill_widens(int n, int n_heads, int n_kv, int hd) {
+    return hd == 256 || (long long)n * (n_heads / n_kv) > kPrefillWidenRows;
+}
+
 // A launch has one workgroup per (kv head, tile of packed query rows), and a CU holds one workgroup.
 //  - Waves: 8 (256 rows, two waves per SIMD) or 4 (128 rows, one per SIMD). One wave takes a key tile in about 0.7 of
 //    the time that two on its SIMD take for theirs together, so 4 waves win where the workgroups are few or unequal
@@ -45,6 +54,13 @@ inline size_t prefill_part_bytes(int nslice, int waves, PrefillKind kind, int n,
 //    tiles of every row tile into slices, one workgroup each, whose partial results a second launch merges (137 us).
 //    An f32 tile takes three to five times as long, so those launches gain from shorter spans on (200 tokens of 32/32
 //    heads of 96 at 1800: 64 workgroups of 32 tiles, 227 us; sliced 69 us).
+//  - Tiles widened through registers have the larger workgroup only. Where a call with a workspace would stage widened
+//    keys, the slices are those of that call, rated by its forms, so that both give the same bits. Up to kPrefillWidenRows
+//    no call does, and the slices are rated by what such a tile takes: 1.9 us (57 tokens of 32/8 heads of 128 at 16000
+//    int8 keys, 2 slices 242 us), 1.27 of a staged one, and 0.09 us a slice in the merge (rated by the staged forms: 57
+//    tokens at 6100 keys took 14 slices, 32.2 us, now 20, 30.8; 64 of 32/8 heads of 64 at 16000 33.3, now 30.2; 40 of 9/3
+//    at 6100 19.1, now 17.4; at worst 40 of 9/3 at 40000 31.3, now 32.6). Over 40 calls of 16 to 64 tokens, prefixes 1000 to
+//    40000, that is 0.8% in the mean above the best of 1 to 64 slices, 5% at most; it was 2.2 and 13.
 // A row's arithmetic does not depend on the waves or the set, only on the slices. Of a sliced launch the partials fit
 // `room` bytes.
 inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, PrefillKind kind, size_t room) {
@@ -52,6 +68,7 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
     const int G = n_heads / n_kv, cus = kPrefillCUs, tmax = (pos0 + n + kPrefillKeys - 1) / kPrefillKeys;
     const long long P = (long long)n * G;
     const int most = prefill_most_waves(kind, hd), rw = prefill_wave_rows(kind);
+    const bool tile_only = kind == kPrefillTile && !prefill_widens(n, n_heads, n_kv, hd);
     PrefillPlan p{most, G, tmax, 1};
     if ((long long)prefill_row_tiles(P, rw * most) * n_kv >= 2 * cus) return p; // longest tiles first balances these
     // Below 16 key tiles slices save less than the merge launch costs. A prompt of up to 4096 keys taken in chunks of
@@ -65,11 +82,12 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
     // workgroups over the CUs, each with a fixed cost until its first tile is in and for its output (~6 us), and for a
     // sliced launch the merge launch (~5 us) and its read of the partials (~4 TB/s).
     const double tile_s = f32 ? 5e-6 : 1.5e-6, per_wg = f32 ? 1.2 : 4.0, merge = f32 ? 1.0 : 3.3;
+    const double per_slice = tile_only ? 0.06 : 0.0, less = tile_only ? 0.97 : 0.95;
     double best = 0;
-    for (int waves = most; waves >= (f32 ? most : most / 2); waves -= most / 2) {
+    for (int waves = most; waves >= (f32 || tile_only ? most : most / 2); waves -= most / 2) {
         const int rows = rw * waves, items = prefill_row_tiles(P, rows);
         const long long wgs = (long long)items * n_kv;
-        const double tile = waves == most ? 1.0 : hd == 256 ? 0.85 : 0.7;
+        const double tile = tile_only ? 1.27 : waves == most ? 1.0 : hd == 256 ? 0.85 : 0.7;
         auto tiles_of = [&](int i) { // key tiles of row tile i
             const long long last = std::min<long long>(n - 1, ((long long)(i + 1) * rows - 1) / G);
             return (int)((pos0 + last) / kPrefillKeys + 1);
@@ -87,8 +105,8 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
             if (tiles_of(0) + C > tmax) u = wgs * slices; // (every row tile has tmax tiles or nearly)
             else
                 for (int i = 0; i < items; i++) u += (long long)n_kv * ((tiles_of(i) + C - 1) / C);
-            const double cost = (double)((u + cus - 1) / cus) * (tile * C + per_wg) + merge + u * part;
-            if (cost < 0.95 * best) best = cost, p = PrefillPlan{waves, G, C, slices};
+            const double cost = (double)((u + cus - 1) / cus) * (tile * C + per_wg) + merge + per_slice * slices + u * part;
+            if (cost < less * best) best = cost, p = PrefillPlan{waves, G, C, slices};
         }
     }
     return p;

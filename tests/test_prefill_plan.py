@@ -99,6 +99,19 @@ def test_short_prompts_have_no_fewer_workgroups_than_heads_give(host):
         assert plan(host, 0, n, 32, 8, 96, F32, 0)[1] == 1
 
 
+def test_tiles_widened_in_the_prefill_are_planned_as_they_are_launched(host):
+    # up to 256 rows a kv head no call stages widened keys: these plans rate the larger workgroup alone, which is what the
+    # kernels have (with the smaller one rated too, 57 tokens at 6100 keys had 112 workgroups on 256 CUs)
+    for n, pos0, heads, kv, hd in ((57, 6100, 32, 8, 128), (32, 16000, 32, 8, 128), (40, 16000, 9, 3, 64), (64, 6100, 32, 8, 64)):
+        waves, group, _, nslice, wgs = plan(host, pos0, n, heads, kv, hd, TILE, ANY_ROOM)
+        assert waves == 8 and group == heads // kv and nslice * wgs > 128, (n, pos0, nslice, wgs)
+    # above, and at head size 256, the slices are those of the call that stages widened keys: the same bits from both
+    for n, pos0, heads, kv, hd in ((65, 6100, 32, 8, 128), (200, 3000, 32, 8, 128), (400, 16000, 9, 3, 64), (16, 6100, 16, 2, 256),
+                                   (200, 16000, 16, 2, 256)):
+        tile, staged = (plan(host, pos0, n, heads, kv, hd, kind, ANY_ROOM) for kind in (TILE, STAGED))
+        assert tile[0] == (4 if hd == 256 else 8) and tile[1:4] == staged[1:4], (n, pos0, tile, staged)
+
+
 def test_a_plan_fits_its_room(host):
     rng = random.Random(5)
     cut = 0
