@@ -83,7 +83,8 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
     // sliced launch the merge launch (~5 us) and its read of the partials (~4 TB/s).
     const double tile_s = f32 ? 5e-6 : 1.5e-6, per_wg = f32 ? 1.2 : 4.0, merge = f32 ? 1.0 : 3.3;
     const double per_slice = tile_only ? 0.06 : 0.0, less = tile_only ? 0.97 : 0.95;
-    double best = 0;
+    double best = 0, uncut = 0;
+    int uncut_waves = most;
     for (int waves = most; waves >= (f32 || tile_only ? most : most / 2); waves -= most / 2) {
         const int rows = rw * waves, items = prefill_row_tiles(P, rows);
         const long long wgs = (long long)items * n_kv;
@@ -95,6 +96,14 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
         // one slice: the longest workgroup, or the mean load of a CU where there are several rounds
         const double mean = (double)wgs / cus * (tile * (tiles_of(0) + tmax) / 2 + (wgs > cus ? per_wg : 0));
         const double one = std::max(tile * tmax, mean) + per_wg;
+        // and where one round of them is about as long as the next (a long prefix under them all): r + 1 rounds take r + 1
+        // times what the longest workgroup of the last of them does (f16, uncut, 4 / 8 waves: 1500 tokens at 3000, 32/8
+        // heads of 128, 376 workgroups or 192, 123 / 114 us; 4096 at 16000, 9/3 heads of 64, 288 or 144, 352 / 283). It
+        // decides between the two sizes only: whether a launch is cut does not depend on it.
+        double rounds = one;
+        for (int r = 1; (long long)r * cus < wgs; r++)
+            rounds = std::max(rounds, (r + 1) * (tile * tiles_of(items - 1 - r * cus / n_kv) + per_wg));
+        if (waves == most || rounds < 0.95 * uncut) uncut = rounds, uncut_waves = waves;
         if (waves == most || one < 0.95 * best) best = one, p = PrefillPlan{waves, G, tmax, 1};
         if (!may_slice) continue;
         const double part = std::min<long long>(P, rows) * (hd + 2) * 4.0 / 4e12 / tile_s;
@@ -109,6 +118,7 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
             if (cost < less * best) best = cost, p = PrefillPlan{waves, G, C, slices};
         }
     }
+    if (p.nslice == 1) p.waves = uncut_waves;
     return p;
 }
 

@@ -112,6 +112,16 @@ def test_tiles_widened_in_the_prefill_are_planned_as_they_are_launched(host):
         assert tile[0] == (4 if hd == 256 else 8) and tile[1:4] == staged[1:4], (n, pos0, tile, staged)
 
 
+def test_an_uncut_launch_of_equal_workgroups_fills_whole_rounds(host):
+    # workgroups of nearly one length (a long prefix), a few more of the smaller size than CUs: a second round as long as the
+    # first, where the larger size takes one
+    for n, pos0, heads, kv, hd in ((1500, 3000, 32, 8, 128), (4096, 16000, 9, 3, 64), (6000, 8000, 8, 8, 128)):
+        waves, _, _, nslice, wgs = plan(host, pos0, n, heads, kv, hd, STAGED, 0)
+        assert waves == 8 and nslice == 1 and wgs <= 256, (n, pos0, waves, wgs)
+    assert plan(host, 0, 1024, 32, 8, 128, STAGED, 0)[0] == 4  # unequal ones even out
+    assert plan(host, 1000, 512, 32, 8, 128, STAGED, 0)[0] == 4  # one round of either
+
+
 def test_a_plan_fits_its_room(host):
     rng = random.Random(5)
     cut = 0
