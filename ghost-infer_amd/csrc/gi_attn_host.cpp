@@ -153,10 +153,10 @@ struct GiPrefillArgs {
     float* part;
     int slice_tiles;
     int nslice;
-    int pwaves;
+    int rows;
     int items;
     uint32_t gmul;
-    int rows;
+    int pwaves;
     int group;
     int sets;
 };
@@ -755,7 +755,7 @@ int prefill_impl(void* stream, const void* q, int q_dtype, long long q_stride, c
     auto run_plan = [&](PrefillKind kind, unsigned char* free, size_t left, auto kernel) {
         const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd, kind, free && aligned16(free) ? left : 0);
         const int rw = prefill_wave_rows(kind), sets = n_heads / n_kv / p.group;
-        a.rows = rw * p.waves;
+        a.rows = p.rows;
         a.group = p.group;
         a.sets = sets;
         a.gmul = gi_row_mul(n, p.group);

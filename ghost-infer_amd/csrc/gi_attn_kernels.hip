@@ -1492,10 +1492,10 @@ struct GiPrefillArgs {
     float* part;
     int slice_tiles;
     int nslice;
-    int pwaves;            // waves of a row tile that hold rows (the workgroup's, or fewer where one tile holds all rows)
+    int rows;              // rows of a row tile: 32 a wave, or fewer (the first waves', the others only stage)
     int items;             // row tiles per kv head
     uint32_t gmul;         // gi_row_mul: a packed row's token without a division (pf_token)
-    int rows;              // rows of a row tile
+    int pwaves;            // waves of a row tile that hold rows (the workgroup's, or fewer where one tile holds all rows)
     int group;             // query heads of a set, whose rows are packed together: a kv head's group, or a part of it
     int sets;              // sets per kv head
 };
@@ -1657,7 +1657,8 @@ template <int N, int I = 0, typename F> __device__ __forceinline__ void gi_unrol
         gi_unroll<N, I + 1>(f);
     }
 }
-// One workgroup = (set of a kv head's query heads, 32 * WAVES packed query rows, key slice); wave w owns rows 32w..32w+31 of the tile. Per
+// One workgroup = (set of a kv head's query heads, a.rows <= 32 * WAVES packed query rows, key slice); wave w owns rows
+// 32w..32w+31 of the tile. Per
 // 64-key tile:
 //   S^T[key, q] = K[key, :] . Q[q, :]       v_mfma_f32_32x32x16_f16, K from LDS (A), Q in registers (B)
 //   O^T[d, q]  += V^T[d, key] . P^T[key, q]  V^T from LDS (A, by transposing reads), P^T from S^T (B)
@@ -1714,7 +1715,6 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     constexpr int IMG = WIDE ? 2 : 1;       // 16 KB images of a K or V tile (128 dims each)
     constexpr int NKB = WIDE ? 2 : 4, NVB = NKB; // K and V tile buffers
     constexpr float VB = WIDE ? 1024.f : PF_I8_VBIAS; // int8: the probabilities' bias
-    constexpr int BQ = 32 * WAVES;  // query rows per workgroup
     constexpr int SW = WAVES / 2;   // waves staging each of K and V
     constexpr int LPW = 16 * IMG / SW; // 1 KB loads per staging wave and tile
     constexpr int LPT = LPW + (STG ? 1 : 0); // loads per staging wave and tile (STG: plus its share of the scales)
@@ -1734,8 +1734,9 @@ __device__ __forceinline__ void gi_prefill_t(const GiPrefillArgs& a) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G = a.group;
-    const PfUnit un = pf_unit(a, BQ, BK);
-    const int kvh = un.kvh, q0 = un.row0, t_begin = un.t_begin, ntiles = un.t_end; // key tiles t_begin .. ntiles - 1
+    const PfUnit un = pf_unit(a, a.rows, BK);
+    const int kvh = un.kvh, t_begin = un.t_begin, ntiles = un.t_end; // key tiles t_begin .. ntiles - 1
+    const int q0 = 32 * wave < a.rows ? un.row0 : a.n * G;           // (a wave past the tile's rows: as past the last one)
     if (t_begin >= ntiles) return; // a slice past the tile's last key
     const int kv_len = a.pos0 + a.n;
     const long long kvs = a.kv_stride;
@@ -2266,11 +2267,9 @@ GI_PREFILL_KERNEL(gi_prefill_fwd_i8s_w4, 1, 128, true, 4, 6)
 GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s, 1, 64, true, 8, 6)
 GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8s_w4, 1, 64, true, 4, 6)
 // int8 tiles widened through registers (the chunks in flight leave room for a ring of 2; with 4 waves, twice the
-// chunks a thread, 36 registers spill and a tile takes twice as long). With 8 waves 7 registers spill at head size 128:
-// the row's token, head and output addresses, stored once before the loop and loaded once behind it. (Computed again
-// behind the loop instead, nothing spills, and the loop's registers fall so that 57 tokens at 6,100 keys take 34.0 us
-// instead of 32.2.) The 20-byte stack frames of the other int8 and 4-bit forms are reserved for scalar registers and never
-// accessed.
+// chunks a thread, 36 registers spill and a tile takes twice as long). With 8 waves 3 registers spill at head size 128,
+// stored once before the loop and loaded once behind it. (The row's token, head and output addresses computed again behind the
+// loop instead: nothing spills, and the loop's registers fall so that 57 tokens at 6,100 keys take 34.0 us instead of 32.2.)
 GI_PREFILL_KERNEL(gi_prefill_fwd_i8, 1, 128, false, 8, 2)
 GI_PREFILL_KERNEL(gi_prefill_fwd_h64_i8, 1, 64, false, 8, 2)
 

@@ -17,6 +17,7 @@ enum PrefillKind { kPrefillStaged, kPrefillTile, kPrefillF32 };
 struct PrefillPlan {
     int waves;      // per workgroup: 8 or 4; head size 256: 4 or 2; f32: 8
     int group;      // query heads that share row tiles
+    int rows;       // of a row tile: the workgroup's, or where an uncut launch leaves CUs idle half of them or fewer
     int tiles;      // key tiles per slice
     int nslice;     // slices of the longest row tile
 };
@@ -61,7 +62,7 @@ inline bool prefill_widens(int n, int n_heads, int n_kv, int hd) {
 //    tokens at 6100 keys took 14 slices, 32.2 us, now 20, 30.8; 64 of 32/8 heads of 64 at 16000 33.3, now 30.2; 40 of 9/3
 //    at 6100 19.1, now 17.4; at worst 40 of 9/3 at 40000 31.3, now 32.6). Over 40 calls of 16 to 64 tokens, prefixes 1000 to
 //    40000, that is 0.8% in the mean above the best of 1 to 64 slices, 5% at most; it was 2.2 and 13.
-// A row's arithmetic does not depend on the waves or the set, only on the slices. Of a sliced launch the partials fit
+// A row's arithmetic does not depend on the waves, the set or the rows of its tile, only on the slices. Of a sliced launch the partials fit
 // `room` bytes.
 inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, PrefillKind kind, size_t room) {
     const bool f32 = kind == kPrefillF32;
@@ -69,7 +70,7 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
     const long long P = (long long)n * G;
     const int most = prefill_most_waves(kind, hd), rw = prefill_wave_rows(kind);
     const bool tile_only = kind == kPrefillTile && !prefill_widens(n, n_heads, n_kv, hd);
-    PrefillPlan p{most, G, tmax, 1};
+    PrefillPlan p{most, G, rw * most, tmax, 1};
     if ((long long)prefill_row_tiles(P, rw * most) * n_kv >= 2 * cus) return p; // longest tiles first balances these
     // Below 16 key tiles slices save less than the merge launch costs. A prompt of up to 4096 keys taken in chunks of
     // 256 tokens or more keeps each row's arithmetic independent of the chunking (one slice always); beyond, and in
@@ -104,7 +105,7 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
         for (int r = 1; (long long)r * cus < wgs; r++)
             rounds = std::max(rounds, (r + 1) * (tile * tiles_of(items - 1 - r * cus / n_kv) + per_wg));
         if (waves == most || rounds < 0.95 * uncut) uncut = rounds, uncut_waves = waves;
-        if (waves == most || one < 0.95 * best) best = one, p = PrefillPlan{waves, G, tmax, 1};
+        if (waves == most || one < 0.95 * best) best = one, p = PrefillPlan{waves, G, rows, tmax, 1};
         if (!may_slice) continue;
         const double part = std::min<long long>(P, rows) * (hd + 2) * 4.0 / 4e12 / tile_s;
         for (int S = 2; S <= std::min(kPrefillMaxSlices, tmax / 2) && wgs * S <= 4 * cus; S++) {
@@ -115,46 +116,49 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
             else
                 for (int i = 0; i < items; i++) u += (long long)n_kv * ((tiles_of(i) + C - 1) / C);
             const double cost = (double)((u + cus - 1) / cus) * (tile * C + per_wg) + merge + per_slice * slices + u * part;
-            if (cost < less * best) best = cost, p = PrefillPlan{waves, G, C, slices};
+            if (cost < less * best) best = cost, p = PrefillPlan{waves, G, rows, C, slices};
         }
     }
-    if (p.nslice == 1) p.waves = uncut_waves;
+    if (p.nslice == 1) p.waves = uncut_waves, p.rows = rw * p.waves;
     return p;
 }
 
 // The plan of a call whose workspace has `room` bytes for partials.
-// A launch that is not cut and leaves CUs idle splits the group of a kv head's query heads into sets, each with row tiles of
-// its own, and takes the smaller workgroup, where that gives more workgroups (at most one each CU): a workgroup loads its
-// rows' queries and stores its outputs by itself, and 128 rows of 256 f32 take it 7 us longer than 16. It has to give a
+// A launch that is not cut and leaves CUs idle takes the smaller workgroup, splits the group of a kv head's query heads into
+// sets with row tiles of their own, and gives a workgroup fewer rows than its waves hold (half, a quarter, 32; the waves
+// without rows stage tiles), each where that gives more workgroups, at most one each CU: a workgroup loads its rows'
+// queries and stores its outputs by itself, and 128 rows of 256 f32 take it 7 us longer than 16. A step has to give a
 // quarter more over a few key tiles (16/2 heads of 256, 200 tokens 15.1 / 13.6 us, 64 workgroups for 50), half as many
 // again over longer spans, where that share counts for less (32/4 heads of 128, 300 tokens at 1500: 96 workgroups for 76
-// take 33.4 us, 76 32.2). Prompts at position 0, replayed graph, whole groups / sets: 32/8 heads of 128, f16, 16 tokens 7.3 / 6.4 us, 64
-// tokens 8.8 / 7.6; 16/2 heads of 256, 16 tokens 14.2 / 8.7, 64 tokens 14.5 / 10.9.
+// take 33.4 us, 76 32.2). Replayed graph, whole groups / sets / sets and fewer rows: 32/8 heads of 128, f16, position 0, 64
+// tokens 8.8 / 7.1 / 6.3 us, 250 tokens - / 11.1 / 8.8; int8 without a workspace, 250 tokens - / 18.9 / 12.0, 512 at
+// 3000 - / 112 / 81; 16/2 heads of 256, f16, 16 tokens 14.2 / 8.4 / 8.4, 64 tokens 14.5 / 10.4 / 8.9.
 // The f32 kernels, bound by their MFMAs with two waves a SIMD, always take one head a set: waves of a tile of 128 tokens of
 // one head skip the key tiles past their own last row, where 128 rows of 4 heads all end at the same one (32/8 heads of
 // 96, whole groups / sets: 32 tokens 19.3 / 10.0 us, 256 tokens 40.2 / 36.3, 4096 tokens 867 / 864).
 inline PrefillPlan prefill_plan(int pos0, int n, int n_heads, int n_kv, int hd, PrefillKind kind, size_t room) {
     PrefillPlan p = prefill_rate(pos0, n, n_heads, n_kv, hd, kind, room ? SIZE_MAX : 0);
     const int most = prefill_most_waves(kind, hd), G = n_heads / n_kv;
-    if (kind == kPrefillTile) p.waves = most;
+    if (kind == kPrefillTile) p.waves = most, p.rows = prefill_wave_rows(kind) * most;
     if (prefill_part_bytes(p.nslice, p.waves, kind, n, n_heads, n_kv, hd) > room) {
         p = prefill_rate(pos0, n, n_heads, n_kv, hd, kind, room);
-        if (kind == kPrefillTile) p.waves = most;
+        if (kind == kPrefillTile) p.waves = most, p.rows = prefill_wave_rows(kind) * most;
     }
     if (p.nslice > 1) return p;
     if (kind == kPrefillF32) {
         p.group = 1;
         return p;
     }
-    auto wgs = [&](int waves, int group) {
-        return (long long)n_heads / group * prefill_row_tiles((long long)n * group, prefill_wave_rows(kind) * waves);
-    };
-    long long have = wgs(p.waves, p.group);
+    auto wgs = [&](int rows, int group) { return (long long)n_heads / group * prefill_row_tiles((long long)n * group, rows); };
+    long long have = wgs(p.rows, p.group);
     const int gain = p.tiles < 16 ? 25 : 50; // percent more workgroups that a split has to give
     auto better = [&](long long w) { return w <= kPrefillCUs && w * 100 >= have * (100 + gain); };
-    if (kind == kPrefillStaged && better(wgs(most / 2, G))) p.waves = most / 2, have = wgs(p.waves, G);
+    const int half = prefill_wave_rows(kind) * most / 2;
+    if (kind == kPrefillStaged && p.waves == most && better(wgs(half, G))) p.waves = most / 2, p.rows = half, have = wgs(half, G);
     for (int g = G - 1; g >= 1; g--)
-        if (G % g == 0 && better(wgs(p.waves, g))) p.group = g, have = wgs(p.waves, g);
+        if (G % g == 0 && better(wgs(p.rows, g))) p.group = g, have = wgs(p.rows, g);
+    for (int rows = p.rows / 2; rows >= prefill_wave_rows(kind); rows /= 2)
+        if (better(wgs(rows, p.group))) p.rows = rows, have = wgs(rows, p.group);
     return p;
 }
 

@@ -17,7 +17,7 @@ uint32_t row_mul(long long n, int group) { return gi_row_mul(n, group); }
 int row_token(int row, uint32_t mul, int group) { return gi_row_token(row, mul, group); }
 void plan(int pos0, int n, int n_heads, int n_kv, int hd, int kind, size_t room, int* out) {
     const PrefillPlan p = prefill_plan(pos0, n, n_heads, n_kv, hd, (PrefillKind)kind, room);
-    out[0] = p.waves, out[1] = p.group, out[2] = p.tiles, out[3] = p.nslice;
+    out[0] = p.waves, out[1] = p.group, out[2] = p.tiles, out[3] = p.nslice, out[4] = p.rows;
 }
 size_t part_bytes(int nslice, int waves, int kind, int n, int n_heads, int n_kv, int hd) {
     return prefill_part_bytes(nslice, waves, (PrefillKind)kind, n, n_heads, n_kv, hd);
@@ -45,10 +45,11 @@ def host(tmp_path_factory):
 
 def plan(host, pos0, n, heads, kv, hd, kind, room):
     """(waves, group, key tiles a slice, slices, workgroups of a slice)"""
-    out = (ctypes.c_int * 4)()
+    out = (ctypes.c_int * 5)()
     host.plan(pos0, n, heads, kv, hd, kind, room, out)
-    waves, group, tiles, nslice = out
-    rows = (16 if kind == F32 else 32) * waves
+    waves, group, tiles, nslice, rows = out
+    most = (16 if kind == F32 else 32) * waves
+    assert rows == most if nslice > 1 or kind == F32 else rows in (most, most // 2, most // 4, most // 8) and rows >= 32
     return waves, group, tiles, nslice, heads // group * -(-n * group // rows)
 
 
@@ -97,6 +98,9 @@ def test_short_prompts_have_no_fewer_workgroups_than_heads_give(host):
                 assert nslice == 1 and heads // kv % group == 0
                 assert heads <= wgs * 1.5 and wgs <= 256, (n, heads, kv, hd, kind, wgs)
         assert plan(host, 0, n, 32, 8, 96, F32, 0)[1] == 1
+    # tiles of 32 rows where those of a workgroup's waves are few (64 rows at head size 256: 16 of them)
+    assert plan(host, 0, 64, 16, 2, 256, STAGED, 0)[4] == 32 and plan(host, 0, 64, 32, 8, 128, STAGED, 0)[4] == 64
+    assert plan(host, 0, 250, 32, 8, 128, TILE, 0)[4] == 256
 
 
 def test_tiles_widened_in_the_prefill_are_planned_as_they_are_launched(host):
