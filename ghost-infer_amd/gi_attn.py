@@ -338,7 +338,8 @@ def decode_q4(q, k_cache, v_cache, k_scale, v_scale, pos0, n_heads, n_kv, scale=
 
 def prefill_workspace(kv_len, n_kv, hd, fmt, device):
     """A workspace for the pre-widened prefill over kv_len keys (fmt 1 int8, 2 the 4-bit cache), or None where that
-    path does not apply (gi_attn_prefill_workspace_bytes is 0)."""
+    path does not apply (gi_attn_prefill_workspace_bytes is 0). Calls in it are not cut along their keys: what a call can use
+    for that is in gi_attn_prefill_scratch_bytes."""
     nbytes = load_library().gi_attn_prefill_workspace_bytes(kv_len, n_kv, hd, fmt)
     return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
 

@@ -137,6 +137,7 @@ def test_a_plan_fits_its_room(host):
         n, pos0 = int(2 ** rng.uniform(4, 12)), int(2 ** rng.uniform(0, 17)) - 1
         whole = plan(host, pos0, n, heads, kv, hd, kind, ANY_ROOM)
         need = host.part_bytes(whole[3], whole[0], kind, n, heads, kv, hd)
+        assert need <= 1024 * (128 if hd == 256 or kind == F32 else 256) * (hd + 2) * 4  # a session's room for any call
         assert whole[3] <= 64 and whole[2] * whole[3] * 64 >= pos0 + n
         assert plan(host, pos0, n, heads, kv, hd, kind, need) == whole or whole[3] == 1
         assert plan(host, pos0, n, heads, kv, hd, kind, 0)[3] == 1
