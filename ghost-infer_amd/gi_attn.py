@@ -362,7 +362,7 @@ def _workspace(t):
 
 
 def _prefill_ws(q, k_cache, v_cache, k_scale, v_scale, fmt, flags, strides, out, pos0, n, n_heads, n_kv, hd, scale,
-                workspace=None):
+                workspace=None, out_stride=None):
     """gi_attn_prefill_ws in the workspace given, else with a scratch of its own."""
     if workspace is not None:
         scratch, nbytes = _workspace(workspace)
@@ -372,7 +372,7 @@ def _prefill_ws(q, k_cache, v_cache, k_scale, v_scale, fmt, flags, strides, out,
     _check(load_library().gi_attn_prefill_ws(
         _stream(), _ptr(q), GI_F16 if q.dtype == torch.float16 else GI_F32, q.stride(0), _ptr(k_cache), _ptr(v_cache),
         _ptr(k_scale), _ptr(v_scale), fmt, flags, *strides, _ptr(out), GI_F16 if out.dtype == torch.float16 else GI_F32,
-        out.stride(0), pos0, n, n_heads, n_kv, hd, scale, scratch, nbytes))
+        out.stride(0) if out_stride is None else out_stride, pos0, n, n_heads, n_kv, hd, scale, scratch, nbytes))
 
 
 def prefill_q4(q, k_cache, v_cache, k_scale, v_scale, pos0, n_heads, n_kv, scale=None, out=None, out_dtype=None,
@@ -547,9 +547,10 @@ def attention(qkv, k_cache, v_cache, pos0, n_heads, n_kv, hd=128, exact=False, o
         ws_ptr, ws_bytes = _workspace(workspace)
     elif i8 and not no_tc and posp is None:
         # a prefill batch over the int8 cache with a scratch of its own (gi_attention_i8 would cut the launch only in
-        # what a workspace holds beyond the widened keys); the scale as the library rounds it
+        # what a workspace holds beyond the widened keys); the scale as the library rounds it, the output's rows side by side
+        # whatever its shape, as the library's operators write them
         _prefill_ws(qkv, k_cache, v_cache, k_scale, v_scale, 1, GI_PREFILL_WIDEN, (n_kv * hd, hd, n_kv, 1), out, pos0, n,
-                    n_heads, n_kv, hd, 1.0 / ctypes.c_float(math.sqrt(hd)).value)
+                    n_heads, n_kv, hd, 1.0 / ctypes.c_float(math.sqrt(hd)).value, out_stride=n_heads * hd)
         return out
     else:
         flags = (GI_PREFILL_WIDEN if i8 else 0) if not no_tc else GI_PREFILL_F32

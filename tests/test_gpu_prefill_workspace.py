@@ -108,3 +108,21 @@ def test_f16_and_f32_calls_take_the_workspace_they_are_given(gpu, n, pos0, n_hea
             assert torch.equal(out, uncut)
         with pytest.raises(gi_attn.GiAttnError, match="workspace must be a CUDA tensor"):
             call(torch.empty(part, dtype=torch.uint8))
+
+
+@pytest.mark.parametrize("i8", [False, True])
+def test_operator_writes_rows_side_by_side_into_any_out(gpu, i8):
+    # attention() takes an out of any shape with n * n_heads * hd values: flat, or with the heads apart
+    n, pos0, n_heads, n_kv, hd = 20, 40, 8, 2, 128
+    print("[case] operator out", i8, flush=True)
+    _, k, v, ks, vs = make_inputs_i8(9990, 1, pos0 + n, n_heads, n_kv, hd=hd)
+    kt, vt, kst, vst = dev(k, gpu, -1, n_kv, hd), dev(v, gpu, -1, n_kv, hd), dev(ks, gpu, -1, n_kv), dev(vs, gpu, -1, n_kv)
+    if not i8:
+        kt, vt, kst, vst = kt.half(), vt.half(), None, None
+    gen = torch.Generator(device=gpu).manual_seed(9991)
+    qkv = torch.randn((n, (n_heads + 2 * n_kv) * hd), device=gpu, generator=gen)
+    want = gi_attn.attention(qkv, kt, vt, pos0, n_heads, n_kv, hd=hd, k_scale=kst, v_scale=vst)
+    for shape in ((n * n_heads * hd,), (n, n_heads, hd), (1, n * n_heads * hd)):
+        out = torch.empty(shape, device=gpu)
+        got = gi_attn.attention(qkv, kt, vt, pos0, n_heads, n_kv, hd=hd, k_scale=kst, v_scale=vst, out=out)
+        assert got is out and torch.equal(out.view(n, -1), want), shape
