@@ -355,9 +355,12 @@ def _prefill_scratch(pos0, n, n_heads, n_kv, hd, fmt, flags, device):
 
 
 def _workspace(t):
-    """(pointer, bytes) of a workspace that the caller gives, of any type."""
+    """(pointer, bytes) of a workspace that the caller gives, of any type. One whose elements do not lie side by side (an
+    expanded one has fewer bytes than elements) has no room: the call does without."""
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise GiAttnError("workspace must be a CUDA tensor")
+    if not t.is_contiguous():
+        return None, 0
     return t.data_ptr(), t.numel() * t.element_size()
 
 

@@ -126,3 +126,16 @@ def test_operator_writes_rows_side_by_side_into_any_out(gpu, i8):
         out = torch.empty(shape, device=gpu)
         got = gi_attn.attention(qkv, kt, vt, pos0, n_heads, n_kv, hd=hd, k_scale=kst, v_scale=vst, out=out)
         assert got is out and torch.equal(out.view(n, -1), want), shape
+
+
+def test_an_expanded_workspace_is_not_used(gpu):
+    # one element, 2^28 by its shape: uncut, as with an empty one
+    n, pos0, n_heads, n_kv, hd = 57, 3000, 16, 4, 128
+    print("[case] expanded workspace", flush=True)
+    gen = torch.Generator(device=gpu).manual_seed(9995)
+    q = torch.randn((n, n_heads * hd), device=gpu, generator=gen)
+    kt, vt = (torch.randn((pos0 + n, n_kv, hd), device=gpu, generator=gen).half() for _ in range(2))
+    want = gi_attn.prefill(q, kt, vt, pos0, n_heads, n_kv, hd=hd, workspace=torch.empty(0, dtype=torch.uint8, device=gpu))
+    ws = torch.empty(1, dtype=torch.uint8, device=gpu).expand(1 << 28)
+    call = lambda: gi_attn.prefill(q, kt, vt, pos0, n_heads, n_kv, hd=hd, workspace=ws)
+    assert merges(call) == 0 and torch.equal(call(), want)
