@@ -26,6 +26,7 @@ GI_PREFILL_WIDEN = 1
 GI_PREFILL_F32 = 2
 SPLIT_MAX_BATCH = 15  # src/cuda.rs:119
 TILED_MIN_BATCH = 16  # src/cuda.rs:95
+PREFILL_WIDEN_ROWS = 256  # rows per kv head up to which the library widens no int8 keys into a workspace (head sizes 64, 128)
 
 # Exported symbols of include/gi_attn.h
 SYMBOLS = (
@@ -365,7 +366,7 @@ def _workspace(t):
 
 
 def _prefill_ws(q, k_cache, v_cache, k_scale, v_scale, fmt, flags, strides, out, pos0, n, n_heads, n_kv, hd, scale,
-                workspace=None, out_stride=None):
+                workspace=None):
     """gi_attn_prefill_ws in the workspace given, else with a scratch of its own."""
     if workspace is not None:
         scratch, nbytes = _workspace(workspace)
@@ -375,7 +376,7 @@ def _prefill_ws(q, k_cache, v_cache, k_scale, v_scale, fmt, flags, strides, out,
     _check(load_library().gi_attn_prefill_ws(
         _stream(), _ptr(q), GI_F16 if q.dtype == torch.float16 else GI_F32, q.stride(0), _ptr(k_cache), _ptr(v_cache),
         _ptr(k_scale), _ptr(v_scale), fmt, flags, *strides, _ptr(out), GI_F16 if out.dtype == torch.float16 else GI_F32,
-        out.stride(0) if out_stride is None else out_stride, pos0, n, n_heads, n_kv, hd, scale, scratch, nbytes))
+        out.stride(0), pos0, n, n_heads, n_kv, hd, scale, scratch, nbytes))
 
 
 def prefill_q4(q, k_cache, v_cache, k_scale, v_scale, pos0, n_heads, n_kv, scale=None, out=None, out_dtype=None,
@@ -548,16 +549,19 @@ def attention(qkv, k_cache, v_cache, pos0, n_heads, n_kv, hd=128, exact=False, o
         # a prefill batch in the caller's workspace: the library takes what it holds (the widened keys of the int8 cache,
         # a cut launch's partials) and does without the rest
         ws_ptr, ws_bytes = _workspace(workspace)
-    elif i8 and not no_tc and posp is None:
-        # a prefill batch over the int8 cache with a scratch of its own (gi_attention_i8 would cut the launch only in
-        # what a workspace holds beyond the widened keys); the scale as the library rounds it, the output's rows side by side
-        # whatever its shape, as the library's operators write them
-        _prefill_ws(qkv, k_cache, v_cache, k_scale, v_scale, 1, GI_PREFILL_WIDEN, (n_kv * hd, hd, n_kv, 1), out, pos0, n,
-                    n_heads, n_kv, hd, 1.0 / ctypes.c_float(math.sqrt(hd)).value, out_stride=n_heads * hd)
-        return out
     else:
         flags = (GI_PREFILL_WIDEN if i8 else 0) if not no_tc else GI_PREFILL_F32
         scratch, ws_bytes = _prefill_scratch(pos0, n, n_heads, n_kv, hd, 1 if i8 else 0, flags, qkv.device)
+        if (i8 and not no_tc and posp is None and scratch is not None and hd in (64, 128)
+                and n * (n_heads // n_kv) <= PREFILL_WIDEN_ROWS):
+            # partials alone, no widened keys: gi_attention_i8 cuts a launch only in what a workspace holds beyond those. The
+            # same call as its own, its scale among them (1 / sqrt(hd) in f32) and rows side by side whatever out's shape.
+            # (Called directly: through _prefill_ws, and for every prompt, it cost short ones 1 us of host time.)
+            _check(load_library().gi_attn_prefill_ws(
+                _stream(), qkv.data_ptr(), GI_F32, row, k_cache.data_ptr(), v_cache.data_ptr(), k_scale.data_ptr(),
+                v_scale.data_ptr(), 1, GI_PREFILL_WIDEN, n_kv * hd, hd, n_kv, 1, out.data_ptr(), GI_F32, n_heads * hd, pos0, n,
+                n_heads, n_kv, hd, 0.125 if hd == 64 else 1.0 / ctypes.c_float(math.sqrt(128)).value, scratch.data_ptr(), ws_bytes))
+            return out
         ws_ptr = _ptr(scratch)
     lib = load_library()
     if i8:
