@@ -98,13 +98,16 @@ inline PrefillPlan prefill_rate(int pos0, int n, int n_heads, int n_kv, int hd, 
         const double mean = (double)wgs / cus * (tile * (tiles_of(0) + tmax) / 2 + (wgs > cus ? per_wg : 0));
         const double one = std::max(tile * tmax, mean) + per_wg;
         // and where one round of them is about as long as the next (a long prefix under them all): r + 1 rounds take r + 1
-        // times what the longest workgroup of the last of them does (f16, uncut, 4 / 8 waves: 1500 tokens at 3000, 32/8
-        // heads of 128, 376 workgroups or 192, 123 / 114 us; 4096 at 16000, 9/3 heads of 64, 288 or 144, 352 / 283). It
-        // decides between the two sizes only: whether a launch is cut does not depend on it.
+        // times what the longest workgroup of the last of them does. (f16, uncut, 4 / 8 waves: 1500 tokens at 3000, 32/8
+        // heads of 128, 376 workgroups or 192, 123 / 114 us; 4096 at 16000, 9/3 heads of 64, 288 or 144, 352 / 283; at
+        // position 0 2000 tokens of 32/8 heads of 128 44 / 53. Of 250 calls, 1050 to 4096 tokens at 0 to 12000, five head
+        // shapes, f16 and int8, the size taken costs 0.2% over the better one in the mean, 5.5% at most; with the mean load
+        // alone it was 5.8 and 75.) It decides between the two sizes only: whether a launch is cut does not depend on it.
+        const double later = hd == 64 && waves != most ? 0.75 : tile;
         double rounds = one;
         for (int r = 1; (long long)r * cus < wgs; r++)
-            rounds = std::max(rounds, (r + 1) * (tile * tiles_of(items - 1 - r * cus / n_kv) + per_wg));
-        if (waves == most || rounds < 0.95 * uncut) uncut = rounds, uncut_waves = waves;
+            rounds = std::max(rounds, (r + 1) * (later * tiles_of(items - 1 - r * cus / n_kv) + per_wg));
+        if (waves == most || rounds < 1.05 * uncut) uncut = rounds, uncut_waves = waves; // (rounds overlap a little)
         if (waves == most || one < 0.95 * best) best = one, p = PrefillPlan{waves, G, rows, tmax, 1};
         if (!may_slice) continue;
         const double part = std::min<long long>(P, rows) * (hd + 2) * 4.0 / 4e12 / tile_s;

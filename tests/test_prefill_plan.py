@@ -119,10 +119,12 @@ def test_tiles_widened_in_the_prefill_are_planned_as_they_are_launched(host):
 def test_an_uncut_launch_of_equal_workgroups_fills_whole_rounds(host):
     # workgroups of nearly one length (a long prefix), a few more of the smaller size than CUs: a second round as long as the
     # first, where the larger size takes one
-    for n, pos0, heads, kv, hd in ((1500, 3000, 32, 8, 128), (4096, 16000, 9, 3, 64), (6000, 8000, 8, 8, 128)):
+    # (6000 tokens of 8/8 heads at 8000 are a tie, 317 and 313 us; at 16000 the sizes take 551 and 497)
+    for n, pos0, heads, kv, hd in ((1500, 3000, 32, 8, 128), (4096, 16000, 9, 3, 64), (6000, 16000, 8, 8, 128)):
         waves, _, _, nslice, wgs = plan(host, pos0, n, heads, kv, hd, STAGED, 0)
         assert waves == 8 and nslice == 1 and wgs <= 256, (n, pos0, waves, wgs)
     assert plan(host, 0, 1024, 32, 8, 128, STAGED, 0)[0] == 4  # unequal ones even out
+    assert plan(host, 0, 2000, 32, 8, 128, STAGED, 0)[0] == 4  # (44 us, 53 with 8 waves)
     assert plan(host, 1000, 512, 32, 8, 128, STAGED, 0)[0] == 4  # one round of either
 
 
